@@ -261,7 +261,7 @@ def main():
         "speedup_vs_plain_fp64": round(plain["ms"] / ms_step, 3) if plain else None,
         "autotune": {"vxc_shape": chosen["tuned"][0], "vxc_chunk": chosen["tuned"][1],
                      "shapes": {"0": "128 x 128 blocks over 128-AO super-tile pairs",
-                                "1": "256 x 256 blocks over 8-tile groups of each chunk's alive-tile union"},
+                                "1": "256 x 256 blocks over 8-tile groups of each chunk's AO list"},
                      "ms": {"%d/%d" % k: round(v, 4) for k, v in chosen["tuned"][2].items()}}
         if chosen["tuned"] else None,
         "tflops": round(flops_build / (ms_step * 1e-3) / 1e12, 3),

@@ -356,7 +356,7 @@ class Grid:
         return c.value, dict(zip((8, 16, 32, 128), list(ms)))
 
     def autotuneTiles(self, xc, D_ptr, V_ptr, reps=3):
-        """Mixed form: times both Vxc block shapes (0: 128-AO super-tiles, 1: 256-AO union groups) at
+        """Mixed form: times both Vxc block shapes (0: 128-AO super-tiles, 1: 256-AO groups) at
         each work-item length, keeps the fastest; returns (shape, chunk, {(shape, chunk): ms})."""
         sh, c = ctypes.c_int(), ctypes.c_int()
         ms = (ctypes.c_float * 8)()
@@ -717,7 +717,7 @@ class Pack:
         return c.value, dict(zip((8, 16, 32, 128), list(ms)))
 
     def vxcWideFrom(self):
-        """The autotuned Vxc shape threshold: 256-AO union groups for npad >= it (-1: none)."""
+        """The autotuned Vxc shape threshold: 256-AO groups for npad >= it (-1: none)."""
         v = ctypes.c_int()
         _check(lib().chx_pack_vxc_wide_from(self.h, ctypes.byref(v)))
         return v.value

@@ -134,6 +134,12 @@ void run_functional(chx_grid* g, const chx_xc* xc, bool want_e, bool want_v) {
   g->mark_end(2, e);
 }
 
+// The chunks' dense blocks of a device matrix D (FP64 form).
+void gather_d(chx_grid* g, const double* dD, DevBuf<double>& Dt) {
+  launch_gather_d(g->stream, (int)g->tile_chunk.size(), g->nbasis, dD, g->d_tile_chunk.p, g->d_chunks.p, g->d_ao_of.p,
+                  Dt.alloc_get(std::max<size_t>(1, g->dt_elems)));
+}
+
 // Stage ids of chx_grid_kernel_times.
 enum { kStPermute = 0, kStDensity = 1, kStFunctional = 2, kStVxc = 3, kStFinalize = 4, kStMakeB = 5, kStCore = 6 };
 
@@ -145,8 +151,8 @@ void density_from_device(chx_grid* g, const double* dD, int spin = 0) {
   if (g->precision == CHX_PREC_MIXED) {
     g->mark_begin(kStPermute, &e);
     const int ncg = (int)g->core_grps.size();
-    launch_split_d(g->stream, g->nbasis, g->npad, dD, g->d_int2ref.p, g->d_Dsplit.p,
-                   g->d_Dres.p + (size_t)spin * g->nbasis * g->nbasis);
+    launch_split_d(g->stream, (int)g->tile_chunk.size(), g->nbasis, dD, g->d_tile_chunk.p, g->d_chunks.p, g->d_ao_of.p,
+                   g->d_Dsplit.p, g->d_Dres.p + (size_t)spin * g->nbasis * g->nbasis);
     g->mark_end(kStPermute, e);
     g->mark_begin(kStDensity, &e);
     // meta-GGA: rho, grad rho and the tau partials (A = d_r phi) in one launch that stages D once
@@ -166,25 +172,23 @@ void density_from_device(chx_grid* g, const double* dD, int spin = 0) {
     return;
   }
   g->mark_begin(kStPermute, &e);
-  launch_permute_d(g->stream, g->nbasis, g->npad, dD, g->d_int2ref.p, g->d_Dint.p);
+  gather_d(g, dD, g->d_Dt);
   g->mark_end(kStPermute, e);
   g->mark_begin(kStDensity, &e);
   if (g->cached) {
-    launch_density_c64(g->stream, 0, ng, g->d_grp_batch.p, g->d_grp_tiles.p, g->d_grp_slots.p, g->d_grp_ntiles.p,
-                       g->d_bt_off.p, g->d_bt_list.p, g->d_cache.p, g->d_Dint.p, g->npad, g->d_part.p);
+    launch_density_c64(g->stream, 0, ng, g->d_grp_batch.p, g->d_grp_tile.p, g->d_grp_ntiles.p,
+                           g->d_bt_off.p, g->d_b_chunk.p, g->d_chunks.p, g->d_cache.p, g->d_Dt.p, g->d_part.p);
     if (g->type >= 2)  // tau: three more contractions with A = d_r phi
       for (int r = 1; r <= 3; ++r)
-        launch_density_c64(g->stream, r, ng, g->d_grp_batch.p, g->d_grp_tiles.p, g->d_grp_slots.p, g->d_grp_ntiles.p,
-                           g->d_bt_off.p, g->d_bt_list.p, g->d_cache.p, g->d_Dint.p, g->npad,
-                           g->d_part_tau.p + (size_t)(r - 1) * kBatch);
+        launch_density_c64(g->stream, r, ng, g->d_grp_batch.p, g->d_grp_tile.p, g->d_grp_ntiles.p,
+                           g->d_bt_off.p, g->d_b_chunk.p, g->d_chunks.p, g->d_cache.p, g->d_Dt.p, g->d_part_tau.p + (size_t)(r - 1) * kBatch);
   } else {  // AO values recomputed in the kernels
-    launch_density_f64(g->stream, 0, ng, g->d_grp_batch.p, g->d_grp_tiles.p, g->d_grp_ntiles.p, g->d_bt_off.p,
-                       g->d_bt_list.p, g->d_x.p, g->d_y.p, g->d_z.p, g->view(), g->d_Dint.p, g->npad, g->d_part.p);
+    launch_density_f64(g->stream, 0, ng, g->d_grp_batch.p, g->d_grp_tile.p, g->d_grp_ntiles.p, g->d_b_chunk.p,
+                         g->d_chunks.p, g->d_x.p, g->d_y.p, g->d_z.p, g->view(), g->d_Dt.p, g->d_part.p);
     if (g->type >= 2)
       for (int r = 1; r <= 3; ++r)
-        launch_density_f64(g->stream, r, ng, g->d_grp_batch.p, g->d_grp_tiles.p, g->d_grp_ntiles.p, g->d_bt_off.p,
-                           g->d_bt_list.p, g->d_x.p, g->d_y.p, g->d_z.p, g->view(), g->d_Dint.p, g->npad,
-                           g->d_part_tau.p + (size_t)(r - 1) * kBatch);
+        launch_density_f64(g->stream, r, ng, g->d_grp_batch.p, g->d_grp_tile.p, g->d_grp_ntiles.p, g->d_b_chunk.p,
+                         g->d_chunks.p, g->d_x.p, g->d_y.p, g->d_z.p, g->view(), g->d_Dt.p, g->d_part_tau.p + (size_t)(r - 1) * kBatch);
   }
   g->mark_end(kStDensity, e);
   g->have_density = true;
@@ -202,7 +206,6 @@ void fock_to_device(chx_grid* g, double* dV, int spin = 0) {
     g->mark_begin(kStMakeB, &e);
     launch_make_b_mx(g->stream, nc, g->hmol);
     g->mark_end(kStMakeB, e);
-    launch_fill(g->stream, g->d_Mint.p, (size_t)g->npad * g->npad, 0.0);
     g->mark_begin(kStVxc, &e);
     if (g->mx_wide)
       launch_vxc_mx_wide(g->stream, nc, (int)g->cwork.size(), g->hmol);
@@ -211,36 +214,35 @@ void fock_to_device(chx_grid* g, double* dV, int spin = 0) {
     g->mark_end(kStVxc, e);
     g->mark_begin(kStFinalize, &e);
     if (g->corr_pending)
-      launch_finalize_corr(g->stream, g->nbasis, g->npad, g->d_Mint.p, g->d_ref2int.p, dV,
+      launch_finalize_corr(g->stream, g->nbasis, g->npad, g->d_Mint.p, dV,
                            g->d_Dres.p + (size_t)spin * g->nbasis * g->nbasis,
                            g->d_cpart.p + (size_t)spin * corr_blocks(g->nbasis));
     else
-      launch_finalize_sym(g->stream, g->nbasis, g->npad, g->d_Mint.p, g->d_ref2int.p, dV);
+      launch_finalize_sym(g->stream, g->nbasis, g->npad, g->d_Mint.p, dV);
     g->mark_end(kStFinalize, e);
     return;
   }
   if (g->cached) {
     const int nc = g->v_family >= 2 ? 4 : 1;
     g->mark_begin(kStMakeB, &e);
-    launch_make_b(g->stream, g->nbatches, g->d_bt_off.p, g->d_coef.p, g->d_cache.p, g->d_bmat.p);
+    launch_make_b(g->stream, g->nbatches, g->d_bt_off.p, g->d_coef.p, g->d_cache.p, g->d_bmat.p, g->d_Mint.p,
+                  (size_t)g->npad * g->npad);
     g->mark_end(kStMakeB, e);
-    launch_fill(g->stream, g->d_Mint.p, (size_t)g->npad * g->npad, 0.0);
     g->mark_begin(kStVxc, &e);
-    launch_vxc_c64(g->stream, nc, (int)g->cwork.size(), g->d_cwork.p, g->d_cpair_batches.p, g->d_slot_of.p, g->ntiles,
-                   g->d_cache.p, g->d_bmat.p, g->d_coef.p, g->d_Mint.p, g->npad);
+    launch_vxc_c64(g->stream, nc, (int)g->cwork.size(), g->d_cwork.p, g->d_ao_of.p, g->d_cache.p, g->d_bmat.p, g->d_coef.p, g->d_Mint.p, g->npad);
     g->mark_end(kStVxc, e);
     g->mark_begin(kStFinalize, &e);
-    launch_finalize_sym(g->stream, g->nbasis, g->npad, g->d_Mint.p, g->d_ref2int.p, dV);
+    launch_finalize_sym(g->stream, g->nbasis, g->npad, g->d_Mint.p, dV);
     g->mark_end(kStFinalize, e);
     return;
   }
-  launch_fill(g->stream, g->d_Vint.p, (size_t)g->npad * g->npad, 0.0);
+  launch_fill(g->stream, g->d_Mint.p, (size_t)g->npad * g->npad, 0.0);
   g->mark_begin(kStVxc, &e);
-  launch_vxc_f64(g->stream, g->v_family >= 2 ? 4 : 1, (int)g->vwork.size(), g->d_vwork.p, g->d_pair_batches.p,
-                 g->d_alive.p, g->ntiles, g->d_x.p, g->d_y.p, g->d_z.p, g->d_coef.p, g->view(), g->d_Vint.p, g->npad);
+  launch_vxc_f64(g->stream, g->v_family >= 2 ? 4 : 1, (int)g->vwork.size(), g->d_vwork.p, g->d_ao_of.p, g->d_x.p,
+                 g->d_y.p, g->d_z.p, g->d_coef.p, g->view(), g->d_Mint.p, g->npad);
   g->mark_end(kStVxc, e);
   g->mark_begin(kStFinalize, &e);
-  launch_finalize_v(g->stream, g->nbasis, g->npad, g->d_Vint.p, g->d_ref2int.p, dV);
+  launch_finalize_sym(g->stream, g->nbasis, g->npad, g->d_Mint.p, dV);
   g->mark_end(kStFinalize, e);
 }
 
@@ -403,20 +405,18 @@ int chx_grid_copy(const chx_grid* s, chx_grid** out) {
     g->core_radius = s->core_radius;
     g->mol = s->mol;
     g->nbasis = s->nbasis; g->npad = s->npad; g->ntiles = s->ntiles;
-    g->int2ref = s->int2ref; g->ref2int = s->ref2int;
     g->sh_xyz = s->sh_xyz; g->sh_type = s->sh_type; g->sh_nprim = s->sh_nprim; g->sh_poff = s->sh_poff;
-    g->p_exp = s->p_exp; g->p_coef = s->p_coef; g->tile_seg_off = s->tile_seg_off; g->seg = s->seg;
+    g->p_exp = s->p_exp; g->p_coef = s->p_coef; g->sh_ao = s->sh_ao;
     g->npoints = s->npoints; g->nbatches = s->nbatches; g->batch_n = s->batch_n;
     g->hx = s->hx; g->hy = s->hy; g->hz = s->hz; g->hw = s->hw;
     make_stream(g);
     hipStream_t st = g->stream;
     CHX_HIP(hipStreamSynchronize(s->stream));
     g->d_sh_xyz.copy_from(s->d_sh_xyz, st); g->d_p_exp.copy_from(s->d_p_exp, st); g->d_p_coef.copy_from(s->d_p_coef, st);
-    g->d_segrec.copy_from(s->d_segrec, st); g->max_nprim = s->max_nprim;
+    g->max_nprim = s->max_nprim;
     g->sh_atom = s->sh_atom; g->d_sh_atom.copy_from(s->d_sh_atom, st);
     g->d_sh_type.copy_from(s->d_sh_type, st); g->d_sh_nprim.copy_from(s->d_sh_nprim, st);
-    g->d_sh_poff.copy_from(s->d_sh_poff, st); g->d_tile_seg_off.copy_from(s->d_tile_seg_off, st);
-    g->d_seg.copy_from(s->d_seg, st); g->d_int2ref.copy_from(s->d_int2ref, st); g->d_ref2int.copy_from(s->d_ref2int, st);
+    g->d_sh_poff.copy_from(s->d_sh_poff, st);
     g->d_x.copy_from(s->d_x, st); g->d_y.copy_from(s->d_y, st); g->d_z.copy_from(s->d_z, st);
     g->d_w.copy_from(s->d_w, st); g->d_bn.copy_from(s->d_bn, st);
     CHX_HIP(hipStreamSynchronize(st));
@@ -504,7 +504,8 @@ int chx_grid_get_density_skeleton(chx_grid* g, const double* D, int nspin, int n
     require(g->precision == CHX_PREC_FP64 && g->cached, CHX_ERR_UNSUPPORTED,
             "the XC gradient is built for the FP64 form with the AO tables in HBM");
     CHX_HIP(hipMemcpyAsync(g->d_Din.p, D, sizeof(double) * (size_t)nbasis * nbasis, hipMemcpyHostToDevice, g->stream));
-    launch_permute_d(g->stream, g->nbasis, g->npad, g->d_Din.p, g->d_int2ref.p, g->d_Dskel.alloc_get((size_t)g->npad * g->npad));
+    launch_pad_d(g->stream, g->nbasis, g->npad, g->d_Din.p, g->d_Dskel.alloc_get((size_t)g->npad * g->npad));
+    gather_d(g, g->d_Din.p, g->d_Dskel_t);
     g->have_skeleton = true;
   });
 }
@@ -520,13 +521,13 @@ int chx_grid_get_density_u(chx_grid* g, const double* D, int nmats, int nspin, i
     double* rhou = g->d_rhou.alloc_get(std::max<size_t>(1, (size_t)nspin * nmats * 4 * nslots));
     for (int m = 0; m < nspin * nmats; ++m) {  // rho^x and grad rho^x of each matrix ([spin][mat]), per point
       CHX_HIP(hipMemcpyAsync(g->d_Din.p, D + m * nb2, sizeof(double) * nb2, hipMemcpyHostToDevice, g->stream));
-      launch_permute_d(g->stream, g->nbasis, g->npad, g->d_Din.p, g->d_int2ref.p, g->d_Dint.p);
+      gather_d(g, g->d_Din.p, g->d_Dt);
       if (g->cached)
-        launch_density_c64(g->stream, 0, ng, g->d_grp_batch.p, g->d_grp_tiles.p, g->d_grp_slots.p, g->d_grp_ntiles.p,
-                           g->d_bt_off.p, g->d_bt_list.p, g->d_cache.p, g->d_Dint.p, g->npad, part);
+        launch_density_c64(g->stream, 0, ng, g->d_grp_batch.p, g->d_grp_tile.p, g->d_grp_ntiles.p,
+                           g->d_bt_off.p, g->d_b_chunk.p, g->d_chunks.p, g->d_cache.p, g->d_Dt.p, part);
       else
-        launch_density_f64(g->stream, 0, ng, g->d_grp_batch.p, g->d_grp_tiles.p, g->d_grp_ntiles.p, g->d_bt_off.p,
-                           g->d_bt_list.p, g->d_x.p, g->d_y.p, g->d_z.p, g->view(), g->d_Dint.p, g->npad, part);
+        launch_density_f64(g->stream, 0, ng, g->d_grp_batch.p, g->d_grp_tile.p, g->d_grp_ntiles.p, g->d_b_chunk.p,
+                         g->d_chunks.p, g->d_x.p, g->d_y.p, g->d_z.p, g->view(), g->d_Dt.p, part);
       launch_point_rho(g->stream, g->nbatches, g->d_grp_off.p, part, rhou + (size_t)m * 4 * nslots);
     }
     CHX_HIP(hipStreamSynchronize(g->stream));
@@ -554,16 +555,15 @@ static void response_fock(chx_grid* g, const double* rhou, int nmats, double* F,
       launch_response_coef(g->stream, g->nbatches, rhou + (size_t)m * 4 * nslots, g->d_fx.p, g->d_w.p, g->fx_family,
                            coef);
     if (g->cached) {  // B = a phi + c . grad phi from the tables, M = Phi^T B, V = M + M^T
-      launch_make_b(g->stream, g->nbatches, g->d_bt_off.p, coef, g->d_cache.p, g->d_bmat.p);
-      launch_fill(g->stream, g->d_Mint.p, (size_t)g->npad * g->npad, 0.0);
-      launch_vxc_c64(g->stream, 1, (int)g->cwork.size(), g->d_cwork.p, g->d_cpair_batches.p, g->d_slot_of.p,
-                     g->ntiles, g->d_cache.p, g->d_bmat.p, coef, g->d_Mint.p, g->npad);
-      launch_finalize_sym(g->stream, g->nbasis, g->npad, g->d_Mint.p, g->d_ref2int.p, g->d_Vout.p);
+      launch_make_b(g->stream, g->nbatches, g->d_bt_off.p, coef, g->d_cache.p, g->d_bmat.p, g->d_Mint.p,
+                    (size_t)g->npad * g->npad);
+      launch_vxc_c64(g->stream, 1, (int)g->cwork.size(), g->d_cwork.p, g->d_ao_of.p, g->d_cache.p, g->d_bmat.p, coef, g->d_Mint.p, g->npad);
+      launch_finalize_sym(g->stream, g->nbasis, g->npad, g->d_Mint.p, g->d_Vout.p);
     } else {
-      launch_fill(g->stream, g->d_Vint.p, (size_t)g->npad * g->npad, 0.0);
-      launch_vxc_f64(g->stream, 1, (int)g->vwork.size(), g->d_vwork.p, g->d_pair_batches.p, g->d_alive.p,
-                     g->ntiles, g->d_x.p, g->d_y.p, g->d_z.p, coef, g->view(), g->d_Vint.p, g->npad);
-      launch_finalize_v(g->stream, g->nbasis, g->npad, g->d_Vint.p, g->d_ref2int.p, g->d_Vout.p);
+      launch_fill(g->stream, g->d_Mint.p, (size_t)g->npad * g->npad, 0.0);
+      launch_vxc_f64(g->stream, 1, (int)g->vwork.size(), g->d_vwork.p, g->d_ao_of.p, g->d_x.p, g->d_y.p, g->d_z.p,
+                     coef, g->view(), g->d_Mint.p, g->npad);
+      launch_finalize_sym(g->stream, g->nbasis, g->npad, g->d_Mint.p, g->d_Vout.p);
     }
     CHX_HIP(hipMemcpyAsync(F + m * nb2, g->d_Vout.p, sizeof(double) * nb2, hipMemcpyDeviceToHost, g->stream));
   }
@@ -586,16 +586,17 @@ int chx_grid_fock_u(chx_grid* g, double* F, int nmats, int nspin, int nbasis) {
 
 // slot -> (density group, column tile in the group), for the per-slot epilogues
 static void ensure_slot_groups(chx_grid* g) {
-  const int ng = (int)g->grp_batch.size(), ns = (int)g->bt_list.size();
+  const int ng = (int)g->grp_batch.size(), ns = (int)g->slot_tile.size();
   if (g->slot_grp.size() == (size_t)ns) return;
   g->slot_grp.assign(ns, 0);
   g->slot_q.assign(ns, 0);
-  for (int k = 0; k < ng; ++k)
+  for (int k = 0; k < ng; ++k) {
+    const int b = g->grp_batch[k], s0 = g->bt_off[b] + g->grp_tile[k] - g->chunks[g->b_chunk[b]].tile0;
     for (int q = 0; q < g->grp_ntiles[k]; ++q) {
-      const int sl = g->grp_slots[(size_t)k * kGroup + q];
-      g->slot_grp[sl] = k;
-      g->slot_q[sl] = q;
+      g->slot_grp[s0 + q] = k;
+      g->slot_q[s0 + q] = q;
     }
+  }
   g->d_slot_grp.upload(g->slot_grp, g->stream);
   g->d_slot_q.upload(g->slot_q, g->stream);
 }
@@ -610,7 +611,7 @@ int chx_grid_fock_s(chx_grid* g, double* F, int nspin, int nbasis) {
     require(g->fx_nspin == 1, CHX_ERR_UNSUPPORTED, "the skeleton response is built for the closed-shell path");
     require(g->precision == CHX_PREC_FP64 && g->cached, CHX_ERR_UNSUPPORTED,
             "the skeleton response is built for the FP64 form with the AO tables in HBM");
-    const int na = g->mol.natoms, ng = (int)g->grp_batch.size(), ns = (int)g->bt_list.size();
+    const int na = g->mol.natoms, ng = (int)g->grp_batch.size(), ns = (int)g->slot_tile.size();
     const long npt = (long)g->nbatches * kBatch;
     ensure_slot_groups(g);
     // per point and nuclear coordinate: rho^{A,t}, grad rho^{A,t}
@@ -620,10 +621,10 @@ int chx_grid_fock_s(chx_grid* g, double* F, int nspin, int nbasis) {
     xz2.alloc(nxz);
     double* rhos = g->d_rhou.alloc_get(std::max<size_t>(1, (size_t)3 * na * 4 * npt));
     launch_fill(g->stream, rhos, (size_t)3 * na * 4 * npt, 0.0);
-    launch_xgrad_xz(g->stream, ng, g->d_grp_batch.p, g->d_grp_tiles.p, g->d_grp_ntiles.p, g->d_bt_off.p,
-                    g->d_bt_list.p, g->d_cache.p, g->d_bmat.p, g->d_Dskel.p, g->npad, 0, 1, xz1.p);
-    launch_xgrad_xz(g->stream, ng, g->d_grp_batch.p, g->d_grp_tiles.p, g->d_grp_ntiles.p, g->d_bt_off.p,
-                    g->d_bt_list.p, g->d_cache.p, g->d_bmat.p, g->d_Dskel.p, g->npad, 2, 3, xz2.p);
+    launch_xgrad_xz(g->stream, ng, g->d_grp_batch.p, g->d_grp_tile.p, g->d_grp_ntiles.p, g->d_bt_off.p,
+                    g->d_b_chunk.p, g->d_chunks.p, g->d_cache.p, g->d_bmat.p, g->d_Dskel_t.p, 0, 1, xz1.p);
+    launch_xgrad_xz(g->stream, ng, g->d_grp_batch.p, g->d_grp_tile.p, g->d_grp_ntiles.p, g->d_bt_off.p,
+                    g->d_b_chunk.p, g->d_chunks.p, g->d_cache.p, g->d_bmat.p, g->d_Dskel_t.p, 2, 3, xz2.p);
     launch_skel_rho(g->stream, ns, g->d_slot_batch.p, g->d_slot_tile.p, g->d_slot_grp.p, g->d_slot_q.p, g->d_x.p,
                     g->d_y.p, g->d_z.p, g->view(), xz1.p, xz2.p, npt, rhos);
     g->nmats_u = 0;  // rhou now holds the skeleton densities, not getDensityU's
@@ -642,7 +643,7 @@ int chx_grid_fock_skeleton(chx_grid* g, double* F, int nspin, int nbasis) {
     require(g->v_nspin == 1, CHX_ERR_UNSUPPORTED, "the skeleton Fock derivative is built for the closed-shell path");
     require(g->precision == CHX_PREC_FP64 && g->cached, CHX_ERR_UNSUPPORTED,
             "the skeleton Fock derivative is built for the FP64 form with the AO tables in HBM");
-    const int na = g->mol.natoms, ns = (int)g->bt_list.size(), n = g->nbasis;
+    const int na = g->mol.natoms, ns = (int)g->slot_tile.size(), n = g->nbasis;
     const size_t pp = (size_t)g->npad * g->npad, sb = (size_t)kBatch * kTile;
     // atom of each AO, reference order
     std::vector<int> ao_atom(n, 0);
@@ -650,7 +651,7 @@ int chx_grid_fock_skeleton(chx_grid* g, double* F, int nspin, int nbasis) {
       for (int k = 0; k < chx::shell_size(sh.type); ++k) ao_atom[sh.ao_off + k] = sh.center;
     DevBuf<int> d_atom;
     d_atom.upload(ao_atom, g->stream);
-    launch_make_b(g->stream, g->nbatches, g->d_bt_off.p, g->d_coef.p, g->d_cache.p, g->d_bmat.p);
+    launch_make_b(g->stream, g->nbatches, g->d_bt_off.p, g->d_coef.p, g->d_cache.p, g->d_bmat.p, nullptr, 0);
     DevBuf<double> etab, qp, out;
     etab.alloc(std::max<size_t>(1, 3 * (size_t)ns * sb));
     launch_fill(g->stream, etab.p, 3 * (size_t)ns * sb, 0.0);
@@ -660,17 +661,15 @@ int chx_grid_fock_skeleton(chx_grid* g, double* F, int nspin, int nbasis) {
     launch_fill(g->stream, qp.p, 6 * pp, 0.0);
     for (int t = 0; t < 3; ++t) {
       // Q^t = (d_t Phi)^T B: the cached component t + 1 as the row operand
-      launch_vxc_c64(g->stream, 1, (int)g->cwork.size(), g->d_cwork.p, g->d_cpair_batches.p, g->d_slot_of.p,
-                     g->ntiles, g->d_cache.p + (size_t)(t + 1) * sb, g->d_bmat.p, g->d_coef.p, qp.p + t * pp,
+      launch_vxc_c64(g->stream, 1, (int)g->cwork.size(), g->d_cwork.p, g->d_ao_of.p, g->d_cache.p + (size_t)(t + 1) * sb, g->d_bmat.p, g->d_coef.p, qp.p + t * pp,
                      g->npad);
       // P^t = Phi^T E^t: E^t in the B table's place
-      launch_vxc_c64(g->stream, 1, (int)g->cwork.size(), g->d_cwork.p, g->d_cpair_batches.p, g->d_slot_of.p,
-                     g->ntiles, g->d_cache.p, etab.p + (size_t)t * ns * sb, g->d_coef.p, qp.p + (3 + t) * pp,
+      launch_vxc_c64(g->stream, 1, (int)g->cwork.size(), g->d_cwork.p, g->d_ao_of.p, g->d_cache.p, etab.p + (size_t)t * ns * sb, g->d_coef.p, qp.p + (3 + t) * pp,
                      g->npad);
     }
     const size_t tot = (size_t)3 * na * n * n;
     out.alloc(std::max<size_t>(1, tot));
-    launch_fock_skel_fin(g->stream, n, g->npad, na, qp.p, g->d_ref2int.p, d_atom.p, out.p);
+    launch_fock_skel_fin(g->stream, n, g->npad, na, qp.p, d_atom.p, out.p);
     CHX_HIP(hipMemcpyAsync(F, out.p, sizeof(double) * tot, hipMemcpyDeviceToHost, g->stream));
     CHX_HIP(hipStreamSynchronize(g->stream));
   });
@@ -692,33 +691,31 @@ int chx_grid_energy_hess(chx_grid* g, double* H) {
     require(g->v_nspin == 1 && g->fx_nspin == 1, CHX_ERR_UNSUPPORTED, "the XC Hessian is built for the closed-shell path");
     require(g->precision == CHX_PREC_FP64 && g->cached, CHX_ERR_UNSUPPORTED,
             "the XC Hessian is built for the FP64 form with the AO tables in HBM");
-    const int na = g->mol.natoms, np = 3 * na, ng = (int)g->grp_batch.size(), ns = (int)g->bt_list.size();
+    const int na = g->mol.natoms, np = 3 * na, ng = (int)g->grp_batch.size(), ns = (int)g->slot_tile.size();
     const long npt = (long)g->nbatches * kBatch;
     const size_t pp = (size_t)g->npad * g->npad, sb = (size_t)kBatch * kTile;
     ensure_slot_groups(g);
-    // atom of each internal AO (-1: padding)
-    std::vector<int> ao_atom(g->nbasis, 0), atom_int(g->npad, -1);
+    // atom of each AO (-1: padding)
+    std::vector<int> ao_atom(g->npad, -1);
     for (const chx::ShellH& sh : g->mol.shells)
       for (int k = 0; k < chx::shell_size(sh.type); ++k) ao_atom[sh.ao_off + k] = sh.center;
-    for (int i = 0; i < g->npad; ++i)
-      if (g->int2ref[i] >= 0) atom_int[i] = ao_atom[g->int2ref[i]];
     DevBuf<int> d_atom;
-    d_atom.upload(atom_int, g->stream);
+    d_atom.upload(ao_atom, g->stream);
     // X = D phi, Y^x = D d_x phi (xz1); Y^y, Y^z (xz2); first-order skeleton densities
     const size_t nxz = std::max<size_t>(1, (size_t)ng * 2 * kGroup * kTile * kBatch);
     DevBuf<double> xz1, xz2, rhos, etab, rr, dH;
     xz1.alloc(nxz);
     xz2.alloc(nxz);
-    launch_xgrad_xz(g->stream, ng, g->d_grp_batch.p, g->d_grp_tiles.p, g->d_grp_ntiles.p, g->d_bt_off.p,
-                    g->d_bt_list.p, g->d_cache.p, g->d_bmat.p, g->d_Dskel.p, g->npad, 0, 1, xz1.p);
-    launch_xgrad_xz(g->stream, ng, g->d_grp_batch.p, g->d_grp_tiles.p, g->d_grp_ntiles.p, g->d_bt_off.p,
-                    g->d_bt_list.p, g->d_cache.p, g->d_bmat.p, g->d_Dskel.p, g->npad, 2, 3, xz2.p);
+    launch_xgrad_xz(g->stream, ng, g->d_grp_batch.p, g->d_grp_tile.p, g->d_grp_ntiles.p, g->d_bt_off.p,
+                    g->d_b_chunk.p, g->d_chunks.p, g->d_cache.p, g->d_bmat.p, g->d_Dskel_t.p, 0, 1, xz1.p);
+    launch_xgrad_xz(g->stream, ng, g->d_grp_batch.p, g->d_grp_tile.p, g->d_grp_ntiles.p, g->d_bt_off.p,
+                    g->d_b_chunk.p, g->d_chunks.p, g->d_cache.p, g->d_bmat.p, g->d_Dskel_t.p, 2, 3, xz2.p);
     rhos.alloc(std::max<size_t>(1, (size_t)np * 4 * npt));
     launch_fill(g->stream, rhos.p, (size_t)np * 4 * npt, 0.0);
     launch_skel_rho(g->stream, ns, g->d_slot_batch.p, g->d_slot_tile.p, g->d_slot_grp.p, g->d_slot_q.p, g->d_x.p,
                     g->d_y.p, g->d_z.p, g->view(), xz1.p, xz2.p, npt, rhos.p);
     // rr[3 t + s] = (d_t Phi)^T E^s over the cached contraction
-    launch_make_b(g->stream, g->nbatches, g->d_bt_off.p, g->d_coef.p, g->d_cache.p, g->d_bmat.p);
+    launch_make_b(g->stream, g->nbatches, g->d_bt_off.p, g->d_coef.p, g->d_cache.p, g->d_bmat.p, nullptr, 0);
     etab.alloc(std::max<size_t>(1, 3 * (size_t)ns * sb));
     launch_fill(g->stream, etab.p, 3 * (size_t)ns * sb, 0.0);
     launch_skel_etab(g->stream, ns, g->d_slot_batch.p, g->d_slot_tile.p, g->d_x.p, g->d_y.p, g->d_z.p, g->view(),
@@ -727,8 +724,7 @@ int chx_grid_energy_hess(chx_grid* g, double* H) {
     launch_fill(g->stream, rr.p, 9 * pp, 0.0);
     for (int t = 0; t < 3; ++t)
       for (int u = 0; u < 3; ++u)
-        launch_vxc_c64(g->stream, 1, (int)g->cwork.size(), g->d_cwork.p, g->d_cpair_batches.p, g->d_slot_of.p,
-                       g->ntiles, g->d_cache.p + (size_t)(t + 1) * sb, etab.p + (size_t)u * ns * sb, g->d_coef.p,
+        launch_vxc_c64(g->stream, 1, (int)g->cwork.size(), g->d_cwork.p, g->d_ao_of.p, g->d_cache.p + (size_t)(t + 1) * sb, etab.p + (size_t)u * ns * sb, g->d_coef.p,
                        rr.p + (size_t)(3 * t + u) * pp, g->npad);
     dH.alloc((size_t)np * np);
     launch_fill(g->stream, dH.p, (size_t)np * np, 0.0);
@@ -747,15 +743,15 @@ int chx_grid_energy_grad(chx_grid* g, double* grad) {
     require(g->have_v, CHX_ERR_STATE, "ExchangeCorrelation::Evaluate(\"ev\") must precede Grid::getEnergyGrad");
     require(g->v_family <= 1 && g->type <= 1, CHX_ERR_UNSUPPORTED, "the XC gradient is built for LDA and GGA");
     require(g->v_nspin == 1, CHX_ERR_UNSUPPORTED, "the XC gradient is built for the closed-shell path");
-    const int na = g->mol.natoms, ng = (int)g->grp_batch.size(), ns = (int)g->bt_list.size();
+    const int na = g->mol.natoms, ng = (int)g->grp_batch.size(), ns = (int)g->slot_tile.size();
     ensure_slot_groups(g);
-    launch_make_b(g->stream, g->nbatches, g->d_bt_off.p, g->d_coef.p, g->d_cache.p, g->d_bmat.p);
+    launch_make_b(g->stream, g->nbatches, g->d_bt_off.p, g->d_coef.p, g->d_cache.p, g->d_bmat.p, nullptr, 0);
     DevBuf<double> xz, dg;
     xz.alloc(std::max<size_t>(1, (size_t)ng * 2 * kGroup * kTile * kBatch));
     dg.alloc(3 * (size_t)na);
     launch_fill(g->stream, dg.p, 3 * (size_t)na, 0.0);
-    launch_xgrad_xz(g->stream, ng, g->d_grp_batch.p, g->d_grp_tiles.p, g->d_grp_ntiles.p, g->d_bt_off.p, g->d_bt_list.p,
-                    g->d_cache.p, g->d_bmat.p, g->d_Dskel.p, g->npad, 0, -1, xz.p);
+    launch_xgrad_xz(g->stream, ng, g->d_grp_batch.p, g->d_grp_tile.p, g->d_grp_ntiles.p, g->d_bt_off.p, g->d_b_chunk.p,
+                    g->d_chunks.p, g->d_cache.p, g->d_bmat.p, g->d_Dskel_t.p, 0, -1, xz.p);
     launch_xgrad_epi(g->stream, ns, g->d_slot_batch.p, g->d_slot_tile.p, g->d_slot_grp.p, g->d_slot_q.p, g->d_x.p,
                      g->d_y.p, g->d_z.p, g->view(), g->d_coef.p, xz.p, dg.p);
     CHX_HIP(hipMemcpyAsync(grad, dg.p, sizeof(double) * 3 * na, hipMemcpyDeviceToHost, g->stream));

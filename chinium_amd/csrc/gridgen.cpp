@@ -176,19 +176,6 @@ void bisect(const std::vector<double>& x, const std::vector<double>& y, const st
   bisect(x, y, z, idx, lo + left, hi, out);
 }
 
-uint64_t morton3(double fx, double fy, double fz) {
-  auto spread = [](uint64_t v) {
-    uint64_t r = 0;
-    for (int i = 0; i < 21; ++i) r |= ((v >> i) & 1ull) << (3 * i);
-    return r;
-  };
-  auto q = [](double f) {
-    f = std::min(std::max(f, 0.0), 1.0);
-    return (uint64_t)(f * 2097151.0);
-  };
-  return spread(q(fx)) | (spread(q(fy)) << 1) | (spread(q(fz)) << 2);
-}
-
 }  // namespace
 
 const std::vector<std::array<double, 4>>& lebedev_rule(int n) { return lebedev(n); }
@@ -295,71 +282,279 @@ void grid_build(chx_grid* g, const std::string& grid_name, const std::string& da
       g->hw[s] = k < n ? pw[src] : 0.0;
     }
   }
-  // ---- internal AO order: atoms along a Morton curve, shells in file order
-  double mn[3] = {1e300, 1e300, 1e300}, mx[3] = {-1e300, -1e300, -1e300};
-  for (int a = 0; a < nat; ++a)
-    for (int d = 0; d < 3; ++d) { mn[d] = std::min(mn[d], m.xyz[3 * a + d]); mx[d] = std::max(mx[d], m.xyz[3 * a + d]); }
-  const double span = std::max({mx[0] - mn[0], mx[1] - mn[1], mx[2] - mn[2], 1e-9});
-  std::vector<int> aorder(nat);
-  std::iota(aorder.begin(), aorder.end(), 0);
-  std::vector<uint64_t> key(nat);
-  for (int a = 0; a < nat; ++a)
-    key[a] = morton3((m.xyz[3 * a] - mn[0]) / span, (m.xyz[3 * a + 1] - mn[1]) / span, (m.xyz[3 * a + 2] - mn[2]) / span);
-  std::stable_sort(aorder.begin(), aorder.end(), [&](int p, int q) { return key[p] < key[q]; });
+  // ---- shells in the reference's AO order
   g->nbasis = m.nbasis;
   g->npad = ((m.nbasis + kPadAO - 1) / kPadAO) * kPadAO;
   g->ntiles = g->npad / kTile;
-  g->int2ref.assign(g->npad, -1);
-  g->ref2int.assign(g->nbasis, -1);
   g->sh_xyz.clear(); g->sh_type.clear(); g->sh_nprim.clear(); g->sh_poff.clear(); g->sh_atom.clear();
-  g->p_exp.clear(); g->p_coef.clear();
-  std::vector<int> sh_int_ao;  // internal AO offset per internal shell
-  int ao = 0;
-  for (int a : aorder)
-    for (const ShellH& s : m.shells) {
-      if (s.center != a) continue;
-      const int n = shell_size(s.type);
-      for (int k = 0; k < n; ++k) {
-        g->int2ref[ao + k] = s.ao_off + k;
-        g->ref2int[s.ao_off + k] = ao + k;
-      }
-      g->sh_xyz.push_back(m.xyz[3 * a]); g->sh_xyz.push_back(m.xyz[3 * a + 1]); g->sh_xyz.push_back(m.xyz[3 * a + 2]);
-      g->sh_type.push_back(s.type);
-      g->sh_atom.push_back(a);
-      g->sh_nprim.push_back(s.nprim);
-      g->sh_poff.push_back((int)g->p_exp.size());
-      for (int p = 0; p < s.nprim; ++p) {
-        g->p_exp.push_back(m.exps[s.prim_off + p]);
-        g->p_coef.push_back(m.coefs[s.prim_off + p]);
-      }
-      sh_int_ao.push_back(ao);
-      ao += n;
-    }
-  // ---- tile segments
-  g->tile_seg_off.assign(g->ntiles + 1, 0);
-  g->seg.clear();
-  for (int t = 0; t < g->ntiles; ++t) {
-    g->tile_seg_off[t] = (int)g->seg.size();
-    const int lo = t * kTile, hi = lo + kTile;
-    for (size_t s = 0; s < sh_int_ao.size(); ++s) {
-      const int a0 = sh_int_ao[s], a1 = a0 + shell_size(g->sh_type[s]);
-      const int b0 = std::max(a0, lo), b1 = std::min(a1, hi);
-      if (b0 >= b1) continue;
-      g->seg.push_back(make_int4((int)s, b0 - a0, b1 - b0, b0 - lo));
+  g->sh_ao.clear(); g->p_exp.clear(); g->p_coef.clear();
+  g->max_nprim = 0;
+  for (const ShellH& s : m.shells) {
+    const int a = s.center;
+    g->sh_xyz.push_back(m.xyz[3 * a]); g->sh_xyz.push_back(m.xyz[3 * a + 1]); g->sh_xyz.push_back(m.xyz[3 * a + 2]);
+    g->sh_type.push_back(s.type);
+    g->sh_atom.push_back(a);
+    g->sh_nprim.push_back(s.nprim);
+    g->sh_ao.push_back(s.ao_off);
+    g->sh_poff.push_back((int)g->p_exp.size());
+    g->max_nprim = std::max(g->max_nprim, s.nprim);
+    for (int p = 0; p < s.nprim; ++p) {
+      g->p_exp.push_back(m.exps[s.prim_off + p]);
+      g->p_coef.push_back(m.coefs[s.prim_off + p]);
     }
   }
-  g->tile_seg_off[g->ntiles] = (int)g->seg.size();
   // ---- device copies
   hipStream_t st = g->stream;
   g->d_sh_xyz.upload(g->sh_xyz, st); g->d_sh_type.upload(g->sh_type, st); g->d_sh_nprim.upload(g->sh_nprim, st);
   g->d_sh_atom.upload(g->sh_atom, st);
   g->d_sh_poff.upload(g->sh_poff, st); g->d_p_exp.upload(g->p_exp, st); g->d_p_coef.upload(g->p_coef, st);
-  std::vector<SegRec> rec(g->seg.size());  // lives until the synchronisation below
-  g->max_nprim = 0;
+  g->d_x.upload(g->hx, st); g->d_y.upload(g->hy, st); g->d_z.upload(g->hz, st); g->d_w.upload(g->hw, st);
+  g->d_bn.upload(g->batch_n, st);
+  CHX_HIP(hipStreamSynchronize(st));
+  g->ao_ready = false;
+}
+
+// The distance from a shell's centre beyond which neither |phi| nor any
+// |d phi / d x_k| of its components exceeds thr, from the bounds
+//   |phi| <= r^l F(r),  |d phi| <= r^l G(r) + l r^(l-1) F(r),
+//   F = sum_p |c_p| exp(-a_p r^2),  G = sum_p 2 a_p r |c_p| exp(-a_p r^2)
+// (the components' angular parts are at most 1 and their derivatives at most l
+// on the unit sphere). Every term falls beyond sqrt((l + 1) / (2 a_min)), so
+// the last crossing is bisected there, or searched below when the threshold is
+// that coarse. A zero threshold keeps a shell until its exponentials underflow.
+static double shell_reach(int type, int np, const double* e, const double* c, double thr) {
+  const int l = std::abs(type);
+  auto bound = [&](double r) {
+    double F = 0, G = 0;
+    for (int p = 0; p < np; ++p) {
+      const double t = std::fabs(c[p]) * std::exp(-e[p] * r * r);
+      F += t;
+      G += 2 * e[p] * r * t;
+    }
+    const double rl = std::pow(r, l);
+    return std::max(rl * F, rl * G + (l ? l * std::pow(r, l - 1) * F : 0.0));
+  };
+  double amin = e[0];
+  for (int p = 1; p < np; ++p) amin = std::min(amin, e[p]);
+  double lo = std::sqrt((l + 1) / (2 * amin)), hi = lo + std::sqrt(800 / amin);
+  if (bound(lo) > thr) {
+    for (int k = 0; k < 100; ++k) {
+      const double mid = 0.5 * (lo + hi);
+      if (bound(mid) > thr) lo = mid; else hi = mid;
+    }
+    return hi * (1 + 1e-9);
+  }
+  const int steps = 4096;
+  for (int k = steps; k >= 0; --k)
+    if (bound(lo * k / steps) > thr) return lo * (k + 1) / steps;
+  return 0.0;
+}
+
+// Cuts the batches into chunks with one AO list each. A batch's own list is
+// short (a few hundred of a large molecule's thousands of AOs), which is what
+// makes the contractions cheap, but a chunk's list is gathered from D and
+// scattered to M once per chunk, so neighbours are merged while the merged
+// list's cost stays below that of the two: cost = n^2 (points + kChunkCost), n
+// the list's length in whole tiles, the second term the gather and the scatter
+// in units of one point's contraction. Over (H2O)1 .. (H2O)128, C18 and
+// alkanes, kChunkCost = 256 gives 7 to 23 batches per chunk at 1.2 to 1.7 times
+// the work of single batches' lists.
+static void build_chunks(chx_grid* g, int nwords, const std::vector<unsigned long long>& alive) {
+  constexpr double kChunkCost = 256.0;
+  const int nb = g->nbatches, nsh = (int)g->sh_type.size();
+  std::vector<int> sizes;  // shell sizes present, with the mask of the shells of that size
+  std::vector<std::vector<unsigned long long>> mask;
+  for (int s = 0; s < nsh; ++s) {
+    const int n = shell_size(g->sh_type[s]);
+    size_t k = std::find(sizes.begin(), sizes.end(), n) - sizes.begin();
+    if (k == sizes.size()) {
+      sizes.push_back(n);
+      mask.emplace_back(nwords, 0ull);
+    }
+    mask[k][s >> 6] |= 1ull << (s & 63);
+  }
+  auto cost = [&](const unsigned long long* w, const unsigned long long* v, int batches) {
+    int n = 0;
+    for (size_t k = 0; k < sizes.size(); ++k)
+      for (int i = 0; i < nwords; ++i) n += sizes[k] * __builtin_popcountll((w[i] | (v ? v[i] : 0ull)) & mask[k][i]);
+    const double t = (n + kTile - 1) / kTile * kTile;
+    return t * t * (double(kBatch) * batches + kChunkCost);
+  };
+  g->chunks.clear(); g->chunk_b0.clear(); g->tile_chunk.clear(); g->ao_of.clear();
+  g->tile_seg_off.clear(); g->seg.clear();
+  g->b_chunk.assign(nb, 0);
+  g->dt_elems = 0;
+  std::vector<unsigned long long> cur(nwords);
+  for (int b0 = 0; b0 < nb;) {
+    std::copy_n(&alive[(size_t)b0 * nwords], nwords, cur.begin());
+    int b1 = b0 + 1;
+    double c = cost(cur.data(), nullptr, 1);
+    while (b1 < nb && b1 - b0 < kChunkMax) {
+      const unsigned long long* v = &alive[(size_t)b1 * nwords];
+      const double cm = cost(cur.data(), v, b1 - b0 + 1);
+      if (cm > c + cost(v, nullptr, 1)) break;
+      for (int i = 0; i < nwords; ++i) cur[i] |= v[i];
+      c = cm;
+      ++b1;
+    }
+    // the list, packed: shells in AO order, one that does not fit a tile continues in the next
+    ChunkDev ch{(long)g->dt_elems, (int)g->tile_chunk.size(), 0};
+    int col = kTile;
+    for (int s = 0; s < nsh; ++s) {
+      if (!(cur[s >> 6] >> (s & 63) & 1ull)) continue;
+      for (int k = 0, n = shell_size(g->sh_type[s]); k < n;) {
+        if (col == kTile) {  // next tile
+          g->tile_seg_off.push_back((int)g->seg.size());
+          g->tile_chunk.push_back((int)g->chunks.size());
+          g->ao_of.resize(g->ao_of.size() + kTile, -1);
+          ++ch.ntl;
+          col = 0;
+        }
+        const int cnt = std::min(n - k, kTile - col);
+        g->seg.push_back(make_int4(s, k, cnt, col));
+        for (int i = 0; i < cnt; ++i) g->ao_of[g->ao_of.size() - kTile + col + i] = g->sh_ao[s] + k + i;
+        k += cnt;
+        col += cnt;
+      }
+    }
+    g->dt_elems += (size_t)ch.ntl * kTile * ch.ntl * kTile;
+    for (int b = b0; b < b1; ++b) g->b_chunk[b] = (int)g->chunks.size();
+    g->chunks.push_back(ch);
+    g->chunk_b0.push_back(b0);
+    b0 = b1;
+  }
+  g->chunk_b0.push_back(nb);
+  g->tile_seg_off.push_back((int)g->seg.size());
+}
+
+// Vxc work items: per chunk every block (I, J) of super-tiles of `sup` tiles
+// (upper: only I <= J), cut into runs of at most `len` of its batches.
+// Chunk-major, so that the items that run together on one XCD share the
+// chunk's operand slots in its L2.
+static void build_items(const chx_grid* g, int sup, bool upper, int len, std::vector<VxcItem>& out) {
+  out.clear();
+  for (size_t c = 0; c < g->chunks.size(); ++c) {
+    const ChunkDev& ch = g->chunks[c];
+    const int ns = (ch.ntl + sup - 1) / sup;
+    for (int b = g->chunk_b0[c]; b < g->chunk_b0[c + 1]; b += len) {
+      const int nbat = std::min(len, g->chunk_b0[c + 1] - b);
+      for (int I = 0; I < ns; ++I)
+        for (int J = upper ? I : 0; J < ns; ++J)
+          out.push_back(VxcItem{I, J, g->bt_off[b], nbat, ch.ntl, ch.tile0, b, 0});
+    }
+  }
+}
+
+// The longest run (a power of two up to the chunk length) that still leaves
+// enough items: each item ends in one FP64 atomic per element of its block, a
+// short list of long items leaves CUs idle. Times by run length, in us, Vxc
+// launch: (H2O)16 / def2-SVP mixed 1111 (1), 201 (8), 127 (32); (H2O)4 67 (1),
+// 27 (4), 67 (32); C7H16 FP64 323 (1), 179 (8), 307 (32); H2O FP64 18 (1), 260 (32).
+static int default_len(const chx_grid* g, int sup, bool upper) {
+  const long kMinItems = g->precision == CHX_PREC_MIXED ? 160 : 384;
+  for (int len = kChunkMax; len > 1; len /= 2) {
+    long n = 0;
+    for (size_t c = 0; c < g->chunks.size(); ++c) {
+      const long ns = (g->chunks[c].ntl + sup - 1) / sup, nb = g->chunk_b0[c + 1] - g->chunk_b0[c];
+      n += (upper ? ns * (ns + 1) / 2 : ns * ns) * ((nb + len - 1) / len);
+    }
+    if (n >= kMinItems) return len;
+  }
+  return 1;
+}
+
+// Vxc work items of the cached / mixed paths: 128-AO super-tiles, or (mixed
+// form, large bases) 256-AO groups whose items cover (I, J) and (J, I).
+void build_cwork(chx_grid* g) {
+  const bool wide = g->precision == CHX_PREC_MIXED && g->mx_wide;
+  const int sup = wide ? 2 * kCacheSuper : kCacheSuper;
+  build_items(g, sup, wide, g->vxc_chunk > 0 ? g->vxc_chunk : default_len(g, sup, wide), g->cwork);
+}
+
+// Rebuilds the Vxc work items for another chunk length (autotuning) without
+// touching the AO tables.
+void set_vxc_chunk(chx_grid* g, int chunk) {
+  g->vxc_chunk = chunk;
+  if (!g->ao_ready || !g->cached) return;
+  ++g->plan_gen;
+  build_cwork(g);
+  hipStream_t st = g->stream;
+  g->d_cwork.upload(g->cwork, st);
+  g->hmol.cwork = g->d_cwork.p;
+  CHX_HIP(hipStreamSynchronize(st));
+}
+
+// Vxc block shape of the mixed form (-1: 256-AO groups from npad 1024
+// on, 128-AO super-tiles below; 0, 1: either), rebuilding the work items.
+void set_vxc_shape(chx_grid* g, int shape) {
+  g->vxc_shape = shape;
+  if (!g->ao_ready || g->precision != CHX_PREC_MIXED) return;
+  g->mx_wide = (shape == 1 || (shape < 0 && g->npad >= 1024)) ? 1 : 0;
+  set_vxc_chunk(g, g->vxc_chunk);
+}
+
+// Screening and work plans (Grid::getAO counterpart).
+void grid_plan(chx_grid* g) {
+  hipStream_t st = g->stream;
+  const int nb = g->nbatches, nsh = (int)g->sh_type.size(), nwords = (nsh + 63) / 64;
+  std::vector<double> reach2(nsh);
+  for (int s = 0; s < nsh; ++s) {
+    const double r = shell_reach(g->sh_type[s], g->sh_nprim[s], &g->p_exp[g->sh_poff[s]], &g->p_coef[g->sh_poff[s]],
+                                 g->screen_thr);
+    reach2[s] = r * r;
+  }
+  std::vector<unsigned long long> alive((size_t)nb * nwords, 0ull);
+  {
+    DevBuf<double> d_reach;
+    DevBuf<unsigned long long> d_alive;
+    d_reach.upload(reach2, st);
+    d_alive.alloc(std::max<size_t>(1, alive.size()));
+    launch_screen(st, nb, nsh, nwords, g->d_x.p, g->d_y.p, g->d_z.p, g->d_bn.p, g->d_sh_xyz.p, d_reach.p,
+                  d_alive.p);
+    if (nb)
+      CHX_HIP(hipMemcpyAsync(alive.data(), d_alive.p, sizeof(alive[0]) * alive.size(), hipMemcpyDeviceToHost, st));
+    CHX_HIP(hipStreamSynchronize(st));
+  }
+  build_chunks(g, nwords, alive);
+  g->bt_off.assign(nb + 1, 0);
+  g->batch_work.assign(nb, 0.0);
+  g->slot_batch.clear(); g->slot_tile.clear();
+  g->grp_batch.clear(); g->grp_tile.clear(); g->grp_ntiles.clear();
+  g->grp_off.assign(nb + 1, 0);
+  std::vector<int> chunk_nao(g->chunks.size(), 0);
+  for (size_t i = 0; i < g->ao_of.size(); ++i)
+    if (g->ao_of[i] >= 0) ++chunk_nao[g->tile_chunk[i / kTile]];
+  double flops = 0, tiles = 0;
+  for (int b = 0; b < nb; ++b) {
+    const ChunkDev& ch = g->chunks[g->b_chunk[b]];
+    g->bt_off[b] = (int)g->slot_tile.size();
+    g->grp_off[b] = (int)g->grp_batch.size();
+    for (int q = 0; q < ch.ntl; ++q) {
+      g->slot_batch.push_back(b);
+      g->slot_tile.push_back(ch.tile0 + q);
+    }
+    for (int q = 0; q < ch.ntl; q += kGroup) {
+      g->grp_batch.push_back(b);
+      g->grp_tile.push_back(ch.tile0 + q);
+      g->grp_ntiles.push_back(std::min(kGroup, ch.ntl - q));
+    }
+    tiles += ch.ntl;
+    const double n = chunk_nao[g->b_chunk[b]];
+    g->batch_work[b] = (double)g->batch_n[b] * n * n;
+    flops += g->batch_work[b];
+  }
+  g->bt_off[nb] = (int)g->slot_tile.size();
+  g->grp_off[nb] = (int)g->grp_batch.size();
+  g->mean_tiles = nb ? tiles / nb : 0;
+  // k contractions per build (GGA: Phi D and Phi^T B; meta-GGA adds three of
+  // each for tau), 2 flops per multiply-add
+  g->flops_build = (g->type >= 2 ? 8.0 : 2.0) * 2.0 * flops;
+  const size_t nslot = g->slot_tile.size();
+  // the tiles' segment records, and the plan's tables on the device
+  std::vector<SegRec> rec(g->seg.size());  // lives until the synchronisation at the end
   for (size_t k = 0; k < g->seg.size(); ++k) {
     const int4 sg = g->seg[k];
     const int sh = sg.x, np = g->sh_nprim[sh], po = g->sh_poff[sh];
-    g->max_nprim = std::max(g->max_nprim, np);
     SegRec& r = rec[k];
     std::memset(&r, 0, sizeof(r));
     r.ax = g->sh_xyz[3 * sh]; r.ay = g->sh_xyz[3 * sh + 1]; r.az = g->sh_xyz[3 * sh + 2];
@@ -372,254 +567,9 @@ void grid_build(chx_grid* g, const std::string& grid_name, const std::string& da
   }
   g->d_segrec.upload(rec, st);
   g->d_tile_seg_off.upload(g->tile_seg_off, st); g->d_seg.upload(g->seg, st);
-  g->d_int2ref.upload(g->int2ref, st); g->d_ref2int.upload(g->ref2int, st);
-  g->d_x.upload(g->hx, st); g->d_y.upload(g->hy, st); g->d_z.upload(g->hz, st); g->d_w.upload(g->hw, st);
-  g->d_bn.upload(g->batch_n, st);
-  CHX_HIP(hipStreamSynchronize(st));
-  g->ao_ready = false;
-}
-
-// Vxc work items of the mixed form for large bases: the batches are cut into
-// chunks of `chunk` consecutive batches (the batch order is spatial, so a
-// chunk covers a compact region), and the union of the alive tiles of a
-// chunk's batches is cut into groups of 8 tiles in tile order. An item is an
-// pair of groups I <= J of one chunk: the 256 x 256 blocks of M at those
-// tiles' rows and columns, (I, J) and for I < J (J, I), accumulated over the
-// chunk's batches. Tiles of a
-// group that are not alive in a batch read the all-zero slot in the table,
-// and the kernel skips their loads and products, so no MFMA multiplies a
-// tile-pair block that the screening dropped. Items are chunk-major: the
-// items that run together on one XCD share the chunk's operand slots in its
-// L2.
-static void build_union_plan(chx_grid* g, int chunk) {
-  const int nb = g->nbatches, nt = g->ntiles, G = 2 * kCacheSuper;
-  const int zero = (int)g->bt_list.size();
-  g->cwork.clear();
-  g->cpair_batches.clear();
-  g->cslot.clear();
-  g->vchunk.clear();
-  g->vtab.clear();
-  g->vtile.clear();
-  std::vector<char> in_u(nt);
-  std::vector<int> U;
-  double useful = 0, dense = 0;
-  for (int b0 = 0; b0 < nb; b0 += chunk) {
-    const int b1 = std::min(nb, b0 + chunk);
-    std::fill(in_u.begin(), in_u.end(), 0);
-    for (int b = b0; b < b1; ++b)
-      for (int it = g->bt_off[b]; it < g->bt_off[b + 1]; ++it) in_u[g->bt_list[it]] = 1;
-    U.clear();
-    for (int t = 0; t < nt; ++t)
-      if (in_u[t]) U.push_back(t);
-    if (U.empty()) continue;
-    const int nu = (int)U.size(), ng = (nu + G - 1) / G, npos = ng * G;
-    const int ci = (int)g->vchunk.size();
-    g->vchunk.push_back(make_int4((int)g->vtab.size(), b1 - b0, npos, (int)g->vtile.size()));
-    for (int u = 0; u < npos; ++u) g->vtile.push_back(u < nu ? U[u] : -1);
-    for (int b = b0; b < b1; ++b) {
-      for (int u = 0; u < npos; ++u) {
-        const int si = u < nu ? g->slot_of[(size_t)b * nt + U[u]] : -1;
-        g->vtab.push_back(si >= 0 ? si : zero);
-      }
-      const double n = g->bt_off[b + 1] - g->bt_off[b];
-      useful += n * n;
-    }
-    dense += (double)(b1 - b0) * nu * nu;
-    for (int I = 0; I < ng; ++I)  // an item covers the blocks (I, J) and (J, I)
-      for (int J = I; J < ng; ++J) g->cwork.push_back(make_int4(I, J, ci, 0));
-  }
-  g->vxc_exec_frac = dense > 0 ? useful / dense : 1.0;
-}
-
-// Vxc work items of the cached / mixed paths: (super-tile I, super-tile J,
-// range of pair_batches) over 128-AO super-tiles, a chunk of batches where
-// both are alive. Chunk-major order: blocks that run at the same time work on
-// the same batches of different (I, J) pairs, so their operand tiles meet in
-// L2. Fewer, longer items mean fewer FP64 atomics into M. Large bases in the
-// mixed form take the chunk tile-group plan above.
-void build_cwork(chx_grid* g) {
-  const int nb = g->nbatches, nt = g->ntiles;
-  const bool mixed = g->precision == CHX_PREC_MIXED;
-  size_t chunk = g->vxc_chunk > 0 ? (size_t)g->vxc_chunk : (mixed ? 32 : kCacheChunk);
-  if (mixed) chunk = std::min<size_t>(chunk, kMxMaxChunk);  // the kernel stages one item's slot table
-  if (mixed && g->mx_wide) {
-    build_union_plan(g, (int)chunk);
-    return;
-  }
-  g->vchunk.clear();
-  g->vtab.clear();
-  g->vtile.clear();
-  const int sup = kCacheSuper;  // tiles per super-tile
-  const int nsc = g->npad / (sup * kTile);
-  std::vector<std::vector<int>> cp((size_t)nsc * nsc);
-  std::vector<int> alive_sup;
-  for (int b = 0; b < nb; ++b) {
-    alive_sup.clear();
-    for (int sI = 0; sI < nsc; ++sI) {
-      bool any = false;
-      for (int h = 0; h < sup; ++h) any |= g->alive[(size_t)b * nt + sI * sup + h] != 0;
-      if (any) alive_sup.push_back(sI);
-    }
-    for (int I : alive_sup)
-      for (int J : alive_sup) cp[(size_t)I * nsc + J].push_back(b);
-  }
-  g->cwork.clear();
-  g->cpair_batches.clear();
-  size_t maxlen = 0;
-  for (const auto& L : cp) maxlen = std::max(maxlen, L.size());
-  for (size_t k = 0; k < maxlen; k += chunk)
-    for (int I = 0; I < nsc; ++I)
-      for (int J = 0; J < nsc; ++J) {
-        const auto& L = cp[(size_t)I * nsc + J];
-        if (k >= L.size()) continue;
-        const int begin = (int)g->cpair_batches.size();
-        const size_t e = std::min(L.size(), k + chunk);
-        g->cpair_batches.insert(g->cpair_batches.end(), L.begin() + k, L.begin() + e);
-        g->cwork.push_back(make_int4(I, J, begin, (int)g->cpair_batches.size()));
-      }
-  g->cslot.clear();
-  if (mixed) {  // per batch of an item: the slots of I's and J's tiles, the all-zero slot if not alive
-    const int zero = (int)g->bt_list.size();
-    g->cslot.resize(g->cpair_batches.size() * 2 * sup);
-    for (const int4& w : g->cwork)
-      for (int k = w.z; k < w.w; ++k) {
-        const int b = g->cpair_batches[k];
-        for (int t = 0; t < sup; ++t) {
-          const int si = g->slot_of[(size_t)b * nt + w.x * sup + t];
-          const int sj = g->slot_of[(size_t)b * nt + w.y * sup + t];
-          g->cslot[(size_t)k * 2 * sup + t] = si >= 0 ? si : zero;
-          g->cslot[(size_t)k * 2 * sup + sup + t] = sj >= 0 ? sj : zero;
-        }
-      }
-  }
-}
-
-// Uploads the mixed form's Vxc plan and points the descriptor at it.
-static void upload_mx_plan(chx_grid* g, hipStream_t st) {
-  // the plan the grid does not use stays a one-element placeholder (the copies
-  // are asynchronous, so their sources outlive the call)
-  static const std::vector<int> one{0};
-  static const std::vector<int4> one4{make_int4(0, 0, 0, 0)};
-  g->d_cslot.upload(g->cslot.empty() ? one : g->cslot, st);
-  g->d_vchunk.upload(g->vchunk.empty() ? one4 : g->vchunk, st);
-  g->d_vtab.upload(g->vtab.empty() ? one : g->vtab, st);
-  g->d_vtile.upload(g->vtile.empty() ? one : g->vtile, st);
-  g->hmol.cwork = g->d_cwork.p;
-  g->hmol.pair_batches = g->d_cpair_batches.p;
-  g->hmol.cslot = g->d_cslot.p;
-  g->hmol.vchunk = g->d_vchunk.p;
-  g->hmol.vtab = g->d_vtab.p;
-  g->hmol.vtile = g->d_vtile.p;
-}
-
-// Rebuilds the Vxc work items for another chunk length (autotuning) without
-// touching the AO tables.
-void set_vxc_chunk(chx_grid* g, int chunk) {
-  g->vxc_chunk = chunk;
-  if (!g->ao_ready || !g->cached) return;
-  ++g->plan_gen;
-  build_cwork(g);
-  hipStream_t st = g->stream;
-  g->d_cwork.upload(g->cwork, st);
-  g->d_cpair_batches.upload(g->cpair_batches, st);
-  if (g->precision == CHX_PREC_MIXED) upload_mx_plan(g, st);
-  CHX_HIP(hipStreamSynchronize(st));
-}
-
-// Vxc block shape of the mixed form (-1: 256-AO union groups from npad 1024
-// on, 128-AO super-tiles below; 0, 1: either), rebuilding the work items.
-void set_vxc_shape(chx_grid* g, int shape) {
-  g->vxc_shape = shape;
-  if (!g->ao_ready || g->precision != CHX_PREC_MIXED) return;
-  g->mx_wide = (shape == 1 || (shape < 0 && g->npad >= 1024)) ? 1 : 0;
-  set_vxc_chunk(g, g->vxc_chunk);
-}
-
-// Screening and work plans (Grid::getAO counterpart).
-void grid_plan(chx_grid* g) {
-  hipStream_t st = g->stream;
-  const int nb = g->nbatches, nt = g->ntiles;
-  g->d_alive.alloc((size_t)std::max(1, nb * nt));
-  launch_screen(st, nb, nt, g->d_x.p, g->d_y.p, g->d_z.p, g->d_bn.p, g->view(), g->screen_thr, g->d_alive.p);
-  g->alive.assign((size_t)nb * nt, 0);
-  if (nb) CHX_HIP(hipMemcpyAsync(g->alive.data(), g->d_alive.p, (size_t)nb * nt, hipMemcpyDeviceToHost, st));
-  CHX_HIP(hipStreamSynchronize(st));
-  // real AO count per tile
-  std::vector<int> tile_nao(nt, 0);
-  for (int t = 0; t < nt; ++t)
-    for (int k = 0; k < kTile; ++k) tile_nao[t] += g->int2ref[t * kTile + k] >= 0 ? 1 : 0;
-  g->bt_off.assign(nb + 1, 0);
-  g->batch_work.assign(nb, 0.0);
-  g->bt_list.clear();
-  g->grp_batch.clear(); g->grp_tiles.clear(); g->grp_ntiles.clear();
-  g->grp_off.assign(nb + 1, 0);
-  double flops = 0, tiles = 0;
-  for (int b = 0; b < nb; ++b) {
-    g->bt_off[b] = (int)g->bt_list.size();
-    g->grp_off[b] = (int)g->grp_batch.size();
-    int nao = 0;
-    std::vector<int> lst;
-    for (int t = 0; t < nt; ++t)
-      if (g->alive[(size_t)b * nt + t]) { lst.push_back(t); nao += tile_nao[t]; }
-    g->bt_list.insert(g->bt_list.end(), lst.begin(), lst.end());
-    for (size_t k = 0; k < lst.size(); k += kGroup) {
-      g->grp_batch.push_back(b);
-      const int cnt = (int)std::min<size_t>(kGroup, lst.size() - k);
-      g->grp_ntiles.push_back(cnt);
-      for (int q = 0; q < kGroup; ++q) g->grp_tiles.push_back(q < cnt ? lst[k + q] : 0);
-    }
-    tiles += (double)lst.size();
-    g->batch_work[b] = (double)g->batch_n[b] * (double)nao * (double)nao;
-    flops += g->batch_work[b];
-  }
-  g->bt_off[nb] = (int)g->bt_list.size();
-  g->grp_off[nb] = (int)g->grp_batch.size();
-  g->mean_tiles = nb ? tiles / nb : 0;
-  // k contractions per build (GGA: Phi D and Phi^T B; meta-GGA adds three of
-  // each for tau), 2 flops per multiply-add
-  g->flops_build = (g->type >= 2 ? 8.0 : 2.0) * 2.0 * flops;
-  // Vxc work items over super-tile pairs
-  const int nsup = g->npad / (kSuper * kTile);
-  std::vector<std::vector<int>> pairs((size_t)nsup * nsup);
-  std::vector<int> sup;
-  for (int b = 0; b < nb; ++b) {
-    sup.clear();
-    for (int s = 0; s < nsup; ++s) {
-      bool any = false;
-      for (int h = 0; h < kSuper; ++h) any |= g->alive[(size_t)b * nt + s * kSuper + h] != 0;
-      if (any) sup.push_back(s);
-    }
-    for (size_t i = 0; i < sup.size(); ++i)
-      for (size_t j = i; j < sup.size(); ++j) pairs[(size_t)sup[i] * nsup + sup[j]].push_back(b);
-  }
-  g->vwork.clear();
-  g->pair_batches.clear();
-  for (int I = 0; I < nsup; ++I)
-    for (int J = I; J < nsup; ++J) {
-      const auto& L = pairs[(size_t)I * nsup + J];
-      for (size_t k = 0; k < L.size(); k += kVxcChunk) {
-        const int begin = (int)g->pair_batches.size();
-        const size_t e = std::min(L.size(), k + kVxcChunk);
-        g->pair_batches.insert(g->pair_batches.end(), L.begin() + k, L.begin() + e);
-        g->vwork.push_back(make_int4(I, J, begin, (int)g->pair_batches.size()));
-      }
-    }
-  // Cached-AO plan: slots are the entries of bt_list.
-  const size_t nslot = g->bt_list.size();
-  g->slot_batch.assign(nslot, 0);
-  g->slot_tile.assign(nslot, 0);
-  g->slot_of.assign((size_t)nb * nt, -1);
-  for (int b = 0; b < nb; ++b)
-    for (int it = g->bt_off[b]; it < g->bt_off[b + 1]; ++it) {
-      g->slot_batch[it] = b;
-      g->slot_tile[it] = g->bt_list[it];
-      g->slot_of[(size_t)b * nt + g->bt_list[it]] = it;
-    }
-  g->tile_nao = tile_nao;
-  g->grp_slots.assign(g->grp_batch.size() * kGroup, 0);
-  for (size_t k = 0; k < g->grp_batch.size(); ++k)
-    for (int q = 0; q < g->grp_ntiles[k]; ++q)
-      g->grp_slots[k * kGroup + q] = g->slot_of[(size_t)g->grp_batch[k] * nt + g->grp_tiles[k * kGroup + q]];
+  g->d_chunks.upload(g->chunks, st); g->d_b_chunk.upload(g->b_chunk, st);
+  g->d_tile_chunk.upload(g->tile_chunk, st); g->d_ao_of.upload(g->ao_of, st);
+  g->d_slot_batch.upload(g->slot_batch, st); g->d_slot_tile.upload(g->slot_tile, st);
   // The mixed form always runs from the split operand cache (nT components
   // in two layouts per slot, 2 bytes per element) plus B^T of nT components.
   const bool mixed = g->precision == CHX_PREC_MIXED;
@@ -643,21 +593,20 @@ void grid_plan(chx_grid* g) {
     throw Error(CHX_ERR_DEVICE, "the mixed-precision form needs " + std::to_string(cache_bytes / 1e9) +
                                     " GB of device memory for its AO cache");
   g->cached = mixed || g->cache_mode == 1 || (g->cache_mode == -1 && cache_bytes < 0.8 * (double)free_b);
-  // large bases: Vxc items over tile groups of batch chunks, 256 x 256 blocks
+  // large bases: Vxc items over 256 x 256 blocks
   g->mx_wide = mixed && (g->vxc_shape == 1 || (g->vxc_shape < 0 && g->npad >= 1024)) ? 1 : 0;
+  g->vwork.clear();
+  g->cwork.clear();
+  g->d_Mint.alloc((size_t)g->npad * g->npad);
   if (g->cached) {
     build_cwork(g);
-    g->d_slot_batch.upload(g->slot_batch, st); g->d_slot_tile.upload(g->slot_tile, st);
-    g->d_slot_of.upload(g->slot_of, st); g->d_tile_nao.upload(g->tile_nao, st);
-    g->d_grp_slots.upload(g->grp_slots, st);
-    g->d_cwork.upload(g->cwork, st); g->d_cpair_batches.upload(g->cpair_batches, st);
-    g->d_Mint.alloc((size_t)g->npad * g->npad);
+    g->d_cwork.upload(g->cwork, st);
     if (mixed) {
       g->d_cache.release();
       g->d_bmat.release();
       g->mx_nT = nT;
       g->mx_sstride = 2 * nT * kMxComp;  // AOg then AOt, nT components each
-      // one extra all-zero slot at index nslot stands in for tiles that are not alive
+      // one extra all-zero slot at index nslot stands in for tiles past a list
       g->d_cmx.alloc((nslot + 1) * (size_t)g->mx_sstride);
       CHX_HIP(hipMemsetAsync(g->d_cmx.p + nslot * (size_t)g->mx_sstride, 0,
                              sizeof(unsigned short) * g->mx_sstride, st));
@@ -665,9 +614,9 @@ void grid_plan(chx_grid* g) {
       // B^T of every slot, plus the all-zero slot that make_b rewrites for the
       // component count of each build's potential
       g->d_bmx.alloc((nslot + 1) * (size_t)nT * kMxComp);
-      g->d_Dsplit.alloc(2 * (size_t)g->npad * g->npad);
+      g->d_Dsplit.alloc(std::max<size_t>(1, 2 * g->dt_elems));
       // core batches: any real point within core_radius of a nucleus with Z > 2
-      std::vector<int> core_off(nb, -1), slot_core(nslot, -1);
+      std::vector<int> core_off(nb, -1), slot_core(std::max<size_t>(1, nslot), -1);
       g->core_grps.clear();
       g->main_grps.clear();
       g->ncore_batches = 0;
@@ -700,8 +649,8 @@ void grid_plan(chx_grid* g) {
       if (g->core_grps.empty()) g->main_grps.clear();  // no core batches: the launch takes every group
       g->d_main_grps.upload(g->main_grps.empty() ? zero1 : g->main_grps, st);
       g->d_cmx3.alloc(std::max<size_t>(1, (size_t)ncore_slots * nT * kBatch * kTile));
-      launch_ao_cache_mx(st, (int)nslot, g->d_slot_batch.p, g->d_slot_tile.p, g->d_tile_nao.p, g->d_x.p, g->d_y.p,
-                         g->d_z.p, g->view(), nT, g->mx_sstride, g->d_cmx.p, ncore_slots ? g->d_slot_core.p : nullptr,
+      launch_ao_cache_mx(st, (int)nslot, g->d_slot_batch.p, g->d_slot_tile.p, g->d_x.p, g->d_y.p, g->d_z.p,
+                         g->view(), nT, g->mx_sstride, g->d_cmx.p, ncore_slots ? g->d_slot_core.p : nullptr,
                          g->d_cmx3.p);
       CHX_HIP(hipStreamSynchronize(st));  // the host vectors above go out of scope
     } else {
@@ -713,27 +662,27 @@ void grid_plan(chx_grid* g) {
       g->mx_nT = g->mx_sstride = g->bmx_comps = 0;
       g->d_cache.alloc(std::max<size_t>(1, nslot * (size_t)4 * kBatch * kTile));
       g->d_bmat.alloc(std::max<size_t>(1, nslot * (size_t)kBatch * kTile));
-      launch_ao_cache(st, (int)nslot, g->d_slot_batch.p, g->d_slot_tile.p, g->d_tile_nao.p, g->d_x.p, g->d_y.p,
-                      g->d_z.p, g->view(), g->d_cache.p);
+      launch_ao_cache(st, (int)nslot, g->d_slot_batch.p, g->d_slot_tile.p, g->d_x.p, g->d_y.p, g->d_z.p, g->view(),
+                      g->d_cache.p);
     }
   } else {
     g->d_cache.release();
     g->d_bmat.release();
-    g->d_Mint.release();
+    build_items(g, kSuper, true, default_len(g, kSuper, true), g->vwork);
+    g->d_vwork.upload(g->vwork, st);
     g->d_cmx.release();
     g->d_bmx.release();
     g->d_Dsplit.release();
     g->d_Dres.release();
     g->d_cpart.release();
   }
-  g->d_bt_off.upload(g->bt_off, st); g->d_bt_list.upload(g->bt_list, st);
-  g->d_grp_batch.upload(g->grp_batch, st); g->d_grp_tiles.upload(g->grp_tiles, st);
+  g->d_bt_off.upload(g->bt_off, st);
+  g->d_grp_batch.upload(g->grp_batch, st); g->d_grp_tile.upload(g->grp_tile, st);
   g->d_grp_ntiles.upload(g->grp_ntiles, st); g->d_grp_off.upload(g->grp_off, st);
-  g->d_vwork.upload(g->vwork, st); g->d_pair_batches.upload(g->pair_batches, st);
   // per-iteration buffers
   const size_t nslots = (size_t)nb * kBatch;
-  g->d_Dint.alloc((size_t)g->npad * g->npad);
-  g->d_Vint.alloc((size_t)g->npad * g->npad);
+  if (mixed) g->d_Dt.release();
+  else g->d_Dt.alloc(std::max<size_t>(1, g->dt_elems));
   g->d_Din.alloc((size_t)g->nbasis * g->nbasis);
   g->d_Vout.alloc((size_t)g->nbasis * g->nbasis);
   g->d_part.alloc(std::max<size_t>(1, g->grp_batch.size() * 4 * kBatch));
@@ -751,22 +700,21 @@ void grid_plan(chx_grid* g) {
   if (mixed) {  // descriptor of this grid for the mixed kernels
     MolDev& m = g->hmol;
     m = MolDev{};
-    m.grp_batch = g->d_grp_batch.p; m.grp_tiles = g->d_grp_tiles.p; m.grp_ntiles = g->d_grp_ntiles.p;
-    m.bt_off = g->d_bt_off.p; m.bt_list = g->d_bt_list.p;
+    m.grp_batch = g->d_grp_batch.p; m.grp_tile = g->d_grp_tile.p; m.grp_ntiles = g->d_grp_ntiles.p;
+    m.bt_off = g->d_bt_off.p; m.b_chunk = g->d_b_chunk.p; m.chunks = g->d_chunks.p; m.ao_of = g->d_ao_of.p;
     m.bx = g->d_x.p; m.by = g->d_y.p; m.bz = g->d_z.p;
     m.bv = g->view();
     m.cache = g->d_cmx.p; m.sstride = g->mx_sstride; m.toff = g->mx_nT * kMxComp;
-    m.Ds = g->d_Dsplit.p; m.npad = g->npad; m.ntiles = g->ntiles; m.nslots = (int)g->bt_list.size();
+    m.Ds = g->d_Dsplit.p; m.npad = g->npad; m.ntiles = g->ntiles; m.nslots = (int)nslot;
     m.part = g->d_part.p; m.part_tau = g->d_part_tau.p;
     m.slot_batch = g->d_slot_batch.p; m.slot_tile = g->d_slot_tile.p;
     m.coef = g->d_coef.p; m.bt = g->d_bmx.p;
-    m.slot_of = g->d_slot_of.p;
     m.Mint = g->d_Mint.p;
+    m.cwork = g->d_cwork.p;
     m.cache3 = g->d_cmx3.p;
     m.core_off = g->d_core_off.p;
     m.core_grps = g->d_core_grps.p;
     m.main_grps = g->core_grps.empty() ? nullptr : g->d_main_grps.p;
-    upload_mx_plan(g, st);
   }
   CHX_HIP(hipStreamSynchronize(st));
   g->ao_ready = true;

@@ -16,10 +16,9 @@ constexpr int kBatch = 64;     // quadrature points per batch (MFMA K for Vxc, M
 constexpr int kTile = 32;      // AOs per screening tile
 constexpr int kGroup = 4;      // AO tiles per density work group (128 output columns)
 constexpr int kSuper = 2;      // AO tiles per Vxc super-tile (64 x 64 output block)
-constexpr int kVxcChunk = 32;  // batches per Vxc work item
 constexpr int kPadAO = 128;    // nbasis is padded to a multiple of this (4 tiles)
 constexpr int kCacheSuper = 4; // tiles per Vxc super-tile in the cached path
-constexpr int kCacheChunk = 16;  // batches per cached-path Vxc work item (FP64 form default)
+constexpr int kChunkMax = 32;  // most consecutive batches that share one AO list
 constexpr int kCoef = 5;       // Vxc integrand coefficients per point: a, c_x, c_y, c_z, t
 constexpr double kCoreRadius = 0.3;  // bohr: points this close to a nucleus with Z > 2 are batched apart
 
@@ -100,7 +99,9 @@ struct SegRec {
 };
 static_assert(sizeof(SegRec) == 128, "segment record is two 64-byte scalar loads");
 
-// Kernel-side view of the basis in the internal AO order.
+// Kernel-side view of the basis. Tiles are the chunks' own: every chunk of
+// batches (see ChunkDev) holds the AOs alive in it, packed in 32-AO tiles, and
+// tile_seg_off / seg / segrec list each tile's shell segments.
 struct BasisView {
   const double* sh_xyz;   // 3 per shell
   const int* sh_type;
@@ -108,23 +109,46 @@ struct BasisView {
   const int* sh_poff;
   const double* p_exp;
   const double* p_coef;
-  const int* tile_seg_off;  // ntiles + 1
+  const int* tile_seg_off;  // tiles of all chunks + 1
   const int4* seg;          // (shell, first component, count, local AO offset in tile)
   const SegRec* segrec;     // per segment, same index as seg (mixed-precision form)
   const int* sh_atom;       // atom of each shell (XC gradient)
 };
 
+// A chunk: up to kChunkMax consecutive batches (the batch order is spatial) and
+// the list of the AOs above the screening threshold in any of them, packed in
+// ntl tiles of 32 AOs (tiles tile0 .. tile0 + ntl - 1 of the grid's list). Every
+// batch of the chunk carries all ntl tiles, so slot (batch, tile q) is
+// bt_off[batch] + q, and the chunk's part of D is a dense (32 ntl)^2 matrix at
+// doff in the gathered copy (elements; the split form holds hi, then lo).
+struct ChunkDev {
+  long doff;
+  int tile0, ntl;
+};
+// A Vxc work item: the block (I, J) of super-tiles of one chunk over nbat of
+// its batches; slot0 is the first batch's first slot.
+struct VxcItem {
+  int I, J, slot0, nbat, ntl, tile0, batch0, pad_;
+};
+
 // Launchers (kernels.hip).
 void launch_becke(hipStream_t s, long npts, const double* px, const double* py, const double* pz, double* w,
                   const int* owner, int natoms, const double* atom_xyz, const double* inv_rab);
-void launch_screen(hipStream_t s, int nbatches, int ntiles, const double* bx, const double* by, const double* bz,
-                   const int* bn, BasisView bv, double thr, unsigned char* alive);
-void launch_permute_d(hipStream_t s, int n, int npad, const double* D, const int* int2ref, double* Dint);
+// alive: per batch nwords 64-bit words, bit k of word w set when shell 64 w + k
+// comes closer than its reach (reach2: squared) to one of the batch's points
+void launch_screen(hipStream_t s, int nbatches, int nshells, int nwords, const double* bx, const double* by,
+                   const double* bz, const int* bn, const double* sh_xyz, const double* reach2,
+                   unsigned long long* alive);
+// The chunks' dense blocks of D (FP64): block r of the launch gathers the 32
+// rows of tile r from D (reference order, column-major n x n), zero for padding.
+void launch_gather_d(hipStream_t s, int ntiles, int n, const double* D, const int* tile_chunk, const ChunkDev* chunks,
+                     const int* ao_of, double* Dt);
+void launch_pad_d(hipStream_t s, int n, int npad, const double* D, double* Dpad);
 // mode 0: rho, grad rho / 2 into part ([group][4][64]); mode r = 1..3: the tau
 // partial of direction r (part = component r - 1 of [group][3][64]).
-void launch_density_f64(hipStream_t s, int mode, int ngroups, const int* grp_batch, const int* grp_tiles,
-                        const int* grp_ntiles, const int* bt_off, const int* bt_list, const double* bx,
-                        const double* by, const double* bz, BasisView bv, const double* Dint, int npad, double* part);
+void launch_density_f64(hipStream_t s, int mode, int ngroups, const int* grp_batch, const int* grp_tile,
+                        const int* grp_ntiles, const int* b_chunk, const ChunkDev* chunks, const double* bx,
+                        const double* by, const double* bz, BasisView bv, const double* Dt, double* part);
 // One molecule of a multi-molecule functional launch: byte offsets of its
 // buffers from the launch's base pointer, its slot count, its first block
 // (entry nmol is a sentinel whose blk0 is the total block count) and its E/N slot.
@@ -142,13 +166,11 @@ void launch_eval_functional(hipStream_t s, long n, const int* codes, int ncodes,
 void launch_reduce_en(hipStream_t s, int nparts, const double* en_part, double* en);
 void launch_fill(hipStream_t s, double* p, size_t n, double v);
 // ncomp 1: a phi + c . grad phi; ncomp 4 adds the tau term (t = coef[4]).
-void launch_vxc_f64(hipStream_t s, int ncomp, int nwork, const int4* work, const int* pair_batches,
-                    const unsigned char* alive, int ntiles, const double* bx, const double* by, const double* bz,
-                    const double* coef, BasisView bv, double* Vint, int npad);
-void launch_finalize_v(hipStream_t s, int n, int npad, const double* Vint, const int* ref2int, double* V);
+void launch_vxc_f64(hipStream_t s, int ncomp, int nwork, const VxcItem* work, const int* ao_of, const double* bx,
+                    const double* by, const double* bz, const double* coef, BasisView bv, double* Mint, int npad);
 void launch_vrho_coef(hipStream_t s, long nslots, const double* vrho_w, double* coef);
 // Cached-AO FP64 path (kernels_cached.hip).
-void launch_ao_cache(hipStream_t s, int nslots, const int* slot_batch, const int* slot_tile, const int* tile_nao,
+void launch_ao_cache(hipStream_t s, int nslots, const int* slot_batch, const int* slot_tile,
                      const double* bx, const double* by, const double* bz, BasisView bv, double* cache);
 // response path (closed shell, LDA/GGA)
 constexpr int kFx = 8;  // per slot: v2rho2, v2rhosigma, v2sigma2, v_sigma, grad rho (3), -
@@ -212,42 +234,36 @@ void launch_functional_mlp(hipStream_t s, int nbatches, const int* grp_off, cons
 void launch_point_density(hipStream_t s, int nbatches, const int* grp_off, const double* part,
                           const double* part_tau, int has_tau, const double* bw, double* rho, double* sigma,
                           double* tau, double* w);
-void launch_density_c64(hipStream_t s, int mode, int ngroups, const int* grp_batch, const int* grp_tiles,
-                        const int* grp_slots, const int* grp_ntiles, const int* bt_off, const int* bt_list,
-                        const double* cache, const double* Dint, int npad, double* part);
-// B = a phi + c . grad phi per slot (one component for every family)
+void launch_density_c64(hipStream_t s, int mode, int ngroups, const int* grp_batch, const int* grp_tile,
+                        const int* grp_ntiles, const int* bt_off, const int* b_chunk, const ChunkDev* chunks,
+                        const double* cache, const double* Dt, double* part);
+// B = a phi + c . grad phi per slot (one component for every family); clears the nfill elements at M
 void launch_make_b(hipStream_t s, int nbatches, const int* bt_off, const double* coef, const double* cache,
-                   double* bmat);
+                   double* bmat, double* M, size_t nfill);
 // ncomp 4 adds the tau term, its operand t d_r phi formed from the cache and coef[4] as it is loaded
-void launch_vxc_c64(hipStream_t s, int ncomp, int nwork, const int4* work, const int* pair_batches, const int* slot_of,
-                    int ntiles, const double* cache, const double* bmat, const double* coef, double* Mint, int npad);
-void launch_finalize_sym(hipStream_t s, int n, int npad, const double* Mint, const int* ref2int, double* V);
+void launch_vxc_c64(hipStream_t s, int ncomp, int nwork, const VxcItem* work, const int* ao_of, const double* cache,
+                    const double* bmat, const double* coef, double* Mint, int npad);
+void launch_finalize_sym(hipStream_t s, int n, int npad, const double* Mint, double* V);
 // Device descriptor of one grid for the mixed-precision kernels. A kernel
 // launch covers a list of (grid, item) pairs, so one launch can serve many
 // molecules (a pack) as well as a single grid.
 struct MolDev {
-  const int *grp_batch, *grp_tiles, *grp_ntiles, *bt_off, *bt_list;  // density work groups
+  const int *grp_batch, *grp_tile, *grp_ntiles, *bt_off;  // density work groups: batch, first tile, tiles
+  const int* b_chunk;       // chunk of each batch
+  const ChunkDev* chunks;
+  const int* ao_of;         // AO of each column of the chunks' tiles (-1: padding)
   const double *bx, *by, *bz;                                          // points
   BasisView bv;
   const unsigned short* cache;  // split operand cache
   int sstride, toff;            // slot stride; offset of the transposed layout
-  const unsigned short* Ds;     // split D
+  const unsigned short* Ds;     // the chunks' dense blocks of D, split: [hi, lo][nu][mu] per chunk
   int npad, ntiles, nslots, pad_;
   double *part, *part_tau;      // density partials
   const int *slot_batch, *slot_tile;
   const double* coef;           // Vxc integrand coefficients per point
   unsigned short* bt;           // B^T per slot
-  const int4* cwork;            // Vxc work items
-  const int *pair_batches, *slot_of;
-  const int* cslot;             // per pair_batches entry: slots of I's 4 tiles, then J's (zero slot if absent)
+  const VxcItem* cwork;         // Vxc work items
   double* Mint;                 // M accumulator, npad^2
-  // Vxc over chunk tile groups (large bases): per chunk of consecutive batches
-  // (table offset, batches, table width = padded alive-tile union, tile-list
-  // offset); per (chunk batch, union position) the slot (zero slot if the tile
-  // is not alive in that batch); per union position the tile (-1: padding).
-  const int4* vchunk;
-  const int* vtab;
-  const int* vtile;
   // core batches (points within the core radius of a nucleus with Z > 2): their
   // density runs with the AO operands split in three bf16 terms; cache3 holds
   // the third term of their slots' AOg blocks [core slot][c][g][mu],
@@ -257,13 +273,13 @@ struct MolDev {
   const unsigned short* cache3;
   const int *core_off, *core_grps, *main_grps;
 };
-constexpr int kMxMaxTiles = 512;  // alive tiles per batch the mixed density kernel stages (npad <= 16384)
+constexpr int kMxMaxTiles = 512;  // basis size the mixed form takes (npad <= 16384)
 constexpr int kMxMaxChunk = 128;  // batches per Vxc work item in the mixed form
 
 // XC nuclear gradient (kernels_grad.hip), FP64 cached form.
-void launch_xgrad_xz(hipStream_t s, int ngroups, const int* grp_batch, const int* grp_tiles, const int* grp_ntiles,
-                     const int* bt_off, const int* bt_list, const double* cache, const double* bmat,
-                     const double* Dint, int npad, int c1, int c2, double* xz);
+void launch_xgrad_xz(hipStream_t s, int ngroups, const int* grp_batch, const int* grp_tile, const int* grp_ntiles,
+                     const int* bt_off, const int* b_chunk, const ChunkDev* chunks, const double* cache,
+                     const double* bmat, const double* Dt, int c1, int c2, double* xz);
 void launch_xgrad_epi(hipStream_t s, int nslots, const int* slot_batch, const int* slot_tile, const int* slot_grp,
                       const int* slot_q, const double* bx, const double* by, const double* bz, BasisView bv,
                       const double* coef, const double* xz, double* grad);
@@ -274,7 +290,7 @@ void launch_xgrad_epi(hipStream_t s, int nslots, const int* slot_batch, const in
 // order from Q^t = (d_t Phi)^T B (qp[t]) and P^t = Phi^T E^t (qp[3 + t]).
 void launch_skel_etab(hipStream_t s, int nslots, const int* slot_batch, const int* slot_tile, const double* bx,
                       const double* by, const double* bz, BasisView bv, const double* coef, double* etab);
-void launch_fock_skel_fin(hipStream_t s, int n, int npad, int natoms, const double* qp, const int* ref2int,
+void launch_fock_skel_fin(hipStream_t s, int n, int npad, int natoms, const double* qp,
                           const int* ao_atom, double* F);
 // XC energy Hessian terms added to H (np x np, np = 3 natoms; clear it first):
 // the per-slot diagonal-atom term (AO third derivatives, X and Y^r from xz1 /
@@ -295,19 +311,20 @@ void launch_skel_rho(hipStream_t s, int nslots, const int* slot_batch, const int
 constexpr int kMxComp = 2 * kTile * kBatch;  // elements per component and layout of a slot
 // slot_core / cache3 (may be null): the third bf16 term of the AOg block of each
 // slot with slot_core >= 0, at cache3 + slot_core * nT * kBatch * kTile
-void launch_ao_cache_mx(hipStream_t s, int nslots, const int* slot_batch, const int* slot_tile, const int* tile_nao,
+void launch_ao_cache_mx(hipStream_t s, int nslots, const int* slot_batch, const int* slot_tile,
                         const double* bx, const double* by, const double* bz, BasisView bv, int nT, int sstride,
                         unsigned short* cache, const int* slot_core, unsigned short* cache3);
-// R (may be null): what the two terms leave of D, D - hi - lo, in FP32 and in
-// D's own (reference, column-major) order
-void launch_split_d(hipStream_t s, int n, int npad, const double* D, const int* int2ref, unsigned short* Ds,
-                    float* R);
+// The chunks' dense blocks of D in split form (as launch_gather_d), and (all n^2
+// elements) R: what the two terms leave of D, D - hi - lo, in FP32 and in D's
+// own (reference, column-major) order
+void launch_split_d(hipStream_t s, int ntiles, int n, const double* D, const int* tile_chunk, const ChunkDev* chunks,
+                    const int* ao_of, unsigned short* Ds, float* R);
 // First-order energy correction for the split of D: V = M + M^T as
 // launch_finalize_sym, and per block the partial sum of V . R into cpart
 // (corr_blocks(n) blocks); launch_reduce_corr sums nparts partials into *out.
 int corr_blocks(int n);
-void launch_finalize_corr(hipStream_t s, int n, int npad, const double* Mint, const int* ref2int, double* V,
-                          const float* R, double* cpart);
+void launch_finalize_corr(hipStream_t s, int n, int npad, const double* Mint, double* V, const float* R,
+                          double* cpart);
 void launch_reduce_corr(hipStream_t s, int nparts, const double* cpart, double* out);
 // the packed form: per molecule of the table, en[2 slot_en] += its ncpart partials
 void launch_corr_multi(hipStream_t s, const char* base, const FnMolecule* fm, int nmol, double* en);
@@ -319,7 +336,7 @@ void launch_fill_u32(hipStream_t s, unsigned* p, size_t n, unsigned v);
 void launch_density_mx(hipStream_t s, int mode, int nitems, const MolDev& one);
 // the core groups again with three-term operands: mode 0 (rho, grad rho) or r = 1..3 (tau partial r)
 void launch_density_mx_core(hipStream_t s, int mode, int ncore_groups, const MolDev& one);
-// B^T of every slot plus the all-zero slot (index nslots) for ncomp components
+// B^T of every slot plus the all-zero slot (index nslots) for ncomp components; clears M
 void launch_make_b_mx(hipStream_t s, int ncomp, const MolDev& one);
 void launch_vxc_mx(hipStream_t s, int ncomp, int nitems, const MolDev& one);
 // Persistent stage launches over many molecules (packs, LDA/GGA): tab holds one
@@ -328,8 +345,7 @@ void launch_vxc_mx(hipStream_t s, int ncomp, int nitems, const MolDev& one);
 enum { kStageDensity = 0, kStageCore = 1, kStageMakeB = 2, kStageVxc = 3, kStageVxcWide = 4 };
 void launch_stage_multi(hipStream_t s, int stage, int ncomp, const char* base, const MolDev* tab, const int* starts,
                         int nmol, int total);
-// 256 x 256 output blocks over groups of 8 tiles of each batch chunk's alive-tile
-// union (vchunk / vtab / vtile); items (group I, group J, chunk)
+// 256 x 256 output blocks over groups of 8 of a chunk's tiles; items (I <= J)
 void launch_vxc_mx_wide(hipStream_t s, int ncomp, int nitems, const MolDev& one);
 
 }  // namespace chx
@@ -380,12 +396,10 @@ struct chx_grid {
   double screen_thr = 1e-14;
   chx_mol mol;
 
-  // AO layout: internal order groups AOs of spatially sorted atoms.
+  // AOs in the reference's order; matrices of the build (M) have npad rows.
   int nbasis = 0, npad = 0, ntiles = 0;
-  std::vector<int> int2ref;  // npad, -1 for padding
-  std::vector<int> ref2int;  // nbasis
   std::vector<double> sh_xyz;
-  std::vector<int> sh_type, sh_nprim, sh_poff, sh_atom;
+  std::vector<int> sh_type, sh_nprim, sh_poff, sh_atom, sh_ao;  // sh_ao: first AO of the shell
   std::vector<double> p_exp, p_coef;
   std::vector<int> tile_seg_off;
   std::vector<int4> seg;
@@ -401,28 +415,21 @@ struct chx_grid {
   // Bumped whenever the plan, the work lists or a buffer a captured pack graph
   // addresses may change (grid_plan, set_vxc_chunk, reallocations).
   unsigned long plan_gen = 0;
-  std::vector<unsigned char> alive;  // nbatches x ntiles
-  std::vector<int> bt_off, bt_list;  // alive tiles per batch (CSR)
-  std::vector<int> grp_batch, grp_tiles, grp_ntiles, grp_off;  // density work groups
-  std::vector<int4> vwork;           // Vxc work items (tile I, tile J, begin, end)
-  std::vector<int> pair_batches;
+  std::vector<chx::ChunkDev> chunks;   // consecutive batches that share an AO list
+  std::vector<int> chunk_b0;           // first batch of each chunk (and the end)
+  std::vector<int> b_chunk, tile_chunk, ao_of;
+  size_t dt_elems = 0;                 // elements of the chunks' dense blocks of D
+  std::vector<int> bt_off;             // first slot of each batch
+  std::vector<int> grp_batch, grp_tile, grp_ntiles, grp_off;  // density work groups
+  std::vector<chx::VxcItem> vwork;     // Vxc work items (64-AO super-tiles I <= J), AO values recomputed
   // Cached-AO path: phi and grad phi per alive (batch, tile) slot kept in HBM.
   bool cached = false;
   int cache_mode = -1;               // -1 automatic, 0 never, 1 always
-  std::vector<int> slot_batch, slot_tile, slot_of, tile_nao, grp_slots;
-  int vxc_chunk = 0;                 // batches per Vxc work item; 0 = the form's default
-  int vxc_shape = -1;                // mixed form's Vxc blocks: -1 by basis size, 0 128-AO super-tiles, 1 256-AO union groups
-  int mx_wide = 0;                   // mixed form: Vxc over 256-AO super-tiles (large bases)
-  std::vector<int4> cwork;
-  std::vector<int> cpair_batches;
-  std::vector<int> cslot;              // mixed form: slot table per cpair_batches entry
-  chx::DevBuf<int> d_cslot;
-  // mixed form, large bases: Vxc items over groups of each batch chunk's alive-tile union
-  std::vector<int4> vchunk;
-  std::vector<int> vtab, vtile;
-  chx::DevBuf<int4> d_vchunk;
-  chx::DevBuf<int> d_vtab, d_vtile;
-  double vxc_exec_frac = 1.0;          // useful / executed tile-pair products of the mixed Vxc plan
+  std::vector<int> slot_batch, slot_tile;
+  int vxc_chunk = 0;                 // batches per Vxc work item; 0 = by the item count
+  int vxc_shape = -1;                // mixed form's Vxc blocks: -1 by basis size, 0 128-AO super-tiles, 1 256-AO groups
+  int mx_wide = 0;                   // mixed form: Vxc over 256-AO groups (large bases)
+  std::vector<chx::VxcItem> cwork;
   // mixed form: core batches (density with three-term operands)
   double core_radius = chx::kCoreRadius;  // bohr; 0 turns the core treatment off
   int ncore_batches = 0;
@@ -430,8 +437,8 @@ struct chx_grid {
   chx::DevBuf<unsigned short> d_cmx3;
   chx::DevBuf<int> d_core_off, d_core_grps, d_main_grps, d_slot_core;
   chx::DevBuf<double> d_cache, d_bmat, d_Mint;
-  chx::DevBuf<int> d_slot_batch, d_slot_tile, d_slot_of, d_tile_nao, d_grp_slots, d_cpair_batches;
-  chx::DevBuf<int4> d_cwork;
+  chx::DevBuf<int> d_slot_batch, d_slot_tile;
+  chx::DevBuf<chx::VxcItem> d_cwork;
   double flops_build = 0, mean_tiles = 0;
   std::vector<double> batch_work;  // g_b n_b^2 per batch (points x kept AOs squared)
   double core_flops = 0;           // the core batches' three-term (rho, grad rho) launch: 2 sum g_b n_b^2
@@ -446,18 +453,17 @@ struct chx_grid {
   int mx_sstride = 0, mx_nT = 0, bmx_comps = 0;
   chx::DevBuf<int> d_sh_type, d_sh_nprim, d_sh_poff, d_tile_seg_off, d_sh_atom;
   chx::DevBuf<int4> d_seg;
-  chx::DevBuf<int> d_int2ref, d_ref2int;
   chx::DevBuf<double> d_x, d_y, d_z, d_w;
   chx::DevBuf<int> d_bn;
-  chx::DevBuf<unsigned char> d_alive;
-  chx::DevBuf<int> d_bt_off, d_bt_list, d_grp_batch, d_grp_tiles, d_grp_ntiles, d_grp_off;
-  chx::DevBuf<int4> d_vwork;
-  chx::DevBuf<int> d_pair_batches;
+  chx::DevBuf<chx::ChunkDev> d_chunks;
+  chx::DevBuf<int> d_b_chunk, d_tile_chunk, d_ao_of;
+  chx::DevBuf<int> d_bt_off, d_grp_batch, d_grp_tile, d_grp_ntiles, d_grp_off;
+  chx::DevBuf<chx::VxcItem> d_vwork;
   chx::DevBuf<int> d_codes;
 
   // Per-iteration state.
   // d_en: E, N and (mixed form) the first-order correction for the split of D
-  chx::DevBuf<double> d_Din, d_Dint, d_part, d_part_tau, d_rho, d_coef, d_en_part, d_en, d_Vint, d_Vout;
+  chx::DevBuf<double> d_Din, d_Dt, d_part, d_part_tau, d_rho, d_coef, d_en_part, d_en, d_Vout;
   // mixed form: D - hi - lo per spin (FP32, reference order) and the partial sums of V . (D - hi - lo)
   chx::DevBuf<float> d_Dres;
   chx::DevBuf<double> d_cpart;
@@ -469,7 +475,7 @@ struct chx_grid {
   int v_family = 0;    // family of the potential on the grid (set by Evaluate / set_vrho)
   int en_blocks = 0;
   // XC gradient (Grid::getDensitySkeleton / getEnergyGrad)
-  chx::DevBuf<double> d_Dskel;
+  chx::DevBuf<double> d_Dskel, d_Dskel_t;  // D of the skeleton calls: npad^2, and its chunk blocks
   std::vector<int> slot_grp, slot_q;
   chx::DevBuf<int> d_slot_grp, d_slot_q;
   bool have_skeleton = false;

@@ -3,10 +3,10 @@
 // Data layout in HBM
 //   points   : batch-major slots, kBatch (64) slots per batch, SoA x/y/z/w;
 //              padding slots repeat the batch's first point with w = 0.
-//   basis    : internal AO order (atoms sorted along a space-filling order),
-//              split into 32-AO tiles; per tile a list of shell segments.
-//   D, V     : npad x npad, row-major, internal order (npad = nbasis rounded
-//              up to 64). D is symmetric; V holds the upper 64x64 blocks.
+//   chunks   : up to 32 consecutive batches with one list of the AOs alive in
+//              them, packed into 32-AO tiles; per tile a list of shell segments.
+//   D        : per chunk, the dense block of its AOs (gathered each build).
+//   M        : npad x npad (nbasis rounded up to 128), V = M + M^T.
 //   partials : density per (batch, tile group): 4 x 64 doubles (rho, drho/2).
 //   coef     : per slot (a, c_x, c_y, c_z) with the Vxc integrand
 //              B_nu = a phi_nu + c . grad phi_nu, a = w v_rho / 2, c = 2 w v_sigma grad rho.
@@ -64,62 +64,103 @@ void launch_becke(hipStream_t s, long npts, const double* px, const double* py, 
 }
 
 // ---------------------------------------------------------------------------
-// AO screening: one wavefront per batch, one lane per slot. A tile is alive
-// when some AO in it has |phi| or |grad phi| above thr at some real point.
-__global__ __launch_bounds__(64) void k_screen(int ntiles, const double* __restrict__ bx, const double* __restrict__ by,
-                                               const double* __restrict__ bz, const int* __restrict__ bn, BasisView bv,
-                                               double thr, unsigned char* __restrict__ alive) {
-  const int b = blockIdx.x;
-  const int g = threadIdx.x;
-  const bool real = g < bn[b];
-  const double x = bx[b * kBatch + g], y = by[b * kBatch + g], z = bz[b * kBatch + g];
-  for (int t = 0; t < ntiles; ++t) {
-    bool any = false;
-    for (int s = bv.tile_seg_off[t]; s < bv.tile_seg_off[t + 1] && !any; ++s) {
-      const int4 sg = bv.seg[s];
-      double v[7], gx[7], gy[7], gz[7];
-      shell_eval<true>(bv, sg.x, x, y, z, v, gx, gy, gz);
-      double mx = 0;
-      for (int m = 0; m < 7; ++m) {
-        if (m >= sg.y && m < sg.y + sg.z) {
-          mx = fmax(mx, fabs(v[m]));
-          mx = fmax(mx, fmax(fabs(gx[m]), fmax(fabs(gy[m]), fabs(gz[m]))));
-        }
+// AO screening: one block per batch. A shell is alive when its centre comes
+// closer to one of the batch's points than the shell's reach, the distance
+// beyond which neither |phi| nor |grad phi| of any of its components exceeds
+// the threshold (shell_reach in gridgen.cpp). Bound by the FP64 distances
+// (64 per batch and shell); no exponential is taken here, and the batch's bit
+// mask comes out of a wave ballot. Padding slots repeat the first point.
+__global__ __launch_bounds__(256) void k_screen(int nshells, int nwords, const double* __restrict__ bx,
+                                                const double* __restrict__ by, const double* __restrict__ bz,
+                                                const int* __restrict__ bn, const double* __restrict__ sh_xyz,
+                                                const double* __restrict__ reach2,
+                                                unsigned long long* __restrict__ alive) {
+  __shared__ double px[kBatch], py[kBatch], pz[kBatch];
+  const int b = blockIdx.x, tid = threadIdx.x, n = bn[b];
+  if (tid < kBatch) {
+    px[tid] = bx[b * kBatch + tid];
+    py[tid] = by[b * kBatch + tid];
+    pz[tid] = bz[b * kBatch + tid];
+  }
+  __syncthreads();
+  for (int s0 = 0; s0 < nwords * 64; s0 += 256) {
+    const int s = s0 + tid;
+    bool on = false;
+    if (s < nshells) {
+      const double x = sh_xyz[3 * s], y = sh_xyz[3 * s + 1], z = sh_xyz[3 * s + 2];
+      double d2 = 1e300;
+      for (int g = 0; g < n; ++g) {
+        const double dx = px[g] - x, dy = py[g] - y, dz = pz[g] - z;
+        d2 = fmin(d2, dx * dx + dy * dy + dz * dz);
       }
-      any = __ballot(real && mx > thr) != 0;
+      on = d2 < reach2[s];
     }
-    if (g == 0) alive[(size_t)b * ntiles + t] = any ? 1 : 0;
+    const unsigned long long w = __ballot(on);
+    if ((tid & 63) == 0 && (s >> 6) < nwords) alive[(size_t)b * nwords + (s >> 6)] = w;
   }
 }
 
-void launch_screen(hipStream_t s, int nbatches, int ntiles, const double* bx, const double* by, const double* bz,
-                   const int* bn, BasisView bv, double thr, unsigned char* alive) {
+void launch_screen(hipStream_t s, int nbatches, int nshells, int nwords, const double* bx, const double* by,
+                   const double* bz, const int* bn, const double* sh_xyz, const double* reach2,
+                   unsigned long long* alive) {
   if (nbatches == 0) return;
-  hipLaunchKernelGGL(k_screen, dim3(nbatches), dim3(64), 0, s, ntiles, bx, by, bz, bn, bv, thr, alive);
+  hipLaunchKernelGGL(k_screen, dim3(nbatches), dim3(256), 0, s, nshells, nwords, bx, by, bz, bn, sh_xyz, reach2, alive);
   CHX_HIP(hipGetLastError());
 }
 
 // ---------------------------------------------------------------------------
-// D (reference order, column-major n x n) -> internal order, npad x npad, zero padded.
-__global__ void k_permute_d(int n, int npad, const double* __restrict__ D, const int* __restrict__ int2ref,
-                            double* __restrict__ Dint) {
+// D (reference order, column-major n x n) -> row-major npad x npad, zero padded.
+__global__ void k_pad_d(int n, int npad, const double* __restrict__ D, double* __restrict__ Dpad) {
   const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (idx >= (long)npad * npad) return;
   const int r = (int)(idx / npad), c = (int)(idx % npad);
-  const int rr = int2ref[r], cc = int2ref[c];
-  Dint[idx] = (rr >= 0 && cc >= 0) ? D[(size_t)cc * n + rr] : 0.0;
+  Dpad[idx] = r < n && c < n ? D[(size_t)c * n + r] : 0.0;
 }
 
-void launch_permute_d(hipStream_t s, int n, int npad, const double* D, const int* int2ref, double* Dint) {
+void launch_pad_d(hipStream_t s, int n, int npad, const double* D, double* Dpad) {
   const long tot = (long)npad * npad;
-  hipLaunchKernelGGL(k_permute_d, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, s, n, npad, D, int2ref, Dint);
+  hipLaunchKernelGGL(k_pad_d, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, s, n, npad, D, Dpad);
+  CHX_HIP(hipGetLastError());
+}
+
+// The chunks' dense blocks of D: Dt[doff + r ld + c] = D(ao_r, ao_c), ld = 32
+// ntl. One block per tile: its 32 rows against the chunk's columns. Reads runs
+// of consecutive rows of a column of D (a shell's AOs), which the chunks that
+// share them find in the caches; bound by the writes.
+__global__ __launch_bounds__(256) void k_gather_d(int n, const double* __restrict__ D,
+                                                  const int* __restrict__ tile_chunk,
+                                                  const ChunkDev* __restrict__ chunks, const int* __restrict__ ao_of,
+                                                  double* __restrict__ Dt) {
+  const int t = blockIdx.x;
+  const ChunkDev c = chunks[tile_chunk[t]];
+  const int ld = c.ntl * kTile;
+  double* __restrict__ out = Dt + c.doff + (size_t)(t - c.tile0) * kTile * ld;
+  const int* __restrict__ cols = ao_of + (size_t)c.tile0 * kTile;
+  __shared__ int rows[kTile];
+  if (threadIdx.x < kTile) rows[threadIdx.x] = ao_of[(size_t)t * kTile + threadIdx.x];
+  __shared__ double T[kTile][kTile + 1];
+  for (int q = 0; q < c.ntl; ++q) {  // 32 x 32 sub-blocks, transposed through LDS so that both sides run along AOs
+    __syncthreads();
+    for (int e = threadIdx.x; e < kTile * kTile; e += 256) {
+      const int r = e & (kTile - 1), k = e >> 5, rr = rows[r], cc = cols[q * kTile + k];
+      T[r][k] = rr >= 0 && cc >= 0 ? D[(size_t)cc * n + rr] : 0.0;
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e < kTile * kTile; e += 256) out[(size_t)(e >> 5) * ld + q * kTile + (e & 31)] = T[e >> 5][e & 31];
+  }
+}
+
+void launch_gather_d(hipStream_t s, int ntiles, int n, const double* D, const int* tile_chunk, const ChunkDev* chunks,
+                     const int* ao_of, double* Dt) {
+  if (ntiles == 0) return;
+  hipLaunchKernelGGL(k_gather_d, dim3(ntiles), dim3(256), 0, s, n, D, tile_chunk, chunks, ao_of, Dt);
   CHX_HIP(hipGetLastError());
 }
 
 // ---------------------------------------------------------------------------
-// Density. One block (4 waves) per work group = (batch b, up to 4 alive AO
-// tiles j as output columns). X[g, nu] = sum_{alive tiles i} A_i[g, :] D[i, nu]
-// accumulates on MFMA over K = the batch's alive tiles, then
+// Density. One block (4 waves) per work group = (batch b, up to 4 tiles j of its
+// AO list as output columns). X[g, nu] = sum_{tiles i} A_i[g, :] D[i, nu]
+// accumulates on MFMA over K = the list's tiles, then
 // MODE 0 (A = phi): rho[g] += sum_nu X phi_nu, drho[g]/2 += sum_nu X grad phi_nu
 //   (4 components per point into part, [group][4][64]);
 // MODE r = 1..3 (A = d_r phi): sum_nu X d_r phi_nu, the tau partial of
@@ -138,20 +179,20 @@ struct DensSmem {
 };
 
 template <int MODE>
-__global__ __launch_bounds__(256) void k_density_f64(const int* __restrict__ grp_batch, const int* __restrict__ grp_tiles,
-                                                     const int* __restrict__ grp_ntiles, const int* __restrict__ bt_off,
-                                                     const int* __restrict__ bt_list, const double* __restrict__ bx,
-                                                     const double* __restrict__ by, const double* __restrict__ bz,
-                                                     BasisView bv, const double* __restrict__ Dint, int npad,
-                                                     double* __restrict__ part) {
+__global__ __launch_bounds__(256) void k_density_f64(const int* __restrict__ grp_batch, const int* __restrict__ grp_tile,
+                                                     const int* __restrict__ grp_ntiles,
+                                                     const int* __restrict__ b_chunk,
+                                                     const ChunkDev* __restrict__ chunks,
+                                                     const double* __restrict__ bx, const double* __restrict__ by,
+                                                     const double* __restrict__ bz, BasisView bv,
+                                                     const double* __restrict__ Dt, double* __restrict__ part) {
   __shared__ DensSmem sm;
   const int grp = blockIdx.x;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int b = grp_batch[grp];
-  const int nt = grp_ntiles[grp];
-  int jt[kGroup];
-#pragma unroll
-  for (int q = 0; q < kGroup; ++q) jt[q] = grp_tiles[grp * kGroup + q];
+  const int nt = grp_ntiles[grp], j0 = grp_tile[grp];
+  const ChunkDev ch = chunks[b_chunk[b]];
+  const int ld = ch.ntl * kTile, col0 = (j0 - ch.tile0) * kTile;
 
   if (tid < kBatch) {
     sm.px[tid] = bx[b * kBatch + tid];
@@ -164,8 +205,9 @@ __global__ __launch_bounds__(256) void k_density_f64(const int* __restrict__ grp
   __syncthreads();
 
   const int lrow = lane & 15, lk = lane >> 4;
-  for (int it = bt_off[b]; it < bt_off[b + 1]; ++it) {
-    const int ti = bt_list[it];
+  for (int k = 0; k < ch.ntl; ++k) {
+    const int ti = ch.tile0 + k;
+    const double* __restrict__ Drow = Dt + ch.doff + (size_t)k * kTile * ld + col0;
     // zero the Phi tile, then fill the AOs this tile holds
     for (int e = tid; e < kTile * kBatch; e += 256) (&sm.k.A[0][0])[e] = 0.0;
     __syncthreads();
@@ -184,7 +226,7 @@ __global__ __launch_bounds__(256) void k_density_f64(const int* __restrict__ grp
     for (int e = tid; e < kTile * kGroup * kTile; e += 256) {
       const int r = e / (kGroup * kTile), c = e % (kGroup * kTile);
       const int q = c / kTile;
-      sm.k.B[r][c] = (q < nt) ? Dint[(size_t)(ti * kTile + r) * npad + jt[q] * kTile + (c % kTile)] : 0.0;
+      sm.k.B[r][c] = (q < nt) ? Drow[(size_t)r * ld + c] : 0.0;
     }
     __syncthreads();
 #pragma unroll
@@ -214,7 +256,7 @@ __global__ __launch_bounds__(256) void k_density_f64(const int* __restrict__ grp
     if (q < nt) {
       for (int e = tid; e < 4 * kBatch * (kTile + 1); e += 256) (&sm.E[0][0][0])[e] = 0.0;
       __syncthreads();
-      const int tj = jt[q];
+      const int tj = j0 + q;
       const int s0 = bv.tile_seg_off[tj], s1 = bv.tile_seg_off[tj + 1];
       for (int item = tid; item < (s1 - s0) * kBatch; item += 256) {
         const int g = item % kBatch;
@@ -268,13 +310,13 @@ __global__ __launch_bounds__(256) void k_density_f64(const int* __restrict__ grp
   if (c < NOUT) part[(size_t)grp * grp_stride + c * kBatch + 16 * wave + 4 * r + lk] = out;
 }
 
-void launch_density_f64(hipStream_t s, int mode, int ngroups, const int* grp_batch, const int* grp_tiles,
-                        const int* grp_ntiles, const int* bt_off, const int* bt_list, const double* bx,
-                        const double* by, const double* bz, BasisView bv, const double* Dint, int npad, double* part) {
+void launch_density_f64(hipStream_t s, int mode, int ngroups, const int* grp_batch, const int* grp_tile,
+                        const int* grp_ntiles, const int* b_chunk, const ChunkDev* chunks, const double* bx,
+                        const double* by, const double* bz, BasisView bv, const double* Dt, double* part) {
   if (ngroups == 0) return;
 #define CHX_DF64(M)                                                                                       \
-  hipLaunchKernelGGL(k_density_f64<M>, dim3(ngroups), dim3(256), 0, s, grp_batch, grp_tiles, grp_ntiles, \
-                     bt_off, bt_list, bx, by, bz, bv, Dint, npad, part);
+  hipLaunchKernelGGL(k_density_f64<M>, dim3(ngroups), dim3(256), 0, s, grp_batch, grp_tile, grp_ntiles, \
+                     b_chunk, chunks, bx, by, bz, bv, Dt, part);
   switch (mode) {
     case 0: CHX_DF64(0); break;
     case 1: CHX_DF64(1); break;
@@ -916,15 +958,15 @@ void launch_vrho_coef(hipStream_t s, long nslots, const double* vrho_w, double* 
 }
 
 // ---------------------------------------------------------------------------
-// Vxc. One block per work item (super-tiles I <= J of 64 AOs, range of
-// batches where both are alive). V_IJ += sum_g P_I^T B_J + B_I^T P_J on
+// Vxc. One block per work item (super-tiles I <= J of 64 of a chunk's AOs, a
+// range of the chunk's batches). V_IJ = sum_g P_I^T B_J + B_I^T P_J on
 // MFMA, K = points, 32 points per LDS stage. Pass 0 has P = phi and
 // B = a phi + c . grad phi; meta-GGA (NC = 4) adds passes r = 1..3 with
 // P = d_r phi and B = t d_r phi (t = w v_tau / 4, so the pair of products
 // gives w v_tau / 2 d_r phi_mu d_r phi_nu). AO values are recomputed for each
 // pass (no tables in HBM). Wave w owns output rows 16w..16w+15 and all 64
-// columns. The block result is added to V with hardware FP64 atomics once per
-// work item.
+// columns. The block result is added to M with hardware FP64 atomics once per
+// work item, halved on the diagonal (V = M + M^T at finalisation).
 constexpr int kVxcK = 32;
 constexpr int kSupAO = kSuper * kTile;  // 64
 
@@ -937,12 +979,11 @@ struct VxcSmem {
 };
 
 __device__ __forceinline__ void vxc_fill_super(VxcSmem& sm, double (*P)[kSupAO + 1], double (*B)[kSupAO + 1],
-                                               int sup, const unsigned char* alive_b, const BasisView& bv, int tid,
-                                               int pass) {
+                                               int sup, int tile0, int ntl, const BasisView& bv, int tid, int pass) {
   for (int half = 0; half < kSuper; ++half) {
-    const int t = sup * kSuper + half;
-    if (!alive_b[t]) continue;
-    const int s0 = bv.tile_seg_off[t], s1 = bv.tile_seg_off[t + 1];
+    const int q = sup * kSuper + half;
+    if (q >= ntl) continue;
+    const int s0 = bv.tile_seg_off[tile0 + q], s1 = bv.tile_seg_off[tile0 + q + 1];
     for (int item = tid; item < (s1 - s0) * kVxcK; item += 256) {
       const int g = item % kVxcK;
       const int4 sg = bv.seg[s0 + item / kVxcK];
@@ -968,14 +1009,13 @@ __device__ __forceinline__ void vxc_fill_super(VxcSmem& sm, double (*P)[kSupAO +
 }
 
 template <int NC>
-__global__ __launch_bounds__(256) void k_vxc_f64(const int4* __restrict__ work, const int* __restrict__ pair_batches,
-                                                 const unsigned char* __restrict__ alive, int ntiles,
+__global__ __launch_bounds__(256) void k_vxc_f64(const VxcItem* __restrict__ work, const int* __restrict__ ao_of,
                                                  const double* __restrict__ bx, const double* __restrict__ by,
                                                  const double* __restrict__ bz, const double* __restrict__ coef,
-                                                 BasisView bv, double* __restrict__ Vint, int npad) {
+                                                 BasisView bv, double* __restrict__ Mint, int npad) {
   __shared__ VxcSmem sm;
-  const int4 wk = work[blockIdx.x];
-  const int I = wk.x, J = wk.y;
+  const VxcItem wk = work[blockIdx.x];
+  const int I = wk.I, J = wk.J;
   const bool diag = (I == J);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int lrow = lane & 15, lk = lane >> 4;
@@ -983,9 +1023,7 @@ __global__ __launch_bounds__(256) void k_vxc_f64(const int4* __restrict__ work, 
 #pragma unroll
   for (int c = 0; c < 4; ++c) acc[c] = dbl4{0, 0, 0, 0};
 
-  for (int it = wk.z; it < wk.w; ++it) {
-    const int b = pair_batches[it];
-    const unsigned char* ab = alive + (size_t)b * ntiles;
+  for (int b = wk.batch0; b < wk.batch0 + wk.nbat; ++b) {
     for (int h = 0; h < kBatch / kVxcK; ++h) {
       // load the points and their coefficients
       if (tid < kVxcK) {
@@ -1000,7 +1038,7 @@ __global__ __launch_bounds__(256) void k_vxc_f64(const int4* __restrict__ work, 
         sm.ct[tid] = NC == 4 ? coef[kCoef * slot + 4] : 0.0;
       }
       for (int pass = 0; pass < NC; ++pass) {
-      // zero the tiles (AOs outside the alive tiles stay zero), then fill them
+      // zero the tiles (columns past the list stay zero), then fill them
       for (int e = tid; e < kVxcK * (kSupAO + 1); e += 256) {
         (&sm.PI[0][0])[e] = 0.0;
         (&sm.BI[0][0])[e] = 0.0;
@@ -1010,8 +1048,8 @@ __global__ __launch_bounds__(256) void k_vxc_f64(const int4* __restrict__ work, 
         }
       }
       __syncthreads();
-      vxc_fill_super(sm, sm.PI, sm.BI, I, ab, bv, tid, pass);
-      if (!diag) vxc_fill_super(sm, sm.PJ, sm.BJ, J, ab, bv, tid, pass);
+      vxc_fill_super(sm, sm.PI, sm.BI, I, wk.tile0, wk.ntl, bv, tid, pass);
+      if (!diag) vxc_fill_super(sm, sm.PJ, sm.BJ, J, wk.tile0, wk.ntl, bv, tid, pass);
       __syncthreads();
       double (*PJ)[kSupAO + 1] = diag ? sm.PI : sm.PJ;
       double (*BJ)[kSupAO + 1] = diag ? sm.BI : sm.BJ;
@@ -1031,43 +1069,26 @@ __global__ __launch_bounds__(256) void k_vxc_f64(const int4* __restrict__ work, 
     }
   }
   // C layout: acc[cb][r] = V[row = 16w + 4r + lk][col = 16 cb + lrow]
+  const int nrow = wk.ntl * kTile;
+  const int* __restrict__ ao = ao_of + (size_t)wk.tile0 * kTile;
 #pragma unroll
   for (int cb = 0; cb < 4; ++cb)
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int mu = I * kSupAO + 16 * wave + 4 * r + lk;
-      const int nu = J * kSupAO + 16 * cb + lrow;
-      unsafeAtomicAdd(&Vint[(size_t)mu * npad + nu], acc[cb][r]);
+      const int lr = I * kSupAO + 16 * wave + 4 * r + lk, lc = J * kSupAO + 16 * cb + lrow;
+      const int mu = lr < nrow ? ao[lr] : -1, nu = lc < nrow ? ao[lc] : -1;
+      if (mu >= 0 && nu >= 0)
+        unsafeAtomicAdd(&Mint[(size_t)mu * npad + nu], diag ? 0.5 * acc[cb][r] : acc[cb][r]);
     }
 }
 
-void launch_vxc_f64(hipStream_t s, int ncomp, int nwork, const int4* work, const int* pair_batches,
-                    const unsigned char* alive, int ntiles, const double* bx, const double* by, const double* bz,
-                    const double* coef, BasisView bv, double* Vint, int npad) {
+void launch_vxc_f64(hipStream_t s, int ncomp, int nwork, const VxcItem* work, const int* ao_of, const double* bx,
+                    const double* by, const double* bz, const double* coef, BasisView bv, double* Mint, int npad) {
   if (nwork == 0) return;
   if (ncomp == 4)
-    hipLaunchKernelGGL(k_vxc_f64<4>, dim3(nwork), dim3(256), 0, s, work, pair_batches, alive, ntiles, bx, by, bz,
-                       coef, bv, Vint, npad);
+    hipLaunchKernelGGL(k_vxc_f64<4>, dim3(nwork), dim3(256), 0, s, work, ao_of, bx, by, bz, coef, bv, Mint, npad);
   else
-    hipLaunchKernelGGL(k_vxc_f64<1>, dim3(nwork), dim3(256), 0, s, work, pair_batches, alive, ntiles, bx, by, bz,
-                       coef, bv, Vint, npad);
-  CHX_HIP(hipGetLastError());
-}
-
-// Internal upper 64x64 blocks -> full symmetric V in reference order, column-major.
-__global__ void k_finalize_v(int n, int npad, const double* __restrict__ Vint, const int* __restrict__ ref2int,
-                             double* __restrict__ V) {
-  const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= (long)n * n) return;
-  const int col = (int)(idx / n), row = (int)(idx % n);
-  const int mu = ref2int[row], nu = ref2int[col];
-  const double v = (mu / kSupAO <= nu / kSupAO) ? Vint[(size_t)mu * npad + nu] : Vint[(size_t)nu * npad + mu];
-  V[idx] = v;
-}
-
-void launch_finalize_v(hipStream_t s, int n, int npad, const double* Vint, const int* ref2int, double* V) {
-  const long tot = (long)n * n;
-  hipLaunchKernelGGL(k_finalize_v, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, s, n, npad, Vint, ref2int, V);
+    hipLaunchKernelGGL(k_vxc_f64<1>, dim3(nwork), dim3(256), 0, s, work, ao_of, bx, by, bz, coef, bv, Mint, npad);
   CHX_HIP(hipGetLastError());
 }
 

@@ -2,7 +2,7 @@
 //
 // phi and grad phi do not change between SCF iterations, so they are computed
 // once per grid (at Grid::getAO, as the reference caches its AO tables,
-// src/Grid/Grid.cpp:22-33) for every alive (batch, 32-AO tile) slot and kept in
+// src/Grid/Grid.cpp:22-33) for every (batch, 32-AO tile of its list) slot and kept in
 // HBM (~80 KB per slot: 4.4 GB at (H2O)16/def2-SVP/SG-2). Each iteration then
 // streams them through two MFMA contractions:
 //   density: X = Phi_b D_b (A = phi tiles, B = D blocks, both staged in LDS,
@@ -29,9 +29,9 @@ constexpr int kHalf = 32;                   // points per Vxc LDS stage
 // ---------------------------------------------------------------------------
 // AO cache: one block per slot.
 __global__ __launch_bounds__(256) void k_ao_cache(const int* __restrict__ slot_batch, const int* __restrict__ slot_tile,
-                                                  const int* __restrict__ tile_nao, const double* __restrict__ bx,
-                                                  const double* __restrict__ by, const double* __restrict__ bz,
-                                                  BasisView bv, double* __restrict__ cache) {
+                                                  const double* __restrict__ bx, const double* __restrict__ by,
+                                                  const double* __restrict__ bz, BasisView bv,
+                                                  double* __restrict__ cache) {
   __shared__ double px[kBatch], py[kBatch], pz[kBatch];
   const int s = blockIdx.x, tid = threadIdx.x;
   const int b = slot_batch[s], t = slot_tile[s];
@@ -41,8 +41,9 @@ __global__ __launch_bounds__(256) void k_ao_cache(const int* __restrict__ slot_b
     py[tid] = by[b * kBatch + tid];
     pz[tid] = bz[b * kBatch + tid];
   }
-  // padding AOs of the last tile are zero
-  const int nao = tile_nao[t];
+  // padding AOs of a chunk's last tile are zero
+  const int4 last = bv.seg[bv.tile_seg_off[t + 1] - 1];
+  const int nao = last.w + last.z;
   for (int e = tid; e < 4 * kBatch * (kTile - nao); e += 256) {
     const int w = kTile - nao;
     const int c = e / (kBatch * w), r = e % (kBatch * w);
@@ -67,17 +68,17 @@ __global__ __launch_bounds__(256) void k_ao_cache(const int* __restrict__ slot_b
   }
 }
 
-void launch_ao_cache(hipStream_t s, int nslots, const int* slot_batch, const int* slot_tile, const int* tile_nao,
+void launch_ao_cache(hipStream_t s, int nslots, const int* slot_batch, const int* slot_tile,
                      const double* bx, const double* by, const double* bz, BasisView bv, double* cache) {
   if (nslots == 0) return;
-  hipLaunchKernelGGL(k_ao_cache, dim3(nslots), dim3(256), 0, s, slot_batch, slot_tile, tile_nao, bx, by, bz, bv, cache);
+  hipLaunchKernelGGL(k_ao_cache, dim3(nslots), dim3(256), 0, s, slot_batch, slot_tile, bx, by, bz, bv, cache);
   CHX_HIP(hipGetLastError());
 }
 
 // ---------------------------------------------------------------------------
-// Density from the cache. Block = (batch, group of <= 4 alive tiles as output
+// Density from the cache. Block = (batch, group of <= 4 tiles of its list as output
 // columns), 8 waves: wave w owns rows g = 16(w%4)..+15 and output columns
-// 64(w/4)..+63 (two tiles). K loop over the batch's alive tiles: phi tile
+// 64(w/4)..+63 (two tiles). K loop over the list's tiles: phi tile
 // [g][mu] and D block [mu][nu] double-buffered in LDS, the next K step
 // prefetched into registers while the MFMAs of the current one run.
 struct DensCSmem {
@@ -90,11 +91,11 @@ struct DensCSmem {
 // MODE r = 1..3: A = d phi / d x_r, epilogue sum X_r d_r phi into part (one
 // component: the tau partial of direction r).
 template <int MODE>
-__global__ __launch_bounds__(512) void k_density_c64(const int* __restrict__ grp_batch, const int* __restrict__ grp_tiles,
-                                                     const int* __restrict__ grp_slots, const int* __restrict__ grp_ntiles,
-                                                     const int* __restrict__ bt_off, const int* __restrict__ bt_list,
-                                                     const double* __restrict__ cache, const double* __restrict__ Dint,
-                                                     int npad, double* __restrict__ part, int grp_stride) {
+__global__ __launch_bounds__(512) void k_density_c64(const int* __restrict__ grp_batch, const int* __restrict__ grp_tile,
+                                                     const int* __restrict__ grp_ntiles, const int* __restrict__ bt_off,
+                                                     const int* __restrict__ b_chunk, const ChunkDev* __restrict__ chunks,
+                                                     const double* __restrict__ cache, const double* __restrict__ Dt,
+                                                     double* __restrict__ part, int grp_stride) {
   constexpr int NOUT = MODE == 0 ? 4 : 1;
   __shared__ DensCSmem sm;
   const int grp = blockIdx.x;
@@ -104,23 +105,22 @@ __global__ __launch_bounds__(512) void k_density_c64(const int* __restrict__ grp
   const int wr = wave & 3, wc = wave >> 2;  // row block, column half
   const int b = grp_batch[grp];
   const int nt = grp_ntiles[grp];
-  int jt[kGroup];
-#pragma unroll
-  for (int q = 0; q < kGroup; ++q) jt[q] = grp_tiles[grp * kGroup + q];
-  const int it0 = bt_off[b], it1 = bt_off[b + 1];
+  const ChunkDev ch = chunks[b_chunk[b]];
+  const int ld = ch.ntl * kTile, j0 = grp_tile[grp] - ch.tile0;  // j0: the group's first tile in the chunk
+  const int it0 = bt_off[b], it1 = it0 + ch.ntl;
+  const double* __restrict__ Dc = Dt + ch.doff + j0 * kTile;
 
   double2 ra[2], rb[4];
   auto load = [&](int it) {
     const double2* src = reinterpret_cast<const double2*>(cache + (size_t)it * kSlotAO + MODE * kSlotB);
 #pragma unroll
     for (int j = 0; j < 2; ++j) ra[j] = src[tid + 512 * j];
-    const int ti = bt_list[it];
+    const double* __restrict__ Drow = Dc + (size_t)(it - it0) * kTile * ld;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int e = 2 * (tid + 512 * j);
       const int r = e / (kGroup * kTile), cc = e % (kGroup * kTile), q = cc / kTile;
-      rb[j] = (q < nt) ? *reinterpret_cast<const double2*>(Dint + (size_t)(ti * kTile + r) * npad + jt[q] * kTile + (cc % kTile))
-                       : double2{0.0, 0.0};
+      rb[j] = (q < nt) ? *reinterpret_cast<const double2*>(Drow + (size_t)r * ld + cc) : double2{0.0, 0.0};
     }
   };
   auto store = [&](int buf) {
@@ -167,7 +167,7 @@ __global__ __launch_bounds__(512) void k_density_c64(const int* __restrict__ grp
   for (int cb = 0; cb < 4; ++cb) {
     if (cb < ncb) {
       const int q = 2 * wc + cb / 2, h = cb % 2;
-      const double* src = cache + (size_t)grp_slots[grp * kGroup + q] * kSlotAO;
+      const double* src = cache + (size_t)(it0 + j0 + q) * kSlotAO;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int g = 16 * wr + 4 * r + lk;
@@ -204,17 +204,21 @@ __global__ __launch_bounds__(512) void k_density_c64(const int* __restrict__ grp
   }
 }
 
-void launch_density_c64(hipStream_t s, int mode, int ngroups, const int* grp_batch, const int* grp_tiles,
-                        const int* grp_slots, const int* grp_ntiles, const int* bt_off, const int* bt_list,
-                        const double* cache, const double* Dint, int npad, double* part) {
+void launch_density_c64(hipStream_t s, int mode, int ngroups, const int* grp_batch, const int* grp_tile,
+                        const int* grp_ntiles, const int* bt_off, const int* b_chunk, const ChunkDev* chunks,
+                        const double* cache, const double* Dt, double* part) {
   if (ngroups == 0) return;
   const int stride = (mode == 0 ? 4 : 3) * kBatch;  // part: [group][4][64]; tau partials: [group][3][64]
+#define CHX_DC64(M)                                                                                        \
+  hipLaunchKernelGGL(k_density_c64<M>, dim3(ngroups), dim3(512), 0, s, grp_batch, grp_tile, grp_ntiles,    \
+                     bt_off, b_chunk, chunks, cache, Dt, part, stride);
   switch (mode) {
-    case 0: hipLaunchKernelGGL(k_density_c64<0>, dim3(ngroups), dim3(512), 0, s, grp_batch, grp_tiles, grp_slots, grp_ntiles, bt_off, bt_list, cache, Dint, npad, part, stride); break;
-    case 1: hipLaunchKernelGGL(k_density_c64<1>, dim3(ngroups), dim3(512), 0, s, grp_batch, grp_tiles, grp_slots, grp_ntiles, bt_off, bt_list, cache, Dint, npad, part, stride); break;
-    case 2: hipLaunchKernelGGL(k_density_c64<2>, dim3(ngroups), dim3(512), 0, s, grp_batch, grp_tiles, grp_slots, grp_ntiles, bt_off, bt_list, cache, Dint, npad, part, stride); break;
-    default: hipLaunchKernelGGL(k_density_c64<3>, dim3(ngroups), dim3(512), 0, s, grp_batch, grp_tiles, grp_slots, grp_ntiles, bt_off, bt_list, cache, Dint, npad, part, stride); break;
+    case 0: CHX_DC64(0); break;
+    case 1: CHX_DC64(1); break;
+    case 2: CHX_DC64(2); break;
+    default: CHX_DC64(3); break;
   }
+#undef CHX_DC64
   CHX_HIP(hipGetLastError());
 }
 
@@ -223,9 +227,17 @@ void launch_density_c64(hipStream_t s, int mode, int ngroups, const int* grp_bat
 // one component per slot for every family: the meta-GGA operand
 // T_r = t d_r phi (t = w v_tau / 4, so that V = M + M^T carries
 // (1/2) w v_tau grad phi_mu . grad phi_nu) is formed from the cached d_r phi
-// while the Vxc kernel loads it, instead of being stored.
+// while the Vxc kernel loads it, instead of being stored. The blocks past the
+// batches clear M for the Vxc launch that follows.
+constexpr int kFillBlock = 4096;
 __global__ __launch_bounds__(256) void k_make_b(const int* __restrict__ bt_off, const double* __restrict__ coef,
-                                                const double* __restrict__ cache, double* __restrict__ bmat) {
+                                                const double* __restrict__ cache, double* __restrict__ bmat,
+                                                int nbatches, double* __restrict__ M, size_t nfill) {
+  if ((int)blockIdx.x >= nbatches) {
+    const size_t e0 = (size_t)(blockIdx.x - nbatches) * kFillBlock;
+    for (size_t i = e0 + threadIdx.x; i < e0 + kFillBlock && i < nfill; i += 256) M[i] = 0.0;
+    return;
+  }
   __shared__ double ca[kBatch], cx[kBatch], cy[kBatch], cz[kBatch];
   const int b = blockIdx.x, tid = threadIdx.x;
   if (tid < kBatch) {
@@ -248,15 +260,16 @@ __global__ __launch_bounds__(256) void k_make_b(const int* __restrict__ bt_off, 
 }
 
 void launch_make_b(hipStream_t s, int nbatches, const int* bt_off, const double* coef, const double* cache,
-                   double* bmat) {
-  if (nbatches == 0) return;
-  hipLaunchKernelGGL(k_make_b, dim3(nbatches), dim3(256), 0, s, bt_off, coef, cache, bmat);
+                   double* bmat, double* M, size_t nfill) {
+  const unsigned nb = (unsigned)(nbatches + (nfill + kFillBlock - 1) / kFillBlock);
+  if (nb == 0) return;
+  hipLaunchKernelGGL(k_make_b, dim3(nb), dim3(256), 0, s, bt_off, coef, cache, bmat, nbatches, M, nfill);
   CHX_HIP(hipGetLastError());
 }
 
 // ---------------------------------------------------------------------------
 // Vxc from the cache: M_IJ += sum_g phi_I[g]^T B_J[g] over the work item's
-// batches, 32 points per LDS stage (double-buffered), 8 waves: wave w owns rows
+// batches, I and J super-tiles of the chunk's AO list, 32 points per LDS stage (double-buffered), 8 waves: wave w owns rows
 // mu = 16w..16w+15 of the 128 x 128 block. One atomic add per element per item.
 struct VxcCSmem {
   double P[2][kHalf][kSupCAO + 1];
@@ -267,14 +280,13 @@ struct VxcCSmem {
 // component streamed as further K stages, T_r = t d_r phi formed from the
 // cached d_r phi and the point's t = coef[4] as it is loaded.
 template <int NC>
-__global__ __launch_bounds__(512) void k_vxc_c64(const int4* __restrict__ work, const int* __restrict__ pair_batches,
-                                                 const int* __restrict__ slot_of, int ntiles,
+__global__ __launch_bounds__(512) void k_vxc_c64(const VxcItem* __restrict__ work, const int* __restrict__ ao_of,
                                                  const double* __restrict__ cache, const double* __restrict__ bmat,
                                                  const double* __restrict__ coef, double* __restrict__ Mint,
                                                  int npad) {
   __shared__ VxcCSmem sm;
-  const int4 wk = work[blockIdx.x];
-  const int I = wk.x, J = wk.y;
+  const VxcItem wk = work[blockIdx.x];
+  const int I = wk.I, J = wk.J;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lrow = lane & 15, lk = lane >> 4;
@@ -283,14 +295,14 @@ __global__ __launch_bounds__(512) void k_vxc_c64(const int4* __restrict__ work, 
   double2 rp[kSupC], rq[kSupC];
   const int r0 = 2 * tid;  // element within a tile's 32 x 32 block
   auto load = [&](int k) {  // stage k -> (batch, half, component)
-    const int it = wk.z + k / (2 * NC), h = (k / NC) % 2, c = k % NC;
-    const int b = pair_batches[it];
+    const int it = k / (2 * NC), h = (k / NC) % 2, c = k % NC;
+    const int b = wk.batch0 + it, s0 = wk.slot0 + it * wk.ntl;
     const int g = h * kHalf + r0 / kTile, mu = r0 % kTile;
     const double t = c ? coef[kCoef * ((size_t)b * kBatch + g) + 4] : 0.0;
 #pragma unroll
     for (int j = 0; j < kSupC; ++j) {
-      const int si = slot_of[(size_t)b * ntiles + I * kSupC + j];
-      const int sj = slot_of[(size_t)b * ntiles + J * kSupC + j];
+      const int si = I * kSupC + j < wk.ntl ? s0 + I * kSupC + j : -1;
+      const int sj = J * kSupC + j < wk.ntl ? s0 + J * kSupC + j : -1;
       rp[j] = si >= 0 ? *reinterpret_cast<const double2*>(cache + (size_t)si * kSlotAO + (size_t)c * kSlotB + g * kTile + mu)
                       : double2{0.0, 0.0};
       if (sj < 0) {
@@ -318,7 +330,7 @@ __global__ __launch_bounds__(512) void k_vxc_c64(const int4* __restrict__ work, 
   dbl4 acc[8];
 #pragma unroll
   for (int cb = 0; cb < 8; ++cb) acc[cb] = dbl4{0, 0, 0, 0};
-  const int nstage = (wk.w - wk.z) * (kBatch / kHalf) * NC;
+  const int nstage = wk.nbat * (kBatch / kHalf) * NC;
   if (nstage > 0) load(0);
   int buf = 0;
   for (int k = 0; k < nstage; ++k) {
@@ -334,41 +346,39 @@ __global__ __launch_bounds__(512) void k_vxc_c64(const int4* __restrict__ work, 
     }
     buf ^= 1;
   }
+  const int nrow = wk.ntl * kTile;
+  const int* __restrict__ ao = ao_of + (size_t)wk.tile0 * kTile;
 #pragma unroll
   for (int cb = 0; cb < 8; ++cb)
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int mu = I * kSupCAO + 16 * wave + 4 * r + lk;
-      const int nu = J * kSupCAO + 16 * cb + lrow;
-      unsafeAtomicAdd(&Mint[(size_t)mu * npad + nu], acc[cb][r]);
+      const int lr = I * kSupCAO + 16 * wave + 4 * r + lk, lc = J * kSupCAO + 16 * cb + lrow;
+      const int mu = lr < nrow ? ao[lr] : -1, nu = lc < nrow ? ao[lc] : -1;
+      if (mu >= 0 && nu >= 0) unsafeAtomicAdd(&Mint[(size_t)mu * npad + nu], acc[cb][r]);
     }
 }
 
-void launch_vxc_c64(hipStream_t s, int ncomp, int nwork, const int4* work, const int* pair_batches, const int* slot_of,
-                    int ntiles, const double* cache, const double* bmat, const double* coef, double* Mint, int npad) {
+void launch_vxc_c64(hipStream_t s, int ncomp, int nwork, const VxcItem* work, const int* ao_of, const double* cache,
+                    const double* bmat, const double* coef, double* Mint, int npad) {
   if (nwork == 0) return;
   if (ncomp == 4)
-    hipLaunchKernelGGL(k_vxc_c64<4>, dim3(nwork), dim3(512), 0, s, work, pair_batches, slot_of, ntiles, cache, bmat,
-                       coef, Mint, npad);
+    hipLaunchKernelGGL(k_vxc_c64<4>, dim3(nwork), dim3(512), 0, s, work, ao_of, cache, bmat, coef, Mint, npad);
   else
-    hipLaunchKernelGGL(k_vxc_c64<1>, dim3(nwork), dim3(512), 0, s, work, pair_batches, slot_of, ntiles, cache, bmat,
-                       coef, Mint, npad);
+    hipLaunchKernelGGL(k_vxc_c64<1>, dim3(nwork), dim3(512), 0, s, work, ao_of, cache, bmat, coef, Mint, npad);
   CHX_HIP(hipGetLastError());
 }
 
 // V (reference order, column-major) = M + M^T.
-__global__ void k_finalize_sym(int n, int npad, const double* __restrict__ Mint, const int* __restrict__ ref2int,
-                               double* __restrict__ V) {
+__global__ void k_finalize_sym(int n, int npad, const double* __restrict__ Mint, double* __restrict__ V) {
   const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (idx >= (long)n * n) return;
   const int col = (int)(idx / n), row = (int)(idx % n);
-  const int mu = ref2int[row], nu = ref2int[col];
-  V[idx] = Mint[(size_t)mu * npad + nu] + Mint[(size_t)nu * npad + mu];
+  V[idx] = Mint[(size_t)row * npad + col] + Mint[(size_t)col * npad + row];
 }
 
-void launch_finalize_sym(hipStream_t s, int n, int npad, const double* Mint, const int* ref2int, double* V) {
+void launch_finalize_sym(hipStream_t s, int n, int npad, const double* Mint, double* V) {
   const long tot = (long)n * n;
-  hipLaunchKernelGGL(k_finalize_sym, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, s, n, npad, Mint, ref2int, V);
+  hipLaunchKernelGGL(k_finalize_sym, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, s, n, npad, Mint, V);
   CHX_HIP(hipGetLastError());
 }
 

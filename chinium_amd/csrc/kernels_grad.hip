@@ -43,11 +43,12 @@ struct XgradSmem {
   double Bd[kTile][kGCols];      // D block [nu][mu]
 };
 
-__global__ __launch_bounds__(256) void k_xgrad_xz(const int* __restrict__ grp_batch, const int* __restrict__ grp_tiles,
+__global__ __launch_bounds__(256) void k_xgrad_xz(const int* __restrict__ grp_batch, const int* __restrict__ grp_tile,
                                                   const int* __restrict__ grp_ntiles, const int* __restrict__ bt_off,
-                                                  const int* __restrict__ bt_list, const double* __restrict__ cache,
-                                                  const double* __restrict__ bmat, const double* __restrict__ Dint,
-                                                  int npad, int c1, int c2, double* __restrict__ xz) {
+                                                  const int* __restrict__ b_chunk, const ChunkDev* __restrict__ chunks,
+                                                  const double* __restrict__ cache, const double* __restrict__ bmat,
+                                                  const double* __restrict__ Dt, int c1, int c2,
+                                                  double* __restrict__ xz) {
   __shared__ XgradSmem sm;
   const int grp = blockIdx.x;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -55,14 +56,14 @@ __global__ __launch_bounds__(256) void k_xgrad_xz(const int* __restrict__ grp_ba
   const int lrow = lane & 15, lk = lane >> 4;
   const int b = grp_batch[grp];
   const int nt = grp_ntiles[grp];
-  int jt[kGroup];
-#pragma unroll
-  for (int q = 0; q < kGroup; ++q) jt[q] = grp_tiles[grp * kGroup + q];
+  const ChunkDev ch = chunks[b_chunk[b]];
+  const int ld = ch.ntl * kTile, it0 = bt_off[b];
+  const double* __restrict__ Dc = Dt + ch.doff + (grp_tile[grp] - ch.tile0) * kTile;
   dbl4 ax[8], az[8];
 #pragma unroll
   for (int c = 0; c < 8; ++c) ax[c] = az[c] = dbl4{0, 0, 0, 0};
-  for (int it = bt_off[b]; it < bt_off[b + 1]; ++it) {
-    const int ti = bt_list[it];
+  for (int it = it0; it < it0 + ch.ntl; ++it) {
+    const double* __restrict__ Drow = Dc + (size_t)(it - it0) * kTile * ld;
     const double* p = cache + (size_t)it * kGSlotAO + (size_t)c1 * kBatch * kTile;  // [g][nu]
     const double* q = c2 < 0 ? bmat + (size_t)it * kGSlotB : cache + (size_t)it * kGSlotAO + (size_t)c2 * kBatch * kTile;
     for (int e = tid; e < kBatch * kTile; e += 256) {
@@ -71,7 +72,7 @@ __global__ __launch_bounds__(256) void k_xgrad_xz(const int* __restrict__ grp_ba
     }
     for (int e = tid; e < kTile * kGCols; e += 256) {
       const int r = e / kGCols, c = e % kGCols, qq = c / kTile;
-      sm.Bd[r][c] = qq < nt ? Dint[(size_t)(ti * kTile + r) * npad + jt[qq] * kTile + (c % kTile)] : 0.0;
+      sm.Bd[r][c] = qq < nt ? Drow[(size_t)r * ld + c] : 0.0;
     }
     __syncthreads();
 #pragma unroll
@@ -99,12 +100,12 @@ __global__ __launch_bounds__(256) void k_xgrad_xz(const int* __restrict__ grp_ba
     }
 }
 
-void launch_xgrad_xz(hipStream_t s, int ngroups, const int* grp_batch, const int* grp_tiles, const int* grp_ntiles,
-                     const int* bt_off, const int* bt_list, const double* cache, const double* bmat,
-                     const double* Dint, int npad, int c1, int c2, double* xz) {
+void launch_xgrad_xz(hipStream_t s, int ngroups, const int* grp_batch, const int* grp_tile, const int* grp_ntiles,
+                     const int* bt_off, const int* b_chunk, const ChunkDev* chunks, const double* cache,
+                     const double* bmat, const double* Dt, int c1, int c2, double* xz) {
   if (ngroups == 0) return;
-  hipLaunchKernelGGL(k_xgrad_xz, dim3(ngroups), dim3(256), 0, s, grp_batch, grp_tiles, grp_ntiles, bt_off, bt_list,
-                     cache, bmat, Dint, npad, c1, c2, xz);
+  hipLaunchKernelGGL(k_xgrad_xz, dim3(ngroups), dim3(256), 0, s, grp_batch, grp_tile, grp_ntiles, bt_off, b_chunk,
+                     chunks, cache, bmat, Dt, c1, c2, xz);
   CHX_HIP(hipGetLastError());
 }
 
@@ -452,19 +453,18 @@ void launch_skel_etab(hipStream_t s, int nslots, const int* slot_batch, const in
   CHX_HIP(hipGetLastError());
 }
 
-// F[3 A + t] in the reference's order (column-major), from the internal Q^t
-// (qp[t]) and P^t (qp[3 + t]), npad x npad row-major [mu][nu]:
-//   F[row, col] = -( [atom(row) = A] N^t[mu][nu] + [atom(col) = A] N^t[nu][mu] ),
-//   N^t[mu][nu] = Q^t[mu][nu] + P^t[nu][mu], mu = ref2int[row], nu = ref2int[col].
+// F[3 A + t] in the reference's order (column-major), from Q^t (qp[t]) and P^t
+// (qp[3 + t]), npad x npad row-major [mu][nu]:
+//   F[row, col] = -( [atom(row) = A] N^t[row][col] + [atom(col) = A] N^t[col][row] ),
+//   N^t[mu][nu] = Q^t[mu][nu] + P^t[nu][mu].
 __global__ void k_fock_skel_fin(int n, int npad, int natoms, const double* __restrict__ qp,
-                                const int* __restrict__ ref2int, const int* __restrict__ ao_atom,
-                                double* __restrict__ F) {
+                                const int* __restrict__ ao_atom, double* __restrict__ F) {
   const size_t nn = (size_t)n * n, tot = (size_t)3 * natoms * nn, pp = (size_t)npad * npad;
   for (size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x; idx < tot; idx += (size_t)gridDim.x * blockDim.x) {
     const int m = (int)(idx / nn), A = m / 3, t = m % 3;
     const size_t e = idx % nn;
     const int col = (int)(e / n), row = (int)(e % n);
-    const size_t mu = ref2int[row], nu = ref2int[col];
+    const size_t mu = row, nu = col;
     const double* Q = qp + (size_t)t * pp;
     const double* P = qp + (size_t)(3 + t) * pp;
     double v = 0.0;
@@ -474,12 +474,12 @@ __global__ void k_fock_skel_fin(int n, int npad, int natoms, const double* __res
   }
 }
 
-void launch_fock_skel_fin(hipStream_t s, int n, int npad, int natoms, const double* qp, const int* ref2int,
+void launch_fock_skel_fin(hipStream_t s, int n, int npad, int natoms, const double* qp,
                           const int* ao_atom, double* F) {
   const size_t tot = (size_t)3 * natoms * n * n;
   if (tot == 0) return;
   const unsigned blocks = (unsigned)std::min<size_t>((tot + 255) / 256, 65536);
-  hipLaunchKernelGGL(k_fock_skel_fin, dim3(blocks), dim3(256), 0, s, n, npad, natoms, qp, ref2int, ao_atom, F);
+  hipLaunchKernelGGL(k_fock_skel_fin, dim3(blocks), dim3(256), 0, s, n, npad, natoms, qp, ao_atom, F);
   CHX_HIP(hipGetLastError());
 }
 
@@ -664,8 +664,8 @@ __global__ __launch_bounds__(256) void k_hess_fx(long npt, int np, const double*
   unsafeAtomicAdd(&H[(size_t)a * np + b], e);
 }
 
-// H2: one thread per internal element (mu, nu) of D (npad^2, internal order),
-// nine products added to H[3 A + t][3 B + s] (atom: atom of each internal AO, -1 padding).
+// H2: one thread per element (mu, nu) of D (npad^2, zero padded), nine products
+// added to H[3 A + t][3 B + s] (atom: atom of each AO, -1 padding).
 __global__ void k_hess_dk(int npad, int np, const double* __restrict__ Dint, const double* __restrict__ rr,
                           const int* __restrict__ atom, double* __restrict__ H) {
   const size_t pp = (size_t)npad * npad;

@@ -96,22 +96,21 @@ __device__ __forceinline__ float pair_at(const u16* p, int off) { return bf2f(p[
 // AO cache in split form: one block per slot. Values are evaluated in FP64,
 // rounded to FP32 and split.
 __global__ __launch_bounds__(256) void k_ao_cache_mx(const int* __restrict__ slot_batch, const int* __restrict__ slot_tile,
-                                                     const int* __restrict__ tile_nao, const double* __restrict__ bx,
-                                                     const double* __restrict__ by, const double* __restrict__ bz,
-                                                     BasisView bv, int nT, int sstride, u16* __restrict__ cache,
+                                                     const double* __restrict__ bx, const double* __restrict__ by,
+                                                     const double* __restrict__ bz, BasisView bv, int nT, int sstride,
+                                                     u16* __restrict__ cache,
                                                      const int* __restrict__ slot_core, u16* __restrict__ cache3) {
   __shared__ float E[4][kBatch][kTile + 1];
   __shared__ double px[kBatch], py[kBatch], pz[kBatch];
   const int s = blockIdx.x, tid = threadIdx.x;
   const int b = slot_batch[s], t = slot_tile[s];
-  for (int e = tid; e < 4 * kBatch * (kTile + 1); e += 256) (&E[0][0][0])[e] = 0.0f;
+  for (int e = tid; e < 4 * kBatch * (kTile + 1); e += 256) (&E[0][0][0])[e] = 0.0f;  // padding AOs stay zero
   if (tid < kBatch) {
     px[tid] = bx[b * kBatch + tid];
     py[tid] = by[b * kBatch + tid];
     pz[tid] = bz[b * kBatch + tid];
   }
   __syncthreads();
-  (void)tile_nao;  // padding AOs stay zero from the clear above
   const int s0 = bv.tile_seg_off[t], s1 = bv.tile_seg_off[t + 1];
   for (int item = tid; item < (s1 - s0) * kBatch; item += 256) {
     const int g = item % kBatch;
@@ -158,43 +157,74 @@ __global__ __launch_bounds__(256) void k_ao_cache_mx(const int* __restrict__ slo
   }
 }
 
-void launch_ao_cache_mx(hipStream_t s, int nslots, const int* slot_batch, const int* slot_tile, const int* tile_nao,
+void launch_ao_cache_mx(hipStream_t s, int nslots, const int* slot_batch, const int* slot_tile,
                         const double* bx, const double* by, const double* bz, BasisView bv, int nT, int sstride,
                         unsigned short* cache, const int* slot_core, unsigned short* cache3) {
   if (nslots == 0) return;
-  hipLaunchKernelGGL(k_ao_cache_mx, dim3(nslots), dim3(256), 0, s, slot_batch, slot_tile, tile_nao, bx, by, bz, bv, nT,
+  hipLaunchKernelGGL(k_ao_cache_mx, dim3(nslots), dim3(256), 0, s, slot_batch, slot_tile, bx, by, bz, bv, nT,
                      sstride, cache, slot_core, cache3);
   CHX_HIP(hipGetLastError());
 }
 
 // ---------------------------------------------------------------------------
-// D (reference order, column-major) -> internal order, split: Ds[hl][mu][nu].
-// R (if set): what the split leaves of D, D - hi - lo (its FP32 rounding
+// The chunks' dense blocks of D in split form: per chunk [hl][nu][mu], ld = 32
+// ntl. One block per tile of the chunks (its 32 rows nu against the chunk's
+// columns mu), as k_gather_d; the blocks past the tiles form R (kRestBlock
+// elements each), what the split leaves of D, D - hi - lo (its FP32 rounding
 // included), at D's own position. The products see hi + lo; sum V . R, with V
 // the potential of this density, is the first-order energy of the remainder
 // (dE/dD = V), which the energy takes back when the potential is built
-// (k_finalize_corr).
-__global__ void k_split_d(int n, int npad, const double* __restrict__ D, const int* __restrict__ int2ref,
-                          u16* __restrict__ Ds, float* __restrict__ R) {
-  const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  const long np2 = (long)npad * npad;
-  if (idx >= np2) return;
-  const int r = (int)(idx / npad), c = (int)(idx % npad);
-  const int rr = int2ref[r], cc = int2ref[c];
-  const bool real = rr >= 0 && cc >= 0;
-  const double v = real ? D[(size_t)cc * n + rr] : 0.0;
-  u16 hi, lo;
-  const float x = (float)v;
-  split_bf(x, hi, lo);
-  Ds[idx] = hi;
-  Ds[np2 + idx] = lo;
-  if (R && real) R[(size_t)cc * n + rr] = (float)(v - (double)bf2f(hi) - (double)bf2f(lo));
+// (k_finalize_corr). One launch: small molecules (and packs of them) are bound
+// by the launches.
+constexpr int kRestBlock = 4096;
+__global__ __launch_bounds__(256) void k_split_gather(int n, const double* __restrict__ D,
+                                                      const int* __restrict__ tile_chunk,
+                                                      const ChunkDev* __restrict__ chunks,
+                                                      const int* __restrict__ ao_of, u16* __restrict__ Ds,
+                                                      int ntiles, long n2, float* __restrict__ R) {
+  const int t = blockIdx.x;
+  if (t >= ntiles) {
+    const long e0 = (long)(t - ntiles) * kRestBlock, e1 = e0 + kRestBlock < n2 ? e0 + kRestBlock : n2;
+    for (long i = e0 + threadIdx.x; i < e1; i += 256) {
+      const double v = D[i];
+      u16 hi, lo;
+      split_bf((float)v, hi, lo);
+      R[i] = (float)(v - (double)bf2f(hi) - (double)bf2f(lo));
+    }
+    return;
+  }
+  const ChunkDev c = chunks[tile_chunk[t]];
+  const int ld = c.ntl * kTile;
+  const size_t plane = (size_t)ld * ld;
+  u16* __restrict__ out = Ds + 2 * c.doff + (size_t)(t - c.tile0) * kTile * ld;
+  const int* __restrict__ cols = ao_of + (size_t)c.tile0 * kTile;
+  __shared__ int rows[kTile];
+  __shared__ float T[kTile][kTile + 1];
+  if (threadIdx.x < kTile) rows[threadIdx.x] = ao_of[(size_t)t * kTile + threadIdx.x];
+  for (int q = 0; q < c.ntl; ++q) {  // 32 x 32 sub-blocks, transposed through LDS so that both sides run along AOs
+    __syncthreads();
+    for (int e = threadIdx.x; e < kTile * kTile; e += 256) {
+      const int r = e & (kTile - 1), k = e >> 5, rr = rows[r], cc = cols[q * kTile + k];
+      T[r][k] = rr >= 0 && cc >= 0 ? (float)D[(size_t)cc * n + rr] : 0.f;
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e < kTile * kTile / 2; e += 256) {  // two columns per thread
+      const int r = e >> 4, k = 2 * (e & 15);
+      u16 h0, l0, h1, l1;
+      split_bf(T[r][k], h0, l0);
+      split_bf(T[r][k + 1], h1, l1);
+      const size_t o = (size_t)r * ld + q * kTile + k;
+      *reinterpret_cast<unsigned*>(out + o) = (unsigned)h0 | ((unsigned)h1 << 16);
+      *reinterpret_cast<unsigned*>(out + plane + o) = (unsigned)l0 | ((unsigned)l1 << 16);
+    }
+  }
 }
 
-void launch_split_d(hipStream_t s, int n, int npad, const double* D, const int* int2ref, unsigned short* Ds,
-                    float* R) {
-  const long tot = (long)npad * npad;
-  hipLaunchKernelGGL(k_split_d, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, s, n, npad, D, int2ref, Ds, R);
+void launch_split_d(hipStream_t s, int ntiles, int n, const double* D, const int* tile_chunk, const ChunkDev* chunks,
+                    const int* ao_of, unsigned short* Ds, float* R) {
+  const long n2 = (long)n * n;
+  const unsigned nb = (unsigned)(ntiles + (n2 + kRestBlock - 1) / kRestBlock);
+  hipLaunchKernelGGL(k_split_gather, dim3(nb), dim3(256), 0, s, n, D, tile_chunk, chunks, ao_of, Ds, ntiles, n2, R);
   CHX_HIP(hipGetLastError());
 }
 
@@ -214,14 +244,13 @@ __device__ __forceinline__ double block_sum_d(double v) {
 }
 
 __global__ __launch_bounds__(256) void k_finalize_corr(int n, int npad, const double* __restrict__ Mint,
-                                                       const int* __restrict__ ref2int, double* __restrict__ V,
-                                                       const float* __restrict__ R, double* __restrict__ cpart) {
+                                                       double* __restrict__ V, const float* __restrict__ R,
+                                                       double* __restrict__ cpart) {
   const long tot = (long)n * n;
   double acc = 0.0;
   for (long idx = (long)blockIdx.x * 256 + threadIdx.x; idx < tot; idx += (long)gridDim.x * 256) {
     const int col = (int)(idx / n), row = (int)(idx % n);
-    const int mu = ref2int[row], nu = ref2int[col];
-    const double v = Mint[(size_t)mu * npad + nu] + Mint[(size_t)nu * npad + mu];
+    const double v = Mint[(size_t)row * npad + col] + Mint[(size_t)col * npad + row];
     V[idx] = v;
     acc += v * (double)R[idx];
   }
@@ -229,9 +258,9 @@ __global__ __launch_bounds__(256) void k_finalize_corr(int n, int npad, const do
   if (threadIdx.x == 0) cpart[blockIdx.x] = acc;
 }
 
-void launch_finalize_corr(hipStream_t s, int n, int npad, const double* Mint, const int* ref2int, double* V,
-                          const float* R, double* cpart) {
-  hipLaunchKernelGGL(k_finalize_corr, dim3((unsigned)corr_blocks(n)), dim3(256), 0, s, n, npad, Mint, ref2int, V, R,
+void launch_finalize_corr(hipStream_t s, int n, int npad, const double* Mint, double* V, const float* R,
+                          double* cpart) {
+  hipLaunchKernelGGL(k_finalize_corr, dim3((unsigned)corr_blocks(n)), dim3(256), 0, s, n, npad, Mint, V, R,
                      cpart);
   CHX_HIP(hipGetLastError());
 }
@@ -437,9 +466,9 @@ struct DensEpi {
 };
 
 // ---------------------------------------------------------------------------
-// Density. Block = (batch, group of <= 4 alive tiles as output columns), 4
+// Density. Block = (batch, group of <= 4 tiles of its list as output columns), 4
 // waves in a 2 x 2 grid: wave (wr, wc) owns rows g = 32 wr..+31 and columns
-// 64 wc..+63 of X = Phi_b D_b (64 x 128). K loop over the batch's alive tiles
+// 64 wc..+63 of X = Phi_b D_b (64 x 128). K loop over the list's tiles
 // (32 AOs = one MFMA K step). A K step's operands (A: 64 points x 32 AOs, D:
 // 128 columns x 32 AOs, hi and lo) are 24 fragments of 1 KB that the waves'
 // DMA loads (global_load_lds_dwordx4: lane i -> bytes 16 i of the fragment)
@@ -463,7 +492,6 @@ struct DensMxSmem {
   };
   float red[kGroup][4][kBatch];
   double px[kBatch], py[kBatch], pz[kBatch];
-  int tl[kMxMaxTiles];  // the batch's alive tiles (K steps)
 };
 
 // MODE 0: A = phi; epilogue rho and grad rho / 2 (4 components into part).
@@ -488,9 +516,7 @@ __device__ __forceinline__ void density_mx_body(const MolDev& m, int r) {
   __shared__ DensMxSmem<P3> sm;
   const int grp = P3 ? m.core_grps[r] : (MODE == 0 && m.main_grps) ? m.main_grps[r] : r;
   const u16* __restrict__ cache = m.cache + (size_t)MODE * kMxT;
-  const u16* __restrict__ Ds = m.Ds;
   const size_t sstride = (size_t)m.sstride;
-  const int npad = m.npad;
   double* __restrict__ part = MODE == 0 ? m.part : m.part_tau + (MODE - 1) * kBatch;
   const BasisView bv = m.bv;  // descriptor fields in registers, read once
   const int tid = threadIdx.x, lane = tid & 63;
@@ -498,17 +524,14 @@ __device__ __forceinline__ void density_mx_body(const MolDev& m, int r) {
   const int lrow = lane & 15, lk = lane >> 4;
   const int wr = wave & 1, wc = wave >> 1;
   const int b = m.grp_batch[grp];
-  const int nt = m.grp_ntiles[grp];
-  int jt[kGroup];
-#pragma unroll
-  for (int q = 0; q < kGroup; ++q) jt[q] = m.grp_tiles[grp * kGroup + q];
-  const int it0 = m.bt_off[b], nk = m.bt_off[b + 1] - it0;  // the batch's slots it0.. are its K steps
+  const int nt = m.grp_ntiles[grp], j0 = m.grp_tile[grp];
+  const ChunkDev ch = m.chunks[m.b_chunk[b]];
+  const int it0 = m.bt_off[b], nk = ch.ntl, ld = nk * kTile;  // the batch's slots it0.. are its K steps
   if (tid < kBatch) {
     sm.px[tid] = m.bx[b * kBatch + tid];
     sm.py[tid] = m.by[b * kBatch + tid];
     sm.pz[tid] = m.bz[b * kBatch + tid];
   }
-  for (int j = tid; j < nk; j += 256) sm.tl[j] = m.bt_list[it0 + j];
   // The wave's fragments are f = wave + 4 j. A (j = 0, 1): row block f >> 1,
   // hl f & 1. D (j = 2..5, f' = f - 8): column block c = f' >> 1 (tile c >> 1,
   // half c & 1), hl f' & 1; columns past the group's tiles read a present
@@ -529,9 +552,9 @@ __device__ __forceinline__ void density_mx_body(const MolDev& m, int r) {
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const int f = wave + 4 * j, c = f >> 1, q = c >> 1;
-    const int t = q == 1 ? jt[1] : q == 2 ? jt[2] : q == 3 ? jt[3] : jt[0];
-    offb[j] = (f & 1) * npad * npad + ((q < nt ? t : jt[0]) * kTile + 16 * (c & 1) + drow) * npad + 8 * dch;
+    offb[j] = (f & 1) * ld * ld + ((j0 - ch.tile0 + (q < nt ? q : 0)) * kTile + 16 * (c & 1) + drow) * ld + 8 * dch;
   }
+  const u16* __restrict__ Ds = m.Ds + 2 * ch.doff;
   const u16* __restrict__ c3 = nullptr;
   if (P3) {
     // this batch's core slots in the side cache: [core slot][c][g][mu]
@@ -544,7 +567,7 @@ __device__ __forceinline__ void density_mx_body(const MolDev& m, int r) {
 #pragma unroll
     for (int j = 0; j < 2; ++j)
       __builtin_amdgcn_global_load_lds(a + offa[j], (lds_ptr)(sm.F + (wave + 4 * j) * kDxFrag), 16, 0, 0);
-    const int ti = sm.tl[k] * kTile;
+    const int ti = k * kTile;
 #pragma unroll
     for (int j = 0; j < 4; ++j)
       __builtin_amdgcn_global_load_lds(Ds + offb[j] + ti, (lds_ptr)(sm.F + (kDxA + wave + 4 * j) * kDxFrag), 16, 0, 0);
@@ -604,7 +627,7 @@ __device__ __forceinline__ void density_mx_body(const MolDev& m, int r) {
   __syncthreads();
   DensEpi<MODE> epi;
   if (wave < nt) {  // wave q = tile q of the group; lane = point
-    const int t = wave == 1 ? jt[1] : wave == 2 ? jt[2] : wave == 3 ? jt[3] : jt[0];
+    const int t = j0 + wave;
     epi.load(&sm.X[kTile * wave][lane]);
     walk_tile_f32<true>(bv, t, sm.px[lane], sm.py[lane], sm.pz[lane], epi);
   }
@@ -636,12 +659,11 @@ struct DensMxTauSmem {
   };
   float red[kGroup][3][kBatch];
   double px[kBatch], py[kBatch], pz[kBatch];
-  int tl[kMxMaxTiles];
 };
 
 template <int R>
 __device__ __forceinline__ void dens_tau_epilogue(DensMxTauSmem& sm, const f32x4 (&acc)[2][4], const BasisView& bv,
-                                                  const int (&jt)[kGroup], int nt, int wave, int lane, int wr,
+                                                  int j0, int nt, int wave, int lane, int wr,
                                                   int wc, int lrow, int lk) {
   __syncthreads();  // the previous user of the X area (fragments or X_{R-1}) is done
 #pragma unroll
@@ -653,7 +675,7 @@ __device__ __forceinline__ void dens_tau_epilogue(DensMxTauSmem& sm, const f32x4
   __syncthreads();
   DensEpi<R> epi;
   if (wave < nt) {
-    const int t = wave == 1 ? jt[1] : wave == 2 ? jt[2] : wave == 3 ? jt[3] : jt[0];
+    const int t = j0 + wave;
     epi.load(&sm.X[kTile * wave][lane]);
     walk_tile_f32<true>(bv, t, sm.px[lane], sm.py[lane], sm.pz[lane], epi);
   }
@@ -665,9 +687,7 @@ __global__ __launch_bounds__(256, 2) void k_density_mx_tau(MolDev m) {
   __shared__ DensMxTauSmem sm;
   const int grp = xcd_remap(blockIdx.x, gridDim.x);
   const u16* __restrict__ cache = m.cache + (size_t)kMxT;  // component 1 (d_x phi); d_y, d_z follow
-  const u16* __restrict__ Ds = m.Ds;
   const size_t sstride = (size_t)m.sstride;
-  const int npad = m.npad;
   double* __restrict__ part = m.part_tau;  // [group][3][64]
   const BasisView bv = m.bv;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -675,17 +695,14 @@ __global__ __launch_bounds__(256, 2) void k_density_mx_tau(MolDev m) {
   const int lrow = lane & 15, lk = lane >> 4;
   const int wr = wave & 1, wc = wave >> 1;
   const int b = m.grp_batch[grp];
-  const int nt = m.grp_ntiles[grp];
-  int jt[kGroup];
-#pragma unroll
-  for (int q = 0; q < kGroup; ++q) jt[q] = m.grp_tiles[grp * kGroup + q];
-  const int it0 = m.bt_off[b], nk = m.bt_off[b + 1] - it0;
+  const int nt = m.grp_ntiles[grp], j0 = m.grp_tile[grp];
+  const ChunkDev ch = m.chunks[m.b_chunk[b]];
+  const int it0 = m.bt_off[b], nk = ch.ntl, ld = nk * kTile;
   if (tid < kBatch) {
     sm.px[tid] = m.bx[b * kBatch + tid];
     sm.py[tid] = m.by[b * kBatch + tid];
     sm.pz[tid] = m.bz[b * kBatch + tid];
   }
-  for (int j = tid; j < nk; j += 256) sm.tl[j] = m.bt_list[it0 + j];
   const int drow = lane >> 2, dch = (lane & 3) ^ ((drow >> 2) & 3);
   const int fidx = 4 * lrow + (lk ^ ((lrow >> 2) & 3));
   int offa[2], offb[4];
@@ -697,9 +714,9 @@ __global__ __launch_bounds__(256, 2) void k_density_mx_tau(MolDev m) {
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const int f = wave + 4 * j, c = f >> 1, q = c >> 1;
-    const int t = q == 1 ? jt[1] : q == 2 ? jt[2] : q == 3 ? jt[3] : jt[0];
-    offb[j] = (f & 1) * npad * npad + ((q < nt ? t : jt[0]) * kTile + 16 * (c & 1) + drow) * npad + 8 * dch;
+    offb[j] = (f & 1) * ld * ld + ((j0 - ch.tile0 + (q < nt ? q : 0)) * kTile + 16 * (c & 1) + drow) * ld + 8 * dch;
   }
+  const u16* __restrict__ Ds = m.Ds + 2 * ch.doff;
   __syncthreads();
   auto dma = [&](int k) {
     const u16* a = cache + (size_t)(it0 + k) * sstride;
@@ -709,7 +726,7 @@ __global__ __launch_bounds__(256, 2) void k_density_mx_tau(MolDev m) {
       for (int j = 0; j < 2; ++j)
         __builtin_amdgcn_global_load_lds(a + (size_t)r * kMxT + offa[j],
                                          (lds_ptr)(sm.F + (r * kDxA + wave + 4 * j) * kDxFrag), 16, 0, 0);
-    const int ti = sm.tl[k] * kTile;
+    const int ti = k * kTile;
 #pragma unroll
     for (int j = 0; j < 4; ++j)
       __builtin_amdgcn_global_load_lds(Ds + offb[j] + ti, (lds_ptr)(sm.F + (3 * kDxA + wave + 4 * j) * kDxFrag), 16,
@@ -751,9 +768,9 @@ __global__ __launch_bounds__(256, 2) void k_density_mx_tau(MolDev m) {
             acc[d][r][c] = mfma3(a[d][r][0], a[d][r][1], bq[c][0], bq[c][1], acc[d][r][c]);
       }
   }
-  dens_tau_epilogue<1>(sm, acc[0], bv, jt, nt, wave, lane, wr, wc, lrow, lk);
-  dens_tau_epilogue<2>(sm, acc[1], bv, jt, nt, wave, lane, wr, wc, lrow, lk);
-  dens_tau_epilogue<3>(sm, acc[2], bv, jt, nt, wave, lane, wr, wc, lrow, lk);
+  dens_tau_epilogue<1>(sm, acc[0], bv, j0, nt, wave, lane, wr, wc, lrow, lk);
+  dens_tau_epilogue<2>(sm, acc[1], bv, j0, nt, wave, lane, wr, wc, lrow, lk);
+  dens_tau_epilogue<3>(sm, acc[2], bv, j0, nt, wave, lane, wr, wc, lrow, lk);
   __syncthreads();
   if (tid < 3 * kBatch) {
     const int c = tid / kBatch, g = tid % kBatch;
@@ -776,12 +793,11 @@ struct DensMxMggaSmem {
   };
   float red[kGroup][4][kBatch];
   double px[kBatch], py[kBatch], pz[kBatch];
-  int tl[kMxMaxTiles];
 };
 
 template <int R>
 __device__ __forceinline__ void dens_mgga_epilogue(DensMxMggaSmem& sm, const f32x4 (&acc)[2][4], const BasisView& bv,
-                                                   const int (&jt)[kGroup], int nt, int wave, int lane, int wr, int wc,
+                                                   int j0, int nt, int wave, int lane, int wr, int wc,
                                                    int lrow, int lk) {
   __syncthreads();  // the previous user of the X area is done
 #pragma unroll
@@ -793,7 +809,7 @@ __device__ __forceinline__ void dens_mgga_epilogue(DensMxMggaSmem& sm, const f32
   __syncthreads();
   DensEpi<R> epi;
   if (wave < nt) {
-    const int t = wave == 1 ? jt[1] : wave == 2 ? jt[2] : wave == 3 ? jt[3] : jt[0];
+    const int t = j0 + wave;
     epi.load(&sm.X[kTile * wave][lane]);
     walk_tile_f32<true>(bv, t, sm.px[lane], sm.py[lane], sm.pz[lane], epi);
   }
@@ -810,26 +826,21 @@ __global__ __launch_bounds__(256, 2) void k_density_mx_mgga(MolDev m) {
   __shared__ DensMxMggaSmem sm;
   const int grp = xcd_remap(blockIdx.x, gridDim.x);
   const u16* __restrict__ cache = m.cache;  // components 0 (phi), 1..3 (d_r phi)
-  const u16* __restrict__ Ds = m.Ds;
   const size_t sstride = (size_t)m.sstride;
-  const int npad = m.npad;
   const BasisView bv = m.bv;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lrow = lane & 15, lk = lane >> 4;
   const int wr = wave & 1, wc = wave >> 1;
   const int b = m.grp_batch[grp];
-  const int nt = m.grp_ntiles[grp];
-  int jt[kGroup];
-#pragma unroll
-  for (int q = 0; q < kGroup; ++q) jt[q] = m.grp_tiles[grp * kGroup + q];
-  const int it0 = m.bt_off[b], nk = m.bt_off[b + 1] - it0;
+  const int nt = m.grp_ntiles[grp], j0 = m.grp_tile[grp];
+  const ChunkDev ch = m.chunks[m.b_chunk[b]];
+  const int it0 = m.bt_off[b], nk = ch.ntl, ld = nk * kTile;
   if (tid < kBatch) {
     sm.px[tid] = m.bx[b * kBatch + tid];
     sm.py[tid] = m.by[b * kBatch + tid];
     sm.pz[tid] = m.bz[b * kBatch + tid];
   }
-  for (int j = tid; j < nk; j += 256) sm.tl[j] = m.bt_list[it0 + j];
   const int drow = lane >> 2, dch = (lane & 3) ^ ((drow >> 2) & 3);
   const int fidx = 4 * lrow + (lk ^ ((lrow >> 2) & 3));
   int offa[2], offb[4];
@@ -841,9 +852,9 @@ __global__ __launch_bounds__(256, 2) void k_density_mx_mgga(MolDev m) {
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const int f = wave + 4 * j, c = f >> 1, q = c >> 1;
-    const int t = q == 1 ? jt[1] : q == 2 ? jt[2] : q == 3 ? jt[3] : jt[0];
-    offb[j] = (f & 1) * npad * npad + ((q < nt ? t : jt[0]) * kTile + 16 * (c & 1) + drow) * npad + 8 * dch;
+    offb[j] = (f & 1) * ld * ld + ((j0 - ch.tile0 + (q < nt ? q : 0)) * kTile + 16 * (c & 1) + drow) * ld + 8 * dch;
   }
+  const u16* __restrict__ Ds = m.Ds + 2 * ch.doff;
   __syncthreads();
   auto dma = [&](int k) {
     const u16* a = cache + (size_t)(it0 + k) * sstride;
@@ -853,7 +864,7 @@ __global__ __launch_bounds__(256, 2) void k_density_mx_mgga(MolDev m) {
       for (int j = 0; j < 2; ++j)
         __builtin_amdgcn_global_load_lds(a + (size_t)r * kMxT + offa[j],
                                          (lds_ptr)(sm.F + (r * kDxA + wave + 4 * j) * kDxFrag), 16, 0, 0);
-    const int ti = sm.tl[k] * kTile;
+    const int ti = k * kTile;
 #pragma unroll
     for (int j = 0; j < 4; ++j)
       __builtin_amdgcn_global_load_lds(Ds + offb[j] + ti, (lds_ptr)(sm.F + (4 * kDxA + wave + 4 * j) * kDxFrag), 16,
@@ -895,7 +906,7 @@ __global__ __launch_bounds__(256, 2) void k_density_mx_mgga(MolDev m) {
             acc[d][r][c] = mfma3(a[d][r][0], a[d][r][1], bq[c][0], bq[c][1], acc[d][r][c]);
       }
   }
-  dens_mgga_epilogue<0>(sm, acc[0], bv, jt, nt, wave, lane, wr, wc, lrow, lk);
+  dens_mgga_epilogue<0>(sm, acc[0], bv, j0, nt, wave, lane, wr, wc, lrow, lk);
   __syncthreads();
   if (tid < 4 * kBatch) {
     const int c = tid / kBatch, g = tid % kBatch;
@@ -903,9 +914,9 @@ __global__ __launch_bounds__(256, 2) void k_density_mx_mgga(MolDev m) {
     for (int q = 0; q < nt; ++q) v += (double)sm.red[q][c][g];
     m.part[(size_t)grp * 4 * kBatch + c * kBatch + g] = v;
   }
-  dens_mgga_epilogue<1>(sm, acc[1], bv, jt, nt, wave, lane, wr, wc, lrow, lk);
-  dens_mgga_epilogue<2>(sm, acc[2], bv, jt, nt, wave, lane, wr, wc, lrow, lk);
-  dens_mgga_epilogue<3>(sm, acc[3], bv, jt, nt, wave, lane, wr, wc, lrow, lk);
+  dens_mgga_epilogue<1>(sm, acc[1], bv, j0, nt, wave, lane, wr, wc, lrow, lk);
+  dens_mgga_epilogue<2>(sm, acc[2], bv, j0, nt, wave, lane, wr, wc, lrow, lk);
+  dens_mgga_epilogue<3>(sm, acc[3], bv, j0, nt, wave, lane, wr, wc, lrow, lk);
   __syncthreads();
   if (tid < 3 * kBatch) {
     const int c = tid / kBatch, g = tid % kBatch;
@@ -1020,19 +1031,28 @@ __device__ __forceinline__ void make_b_slot(const MolDev& m, int slot, int g) {
       col0[c * kMxT + kTile * kBatch + col * kBatch] = 0;
     }
 }
+// The blocks past the slots clear M for the Vxc launch that follows.
+constexpr int kFillBlock = 4096;
 template <int NC>
 __global__ __launch_bounds__(NC == 4 ? 64 : 256) void k_make_b_mx(MolDev m) {
   constexpr int W = NC == 4 ? 1 : 4;  // waves per block
+  const int nsb = (m.nslots + W) / W;
+  if ((int)blockIdx.x >= nsb) {
+    const size_t n2 = (size_t)m.npad * m.npad, e0 = (size_t)(blockIdx.x - nsb) * kFillBlock;
+    for (size_t i = e0 + threadIdx.x; i < e0 + kFillBlock && i < n2; i += 64 * W) m.Mint[i] = 0.0;
+    return;
+  }
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   make_b_slot<NC>(m, blockIdx.x * W + wave, threadIdx.x & 63);
 }
 
 void launch_make_b_mx(hipStream_t s, int ncomp, const MolDev& one) {
   const int waves = one.nslots + 1;  // every slot and the all-zero slot
+  const int fill = (int)(((size_t)one.npad * one.npad + kFillBlock - 1) / kFillBlock);
   if (ncomp == 4)
-    hipLaunchKernelGGL((k_make_b_mx<4>), dim3(waves), dim3(64), 0, s, one);
+    hipLaunchKernelGGL((k_make_b_mx<4>), dim3(waves + fill), dim3(64), 0, s, one);
   else
-    hipLaunchKernelGGL((k_make_b_mx<1>), dim3((waves + 3) / 4), dim3(256), 0, s, one);
+    hipLaunchKernelGGL((k_make_b_mx<1>), dim3((waves + 3) / 4 + fill), dim3(256), 0, s, one);
   CHX_HIP(hipGetLastError());
 }
 
@@ -1052,24 +1072,20 @@ void launch_make_b_mx(hipStream_t s, int ncomp, const MolDev& one) {
 constexpr int kVxA = 16;  // Phi^T fragments per step: [row block (8)][hl]
 struct VxcMxSmem {
   u32x4 F[2 * kVxA * kDxFrag];  // one K step's fragments: Phi^T_I, then B^T_J
-  int sl[kMxMaxChunk][8];       // per batch of the item: slots of I's and J's tiles
 };
 
 template <int NC>
 __device__ __forceinline__ void vxc_mx_body(const MolDev& m, int item) {
   using lds_ptr = __attribute__((address_space(3))) void*;
   __shared__ VxcMxSmem sm;
-  const int4 wk = m.cwork[item];
-  const int I = wk.x, J = wk.y;
+  const VxcItem wk = m.cwork[item];
+  const int I = wk.I, J = wk.J;
   const u16* __restrict__ cache = m.cache + m.toff;
   const u16* __restrict__ bt = m.bt;
   const size_t sstride = (size_t)m.sstride;
   const int npad = m.npad;
   double* __restrict__ Mint = m.Mint;
-  {  // the item's slot table (absent tiles point at the all-zero slot)
-    const int* __restrict__ cs = m.cslot + (size_t)wk.z * 8;
-    for (int e = threadIdx.x; e < (wk.w - wk.z) * 8; e += 256) sm.sl[e >> 3][e & 7] = cs[e];
-  }
+  const int zero = m.nslots;  // the all-zero slot stands in for tiles past the chunk's last
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lrow = lane & 15, lk = lane >> 4;
@@ -1086,8 +1102,7 @@ __device__ __forceinline__ void vxc_mx_body(const MolDev& m, int item) {
     const int f = wave + 4 * j;
     off[j] = (f & 1) * (kTile * kBatch) + (16 * ((f >> 1) & 1) + drow) * kBatch + 8 * dch;
   }
-  __syncthreads();
-  const int nbat = wk.w - wk.z;                       // items hold >= 1 batch
+  const int nbat = wk.nbat;                           // items hold >= 1 batch
   const int ntau = (NC == 4 && I <= J) ? 6 * nbat : 0;  // tau steps, first
   const int nstage = ntau + 2 * nbat;
   // K step k -> (batch of the item, half of its points, component): tau steps
@@ -1101,8 +1116,9 @@ __device__ __forceinline__ void vxc_mx_body(const MolDev& m, int item) {
     }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const u16* pa = cache + (size_t)sm.sl[it][j] * sstride + c * kMxT + h * 32;
-      const u16* pb = bt + ((size_t)sm.sl[it][4 + j] * NC + c) * kMxT + h * 32;
+      const int s0 = wk.slot0 + it * wk.ntl, ta = I * kMxSup + j, tb = J * kMxSup + j;
+      const u16* pa = cache + (size_t)(ta < wk.ntl ? s0 + ta : zero) * sstride + c * kMxT + h * 32;
+      const u16* pb = bt + ((size_t)(tb < wk.ntl ? s0 + tb : zero) * NC + c) * kMxT + h * 32;
       __builtin_amdgcn_global_load_lds(pa + off[j], (lds_ptr)(sm.F + (wave + 4 * j) * kDxFrag), 16, 0, 0);
       __builtin_amdgcn_global_load_lds(pb + off[j], (lds_ptr)(sm.F + (kVxA + wave + 4 * j) * kDxFrag), 16, 0, 0);
     }
@@ -1137,16 +1153,25 @@ __device__ __forceinline__ void vxc_mx_body(const MolDev& m, int item) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) acc[r][c] = mfma3(a[r][0], a[r][1], bq[c][0], bq[c][1], acc[r][c]);
   }
+  const int nrow = wk.ntl * kTile;
+  const int* __restrict__ ao = m.ao_of + (size_t)wk.tile0 * kTile;
+  int nu[4];
+#pragma unroll
+  for (int cb = 0; cb < 4; ++cb) {
+    const int lc = J * kMxSup * kTile + 64 * wc + 16 * cb + lrow;
+    nu[cb] = lc < nrow ? ao[lc] : -1;
+  }
 #pragma unroll
   for (int r = 0; r < 4; ++r)
 #pragma unroll
-    for (int cb = 0; cb < 4; ++cb)
+    for (int i = 0; i < 4; ++i) {
+      const int lr = I * kMxSup * kTile + 64 * wr + 16 * r + 4 * lk + i;
+      const int mu = lr < nrow ? ao[lr] : -1;
+      if (mu < 0) continue;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int mu = I * kMxSup * kTile + 64 * wr + 16 * r + 4 * lk + i;
-        const int nu = J * kMxSup * kTile + 64 * wc + 16 * cb + lrow;
-        unsafeAtomicAdd(&Mint[(size_t)mu * npad + nu], (double)acc[r][cb][i]);
-      }
+      for (int cb = 0; cb < 4; ++cb)
+        if (nu[cb] >= 0) unsafeAtomicAdd(&Mint[(size_t)mu * npad + nu[cb]], (double)acc[r][cb][i]);
+    }
 }
 template <int NC>
 __global__ __launch_bounds__(256, 3) void k_vxc_mx(MolDev m) {
@@ -1154,8 +1179,7 @@ __global__ __launch_bounds__(256, 3) void k_vxc_mx(MolDev m) {
 }
 
 // Vxc for large bases: M_IJ += Phi_I^T B_J over 256 x 256 blocks whose rows
-// and columns are groups of 8 tiles of a batch chunk's alive-tile union, so
-// every operand byte staged in LDS feeds twice the MFMAs of the 128 x 128
+// and columns are groups of 8 of a chunk's tiles, so every operand byte staged in LDS feeds twice the MFMAs of the 128 x 128
 // kernel (64 instead of 32 FLOP per byte). An item is a pair of groups I <= J
 // of one chunk and covers both blocks: first M_IJ (the tau part, symmetric,
 // taken twice for I < J and once for I = J, then the phi part), then for
@@ -1165,18 +1189,14 @@ __global__ __launch_bounds__(256, 3) void k_vxc_mx(MolDev m) {
 // row group and B^T of the column group, 256 rows each, hi and lo, 64
 // fragments of 1 KB brought in by the waves' DMA (same coalesced lane order
 // and swizzle). 8 waves in a 2 x 4 grid, each owning a 128 x 64 block (up to
-// 96 MFMAs per step). Per batch a 16-bit mask (I's 8 tiles, then J's) marks
-// the tiles alive in it: a dead tile's fragments are not loaded and the
-// products that involve it are skipped, so the MFMAs follow each batch's
-// screening.
+// 96 MFMAs per step). A 16-bit mask (I's 8 tiles, then J's) marks the tiles
+// the chunk has: an absent tile's fragments are not loaded and the products
+// that involve it are skipped.
 constexpr int kMxSupW = 8;   // tiles per group (256 AOs)
 constexpr int kVxAW = 32;    // Phi^T fragments per step: [row block (16)][hl]
 constexpr int kVxWStep = 2 * kVxAW * kDxFrag;  // u32x4 per K step: Phi^T of the row group, then B^T of the column group
 struct VxcMxWideSmem {
   u32x4 F[2 * kVxWStep];  // two K steps' fragments: step k in buffer k & 1
-  int sl[kMxMaxChunk][16];       // per batch: slots of I's 8 tiles, then J's
-  unsigned mk[kMxMaxChunk];      // per batch: alive bits of those 16 tiles
-  int tile[16];                  // I's tiles, then J's (-1: padding)
 };
 
 // Two LDS buffers and one barrier per K step: after it, step k's fragments
@@ -1188,34 +1208,16 @@ template <int NC>
 __device__ __forceinline__ void vxc_mx_wide_body(const MolDev& m, int item) {
   using lds_ptr = __attribute__((address_space(3))) void*;
   __shared__ VxcMxWideSmem sm;
-  const int4 wk = m.cwork[item];
-  const int I = wk.x, J = wk.y;    // I <= J
-  const int4 ch = m.vchunk[wk.z];  // (table offset, batches, table width, tile-list offset)
-  const int nbat = ch.y;
-  const int zero = m.nslots;       // the all-zero slot: tile not alive in that batch
+  const VxcItem wk = m.cwork[item];
+  const int I = wk.I, J = wk.J;    // I <= J
+  const int nbat = wk.nbat;
   const u16* __restrict__ cache = m.cache + m.toff;
   const u16* __restrict__ bt = m.bt;
   const size_t sstride = (size_t)m.sstride;
   const int npad = m.npad;
   double* __restrict__ Mint = m.Mint;
-  {
-    const int* __restrict__ tab = m.vtab + ch.x;
-    for (int e = threadIdx.x; e < nbat * 16; e += 512) {
-      const int it = e >> 4, t = e & 15;
-      sm.sl[it][t] = tab[(size_t)it * ch.z + (t < 8 ? I * kMxSupW + t : J * kMxSupW + t - 8)];
-    }
-    if (threadIdx.x < 16) {
-      const int t = threadIdx.x;
-      sm.tile[t] = m.vtile[ch.w + (t < 8 ? I * kMxSupW + t : J * kMxSupW + t - 8)];
-    }
-  }
-  __syncthreads();
-  for (int it = threadIdx.x; it < nbat; it += 512) {
-    unsigned b = 0;
-#pragma unroll
-    for (int t = 0; t < 16; ++t) b |= (sm.sl[it][t] != zero ? 1u : 0u) << t;
-    sm.mk[it] = b;
-  }
+  const int nI = min(kMxSupW, wk.ntl - I * kMxSupW), nJ = min(kMxSupW, wk.ntl - J * kMxSupW);
+  const unsigned mk = ((1u << nI) - 1u) | (((1u << nJ) - 1u) << 8);
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lrow = lane & 15, lk = lane >> 4;
@@ -1227,7 +1229,6 @@ __device__ __forceinline__ void vxc_mx_wide_body(const MolDev& m, int item) {
   const int fidx = 4 * lrow + (lk ^ ((lrow >> 2) & 3));
   const int off = (wave & 1) * (kTile * kBatch) + (16 * ((wave >> 1) & 1) + drow) * kBatch + 8 * dch;
   const int t0 = wave >> 2;
-  __syncthreads();
   const int ntau = NC == 4 ? 6 * nbat : 0;  // tau steps of M_IJ, first
   const int kmirror = ntau + 2 * nbat;      // first step of M_JI (I < J)
   const int nstage = kmirror + (I < J ? 2 * nbat : 0);
@@ -1247,17 +1248,17 @@ __device__ __forceinline__ void vxc_mx_wide_body(const MolDev& m, int item) {
     bool mir;
     decode(k, it, h, c, mir);
     const int ra = mir ? 8 : 0, cb = mir ? 0 : 8;  // table columns of the row and column groups
-    const unsigned mk = __builtin_amdgcn_readfirstlane(sm.mk[it]);
+    const int s0 = wk.slot0 + it * wk.ntl, sa = s0 + (mir ? J : I) * kMxSupW, sb = s0 + (mir ? I : J) * kMxSupW;
     u32x4* F = sm.F + buf * kVxWStep;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int t = t0 + 2 * j;
       if ((mk >> (ra + t)) & 1u) {
-        const u16* pa = cache + (size_t)sm.sl[it][ra + t] * sstride + c * kMxT + h * 32;
+        const u16* pa = cache + (size_t)(sa + t) * sstride + c * kMxT + h * 32;
         __builtin_amdgcn_global_load_lds(pa + off, (lds_ptr)(F + (wave + 8 * j) * kDxFrag), 16, 0, 0);
       }
       if ((mk >> (cb + t)) & 1u) {
-        const u16* pb = bt + ((size_t)sm.sl[it][cb + t] * NC + c) * kMxT + h * 32;
+        const u16* pb = bt + ((size_t)(sb + t) * NC + c) * kMxT + h * 32;
         __builtin_amdgcn_global_load_lds(pb + off, (lds_ptr)(F + (kVxAW + wave + 8 * j) * kDxFrag), 16, 0, 0);
       }
     }
@@ -1267,25 +1268,27 @@ __device__ __forceinline__ void vxc_mx_wide_body(const MolDev& m, int item) {
   for (int r = 0; r < 8; ++r)
 #pragma unroll
     for (int c = 0; c < 4; ++c) acc[r][c] = f32x4{0.f, 0.f, 0.f, 0.f};
-  // one FP64 atomic add per element of the wave's 128 x 64 block; rows from
-  // table columns ro.., columns from co..
+  // one FP64 atomic add per element of the wave's 128 x 64 block of the chunk's rows ro.. and columns co..
+  const int nrow = wk.ntl * kTile;
+  const int* __restrict__ ao = m.ao_of + (size_t)wk.tile0 * kTile;
   auto flush = [&](int ro, int co) {
+    int nu[4];
 #pragma unroll
-    for (int r = 0; r < 8; ++r) {
-      const int ti = sm.tile[ro + 4 * wr + (r >> 1)];
-      if (ti < 0) continue;
-#pragma unroll
-      for (int cb = 0; cb < 4; ++cb) {
-        const int tj = sm.tile[co + 2 * wc + (cb >> 1)];
-        if (tj < 0) continue;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int mu = ti * kTile + 16 * (r & 1) + 4 * lk + i;
-          const int nu = tj * kTile + 16 * (cb & 1) + lrow;
-          unsafeAtomicAdd(&Mint[(size_t)mu * npad + nu], (double)acc[r][cb][i]);
-        }
-      }
+    for (int cb = 0; cb < 4; ++cb) {
+      const int lc = co * kMxSupW * kTile + 64 * wc + 16 * cb + lrow;
+      nu[cb] = lc < nrow ? ao[lc] : -1;
     }
+#pragma unroll
+    for (int r = 0; r < 8; ++r)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int lr = ro * kMxSupW * kTile + 128 * wr + 16 * r + 4 * lk + i;
+        const int mu = lr < nrow ? ao[lr] : -1;
+        if (mu < 0) continue;
+#pragma unroll
+        for (int cb = 0; cb < 4; ++cb)
+          if (nu[cb] >= 0) unsafeAtomicAdd(&Mint[(size_t)mu * npad + nu[cb]], (double)acc[r][cb][i]);
+      }
   };
   dma(0, 0);
   for (int k = 0; k < nstage; ++k) {
@@ -1296,7 +1299,7 @@ __device__ __forceinline__ void vxc_mx_wide_body(const MolDev& m, int item) {
         for (int c = 0; c < 4; ++c) acc[r][c] *= 2.f;
     }
     if (k == kmirror) {  // M_IJ done: write it and start M_JI
-      flush(0, 8);
+      flush(I, J);
 #pragma unroll
       for (int r = 0; r < 8; ++r)
 #pragma unroll
@@ -1305,8 +1308,7 @@ __device__ __forceinline__ void vxc_mx_wide_body(const MolDev& m, int item) {
     int it, h, c;
     bool mir;
     decode(k, it, h, c, mir);
-    // this wave's row tiles 4 wr..4 wr+3 (bits of rmk) and column tiles 2 wc, 2 wc+1 (cmk) alive in the batch
-    const unsigned mk = __builtin_amdgcn_readfirstlane(sm.mk[it]);
+    // this wave's row tiles 4 wr..4 wr+3 (bits of rmk) and column tiles 2 wc, 2 wc+1 (cmk) in the list
     const unsigned rmk = (mk >> ((mir ? 8 : 0) + 4 * wr)) & 15u, cmk = (mk >> ((mir ? 0 : 8) + 2 * wc)) & 3u;
     __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this wave's fragments of step k are in LDS
     __syncthreads();                     // ... and every other wave's, and step k - 1's buffer is read
@@ -1329,8 +1331,8 @@ __device__ __forceinline__ void vxc_mx_wide_body(const MolDev& m, int item) {
           if ((rmk >> (r >> 1)) & 1u) acc[r][cc] = mfma3(a[r][0], a[r][1], bq[cc][0], bq[cc][1], acc[r][cc]);
       }
   }
-  if (I < J) flush(8, 0);
-  else flush(0, 8);
+  if (I < J) flush(J, I);
+  else flush(I, I);
 }
 template <int NC>
 __global__ __launch_bounds__(512, 1) void k_vxc_mx_wide(MolDev m) {
@@ -1354,8 +1356,9 @@ __device__ __forceinline__ T* rb(const char* base, T* off) {
 }
 __device__ __forceinline__ MolDev rebase(const char* base, const MolDev& o) {
   MolDev m = o;
-  m.grp_batch = rb(base, o.grp_batch); m.grp_tiles = rb(base, o.grp_tiles); m.grp_ntiles = rb(base, o.grp_ntiles);
-  m.bt_off = rb(base, o.bt_off); m.bt_list = rb(base, o.bt_list);
+  m.grp_batch = rb(base, o.grp_batch); m.grp_tile = rb(base, o.grp_tile); m.grp_ntiles = rb(base, o.grp_ntiles);
+  m.bt_off = rb(base, o.bt_off);
+  m.b_chunk = rb(base, o.b_chunk); m.chunks = rb(base, o.chunks); m.ao_of = rb(base, o.ao_of);
   m.bx = rb(base, o.bx); m.by = rb(base, o.by); m.bz = rb(base, o.bz);
   m.bv.sh_xyz = rb(base, o.bv.sh_xyz); m.bv.sh_type = rb(base, o.bv.sh_type);
   m.bv.sh_nprim = rb(base, o.bv.sh_nprim); m.bv.sh_poff = rb(base, o.bv.sh_poff);
@@ -1366,9 +1369,7 @@ __device__ __forceinline__ MolDev rebase(const char* base, const MolDev& o) {
   m.part = rb(base, o.part); m.part_tau = rb(base, o.part_tau);
   m.slot_batch = rb(base, o.slot_batch); m.slot_tile = rb(base, o.slot_tile);
   m.coef = rb(base, o.coef); m.bt = rb(base, o.bt);
-  m.cwork = rb(base, o.cwork); m.pair_batches = rb(base, o.pair_batches); m.slot_of = rb(base, o.slot_of);
-  m.cslot = rb(base, o.cslot); m.Mint = rb(base, o.Mint);
-  m.vchunk = rb(base, o.vchunk); m.vtab = rb(base, o.vtab); m.vtile = rb(base, o.vtile);
+  m.cwork = rb(base, o.cwork); m.Mint = rb(base, o.Mint);
   m.cache3 = rb(base, o.cache3);
   m.core_off = rb(base, o.core_off); m.core_grps = rb(base, o.core_grps); m.main_grps = rb(base, o.main_grps);
   return m;

@@ -176,12 +176,12 @@ void build_persistent(chx_pack* p) {
   // every pointer field of a descriptor (the fields rebase() offsets), read and
   // written as addresses through memcpy
   auto fields = [](MolDev& d) {
-    return std::array<void*, 38>{
-        &d.grp_batch, &d.grp_tiles, &d.grp_ntiles, &d.bt_off, &d.bt_list, &d.bx, &d.by, &d.bz,
+    return std::array<void*, 34>{
+        &d.grp_batch, &d.grp_tile, &d.grp_ntiles, &d.bt_off, &d.b_chunk, &d.chunks, &d.ao_of, &d.bx, &d.by, &d.bz,
         &d.bv.sh_xyz, &d.bv.sh_type, &d.bv.sh_nprim, &d.bv.sh_poff, &d.bv.p_exp, &d.bv.p_coef,
         &d.bv.tile_seg_off, &d.bv.seg, &d.bv.segrec, &d.bv.sh_atom, &d.cache, &d.Ds, &d.part, &d.part_tau,
-        &d.slot_batch, &d.slot_tile, &d.coef, &d.bt, &d.cwork, &d.pair_batches, &d.slot_of, &d.cslot, &d.Mint,
-        &d.vchunk, &d.vtab, &d.vtile, &d.cache3, &d.core_off, &d.core_grps, &d.main_grps};
+        &d.slot_batch, &d.slot_tile, &d.coef, &d.bt, &d.cwork, &d.Mint, &d.cache3, &d.core_off, &d.core_grps,
+        &d.main_grps};
   };
   auto get = [](void* f) {
     uintptr_t v;
@@ -208,7 +208,7 @@ void build_persistent(chx_pack* p) {
   for (int m = 0; m < n; ++m) {
     const chx_grid* g = p->grids[m];
     const int ng = (int)g->grp_batch.size(), ncg = (int)g->core_grps.size(), nw = (int)g->cwork.size();
-    const int cnt[5] = {ng - ncg, ncg, (int)g->bt_list.size() + 1, g->mx_wide ? 0 : nw, g->mx_wide ? nw : 0};
+    const int cnt[5] = {ng - ncg, ncg, (int)g->slot_tile.size() + 1, g->mx_wide ? 0 : nw, g->mx_wide ? nw : 0};
     for (int st = 0; st < 5; ++st) starts[(size_t)st * (n + 1) + m + 1] = starts[(size_t)st * (n + 1) + m] + cnt[st];
   }
   for (int st = 0; st < 5; ++st) p->totals[st] = starts[(size_t)st * (n + 1) + n];
@@ -282,7 +282,7 @@ void build_lanes(chx_pack* p) {
   }
 }
 
-// The molecules of a lane on stream s: split D and clear M first; the density
+// The molecules of a lane on stream s: split D first; the density
 // launches wait for `after` (if set) and signal `dens_done` (if set); then the
 // functional and E/N sums of all the lane's molecules in one launch each, per
 // molecule B^T, Vxc and V = M + M^T (with the partial sums of V . (D - hi -
@@ -298,7 +298,8 @@ void enqueue_lane_stages(chx_pack* p, int lane, hipStream_t s, hipEvent_t after,
   const int m0 = p->cut[lane], m1 = p->cut[lane + 1], nl = m1 - m0;
   for (int m = m0; m < m1; ++m) {
     chx_grid* g = p->grids[m];
-    launch_split_d(s, g->nbasis, g->npad, D[m], g->d_int2ref.p, g->d_Dsplit.p, g->d_Dres.p);
+    launch_split_d(s, (int)g->tile_chunk.size(), g->nbasis, D[m], g->d_tile_chunk.p, g->d_chunks.p, g->d_ao_of.p,
+                   g->d_Dsplit.p, g->d_Dres.p);
     launch_fill(s, g->d_Mint.p, (size_t)g->npad * g->npad, 0.0);
   }
   if (after) CHX_HIP(hipStreamWaitEvent(s, after, 0));
@@ -316,7 +317,7 @@ void enqueue_lane_stages(chx_pack* p, int lane, hipStream_t s, hipEvent_t after,
   stage(kStageVxcWide);
   for (int m = m0; m < m1; ++m) {
     chx_grid* g = p->grids[m];
-    launch_finalize_corr(s, g->nbasis, g->npad, g->d_Mint.p, g->d_ref2int.p, V[m], g->d_Dres.p, g->d_cpart.p);
+    launch_finalize_corr(s, g->nbasis, g->npad, g->d_Mint.p, V[m], g->d_Dres.p, g->d_cpart.p);
   }
   launch_corr_multi(s, p->fn_base[lane], p->fn_tab.p + p->fn_off[lane], nl, p->d_en.p);
 }
@@ -330,8 +331,8 @@ void enqueue_lane(chx_pack* p, int lane, hipStream_t s, hipEvent_t after, hipEve
   const int m0 = p->cut[lane], m1 = p->cut[lane + 1];
   for (int m = m0; m < m1; ++m) {
     chx_grid* g = p->grids[m];
-    launch_split_d(s, g->nbasis, g->npad, D[m], g->d_int2ref.p, g->d_Dsplit.p, g->d_Dres.p);
-    launch_fill(s, g->d_Mint.p, (size_t)g->npad * g->npad, 0.0);
+    launch_split_d(s, (int)g->tile_chunk.size(), g->nbasis, D[m], g->d_tile_chunk.p, g->d_chunks.p, g->d_ao_of.p,
+                   g->d_Dsplit.p, g->d_Dres.p);
   }
   if (after) CHX_HIP(hipStreamWaitEvent(s, after, 0));
   for (int m = m0; m < m1; ++m) {
@@ -353,7 +354,7 @@ void enqueue_lane(chx_pack* p, int lane, hipStream_t s, hipEvent_t after, hipEve
       launch_vxc_mx_wide(s, nc, (int)g->cwork.size(), g->hmol);
     else
       launch_vxc_mx(s, nc, (int)g->cwork.size(), g->hmol);
-    launch_finalize_corr(s, g->nbasis, g->npad, g->d_Mint.p, g->d_ref2int.p, V[m], g->d_Dres.p, g->d_cpart.p);
+    launch_finalize_corr(s, g->nbasis, g->npad, g->d_Mint.p, V[m], g->d_Dres.p, g->d_cpart.p);
   }
   launch_corr_multi(s, p->fn_base[lane], p->fn_tab.p + p->fn_off[lane], m1 - m0, p->d_en.p);
 }
@@ -368,7 +369,8 @@ void enqueue_persistent(chx_pack* p, const double* const* D, double* const* V) {
   hipStream_t s = p->stream;
   for (int m = 0; m < n; ++m) {
     chx_grid* g = p->grids[m];
-    launch_split_d(s, g->nbasis, g->npad, D[m], g->d_int2ref.p, g->d_Dsplit.p, g->d_Dres.p);
+    launch_split_d(s, (int)g->tile_chunk.size(), g->nbasis, D[m], g->d_tile_chunk.p, g->d_chunks.p, g->d_ao_of.p,
+                   g->d_Dsplit.p, g->d_Dres.p);
     launch_fill(s, g->d_Mint.p, (size_t)g->npad * g->npad, 0.0);
   }
   const int* st = p->d_starts.p;
@@ -384,7 +386,7 @@ void enqueue_persistent(chx_pack* p, const double* const* D, double* const* V) {
   stage(kStageVxcWide);
   for (int m = 0; m < n; ++m) {
     chx_grid* g = p->grids[m];
-    launch_finalize_corr(s, g->nbasis, g->npad, g->d_Mint.p, g->d_ref2int.p, V[m], g->d_Dres.p, g->d_cpart.p);
+    launch_finalize_corr(s, g->nbasis, g->npad, g->d_Mint.p, V[m], g->d_Dres.p, g->d_cpart.p);
   }
   launch_corr_multi(s, p->fn_all_base, p->fn_all.p, n, p->d_en.p);
 }
@@ -542,7 +544,7 @@ int chx_pack_autotune(chx_pack* p, const chx_xc* xc, const double* const* D_dev,
       }
     }
     for (chx_grid* g : p->grids) set_vxc_chunk(g, cand[best]);
-    // then the Vxc tile shape per molecule, by a basis-size threshold: 256-AO union groups for
+    // then the Vxc tile shape per molecule, by a basis-size threshold: 256-AO groups for
     // npad >= T, 128-AO super-tiles below (T = 0: all groups; -1: none)
     static const int thr[] = {-1, 1024, 512, 0};
     int best_thr = -1;

@@ -209,9 +209,11 @@ int chx_grid_core_batches(const chx_grid* g, long* n);
  * over those batches, the (rho, grad rho) contraction); the LDA/GGA density
  * launch does the rest of that stage's work */
 int chx_grid_core_flops(const chx_grid* g, double* flops);
-/* AO screening threshold: an AO tile is dropped from a batch when every |phi|
- * and |grad phi| in it stays at or below the threshold at every point of the
- * batch. Takes effect at the next chx_grid_get_ao. Default 1e-14. */
+/* AO screening threshold: a shell is left out of a batch only when bounds on
+ * its |phi| and |d phi| stay at or below the threshold at every point of the
+ * batch. Neighbouring batches share one AO list (the union of theirs), so a
+ * batch may also carry shells that only its neighbours need. Takes effect at
+ * the next chx_grid_get_ao. Default 1e-14. */
 int chx_grid_set_screening(chx_grid* g, double threshold);
 /* Autotuner (no reference counterpart): times `reps` XC builds (D_dev ->
  * V_dev, device pointers, column-major nbasis^2) for each Vxc work-item
@@ -220,13 +222,12 @@ int chx_grid_set_screening(chx_grid* g, double threshold);
 int chx_grid_autotune(chx_grid* g, const chx_xc* xc, const double* D_dev, double* V_dev, int reps, int* chunk_out,
                       float* ms_out);
 /* Mixed form's Vxc block shape (no reference counterpart): 0 = 128 x 128
- * blocks over 128-AO super-tile pairs and the batches where both are alive;
- * 1 = 256 x 256 blocks whose rows and columns are groups of 8 tiles of each
- * batch chunk's alive-tile union, dead tiles skipped per batch; -1 (default)
- * = 1 from npad 1024 on, else 0. chx_grid_vxc_shape reports the shape in use. */
+ * blocks, 1 = 256 x 256 blocks of each batch chunk's AO list; -1 (default) = 1
+ * from npad 1024 on, else 0. chx_grid_vxc_shape reports the shape in use. */
 int chx_grid_set_vxc_shape(chx_grid* g, int shape);
-/* Vxc work-item length in batches (0: the form's default, at most 128); the
- * autotuners set it from their timings. */
+/* Vxc work-item length in batches (0: by the number of items, at most 128; an
+ * item ends with its chunk of at most 32 batches); the autotuners set it from
+ * their timings. */
 int chx_grid_set_vxc_chunk(chx_grid* g, int chunk);
 int chx_grid_vxc_shape(const chx_grid* g, int* shape);
 /* chx_grid_autotune over both shapes (mixed form): times the four work
@@ -234,8 +235,9 @@ int chx_grid_vxc_shape(const chx_grid* g, int* shape);
  * ms_out[8] = [shape][length]. */
 int chx_grid_autotune_tiles(chx_grid* g, const chx_xc* xc, const double* D_dev, double* V_dev, int reps,
                             int* shape_out, int* chunk_out, float* ms_out);
-/* Statistics of the batch layout: batches, points, AO tiles per batch (mean),
- * algorithmic FLOPs of one XC build (dense-contraction count, k*2*sum g_b n_b^2). */
+/* Statistics of the batch layout: batches, points, 32-AO tiles per batch (mean),
+ * algorithmic FLOPs of one XC build (dense-contraction count, k*2*sum g_b n_b^2,
+ * n_b the AOs of the batch's list). */
 int chx_grid_stats(const chx_grid* g, long* nbatches, long* npoints, double* mean_tiles, double* flops_per_build);
 
 /* AO tables in HBM (no reference counterpart; the reference caches its own,

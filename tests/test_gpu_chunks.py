@@ -1,0 +1,83 @@
+"""AO lists of batch chunks (shell-level screening, dense blocks gathered from D, M scattered back)
+at the sizes where the packing can go wrong: one AO, less than a tile, one tile exactly, shells that
+straddle tiles, many chunks whose lists differ, and every Vxc run length."""
+import numpy as np
+import pytest
+
+import chinium_amd as ca
+import oracle_lib as ol
+from chinium_amd import workloads as wl
+
+pytestmark = pytest.mark.gpu
+
+
+def _system(name):
+    if name == "H":  # one s function; two electrons' worth of density in it
+        Z, X, basis, nocc = [1], [[0.0, 0.0, 0.0]], "sto-3g", 1
+    elif name == "water sto-3g":  # 7 AOs
+        Z, X = wl.water_monomer_angstrom()
+        basis, nocc = "sto-3g", 5
+    elif name == "far hydrogens":  # 64 s functions, one or two alive in most batches
+        Z, X, basis, nocc = [1] * 64, [[6.0 * (k % 8), 6.0 * (k // 8), 0.0] for k in range(64)], "sto-3g", 32
+    else:  # C12 chain, 298 AOs: lists from 60 to 298 AOs, d shells across tile borders
+        Z, X = wl.alkane_angstrom(12, 3)
+        basis, nocc = "def2-svp", 49
+    mol = ca.Molecule(np.array(Z), np.array(X, float) * ca.ANGSTROM_TO_BOHR, basis)
+    D, _ = wl.workload_density(mol, nocc, 11)
+    return mol, basis, D
+
+
+def _grid(mol, family, form, cache=-1, thr=None, run=0):
+    g = ca.Grid(mol, "SG-1", 1, 0)
+    g.setPrecision(form)
+    g.setAOCache(cache)
+    if thr is not None:
+        g.setScreening(thr)
+    g.setType(family)
+    g.setVxcChunk(run)
+    g.getAO(0, 0)
+    return g
+
+
+@pytest.mark.parametrize("func", ["PBE", "R2SCAN"])
+@pytest.mark.parametrize("name", ["H", "water sto-3g", "far hydrogens", "C12"])
+def test_chunk_lists(name, func):
+    print("chunk lists: %s %s" % (name, func), flush=True)
+    mol, basis, D = _system(name)
+    xc = ca.ExchangeCorrelation()
+    xc.Read(func)
+    fam = xc.family
+    E, V = ca.xc_build(_grid(mol, fam, ca.CHX_PREC_FP64), xc, D)
+    orc = ol.OracleSystem(mol.Z, mol.xyz, "SG-1", basis)
+    orc.set_functional(func)
+    orc.get_ao()
+    Eo, _, Vo = orc.xc(D)
+    assert abs(E - Eo) <= 1e-10 and np.abs(V - Vo).max() <= 1e-9
+    scale = max(1.0, np.abs(V).max())
+    # every list held in full: what the default threshold drops is below it in every factor
+    for form, cache in ((ca.CHX_PREC_FP64, 1), (ca.CHX_PREC_FP64, 0)):
+        E0, V0 = ca.xc_build(_grid(mol, fam, form, cache, thr=0.0), xc, D)
+        assert abs(E0 - E) <= 1e-11 and np.abs(V0 - V).max() <= 1e-11 * scale
+    # other run lengths sum in another order only
+    for run in (1, 5, 128):
+        E1, V1 = ca.xc_build(_grid(mol, fam, ca.CHX_PREC_FP64, 1, run=run), xc, D)
+        assert abs(E1 - E) <= 1e-11 and np.abs(V1 - V).max() <= 1e-12 * scale
+    # mixed form, both block shapes: 16 significant bits per operand
+    for shape in (0, 1):
+        g = _grid(mol, fam, ca.CHX_PREC_MIXED)
+        g.setVxcShape(shape)
+        Em, Vm = ca.xc_build(g, xc, D)
+        assert abs(Em - E) <= 1e-5 * len(mol.Z) and np.abs(Vm - V).max() <= 5e-5 * scale
+
+
+def test_coarse_threshold_moves_little():
+    """A shell below 1e-6 adds less than 1e-6 times the integral of |v| over the points it leaves."""
+    mol, _, D = _system("C12")
+    xc = ca.ExchangeCorrelation()
+    xc.Read("PBE")
+    E, V = ca.xc_build(_grid(mol, 1, ca.CHX_PREC_FP64), xc, D)
+    g = _grid(mol, 1, ca.CHX_PREC_FP64, thr=1e-6)
+    full = _grid(mol, 1, ca.CHX_PREC_FP64, thr=0.0)
+    assert g.stats()["mean_tiles"] < full.stats()["mean_tiles"]
+    E6, V6 = ca.xc_build(g, xc, D)
+    assert abs(E6 - E) <= 1e-4 and np.abs(V6 - V).max() <= 1e-4
