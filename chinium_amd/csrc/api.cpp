@@ -207,18 +207,12 @@ void fock_to_device(chx_grid* g, double* dV, int spin = 0) {
     launch_make_b_mx(g->stream, nc, g->hmol);
     g->mark_end(kStMakeB, e);
     g->mark_begin(kStVxc, &e);
-    if (g->mx_wide)
-      launch_vxc_mx_wide(g->stream, nc, (int)g->cwork.size(), g->hmol);
-    else
-      launch_vxc_mx(g->stream, nc, (int)g->cwork.size(), g->hmol);
+    launch_vxc_mx(g->stream, nc, g->mx_wide, (int)g->mwork.size(), g->hmol);
     g->mark_end(kStVxc, e);
     g->mark_begin(kStFinalize, &e);
-    if (g->corr_pending)
-      launch_finalize_corr(g->stream, g->nbasis, g->npad, g->d_Mint.p, dV,
-                           g->d_Dres.p + (size_t)spin * g->nbasis * g->nbasis,
-                           g->d_cpart.p + (size_t)spin * corr_blocks(g->nbasis));
-    else
-      launch_finalize_sym(g->stream, g->nbasis, g->npad, g->d_Mint.p, dV);
+    launch_assemble_mx(g->stream, g->nbasis, g->d_rowptr.p, g->d_rows.p, g->d_ao_of.p, g->d_U.p, dV,
+                       g->corr_pending ? g->d_Dres.p + (size_t)spin * g->nbasis * g->nbasis : nullptr,
+                       g->d_cpart.p + (size_t)spin * assemble_blocks(g->nbasis));
     g->mark_end(kStFinalize, e);
     return;
   }
@@ -288,7 +282,7 @@ void fock_spin(chx_grid* g, double* dV, int nspin) {
     CHX_HIP(hipMemcpyAsync(g->d_coef.p, g->d_coef_save.p, sizeof(double) * nc, hipMemcpyDeviceToDevice, g->stream));
   }
   if (g->precision == CHX_PREC_MIXED && g->corr_pending) {
-    launch_reduce_corr(g->stream, nspin * corr_blocks(g->nbasis), g->d_cpart.p, g->d_en.p + 2);
+    launch_reduce_corr(g->stream, nspin * assemble_blocks(g->nbasis), g->d_cpart.p, g->d_en.p + 2);
     g->corr_done = true;
   }
 }

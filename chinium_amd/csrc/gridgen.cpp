@@ -446,29 +446,90 @@ static void build_items(const chx_grid* g, int sup, bool upper, int len, std::ve
 }
 
 // The longest run (a power of two up to the chunk length) that still leaves
-// enough items: each item ends in one FP64 atomic per element of its block, a
-// short list of long items leaves CUs idle. Times by run length, in us, Vxc
-// launch: (H2O)16 / def2-SVP mixed 1111 (1), 201 (8), 127 (32); (H2O)4 67 (1),
-// 27 (4), 67 (32); C7H16 FP64 323 (1), 179 (8), 307 (32); H2O FP64 18 (1), 260 (32).
+// enough items. A run's blocks are written once (FP64 form: one atomic per
+// element), so long runs write less; but an item is a serial chain of its run's
+// K steps, which shows unless several times more items than the chip holds are
+// there. Times by run length, in us, Vxc launch and V's assembly: (H2O)16 /
+// def2-SVP / SG-1 mixed 82 + 90 (4), 84 + 40 (8), 173 + 20 (32); (H2O)4 14 + 25
+// (2), 16 + 15 (4), 69 + 10 (32); (H2O)128 2640 + 1300 (8), 2280 + 700 (32);
+// C7H16 FP64 323 (1), 179 (8), 307 (32); H2O FP64 18 (1), 260 (32).
 static int default_len(const chx_grid* g, int sup, bool upper) {
-  const long kMinItems = g->precision == CHX_PREC_MIXED ? 160 : 384;
+  const bool mixed = g->precision == CHX_PREC_MIXED;
   for (int len = kChunkMax; len > 1; len /= 2) {
+    const long want = !mixed ? 384 : len > 8 ? 4096 : 160;
     long n = 0;
     for (size_t c = 0; c < g->chunks.size(); ++c) {
       const long ns = (g->chunks[c].ntl + sup - 1) / sup, nb = g->chunk_b0[c + 1] - g->chunk_b0[c];
       n += (upper ? ns * (ns + 1) / 2 : ns * ns) * ((nb + len - 1) / len);
     }
-    if (n >= kMinItems) return len;
+    if (n >= want) return len;
   }
   return 1;
 }
 
-// Vxc work items of the cached / mixed paths: 128-AO super-tiles, or (mixed
-// form, large bases) 256-AO groups whose items cover (I, J) and (J, I).
+// Mixed form: runs of at most len batches of a chunk; per run the groups of its
+// tiles (at most sup, equal to within one) and an item per pair I <= J. U holds
+// per run and group I the row panel of I's rows, columns from I0 to the list's
+// end; rows/rowptr list for every AO its row in every run that holds it, from
+// the AO's own column on (the upper triangle).
+static void build_mwork(chx_grid* g, int sup, int len, std::vector<RowRef>& rows, std::vector<int>& rowptr) {
+  g->mwork.clear();
+  g->u_elems = 0;
+  rowptr.assign(g->nbasis + 1, 0);
+  const size_t nch = g->chunks.size();
+  for (size_t c = 0; c < nch; ++c) {
+    const int runs = (g->chunk_b0[c + 1] - g->chunk_b0[c] + len - 1) / len, a0 = g->chunks[c].tile0 * kTile;
+    for (int i = 0; i < g->chunks[c].ntl * kTile; ++i)
+      if (g->ao_of[a0 + i] >= 0) rowptr[g->ao_of[a0 + i] + 1] += runs;
+  }
+  for (int i = 0; i < g->nbasis; ++i) rowptr[i + 1] += rowptr[i];
+  rows.resize(rowptr[g->nbasis]);
+  std::vector<int> at(rowptr.begin(), rowptr.end() - 1);
+  for (size_t c = 0; c < nch; ++c) {
+    const ChunkDev& ch = g->chunks[c];
+    if (ch.ntl == 0) continue;
+    const int ng = (ch.ntl + sup - 1) / sup, a0 = ch.tile0 * kTile;
+    int nreal = ch.ntl * kTile;  // the list's AOs: only its last tile is padded
+    while (g->ao_of[a0 + nreal - 1] < 0) --nreal;
+    for (int b = g->chunk_b0[c]; b < g->chunk_b0[c + 1]; b += len) {
+      const int nbat = std::min(len, g->chunk_b0[c + 1] - b);
+      for (int I = 0; I < ng; ++I) {
+        const int I0 = ch.ntl * I / ng, I1 = ch.ntl * (I + 1) / ng, ldu = (ch.ntl - I0) * kTile;
+        for (int J = I; J < ng; ++J) {
+          const int J0 = ch.ntl * J / ng, J1 = ch.ntl * (J + 1) / ng;
+          g->mwork.push_back(MxItem{(long)g->u_elems + (J0 - I0) * kTile, I0, I1 - I0, J0, J1 - J0, g->bt_off[b], nbat,
+                                    ch.ntl, ldu});
+        }
+        for (int r = I0 * kTile; r < std::min(I1 * kTile, nreal); ++r)
+          rows[at[g->ao_of[a0 + r]]++] = RowRef{(long)g->u_elems + (long)(r - I0 * kTile) * (ldu + 1), a0 + r, nreal - r};
+        g->u_elems += (size_t)(I1 - I0) * kTile * ldu;
+      }
+    }
+  }
+}
+
+// Vxc work items: FP64 form over 128-AO super-tiles, mixed form over groups of
+// up to kMxTiles tiles or (wide) kMxWideTiles. Uploads them and points the descriptor at them;
+// the host vectors outlive the copies (synchronises).
 void build_cwork(chx_grid* g) {
-  const bool wide = g->precision == CHX_PREC_MIXED && g->mx_wide;
-  const int sup = wide ? 2 * kCacheSuper : kCacheSuper;
-  build_items(g, sup, wide, g->vxc_chunk > 0 ? g->vxc_chunk : default_len(g, sup, wide), g->cwork);
+  hipStream_t st = g->stream;
+  if (g->precision != CHX_PREC_MIXED) {
+    build_items(g, kCacheSuper, false, g->vxc_chunk > 0 ? g->vxc_chunk : default_len(g, kCacheSuper, false), g->cwork);
+    g->d_cwork.upload(g->cwork, st);
+    CHX_HIP(hipStreamSynchronize(st));
+    return;
+  }
+  const int sup = g->mx_wide ? kMxWideTiles : kMxTiles;
+  std::vector<RowRef> rows;
+  std::vector<int> rowptr;
+  build_mwork(g, sup, g->vxc_chunk > 0 ? g->vxc_chunk : default_len(g, sup, true), rows, rowptr);
+  g->d_mwork.upload(g->mwork, st);
+  g->d_rows.upload(rows, st);
+  g->d_rowptr.upload(rowptr, st);
+  g->d_U.alloc(std::max<size_t>(1, g->u_elems));
+  g->hmol.cwork = g->d_mwork.p;
+  g->hmol.U = g->d_U.p;
+  CHX_HIP(hipStreamSynchronize(st));
 }
 
 // Rebuilds the Vxc work items for another chunk length (autotuning) without
@@ -478,10 +539,6 @@ void set_vxc_chunk(chx_grid* g, int chunk) {
   if (!g->ao_ready || !g->cached) return;
   ++g->plan_gen;
   build_cwork(g);
-  hipStream_t st = g->stream;
-  g->d_cwork.upload(g->cwork, st);
-  g->hmol.cwork = g->d_cwork.p;
-  CHX_HIP(hipStreamSynchronize(st));
 }
 
 // Vxc block shape of the mixed form (-1: 256-AO groups from npad 1024
@@ -597,23 +654,18 @@ void grid_plan(chx_grid* g) {
   g->mx_wide = mixed && (g->vxc_shape == 1 || (g->vxc_shape < 0 && g->npad >= 1024)) ? 1 : 0;
   g->vwork.clear();
   g->cwork.clear();
-  g->d_Mint.alloc((size_t)g->npad * g->npad);
+  g->mwork.clear();
+  if (mixed) g->d_Mint.release();
+  else g->d_Mint.alloc((size_t)g->npad * g->npad);
   if (g->cached) {
-    build_cwork(g);
-    g->d_cwork.upload(g->cwork, st);
     if (mixed) {
       g->d_cache.release();
       g->d_bmat.release();
       g->mx_nT = nT;
       g->mx_sstride = 2 * nT * kMxComp;  // AOg then AOt, nT components each
-      // one extra all-zero slot at index nslot stands in for tiles past a list
-      g->d_cmx.alloc((nslot + 1) * (size_t)g->mx_sstride);
-      CHX_HIP(hipMemsetAsync(g->d_cmx.p + nslot * (size_t)g->mx_sstride, 0,
-                             sizeof(unsigned short) * g->mx_sstride, st));
+      g->d_cmx.alloc(std::max<size_t>(1, nslot * (size_t)g->mx_sstride));
       g->bmx_comps = nT;
-      // B^T of every slot, plus the all-zero slot that make_b rewrites for the
-      // component count of each build's potential
-      g->d_bmx.alloc((nslot + 1) * (size_t)nT * kMxComp);
+      g->d_bmx.alloc(std::max<size_t>(1, nslot * (size_t)nT * kMxComp));
       g->d_Dsplit.alloc(std::max<size_t>(1, 2 * g->dt_elems));
       // core batches: any real point within core_radius of a nucleus with Z > 2
       std::vector<int> core_off(nb, -1), slot_core(std::max<size_t>(1, nslot), -1);
@@ -695,11 +747,12 @@ void grid_plan(chx_grid* g) {
   launch_fill(st, g->d_en.p, 3, 0.0);
   if (mixed) {  // split remainder of D per spin, and the partial sums of V . remainder
     g->d_Dres.alloc(2 * (size_t)g->nbasis * g->nbasis);
-    g->d_cpart.alloc(2 * (size_t)corr_blocks(g->nbasis));
+    g->d_cpart.alloc(2 * (size_t)assemble_blocks(g->nbasis));
   }
+  g->hmol = MolDev{};
+  if (g->cached) build_cwork(g);
   if (mixed) {  // descriptor of this grid for the mixed kernels
     MolDev& m = g->hmol;
-    m = MolDev{};
     m.grp_batch = g->d_grp_batch.p; m.grp_tile = g->d_grp_tile.p; m.grp_ntiles = g->d_grp_ntiles.p;
     m.bt_off = g->d_bt_off.p; m.b_chunk = g->d_b_chunk.p; m.chunks = g->d_chunks.p; m.ao_of = g->d_ao_of.p;
     m.bx = g->d_x.p; m.by = g->d_y.p; m.bz = g->d_z.p;
@@ -709,8 +762,6 @@ void grid_plan(chx_grid* g) {
     m.part = g->d_part.p; m.part_tau = g->d_part_tau.p;
     m.slot_batch = g->d_slot_batch.p; m.slot_tile = g->d_slot_tile.p;
     m.coef = g->d_coef.p; m.bt = g->d_bmx.p;
-    m.Mint = g->d_Mint.p;
-    m.cwork = g->d_cwork.p;
     m.cache3 = g->d_cmx3.p;
     m.core_off = g->d_core_off.p;
     m.core_grps = g->d_core_grps.p;

@@ -18,6 +18,8 @@ constexpr int kGroup = 4;      // AO tiles per density work group (128 output co
 constexpr int kSuper = 2;      // AO tiles per Vxc super-tile (64 x 64 output block)
 constexpr int kPadAO = 128;    // nbasis is padded to a multiple of this (4 tiles)
 constexpr int kCacheSuper = 4; // tiles per Vxc super-tile in the cached path
+constexpr int kMxTiles = 4;    // tiles per Vxc group of the mixed form (128 AOs)
+constexpr int kMxWideTiles = 5;  // ... of its wide shape (160 AOs)
 constexpr int kChunkMax = 32;  // most consecutive batches that share one AO list
 constexpr int kCoef = 5;       // Vxc integrand coefficients per point: a, c_x, c_y, c_z, t
 constexpr double kCoreRadius = 0.3;  // bohr: points this close to a nucleus with Z > 2 are batched apart
@@ -129,6 +131,18 @@ struct ChunkDev {
 // its batches; slot0 is the first batch's first slot.
 struct VxcItem {
   int I, J, slot0, nbat, ntl, tile0, batch0, pad_;
+};
+
+// Mixed form: tiles I0 .. I0 + nI - 1 against J0 .. J0 + nJ - 1 (I0 <= J0) of a
+// run (nbat batches of a chunk); the block's place u in U and its row length.
+struct MxItem {
+  long u;
+  int I0, nI, J0, nJ, slot0, nbat, ntl, ldu;
+};
+// Row of one AO in a run's blocks: element k (k < len) is V at (that AO, ao_of[a0 + k]).
+struct RowRef {
+  long u;
+  int a0, len;
 };
 
 // Launchers (kernels.hip).
@@ -262,8 +276,8 @@ struct MolDev {
   const int *slot_batch, *slot_tile;
   const double* coef;           // Vxc integrand coefficients per point
   unsigned short* bt;           // B^T per slot
-  const VxcItem* cwork;         // Vxc work items
-  double* Mint;                 // M accumulator, npad^2
+  const MxItem* cwork;          // Vxc work items
+  float* U;                     // the runs' blocks of V (upper)
   // core batches (points within the core radius of a nucleus with Z > 2): their
   // density runs with the AO operands split in three bf16 terms; cache3 holds
   // the third term of their slots' AOg blocks [core slot][c][g][mu],
@@ -319,12 +333,12 @@ void launch_ao_cache_mx(hipStream_t s, int nslots, const int* slot_batch, const 
 // own (reference, column-major) order
 void launch_split_d(hipStream_t s, int ntiles, int n, const double* D, const int* tile_chunk, const ChunkDev* chunks,
                     const int* ao_of, unsigned short* Ds, float* R);
-// First-order energy correction for the split of D: V = M + M^T as
-// launch_finalize_sym, and per block the partial sum of V . R into cpart
-// (corr_blocks(n) blocks); launch_reduce_corr sums nparts partials into *out.
-int corr_blocks(int n);
-void launch_finalize_corr(hipStream_t s, int n, int npad, const double* Mint, double* V, const float* R,
-                          double* cpart);
+// V (reference order) from the runs' blocks U and, with R, the first-order energy
+// correction for the split of D: partial sums of V . R into cpart
+// (assemble_blocks(n) of them); launch_reduce_corr sums nparts partials into *out.
+int assemble_blocks(int n);
+void launch_assemble_mx(hipStream_t s, int n, const int* rowptr, const RowRef* rows, const int* ao_of, const float* U,
+                        double* V, const float* R, double* cpart);
 void launch_reduce_corr(hipStream_t s, int nparts, const double* cpart, double* out);
 // the packed form: per molecule of the table, en[2 slot_en] += its ncpart partials
 void launch_corr_multi(hipStream_t s, const char* base, const FnMolecule* fm, int nmol, double* en);
@@ -336,17 +350,16 @@ void launch_fill_u32(hipStream_t s, unsigned* p, size_t n, unsigned v);
 void launch_density_mx(hipStream_t s, int mode, int nitems, const MolDev& one);
 // the core groups again with three-term operands: mode 0 (rho, grad rho) or r = 1..3 (tau partial r)
 void launch_density_mx_core(hipStream_t s, int mode, int ncore_groups, const MolDev& one);
-// B^T of every slot plus the all-zero slot (index nslots) for ncomp components; clears M
+// B^T of every slot for ncomp components
 void launch_make_b_mx(hipStream_t s, int ncomp, const MolDev& one);
-void launch_vxc_mx(hipStream_t s, int ncomp, int nitems, const MolDev& one);
+// wide: groups of up to kMxWideTiles tiles instead of kMxTiles
+void launch_vxc_mx(hipStream_t s, int ncomp, int wide, int nitems, const MolDev& one);
 // Persistent stage launches over many molecules (packs, LDA/GGA): tab holds one
 // descriptor per molecule with byte offsets from base in place of pointers;
 // starts (nmol + 1) the first item of each molecule in the stage's flat list.
 enum { kStageDensity = 0, kStageCore = 1, kStageMakeB = 2, kStageVxc = 3, kStageVxcWide = 4 };
 void launch_stage_multi(hipStream_t s, int stage, int ncomp, const char* base, const MolDev* tab, const int* starts,
                         int nmol, int total);
-// 256 x 256 output blocks over groups of 8 of a chunk's tiles; items (I <= J)
-void launch_vxc_mx_wide(hipStream_t s, int ncomp, int nitems, const MolDev& one);
 
 }  // namespace chx
 
@@ -429,7 +442,9 @@ struct chx_grid {
   int vxc_chunk = 0;                 // batches per Vxc work item; 0 = by the item count
   int vxc_shape = -1;                // mixed form's Vxc blocks: -1 by basis size, 0 128-AO super-tiles, 1 256-AO groups
   int mx_wide = 0;                   // mixed form: Vxc over 256-AO groups (large bases)
-  std::vector<chx::VxcItem> cwork;
+  std::vector<chx::VxcItem> cwork;      // FP64 form
+  std::vector<chx::MxItem> mwork;       // mixed form
+  size_t u_elems = 0;                   // elements of the runs' blocks of V
   // mixed form: core batches (density with three-term operands)
   double core_radius = chx::kCoreRadius;  // bohr; 0 turns the core treatment off
   int ncore_batches = 0;
@@ -439,6 +454,10 @@ struct chx_grid {
   chx::DevBuf<double> d_cache, d_bmat, d_Mint;
   chx::DevBuf<int> d_slot_batch, d_slot_tile;
   chx::DevBuf<chx::VxcItem> d_cwork;
+  chx::DevBuf<chx::MxItem> d_mwork;
+  chx::DevBuf<chx::RowRef> d_rows;
+  chx::DevBuf<int> d_rowptr;
+  chx::DevBuf<float> d_U;
   double flops_build = 0, mean_tiles = 0;
   std::vector<double> batch_work;  // g_b n_b^2 per batch (points x kept AOs squared)
   double core_flops = 0;           // the core batches' three-term (rho, grad rho) launch: 2 sum g_b n_b^2

@@ -33,7 +33,6 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kMxRow = 2 * kTile;             // one AOg row: 32 hi then 32 lo
 constexpr int kMxT = 2 * kTile * kBatch;      // elements per component of AOg, AOt and Bt
-constexpr int kMxSup = 4;                     // tiles per Vxc super-tile (128 AOs)
 // LDS operand tiles: rows of 4 16-byte chunks (32 bf16), chunk c of row r
 // stored at position c ^ ((r >> 2) & 3). A wave's 16-byte accesses then hit
 // distinct banks both when 16 lanes read one chunk of 16 consecutive rows
@@ -228,40 +227,111 @@ void launch_split_d(hipStream_t s, int ntiles, int n, const double* D, const int
   CHX_HIP(hipGetLastError());
 }
 
-// V = M + M^T (reference order, as k_finalize_sym) and the block's partial sum
-// of V . R, the split remainder of D: grid-stride over the n^2 elements with a
-// fixed block count, so the partials have one fixed order of summation.
-constexpr int kCorrBlocks = 1024;
-int corr_blocks(int n) { return (int)std::min<long>(kCorrBlocks, ((long)n * n + 255) / 256); }
-
 __device__ __forceinline__ double block_sum_d(double v) {
-  __shared__ double red[4];
+  __shared__ double red[16];
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
   __syncthreads();
-  return (red[0] + red[1]) + (red[2] + red[3]);
+  double t = 0.0;
+  for (int w = 0; w < (int)(blockDim.x >> 6); ++w) t += red[w];
+  return t;
 }
 
-__global__ __launch_bounds__(256) void k_finalize_corr(int n, int npad, const double* __restrict__ Mint,
-                                                       double* __restrict__ V, const float* __restrict__ R,
-                                                       double* __restrict__ cpart) {
-  const long tot = (long)n * n;
-  double acc = 0.0;
-  for (long idx = (long)blockIdx.x * 256 + threadIdx.x; idx < tot; idx += (long)gridDim.x * 256) {
-    const int col = (int)(idx / n), row = (int)(idx % n);
-    const double v = Mint[(size_t)row * npad + col] + Mint[(size_t)col * npad + row];
-    V[idx] = v;
-    acc += v * (double)R[idx];
+// V from the runs' blocks U (see k_vxc_mx): block mu sums row mu, columns nu >=
+// mu, of every run whose list holds AO mu into FP64 sums in LDS, writes V[mu][nu]
+// and V[nu][mu] (reference order), and with R the partial sum of V . R over them.
+// 16 waves; a run's row is contiguous in U, kAsmUnroll rows are in flight per
+// wave. Up to kAsmLds / 16 = 512 AOs each wave has a copy of the sums (COPIES =
+// 16), so that a plain LDS read-add-write does; larger rows share one (COPIES = 1)
+// through ds_add_f64, which is the bound there, some 130 cycles per wave: fewer
+// waves with copies are slower still. (H2O)16: 48 us against 86 shared; (H2O)48:
+// 250 us shared against 363 with 4 waves; (H2O)128 700 us against 1430 with 2.
+// The FP64 atomics to HBM that all this replaces, one per element of M and run
+// at about 40 G/s, took most of the Vxc launch. kAsmLds sums per block: larger
+// bases take several column ranges (grid y).
+constexpr int kAsmLds = 8192;
+constexpr int kAsmUnroll = 8;
+constexpr int kAsmThreads = 1024;
+static int asm_copies(int n) { return n <= kAsmLds / 16 ? 16 : 1; }
+static int asm_ranges(int n) { return (n + kAsmLds / asm_copies(n) - 1) / (kAsmLds / asm_copies(n)); }
+int assemble_blocks(int n) { return n * asm_ranges(n); }
+
+template <int COPIES>
+__global__ __launch_bounds__(kAsmThreads) void k_assemble_mx(int n, const int* __restrict__ rowptr,
+                                                             const RowRef* __restrict__ rows,
+                                                             const int* __restrict__ ao_of,
+                                                             const float* __restrict__ U, double* __restrict__ V,
+                                                             const float* __restrict__ R,
+                                                             double* __restrict__ cpart) {
+  extern __shared__ double asum[];
+  constexpr int kCols = kAsmLds / COPIES, kWaves = kAsmThreads / 64;
+  const int mu = blockIdx.x, c0 = blockIdx.y * kCols, w = min(kCols, n - c0), tid = threadIdx.x;
+  if (c0 + w <= mu) {  // below the diagonal: the block of row nu writes it
+    if (R && tid == 0) cpart[(size_t)blockIdx.y * n + mu] = 0.0;
+    return;
   }
-  acc = block_sum_d(acc);
-  if (threadIdx.x == 0) cpart[blockIdx.x] = acc;
+  for (int i = tid; i < w * COPIES; i += kAsmThreads) asum[i] = 0.0;
+  __syncthreads();
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  double* sum = COPIES == 1 ? asum : asum + (size_t)wave * w;
+  const int e1 = rowptr[mu + 1];
+  for (int e = rowptr[mu] + wave * kAsmUnroll; e < e1; e += kWaves * kAsmUnroll) {
+    RowRef r[kAsmUnroll];
+    int len = 0;
+#pragma unroll
+    for (int q = 0; q < kAsmUnroll; ++q) {
+      r[q] = rows[min(e + q, e1 - 1)];
+      if (e + q >= e1) r[q].len = 0;
+      len = max(len, r[q].len);
+    }
+    for (int k = lane; k < len; k += 64) {
+      int nu[kAsmUnroll];
+      float v[kAsmUnroll];
+#pragma unroll
+      for (int q = 0; q < kAsmUnroll; ++q) {  // clamped, not skipped: the loads go out together
+        const int kk = min(k, max(r[q].len - 1, 0));
+        nu[q] = ao_of[r[q].a0 + kk] - c0;
+        v[q] = U[r[q].u + kk];
+        if (k >= r[q].len) nu[q] = -1;
+      }
+#pragma unroll
+      for (int q = 0; q < kAsmUnroll; ++q)
+        if (nu[q] >= 0 && nu[q] < w) {
+          if (COPIES == 1)
+            __hip_atomic_fetch_add(&sum[nu[q]], (double)v[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+          else
+            sum[nu[q]] += (double)v[q];
+        }
+    }
+  }
+  __syncthreads();
+  double acc = 0.0;
+  for (int i = max(0, mu - c0) + tid; i < w; i += kAsmThreads) {
+    double v = asum[i];
+#pragma unroll
+    for (int c = 1; c < COPIES; ++c) v += asum[(size_t)c * w + i];
+    const size_t up = (size_t)mu * n + c0 + i, lo = (size_t)(c0 + i) * n + mu;
+    V[up] = v;
+    V[lo] = v;
+    if (R) acc += v * (up == lo ? (double)R[up] : (double)R[up] + (double)R[lo]);
+  }
+  if (R) {
+    acc = block_sum_d(acc);
+    if (tid == 0) cpart[(size_t)blockIdx.y * n + mu] = acc;
+  }
 }
 
-void launch_finalize_corr(hipStream_t s, int n, int npad, const double* Mint, double* V, const float* R,
-                          double* cpart) {
-  hipLaunchKernelGGL(k_finalize_corr, dim3((unsigned)corr_blocks(n)), dim3(256), 0, s, n, npad, Mint, V, R,
-                     cpart);
+void launch_assemble_mx(hipStream_t s, int n, const int* rowptr, const RowRef* rows, const int* ao_of, const float* U,
+                        double* V, const float* R, double* cpart) {
+  if (n == 0) return;
+  const int copies = asm_copies(n);
+  const dim3 grid(n, asm_ranges(n));
+  const size_t lds = (size_t)std::min(n, kAsmLds / copies) * copies * sizeof(double);
+  if (copies == 16)
+    hipLaunchKernelGGL(k_assemble_mx<16>, grid, dim3(kAsmThreads), lds, s, n, rowptr, rows, ao_of, U, V, R, cpart);
+  else
+    hipLaunchKernelGGL(k_assemble_mx<1>, grid, dim3(kAsmThreads), lds, s, n, rowptr, rows, ao_of, U, V, R, cpart);
   CHX_HIP(hipGetLastError());
 }
 
@@ -989,23 +1059,10 @@ struct MakeB {
   __device__ void end() {}
 };
 
-// The wave of slot index nslots clears the all-zero slot that the Vxc items
-// read for tiles that are not alive in a batch: it sits at nslots * NC
-// components, so its place moves with the potential's component count and is
-// rewritten on every build.
 template <int NC>
 __device__ __forceinline__ void make_b_slot(const MolDev& m, int slot, int g) {
-  if (slot > m.nslots) return;
+  if (slot >= m.nslots) return;
   u16* __restrict__ col0 = m.bt + (size_t)slot * NC * kMxT + g;  // [c][hl][nu][g], this lane's point
-  if (slot == m.nslots) {
-    for (int col = 0; col < kTile; ++col)
-#pragma unroll
-      for (int c = 0; c < NC; ++c) {
-        col0[c * kMxT + col * kBatch] = 0;
-        col0[c * kMxT + kTile * kBatch + col * kBatch] = 0;
-      }
-    return;
-  }
   const BasisView bv = m.bv;  // descriptor fields in registers, read once
   const int b = m.slot_batch[slot], t = m.slot_tile[slot];
   const size_t p = (size_t)b * kBatch + g;
@@ -1031,312 +1088,179 @@ __device__ __forceinline__ void make_b_slot(const MolDev& m, int slot, int g) {
       col0[c * kMxT + kTile * kBatch + col * kBatch] = 0;
     }
 }
-// The blocks past the slots clear M for the Vxc launch that follows.
-constexpr int kFillBlock = 4096;
 template <int NC>
 __global__ __launch_bounds__(NC == 4 ? 64 : 256) void k_make_b_mx(MolDev m) {
   constexpr int W = NC == 4 ? 1 : 4;  // waves per block
-  const int nsb = (m.nslots + W) / W;
-  if ((int)blockIdx.x >= nsb) {
-    const size_t n2 = (size_t)m.npad * m.npad, e0 = (size_t)(blockIdx.x - nsb) * kFillBlock;
-    for (size_t i = e0 + threadIdx.x; i < e0 + kFillBlock && i < n2; i += 64 * W) m.Mint[i] = 0.0;
-    return;
-  }
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   make_b_slot<NC>(m, blockIdx.x * W + wave, threadIdx.x & 63);
 }
 
 void launch_make_b_mx(hipStream_t s, int ncomp, const MolDev& one) {
-  const int waves = one.nslots + 1;  // every slot and the all-zero slot
-  const int fill = (int)(((size_t)one.npad * one.npad + kFillBlock - 1) / kFillBlock);
+  const int waves = one.nslots;
+  if (waves == 0) return;
   if (ncomp == 4)
-    hipLaunchKernelGGL((k_make_b_mx<4>), dim3(waves + fill), dim3(64), 0, s, one);
+    hipLaunchKernelGGL((k_make_b_mx<4>), dim3(waves), dim3(64), 0, s, one);
   else
-    hipLaunchKernelGGL((k_make_b_mx<1>), dim3((waves + 3) / 4 + fill), dim3(256), 0, s, one);
+    hipLaunchKernelGGL((k_make_b_mx<1>), dim3((waves + 3) / 4), dim3(256), 0, s, one);
   CHX_HIP(hipGetLastError());
 }
 
 // ---------------------------------------------------------------------------
-// Vxc: M_IJ += sum_g Phi_I[g]^T B_J[g] over the work item's batches, for
-// 128-AO super-tiles I, J. A K step is 32 points of one component: Phi^T_I
-// (128 mu x 32 g) and B^T_J (128 nu x 32 g), hi and lo, 32 fragments of 1 KB
-// (16 rows of 64 bytes) that the waves' DMA loads bring straight into LDS,
-// coalesced and swizzled as in the density kernel. One buffer: wait for the
-// step's fragments, read the wave's 16 into registers, barrier, start the DMA
-// of the next step, run the wave's 48 MFMAs. 4 waves in a 2 x 2 grid, each
-// owning a 64 x 64 block of M. One FP64 atomic add per element per work item.
-// Meta-GGA (NC = 4): the tau part sum_r (d_r Phi)^T (t d_r Phi) is symmetric
-// and V = M + M^T, so an item with I > J skips it, an item with I < J takes it
-// twice (its tau steps run first, then the accumulators are doubled before the
-// phi steps), and I = J takes it once.
-constexpr int kVxA = 16;  // Phi^T fragments per step: [row block (8)][hl]
+// Vxc: one block of one run's V, U_IJ = sum_g Phi_I^T B_J + B_I^T Phi_J over
+// the run's batches, for groups I <= J of at most MT of the chunk's tiles (the
+// groups of a list are equal to within a tile, so no block is mostly padding).
+// For I < J both products go into the same accumulators (second pass: the
+// operands swap roles), so only the upper blocks are formed; for I = J one
+// product M is formed and U = M + M^T through LDS at the end. The tau part
+// (NC = 4) is symmetric, M_tau = sum_r (d_r Phi)^T (t d_r Phi): its steps run
+// first and once, doubled for I < J.
+// A K step is 32 points of one component: the row group's and the column
+// group's operands, hi and lo, fragments of 1 KB (16 rows of 64 bytes) that the
+// waves' DMA loads bring straight into LDS, coalesced and swizzled as in the
+// density kernel. Two LDS buffers and one barrier per step: after it, step k's
+// fragments are in LDS and every wave has read step k - 1's buffer, so the DMA
+// of step k + 1 goes there before step k's fragment reads and products. 4 waves
+// in a 2 x 2 grid, each owning half of the row and of the column blocks (up to
+// MT x MT fragments of 16 x 16; MT = 5 is the largest whose two buffers leave
+// room for two blocks per CU).
+// The result is stored once per run, in FP32 like the accumulators (row-major,
+// the row panel of group I from column I0 on), and summed in FP64 by
+// k_assemble_mx.
+template <int MT>
 struct VxcMxSmem {
-  u32x4 F[2 * kVxA * kDxFrag];  // one K step's fragments: Phi^T_I, then B^T_J
+  u32x4 F[2][8 * MT * kDxFrag];  // step k in buffer k & 1: row group's fragments, then the column group's
 };
 
-template <int NC>
+template <int NC, int MT>
 __device__ __forceinline__ void vxc_mx_body(const MolDev& m, int item) {
   using lds_ptr = __attribute__((address_space(3))) void*;
-  __shared__ VxcMxSmem sm;
-  const VxcItem wk = m.cwork[item];
-  const int I = wk.I, J = wk.J;
+  constexpr int PT = 32 * MT + 4;  // pitch of the transposed strip
+  __shared__ VxcMxSmem<MT> sm;
+  const MxItem wk = m.cwork[item];
+  const int nI = wk.nI, RB = 2 * nI, CB = 2 * wk.nJ, nf = 2 * (RB + CB);
+  const bool diag = wk.I0 == wk.J0;
   const u16* __restrict__ cache = m.cache + m.toff;
   const u16* __restrict__ bt = m.bt;
   const size_t sstride = (size_t)m.sstride;
-  const int npad = m.npad;
-  double* __restrict__ Mint = m.Mint;
-  const int zero = m.nslots;  // the all-zero slot stands in for tiles past the chunk's last
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lrow = lane & 15, lk = lane >> 4;
   const int wr = wave & 1, wc = wave >> 1;
-  // The wave's fragments are f = wave + 4 j, j = 0..3 of Phi^T_I and of B^T_J:
-  // row block f >> 1 (tile j = f >> 2, rows 16 ((f >> 1) & 1)..+15 of it), hl
-  // f & 1. DMA lane i fetches row i >> 2, chunk (i & 3) ^ sw(row); the MFMA
-  // lane that needs (row, chunk) reads it back at fidx.
+  const int r0 = nI * wr, nc = wk.nJ, c0 = nc * wc;  // the wave's row blocks r0 .. r0 + nI - 1, columns c0 ..
+  // The wave's fragments are f = wave + 4 j: hl f & 1, rows 16 ((f >> 1) & 1)..+15
+  // of tile f >> 2 of the row group (f < 2 RB) or of the column group.
   const int drow = lane >> 2, dch = (lane & 3) ^ ((drow >> 2) & 3);
   const int fidx = 4 * lrow + (lk ^ ((lrow >> 2) & 3));
-  int off[4];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int f = wave + 4 * j;
-    off[j] = (f & 1) * (kTile * kBatch) + (16 * ((f >> 1) & 1) + drow) * kBatch + 8 * dch;
-  }
-  const int nbat = wk.nbat;                           // items hold >= 1 batch
-  const int ntau = (NC == 4 && I <= J) ? 6 * nbat : 0;  // tau steps, first
-  const int nstage = ntau + 2 * nbat;
-  // K step k -> (batch of the item, half of its points, component): tau steps
-  // (it, h, c = 1..3) for k < ntau, then the phi steps (it, h, c = 0)
-  auto dma = [&](int k) {
+  const int off = (wave & 1) * (kTile * kBatch) + drow * kBatch + 8 * dch;
+  const int nbat = wk.nbat;
+  const int ntau = NC == 4 ? 6 * nbat : 0;  // tau steps, first
+  const int kswap = ntau + 2 * nbat;        // first step of the second product
+  const int nstage = kswap + (diag ? 0 : 2 * nbat);
+  auto dma = [&](int k, int buf) {  // issue step k's loads: (batch, half of its points, component, product)
+    const bool swap = k >= kswap;
     int it, h, c;
     if (k < ntau) {
       it = k / 6; h = (k / 3) % 2; c = 1 + k % 3;
     } else {
-      it = (k - ntau) >> 1; h = (k - ntau) & 1; c = 0;
-    }
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int s0 = wk.slot0 + it * wk.ntl, ta = I * kMxSup + j, tb = J * kMxSup + j;
-      const u16* pa = cache + (size_t)(ta < wk.ntl ? s0 + ta : zero) * sstride + c * kMxT + h * 32;
-      const u16* pb = bt + ((size_t)(tb < wk.ntl ? s0 + tb : zero) * NC + c) * kMxT + h * 32;
-      __builtin_amdgcn_global_load_lds(pa + off[j], (lds_ptr)(sm.F + (wave + 4 * j) * kDxFrag), 16, 0, 0);
-      __builtin_amdgcn_global_load_lds(pb + off[j], (lds_ptr)(sm.F + (kVxA + wave + 4 * j) * kDxFrag), 16, 0, 0);
-    }
-  };
-  f32x4 acc[4][4];
-#pragma unroll
-  for (int r = 0; r < 4; ++r)
-#pragma unroll
-    for (int c = 0; c < 4; ++c) acc[r][c] = f32x4{0.f, 0.f, 0.f, 0.f};
-  dma(0);
-  for (int k = 0; k < nstage; ++k) {
-    if (NC == 4 && k == ntau && I < J) {  // 2 M_tau for the item's (I, J) and (J, I) blocks
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-#pragma unroll
-        for (int c = 0; c < 4; ++c) acc[r][c] *= 2.f;
-    }
-    __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this wave's fragments of step k are in LDS
-    __syncthreads();                     // ... and every other wave's
-    u32x4 a[4][2], bq[4][2];
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        a[r][h] = sm.F[((4 * wr + r) * 2 + h) * kDxFrag + fidx];
-        bq[r][h] = sm.F[(kVxA + (4 * wc + r) * 2 + h) * kDxFrag + fidx];
-      }
-    __syncthreads();  // every wave holds its fragments: the buffer is free
-    if (k + 1 < nstage) dma(k + 1);
-#pragma unroll
-    for (int c = 0; c < 4; ++c)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) acc[r][c] = mfma3(a[r][0], a[r][1], bq[c][0], bq[c][1], acc[r][c]);
-  }
-  const int nrow = wk.ntl * kTile;
-  const int* __restrict__ ao = m.ao_of + (size_t)wk.tile0 * kTile;
-  int nu[4];
-#pragma unroll
-  for (int cb = 0; cb < 4; ++cb) {
-    const int lc = J * kMxSup * kTile + 64 * wc + 16 * cb + lrow;
-    nu[cb] = lc < nrow ? ao[lc] : -1;
-  }
-#pragma unroll
-  for (int r = 0; r < 4; ++r)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int lr = I * kMxSup * kTile + 64 * wr + 16 * r + 4 * lk + i;
-      const int mu = lr < nrow ? ao[lr] : -1;
-      if (mu < 0) continue;
-#pragma unroll
-      for (int cb = 0; cb < 4; ++cb)
-        if (nu[cb] >= 0) unsafeAtomicAdd(&Mint[(size_t)mu * npad + nu[cb]], (double)acc[r][cb][i]);
-    }
-}
-template <int NC>
-__global__ __launch_bounds__(256, 3) void k_vxc_mx(MolDev m) {
-  vxc_mx_body<NC>(m, xcd_remap(blockIdx.x, gridDim.x));
-}
-
-// Vxc for large bases: M_IJ += Phi_I^T B_J over 256 x 256 blocks whose rows
-// and columns are groups of 8 of a chunk's tiles, so every operand byte staged in LDS feeds twice the MFMAs of the 128 x 128
-// kernel (64 instead of 32 FLOP per byte). An item is a pair of groups I <= J
-// of one chunk and covers both blocks: first M_IJ (the tau part, symmetric,
-// taken twice for I < J and once for I = J, then the phi part), then for
-// I < J the mirror block M_JI (phi part only), so every item does about the
-// same work per batch and the items that run together on an XCD stream the
-// chunk's slots in step. A K step is 32 points of one component: Phi^T of the
-// row group and B^T of the column group, 256 rows each, hi and lo, 64
-// fragments of 1 KB brought in by the waves' DMA (same coalesced lane order
-// and swizzle). 8 waves in a 2 x 4 grid, each owning a 128 x 64 block (up to
-// 96 MFMAs per step). A 16-bit mask (I's 8 tiles, then J's) marks the tiles
-// the chunk has: an absent tile's fragments are not loaded and the products
-// that involve it are skipped.
-constexpr int kMxSupW = 8;   // tiles per group (256 AOs)
-constexpr int kVxAW = 32;    // Phi^T fragments per step: [row block (16)][hl]
-constexpr int kVxWStep = 2 * kVxAW * kDxFrag;  // u32x4 per K step: Phi^T of the row group, then B^T of the column group
-struct VxcMxWideSmem {
-  u32x4 F[2 * kVxWStep];  // two K steps' fragments: step k in buffer k & 1
-};
-
-// Two LDS buffers and one barrier per K step: after it, step k's fragments
-// are in LDS and every wave has read step k - 1's buffer, so the DMA of step
-// k + 1 goes there before step k's fragment reads and products (measured at
-// (H2O)128 / r2SCAN: 114.5 ms per launch against 125.5 ms with one buffer and
-// a second barrier after the fragment reads).
-template <int NC>
-__device__ __forceinline__ void vxc_mx_wide_body(const MolDev& m, int item) {
-  using lds_ptr = __attribute__((address_space(3))) void*;
-  __shared__ VxcMxWideSmem sm;
-  const VxcItem wk = m.cwork[item];
-  const int I = wk.I, J = wk.J;    // I <= J
-  const int nbat = wk.nbat;
-  const u16* __restrict__ cache = m.cache + m.toff;
-  const u16* __restrict__ bt = m.bt;
-  const size_t sstride = (size_t)m.sstride;
-  const int npad = m.npad;
-  double* __restrict__ Mint = m.Mint;
-  const int nI = min(kMxSupW, wk.ntl - I * kMxSupW), nJ = min(kMxSupW, wk.ntl - J * kMxSupW);
-  const unsigned mk = ((1u << nI) - 1u) | (((1u << nJ) - 1u) << 8);
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int lrow = lane & 15, lk = lane >> 4;
-  const int wr = wave & 1, wc = wave >> 1;
-  // The wave's fragments are f = wave + 8 j, j = 0..3, of the row group's Phi^T
-  // and of the column group's B^T: hl f & 1 = wave & 1, rows
-  // 16 ((wave >> 1) & 1)..+15 of tile (wave >> 2) + 2 j.
-  const int drow = lane >> 2, dch = (lane & 3) ^ ((drow >> 2) & 3);
-  const int fidx = 4 * lrow + (lk ^ ((lrow >> 2) & 3));
-  const int off = (wave & 1) * (kTile * kBatch) + (16 * ((wave >> 1) & 1) + drow) * kBatch + 8 * dch;
-  const int t0 = wave >> 2;
-  const int ntau = NC == 4 ? 6 * nbat : 0;  // tau steps of M_IJ, first
-  const int kmirror = ntau + 2 * nbat;      // first step of M_JI (I < J)
-  const int nstage = kmirror + (I < J ? 2 * nbat : 0);
-  // K step k -> (batch, half of its points, component, mirror block?)
-  auto decode = [&](int k, int& it, int& h, int& c, bool& mir) {
-    mir = k >= kmirror;
-    if (k < ntau) {
-      it = k / 6; h = (k / 3) % 2; c = 1 + k % 3;
-    } else {
-      const int q = k - (mir ? kmirror : ntau);
+      const int q = k - (swap ? kswap : ntau);
       it = q >> 1; h = q & 1; c = 0;
     }
-  };
-  // issue step k's loads into buffer buf
-  auto dma = [&](int k, int buf) {
-    int it, h, c;
-    bool mir;
-    decode(k, it, h, c, mir);
-    const int ra = mir ? 8 : 0, cb = mir ? 0 : 8;  // table columns of the row and column groups
-    const int s0 = wk.slot0 + it * wk.ntl, sa = s0 + (mir ? J : I) * kMxSupW, sb = s0 + (mir ? I : J) * kMxSupW;
-    u32x4* F = sm.F + buf * kVxWStep;
+    const int s0 = wk.slot0 + it * wk.ntl;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int t = t0 + 2 * j;
-      if ((mk >> (ra + t)) & 1u) {
-        const u16* pa = cache + (size_t)(sa + t) * sstride + c * kMxT + h * 32;
-        __builtin_amdgcn_global_load_lds(pa + off, (lds_ptr)(F + (wave + 8 * j) * kDxFrag), 16, 0, 0);
-      }
-      if ((mk >> (cb + t)) & 1u) {
-        const u16* pb = bt + ((size_t)(sb + t) * NC + c) * kMxT + h * 32;
-        __builtin_amdgcn_global_load_lds(pb + off, (lds_ptr)(F + (kVxAW + wave + 8 * j) * kDxFrag), 16, 0, 0);
+    for (int j = 0; j < 2 * MT; ++j) {
+      const int f = wave + 4 * j;
+      if (f < nf) {
+        const bool row = f < 2 * RB;
+        const int fr = row ? f : f - 2 * RB;
+        const size_t slot = (size_t)(s0 + (row ? wk.I0 : wk.J0) + (fr >> 2));
+        const u16* p = (row != swap ? cache + slot * sstride : bt + slot * (NC * kMxT)) + c * kMxT + h * 32 +
+                       ((fr >> 1) & 1) * (16 * kBatch);
+        __builtin_amdgcn_global_load_lds(p + off, (lds_ptr)(sm.F[buf] + f * kDxFrag), 16, 0, 0);
       }
     }
   };
-  f32x4 acc[8][4];
+  f32x4 acc[MT][MT];
 #pragma unroll
-  for (int r = 0; r < 8; ++r)
+  for (int r = 0; r < MT; ++r)
 #pragma unroll
-    for (int c = 0; c < 4; ++c) acc[r][c] = f32x4{0.f, 0.f, 0.f, 0.f};
-  // one FP64 atomic add per element of the wave's 128 x 64 block of the chunk's rows ro.. and columns co..
-  const int nrow = wk.ntl * kTile;
-  const int* __restrict__ ao = m.ao_of + (size_t)wk.tile0 * kTile;
-  auto flush = [&](int ro, int co) {
-    int nu[4];
-#pragma unroll
-    for (int cb = 0; cb < 4; ++cb) {
-      const int lc = co * kMxSupW * kTile + 64 * wc + 16 * cb + lrow;
-      nu[cb] = lc < nrow ? ao[lc] : -1;
-    }
-#pragma unroll
-    for (int r = 0; r < 8; ++r)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int lr = ro * kMxSupW * kTile + 128 * wr + 16 * r + 4 * lk + i;
-        const int mu = lr < nrow ? ao[lr] : -1;
-        if (mu < 0) continue;
-#pragma unroll
-        for (int cb = 0; cb < 4; ++cb)
-          if (nu[cb] >= 0) unsafeAtomicAdd(&Mint[(size_t)mu * npad + nu[cb]], (double)acc[r][cb][i]);
-      }
-  };
+    for (int c = 0; c < MT; ++c) acc[r][c] = f32x4{0.f, 0.f, 0.f, 0.f};
   dma(0, 0);
   for (int k = 0; k < nstage; ++k) {
-    if (NC == 4 && k == ntau && I < J) {  // 2 M_tau: the item's (I, J) block and, by symmetry, (J, I)
+    if (NC == 4 && k == ntau && !diag) {  // 2 M_tau
 #pragma unroll
-      for (int r = 0; r < 8; ++r)
+      for (int r = 0; r < MT; ++r)
 #pragma unroll
-        for (int c = 0; c < 4; ++c) acc[r][c] *= 2.f;
+        for (int c = 0; c < MT; ++c) acc[r][c] *= 2.f;
     }
-    if (k == kmirror) {  // M_IJ done: write it and start M_JI
-      flush(I, J);
-#pragma unroll
-      for (int r = 0; r < 8; ++r)
-#pragma unroll
-        for (int c = 0; c < 4; ++c) acc[r][c] = f32x4{0.f, 0.f, 0.f, 0.f};
-    }
-    int it, h, c;
-    bool mir;
-    decode(k, it, h, c, mir);
-    // this wave's row tiles 4 wr..4 wr+3 (bits of rmk) and column tiles 2 wc, 2 wc+1 (cmk) in the list
-    const unsigned rmk = (mk >> ((mir ? 8 : 0) + 4 * wr)) & 15u, cmk = (mk >> ((mir ? 0 : 8) + 2 * wc)) & 3u;
     __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this wave's fragments of step k are in LDS
     __syncthreads();                     // ... and every other wave's, and step k - 1's buffer is read
     if (k + 1 < nstage) dma(k + 1, (k + 1) & 1);
-    const u32x4* F = sm.F + (k & 1) * kVxWStep;
-    u32x4 a[8][2], bq[4][2];
+    const u32x4* F = sm.F[k & 1];
+    u32x4 a[MT][2];
 #pragma unroll
-    for (int r = 0; r < 8; ++r)
+    for (int r = 0; r < MT; ++r)
+      if (r < nI) {
 #pragma unroll
-      for (int hh = 0; hh < 2; ++hh) a[r][hh] = F[((8 * wr + r) * 2 + hh) * kDxFrag + fidx];
+        for (int hh = 0; hh < 2; ++hh) a[r][hh] = F[((r0 + r) * 2 + hh) * kDxFrag + fidx];
+      }
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
+    for (int c = 0; c < MT; ++c)
+      if (c < nc) {
+        const u32x4* Fc = F + (2 * RB + (c0 + c) * 2) * kDxFrag + fidx;
+        const u32x4 bh = Fc[0], bl = Fc[kDxFrag];
 #pragma unroll
-      for (int hh = 0; hh < 2; ++hh) bq[r][hh] = F[(kVxAW + (4 * wc + r) * 2 + hh) * kDxFrag + fidx];
-#pragma unroll
-    for (int cc = 0; cc < 4; ++cc)
-      if ((cmk >> (cc >> 1)) & 1u) {
-#pragma unroll
-        for (int r = 0; r < 8; ++r)
-          if ((rmk >> (r >> 1)) & 1u) acc[r][cc] = mfma3(a[r][0], a[r][1], bq[cc][0], bq[cc][1], acc[r][cc]);
+        for (int r = 0; r < MT; ++r)
+          if (r < nI) acc[r][c] = mfma3(a[r][0], a[r][1], bh, bl, acc[r][c]);
       }
   }
-  if (I < J) flush(J, I);
-  else flush(I, I);
+  float* __restrict__ U = m.U + wk.u;
+  const int ld = wk.ldu;
+  if (!diag) {
+#pragma unroll
+    for (int r = 0; r < MT; ++r)
+      if (r < nI) {
+#pragma unroll
+        for (int c = 0; c < MT; ++c)
+          if (c < nc) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+              U[(size_t)(16 * (r0 + r) + 4 * lk + i) * ld + 16 * (c0 + c) + lrow] = acc[r][c][i];
+          }
+      }
+    return;
+  }
+  // U = M + M^T, 64 rows at a time: the strip's 64 columns of M go to LDS transposed
+  float* T = reinterpret_cast<float*>(&sm.F[0][0]);
+  static_assert(sizeof(float) * 64 * PT <= sizeof(sm), "a strip fits the fragment buffers");
+  for (int s = 0; s < CB; s += 4) {
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < MT; ++c)
+      if (c < nc && c0 + c >= s && c0 + c < s + 4) {
+#pragma unroll
+        for (int r = 0; r < MT; ++r)
+          if (r < nI)
+            *reinterpret_cast<f32x4*>(T + (16 * (c0 + c - s) + lrow) * PT + 16 * (r0 + r) + 4 * lk) = acc[r][c];
+      }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < MT; ++r)
+      if (r < nI && r0 + r >= s && r0 + r < s + 4) {
+#pragma unroll
+        for (int c = 0; c < MT; ++c)
+          if (c < nc) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              const int row = 16 * (r0 + r) + 4 * lk + i, col = 16 * (c0 + c) + lrow;
+              U[(size_t)row * ld + col] = acc[r][c][i] + T[(row - 16 * s) * PT + col];
+            }
+          }
+      }
+  }
 }
-template <int NC>
-__global__ __launch_bounds__(512, 1) void k_vxc_mx_wide(MolDev m) {
-  vxc_mx_wide_body<NC>(m, xcd_remap(blockIdx.x, gridDim.x));
+template <int NC, int MT>
+__global__ __launch_bounds__(256, 2) void k_vxc_mx(MolDev m) {
+  vxc_mx_body<NC, MT>(m, xcd_remap(blockIdx.x, gridDim.x));
 }
 
 // ---------------------------------------------------------------------------
@@ -1369,7 +1293,7 @@ __device__ __forceinline__ MolDev rebase(const char* base, const MolDev& o) {
   m.part = rb(base, o.part); m.part_tau = rb(base, o.part_tau);
   m.slot_batch = rb(base, o.slot_batch); m.slot_tile = rb(base, o.slot_tile);
   m.coef = rb(base, o.coef); m.bt = rb(base, o.bt);
-  m.cwork = rb(base, o.cwork); m.Mint = rb(base, o.Mint);
+  m.cwork = rb(base, o.cwork); m.U = rb(base, o.U);
   m.cache3 = rb(base, o.cache3);
   m.core_off = rb(base, o.core_off); m.core_grps = rb(base, o.core_grps); m.main_grps = rb(base, o.main_grps);
   return m;
@@ -1414,26 +1338,14 @@ __global__ __launch_bounds__(256) void k_make_b_mx_multi(const char* base, const
   }
 }
 
-template <int NC>
-__global__ __launch_bounds__(256, 3) void k_vxc_mx_multi(const char* base, const MolDev* __restrict__ tab,
+template <int NC, int MT>
+__global__ __launch_bounds__(256, 2) void k_vxc_mx_multi(const char* base, const MolDev* __restrict__ tab,
                                                          const int* __restrict__ starts, int nmol, int total) {
   int k = -1;
   for (int v = blockIdx.x; v < total; v += gridDim.x) {
     const int item = xcd_remap(v, total);
     k = item_owner_from(starts, nmol, item, k);
-    vxc_mx_body<NC>(rebase(base, tab[k]), item - starts[k]);
-    __syncthreads();
-  }
-}
-
-template <int NC>
-__global__ __launch_bounds__(512, 1) void k_vxc_mx_wide_multi(const char* base, const MolDev* __restrict__ tab,
-                                                              const int* __restrict__ starts, int nmol, int total) {
-  int k = -1;
-  for (int v = blockIdx.x; v < total; v += gridDim.x) {
-    const int item = xcd_remap(v, total);
-    k = item_owner_from(starts, nmol, item, k);
-    vxc_mx_wide_body<NC>(rebase(base, tab[k]), item - starts[k]);
+    vxc_mx_body<NC, MT>(rebase(base, tab[k]), item - starts[k]);
     __syncthreads();
   }
 }
@@ -1478,14 +1390,14 @@ void launch_stage_multi(hipStream_t s, int stage, int ncomp, const char* base, c
     }
     case kStageVxc: {
       if (ncomp != 1) throw Error(CHX_ERR_UNSUPPORTED, "persistent packs are built for LDA and GGA");
-      auto k = k_vxc_mx_multi<1>;
+      auto k = k_vxc_mx_multi<1, 4>;
       hipLaunchKernelGGL(k, dim3(persistent_blocks(k, 256, total)), dim3(256), 0, s, base, tab, starts, nmol, total);
       break;
     }
     case kStageVxcWide: {
       if (ncomp != 1) throw Error(CHX_ERR_UNSUPPORTED, "persistent packs are built for LDA and GGA");
-      auto k = k_vxc_mx_wide_multi<1>;
-      hipLaunchKernelGGL(k, dim3(persistent_blocks(k, 512, total)), dim3(512), 0, s, base, tab, starts, nmol, total);
+      auto k = k_vxc_mx_multi<1, 5>;
+      hipLaunchKernelGGL(k, dim3(persistent_blocks(k, 256, total)), dim3(256), 0, s, base, tab, starts, nmol, total);
       break;
     }
     default:
@@ -1494,21 +1406,16 @@ void launch_stage_multi(hipStream_t s, int stage, int ncomp, const char* base, c
   CHX_HIP(hipGetLastError());
 }
 
-void launch_vxc_mx_wide(hipStream_t s, int ncomp, int nitems, const MolDev& one) {
+void launch_vxc_mx(hipStream_t s, int ncomp, int wide, int nitems, const MolDev& one) {
   if (nitems == 0) return;
-  if (ncomp == 4)
-    hipLaunchKernelGGL((k_vxc_mx_wide<4>), dim3(nitems), dim3(512), 0, s, one);
+  if (wide && ncomp == 4)
+    hipLaunchKernelGGL((k_vxc_mx<4, 5>), dim3(nitems), dim3(256), 0, s, one);
+  else if (wide)
+    hipLaunchKernelGGL((k_vxc_mx<1, 5>), dim3(nitems), dim3(256), 0, s, one);
+  else if (ncomp == 4)
+    hipLaunchKernelGGL((k_vxc_mx<4, 4>), dim3(nitems), dim3(256), 0, s, one);
   else
-    hipLaunchKernelGGL((k_vxc_mx_wide<1>), dim3(nitems), dim3(512), 0, s, one);
-  CHX_HIP(hipGetLastError());
-}
-
-void launch_vxc_mx(hipStream_t s, int ncomp, int nitems, const MolDev& one) {
-  if (nitems == 0) return;
-  if (ncomp == 4)
-    hipLaunchKernelGGL((k_vxc_mx<4>), dim3(nitems), dim3(256), 0, s, one);
-  else
-    hipLaunchKernelGGL((k_vxc_mx<1>), dim3(nitems), dim3(256), 0, s, one);
+    hipLaunchKernelGGL((k_vxc_mx<1, 4>), dim3(nitems), dim3(256), 0, s, one);
   CHX_HIP(hipGetLastError());
 }
 

@@ -144,7 +144,7 @@ void fn_table(const chx_pack* p, int m0, int m1, std::vector<FnMolecule>& tab, c
     FnMolecule f{};
     f.grp_off = q[0] - base; f.part = q[1] - base; f.part_tau = q[2] - base; f.w = q[3] - base;
     f.rho = q[4] - base; f.coef = q[5] - base; f.en_part = q[6] - base; f.cpart = q[7] - base;
-    f.ncpart = corr_blocks(g->nbasis);
+    f.ncpart = assemble_blocks(g->nbasis);
     f.nslots = g->nbatches * kBatch;
     f.blk0 = blk;
     f.slot_en = m;
@@ -180,7 +180,7 @@ void build_persistent(chx_pack* p) {
         &d.grp_batch, &d.grp_tile, &d.grp_ntiles, &d.bt_off, &d.b_chunk, &d.chunks, &d.ao_of, &d.bx, &d.by, &d.bz,
         &d.bv.sh_xyz, &d.bv.sh_type, &d.bv.sh_nprim, &d.bv.sh_poff, &d.bv.p_exp, &d.bv.p_coef,
         &d.bv.tile_seg_off, &d.bv.seg, &d.bv.segrec, &d.bv.sh_atom, &d.cache, &d.Ds, &d.part, &d.part_tau,
-        &d.slot_batch, &d.slot_tile, &d.coef, &d.bt, &d.cwork, &d.Mint, &d.cache3, &d.core_off, &d.core_grps,
+        &d.slot_batch, &d.slot_tile, &d.coef, &d.bt, &d.cwork, &d.U, &d.cache3, &d.core_off, &d.core_grps,
         &d.main_grps};
   };
   auto get = [](void* f) {
@@ -201,14 +201,13 @@ void build_persistent(chx_pack* p) {
     }
   p->mol_base = (const char*)base;
   p->mol_tab.upload(mols, p->stream);
-  // per stage: density (the groups outside the core batches), core groups, B^T slots (+ the zero
-  // slot), Vxc items of 128-AO molecules, Vxc items of 256-AO molecules
+  // per stage: density (the groups outside the core batches), core groups, B^T slots, Vxc items of 128-AO molecules, Vxc items of 256-AO molecules
   std::vector<int> starts(5 * (size_t)(n + 1), 0);
   p->totals.assign(5, 0);
   for (int m = 0; m < n; ++m) {
     const chx_grid* g = p->grids[m];
-    const int ng = (int)g->grp_batch.size(), ncg = (int)g->core_grps.size(), nw = (int)g->cwork.size();
-    const int cnt[5] = {ng - ncg, ncg, (int)g->slot_tile.size() + 1, g->mx_wide ? 0 : nw, g->mx_wide ? nw : 0};
+    const int ng = (int)g->grp_batch.size(), ncg = (int)g->core_grps.size(), nw = (int)g->mwork.size();
+    const int cnt[5] = {ng - ncg, ncg, (int)g->slot_tile.size(), g->mx_wide ? 0 : nw, g->mx_wide ? nw : 0};
     for (int st = 0; st < 5; ++st) starts[(size_t)st * (n + 1) + m + 1] = starts[(size_t)st * (n + 1) + m] + cnt[st];
   }
   for (int st = 0; st < 5; ++st) p->totals[st] = starts[(size_t)st * (n + 1) + n];
@@ -240,7 +239,7 @@ void build_lanes(chx_pack* p) {
   const int n = (int)p->grids.size();
   std::vector<double> cum(n + 1, 0.0);
   for (int m = 0; m < n; ++m)
-    cum[m + 1] = cum[m] + (double)p->grids[m]->grp_batch.size() + (double)p->grids[m]->cwork.size();
+    cum[m + 1] = cum[m] + (double)p->grids[m]->grp_batch.size() + (double)p->grids[m]->mwork.size();
   const int L = std::max(1, std::min(p->lanes, n));
   p->cut.assign(L + 1, n);
   int c = 0;
@@ -291,6 +290,10 @@ void build_lanes(chx_pack* p) {
 // arguments are those of the single-grid build.
 bool stages_ok(const chx_pack* p) { return p->type <= 1 && p->family <= 1; }
 
+void assemble(hipStream_t s, const chx_grid* g, double* V) {
+  launch_assemble_mx(s, g->nbasis, g->d_rowptr.p, g->d_rows.p, g->d_ao_of.p, g->d_U.p, V, g->d_Dres.p, g->d_cpart.p);
+}
+
 // Form 2: the lane's molecules in one launch per stage (the persistent stage
 // kernels over the lane's part of the descriptor table).
 void enqueue_lane_stages(chx_pack* p, int lane, hipStream_t s, hipEvent_t after, hipEvent_t dens_done,
@@ -300,7 +303,6 @@ void enqueue_lane_stages(chx_pack* p, int lane, hipStream_t s, hipEvent_t after,
     chx_grid* g = p->grids[m];
     launch_split_d(s, (int)g->tile_chunk.size(), g->nbasis, D[m], g->d_tile_chunk.p, g->d_chunks.p, g->d_ao_of.p,
                    g->d_Dsplit.p, g->d_Dres.p);
-    launch_fill(s, g->d_Mint.p, (size_t)g->npad * g->npad, 0.0);
   }
   if (after) CHX_HIP(hipStreamWaitEvent(s, after, 0));
   const int* st = p->d_lane_starts.p + p->lane_soff[lane];
@@ -317,7 +319,7 @@ void enqueue_lane_stages(chx_pack* p, int lane, hipStream_t s, hipEvent_t after,
   stage(kStageVxcWide);
   for (int m = m0; m < m1; ++m) {
     chx_grid* g = p->grids[m];
-    launch_finalize_corr(s, g->nbasis, g->npad, g->d_Mint.p, V[m], g->d_Dres.p, g->d_cpart.p);
+    assemble(s, g, V[m]);
   }
   launch_corr_multi(s, p->fn_base[lane], p->fn_tab.p + p->fn_off[lane], nl, p->d_en.p);
 }
@@ -350,19 +352,16 @@ void enqueue_lane(chx_pack* p, int lane, hipStream_t s, hipEvent_t after, hipEve
   for (int m = m0; m < m1; ++m) {
     chx_grid* g = p->grids[m];
     launch_make_b_mx(s, nc, g->hmol);
-    if (g->mx_wide)
-      launch_vxc_mx_wide(s, nc, (int)g->cwork.size(), g->hmol);
-    else
-      launch_vxc_mx(s, nc, (int)g->cwork.size(), g->hmol);
-    launch_finalize_corr(s, g->nbasis, g->npad, g->d_Mint.p, V[m], g->d_Dres.p, g->d_cpart.p);
+    launch_vxc_mx(s, nc, g->mx_wide, (int)g->mwork.size(), g->hmol);
+    assemble(s, g, V[m]);
   }
   launch_corr_multi(s, p->fn_base[lane], p->fn_tab.p + p->fn_off[lane], m1 - m0, p->d_en.p);
 }
 
 // One XC build of every molecule as persistent stages on the pack's stream
-// (LDA/GGA): per molecule split D and clear M; then one launch per stage over
+// (LDA/GGA): per molecule split D; then one launch per stage over
 // every molecule's items (density, core batches, functional, B^T, Vxc of each
-// block shape); per molecule V = M + M^T with the partial sums of
+// block shape); per molecule the assembly of V with the partial sums of
 // V . (D - hi - lo), and one launch for the energies' corrections.
 void enqueue_persistent(chx_pack* p, const double* const* D, double* const* V) {
   const int n = (int)p->grids.size();
@@ -371,7 +370,6 @@ void enqueue_persistent(chx_pack* p, const double* const* D, double* const* V) {
     chx_grid* g = p->grids[m];
     launch_split_d(s, (int)g->tile_chunk.size(), g->nbasis, D[m], g->d_tile_chunk.p, g->d_chunks.p, g->d_ao_of.p,
                    g->d_Dsplit.p, g->d_Dres.p);
-    launch_fill(s, g->d_Mint.p, (size_t)g->npad * g->npad, 0.0);
   }
   const int* st = p->d_starts.p;
   auto stage = [&](int k) {
@@ -386,7 +384,7 @@ void enqueue_persistent(chx_pack* p, const double* const* D, double* const* V) {
   stage(kStageVxcWide);
   for (int m = 0; m < n; ++m) {
     chx_grid* g = p->grids[m];
-    launch_finalize_corr(s, g->nbasis, g->npad, g->d_Mint.p, V[m], g->d_Dres.p, g->d_cpart.p);
+    assemble(s, g, V[m]);
   }
   launch_corr_multi(s, p->fn_all_base, p->fn_all.p, n, p->d_en.p);
 }
