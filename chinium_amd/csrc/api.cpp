@@ -151,19 +151,20 @@ void density_from_device(chx_grid* g, const double* dD, int spin = 0) {
   if (g->precision == CHX_PREC_MIXED) {
     g->mark_begin(kStPermute, &e);
     const int ncg = (int)g->core_grps.size();
+    g->hmol.gen = ++g->d_gen;
     launch_split_d(g->stream, (int)g->tile_chunk.size(), g->nbasis, dD, g->d_tile_chunk.p, g->d_chunks.p, g->d_ao_of.p,
-                   g->d_Dsplit.p, g->d_Dres.p + (size_t)spin * g->nbasis * g->nbasis);
+                   g->d_Dsplit.p, g->d_Dres.p + (size_t)spin * g->nbasis * g->nbasis, g->d_asym.p, g->hmol.gen);
     g->mark_end(kStPermute, e);
     g->mark_begin(kStDensity, &e);
     // meta-GGA: rho, grad rho and the tau partials (A = d_r phi) in one launch that stages D once
     // (rho, grad rho alone: the core batches' groups are left to the core launch)
-    launch_density_mx(g->stream, g->type >= 2 ? 5 : 0, g->type >= 2 ? ng : ng - ncg, g->hmol);
+    launch_density_mx(g->stream, g->type >= 2, g->type >= 2 ? ng : ng - ncg, g->hmol);
     g->mark_end(kStDensity, e);
     // core batches' rho and grad rho with three-term AO operands (meta-GGA: overwriting their
     // partials; tau keeps two terms: near the nuclei its error is far below rho's effect on E_xc)
     if (ncg) {
       g->mark_begin(kStCore, &e);
-      launch_density_mx_core(g->stream, 0, ncg, g->hmol);
+      launch_density_mx_core(g->stream, ncg, g->hmol);
       g->mark_end(kStCore, e);
     }
     g->have_density = true;

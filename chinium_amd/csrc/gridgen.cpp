@@ -617,6 +617,7 @@ void grid_plan(chx_grid* g) {
     r.ax = g->sh_xyz[3 * sh]; r.ay = g->sh_xyz[3 * sh + 1]; r.az = g->sh_xyz[3 * sh + 2];
     r.meta = (g->sh_type[sh] & 0xff) | (std::min(np, kSegPrim) << 8) | (sg.y << 16) | (sg.z << 24);
     r.col = sg.w;
+    if (k > 0 && sg.w > 0 && g->sh_atom[g->seg[k - 1].x] == g->sh_atom[sh]) r.meta |= kSegSame;
     for (int p = 0; p < np && p < kSegPrim; ++p) {
       r.e[p] = (float)g->p_exp[po + p];
       r.c[p] = (float)g->p_coef[po + p];
@@ -745,6 +746,13 @@ void grid_plan(chx_grid* g) {
   g->d_en_part.alloc(2 * (size_t)g->en_blocks);
   g->d_en.alloc(3);
   launch_fill(st, g->d_en.p, 3, 0.0);
+  if (mixed && g->type >= 2) {
+    g->d_asym.alloc(1);
+    launch_fill_u32(st, (unsigned*)g->d_asym.p, 1, 0u);
+  } else {
+    g->d_asym.release();
+  }
+  g->d_gen = 0;
   if (mixed) {  // split remainder of D per spin, and the partial sums of V . remainder
     g->d_Dres.alloc(2 * (size_t)g->nbasis * g->nbasis);
     g->d_cpart.alloc(2 * (size_t)assemble_blocks(g->nbasis));
@@ -763,6 +771,7 @@ void grid_plan(chx_grid* g) {
     m.slot_batch = g->d_slot_batch.p; m.slot_tile = g->d_slot_tile.p;
     m.coef = g->d_coef.p; m.bt = g->d_bmx.p;
     m.cache3 = g->d_cmx3.p;
+    m.asym = g->d_asym.p;
     m.core_off = g->d_core_off.p;
     m.core_grps = g->d_core_grps.p;
     m.main_grps = g->core_grps.empty() ? nullptr : g->d_main_grps.p;

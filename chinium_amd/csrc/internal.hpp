@@ -93,6 +93,7 @@ template <class T> struct DevBuf {
 // One shell segment of a tile with everything its evaluation reads, so that a
 // wave fetches it with two scalar loads (mixed-precision form).
 constexpr int kSegPrim = 12;  // primitives per record
+constexpr int kSegSame = 1 << 15;  // meta: the same centre as the record before (in the tile)
 struct SegRec {
   double ax, ay, az;  // shell centre
   int meta;           // type & 0xff | nprim << 8 | first component << 16 | count << 24
@@ -286,6 +287,8 @@ struct MolDev {
   // other batches (the (rho, grad rho) launch's groups; null: every group)
   const unsigned short* cache3;
   const int *core_off, *core_grps, *main_grps;
+  const int* asym;  // == gen: this build's D is not symmetric (meta-GGA)
+  int gen, pad2_;
 };
 constexpr int kMxMaxTiles = 512;  // basis size the mixed form takes (npad <= 16384)
 constexpr int kMxMaxChunk = 128;  // batches per Vxc work item in the mixed form
@@ -330,9 +333,10 @@ void launch_ao_cache_mx(hipStream_t s, int nslots, const int* slot_batch, const 
                         unsigned short* cache, const int* slot_core, unsigned short* cache3);
 // The chunks' dense blocks of D in split form (as launch_gather_d), and (all n^2
 // elements) R: what the two terms leave of D, D - hi - lo, in FP32 and in D's
-// own (reference, column-major) order
+// own (reference, column-major) order; asym (may be null): *asym = gen when D is
+// not symmetric to within rounding
 void launch_split_d(hipStream_t s, int ntiles, int n, const double* D, const int* tile_chunk, const ChunkDev* chunks,
-                    const int* ao_of, unsigned short* Ds, float* R);
+                    const int* ao_of, unsigned short* Ds, float* R, int* asym, int gen);
 // V (reference order) from the runs' blocks U and, with R, the first-order energy
 // correction for the split of D: partial sums of V . R into cpart
 // (assemble_blocks(n) of them); launch_reduce_corr sums nparts partials into *out.
@@ -345,11 +349,10 @@ void launch_corr_multi(hipStream_t s, const char* base, const FnMolecule* fm, in
 void launch_bf16_check(hipStream_t s, unsigned n, unsigned* bad);
 void launch_fill_u32(hipStream_t s, unsigned* p, size_t n, unsigned v);
 // One launch over the grid `one` (descriptor by value): density work groups,
-// B^T slot blocks, Vxc work items. Density mode 0: rho, grad rho; 4: the three
-// tau partials in one launch.
-void launch_density_mx(hipStream_t s, int mode, int nitems, const MolDev& one);
-// the core groups again with three-term operands: mode 0 (rho, grad rho) or r = 1..3 (tau partial r)
-void launch_density_mx_core(hipStream_t s, int mode, int ncore_groups, const MolDev& one);
+// B^T slot blocks, Vxc work items. Density: rho, grad rho; with_tau: tau too.
+void launch_density_mx(hipStream_t s, int with_tau, int nitems, const MolDev& one);
+// the core groups' rho, grad rho (again) with three-term operands
+void launch_density_mx_core(hipStream_t s, int ncore_groups, const MolDev& one);
 // B^T of every slot for ncomp components
 void launch_make_b_mx(hipStream_t s, int ncomp, const MolDev& one);
 // wide: groups of up to kMxWideTiles tiles instead of kMxTiles
@@ -458,6 +461,8 @@ struct chx_grid {
   chx::DevBuf<chx::RowRef> d_rows;
   chx::DevBuf<int> d_rowptr;
   chx::DevBuf<float> d_U;
+  chx::DevBuf<int> d_asym;              // number of the last build whose D was not symmetric
+  int d_gen = 0;                        // builds counted
   double flops_build = 0, mean_tiles = 0;
   std::vector<double> batch_work;  // g_b n_b^2 per batch (points x kept AOs squared)
   double core_flops = 0;           // the core batches' three-term (rho, grad rho) launch: 2 sum g_b n_b^2

@@ -173,15 +173,42 @@ void launch_ao_cache_mx(hipStream_t s, int nslots, const int* slot_batch, const 
 // included), at D's own position. The products see hi + lo; sum V . R, with V
 // the potential of this density, is the first-order energy of the remainder
 // (dE/dD = V), which the energy takes back when the potential is built
-// (k_finalize_corr). One launch: small molecules (and packs of them) are bound
-// by the launches.
+// (k_assemble_mx). With asym (meta-GGA) the last blocks compare D with D^T: an
+// element more than 1e-12 sqrt(D_ii D_jj) off (products of FP64 rounding stay far
+// below, as this does below the split) sets *asym = gen, this build's number.
+// One launch: small molecules (and packs of them) are bound by the launches.
 constexpr int kRestBlock = 4096;
 __global__ __launch_bounds__(256) void k_split_gather(int n, const double* __restrict__ D,
                                                       const int* __restrict__ tile_chunk,
                                                       const ChunkDev* __restrict__ chunks,
                                                       const int* __restrict__ ao_of, u16* __restrict__ Ds,
-                                                      int ntiles, long n2, float* __restrict__ R) {
+                                                      int ntiles, long n2, float* __restrict__ R, int nrest,
+                                                      int* __restrict__ asym, int gen) {
   const int t = blockIdx.x;
+  if (t >= ntiles + nrest) {  // 32 x 32 tile pair (i <= j) of the symmetry check
+    __shared__ double P[kTile][kTile + 1];
+    const int k = t - ntiles - nrest;
+    int j = (int)((sqrtf(8.f * (float)k + 1.f) - 1.f) * 0.5f);
+    while ((j + 1) * (j + 2) / 2 <= k) ++j;
+    while (j * (j + 1) / 2 > k) --j;
+    const int i = k - j * (j + 1) / 2;
+    for (int e = threadIdx.x; e < kTile * kTile; e += 256) {  // rows of tile j, columns of tile i
+      const int r = j * kTile + (e & 31), c = i * kTile + (e >> 5);
+      P[e >> 5][e & 31] = r < n && c < n ? D[(size_t)c * n + r] : 0.0;
+    }
+    __syncthreads();
+    bool bad = false;
+    for (int e = threadIdx.x; e < kTile * kTile; e += 256) {
+      const int r = i * kTile + (e & 31), c = j * kTile + (e >> 5);
+      if (r < n && c < n) {
+        const double u = D[(size_t)c * n + r], v = P[e & 31][e >> 5];
+        const double s = ::sqrt(::fabs(D[(size_t)r * n + r] * D[(size_t)c * n + c]));
+        bad = bad || !(::fabs(u - v) <= 1e-12 * s);
+      }
+    }
+    if (__ballot(bad) && (threadIdx.x & 63) == 0) *asym = gen;
+    return;
+  }
   if (t >= ntiles) {
     const long e0 = (long)(t - ntiles) * kRestBlock, e1 = e0 + kRestBlock < n2 ? e0 + kRestBlock : n2;
     for (long i = e0 + threadIdx.x; i < e1; i += 256) {
@@ -220,10 +247,12 @@ __global__ __launch_bounds__(256) void k_split_gather(int n, const double* __res
 }
 
 void launch_split_d(hipStream_t s, int ntiles, int n, const double* D, const int* tile_chunk, const ChunkDev* chunks,
-                    const int* ao_of, unsigned short* Ds, float* R) {
+                    const int* ao_of, unsigned short* Ds, float* R, int* asym, int gen) {
   const long n2 = (long)n * n;
-  const unsigned nb = (unsigned)(ntiles + (n2 + kRestBlock - 1) / kRestBlock);
-  hipLaunchKernelGGL(k_split_gather, dim3(nb), dim3(256), 0, s, n, D, tile_chunk, chunks, ao_of, Ds, ntiles, n2, R);
+  const int nrest = (int)((n2 + kRestBlock - 1) / kRestBlock), nt = (n + kTile - 1) / kTile;
+  const unsigned nb = (unsigned)(ntiles + nrest + (asym ? nt * (nt + 1) / 2 : 0));
+  hipLaunchKernelGGL(k_split_gather, dim3(nb), dim3(256), 0, s, n, D, tile_chunk, chunks, ao_of, Ds, ntiles, n2, R, nrest,
+                     asym, gen);
   CHX_HIP(hipGetLastError());
 }
 
@@ -456,6 +485,7 @@ template <bool PREFETCH = false, class Op>
 __device__ __forceinline__ void walk_tile_f32(const BasisView& bv, int t, double px, double py, double pz, Op& op) {
   using cint = const __attribute__((address_space(4))) int;
   const int s0 = ((cint*)bv.tile_seg_off)[t], s1 = ((cint*)bv.tile_seg_off)[t + 1];
+  float x = 0.f, y = 0.f, z = 0.f, r2 = 0.f;
   SegRec nxt;
   if (PREFETCH && s0 < s1) nxt = load_segrec(bv.segrec, s0);
   for (int k = s0; k < s1; ++k) {
@@ -466,10 +496,14 @@ __device__ __forceinline__ void walk_tile_f32(const BasisView& bv, int t, double
     } else {
       rec = load_segrec(bv.segrec, k);
     }
-    const float x = (float)(px - rec.ax), y = (float)(py - rec.ay), z = (float)(pz - rec.az);
-    const float r2 = x * x + y * y + z * z;
+    if (!(rec.meta & kSegSame)) {  // a new centre (the shells of an atom follow each other)
+      x = (float)(px - rec.ax);
+      y = (float)(py - rec.ay);
+      z = (float)(pz - rec.az);
+      r2 = x * x + y * y + z * z;
+    }
     float A0 = 0.f, A1 = 0.f;
-    switch ((rec.meta >> 8) & 0xff) {  // primitive count: straight-line code per count
+    switch ((rec.meta >> 8) & 0x7f) {  // primitive count: straight-line code per count
       case 1: radial_f32<1>(rec, r2, A0, A1); break;
       case 2: radial_f32<2>(rec, r2, A0, A1); break;
       case 3: radial_f32<3>(rec, r2, A0, A1); break;
@@ -494,44 +528,48 @@ __device__ __forceinline__ void walk_tile_f32(const BasisView& bv, int t, double
   }
 }
 
-// Density epilogue on one tile: sum_nu X[g][nu] phi_nu and sum_nu X[g][nu] grad phi_nu
-// (MODE 0), or sum_nu X_r[g][nu] d_r phi_nu (MODE r), as
-// R sum X Q + grad R sum X Q and R sum X grad Q per shell.
+// Density epilogue on one tile at this lane's point, as sums per shell of X Q
+// and X grad Q times R and grad R: with X = Phi D, o[0] = sum_nu X_nu phi_nu and
+// o[1..3] = sum_nu X_nu grad phi_nu; TAU: with X_r = (d_r Phi) D also
+// o[4] = sum_r sum_nu X_r,nu d_r phi_nu, from the same walk over the shells (the
+// walk, not the MFMAs, is most of a GGA density on lists of a few hundred AOs).
+// X is held in registers (uniform column index: no memory access).
 typedef float f32x32 __attribute__((ext_vector_type(32)));
-template <int MODE>
+template <bool TAU>
 struct DensEpi {
-  f32x32 xv;  // X of this tile at this lane's point, in registers (uniform column index: no memory access)
-  float o[4] = {0.f, 0.f, 0.f, 0.f};
-  float R, Rx, Ry, Rz, S0, Sx, Sy, Sz;
+  f32x32 xv[TAU ? 4 : 1];
+  float o[TAU ? 5 : 4] = {};
+  float R, Rx, Ry, Rz, S0, Sx, Sy, Sz, T0, Tx, Ty, Tz;
   // xq: X^T of this tile at this lane's point, xq[col * (kBatch + 1)]
-  __device__ void load(const float* xq) {
+  __device__ void load(int d, const float* xq) {
 #pragma unroll
-    for (int c = 0; c < kTile; ++c) xv[c] = xq[c * (kBatch + 1)];
+    for (int c = 0; c < kTile; ++c) xv[d][c] = xq[c * (kBatch + 1)];
   }
   __device__ void begin(float a, float ax, float ay, float az) {
     R = a; Rx = ax; Ry = ay; Rz = az;
     S0 = Sx = Sy = Sz = 0.f;
+    if (TAU) T0 = Tx = Ty = Tz = 0.f;
   }
   __device__ void comp(int col, float q, float qx, float qy, float qz) {
-    const float x = xv[col];
-    S0 += x * q;
-    if (MODE == 0 || MODE == 1) Sx += x * qx;
-    if (MODE == 0 || MODE == 2) Sy += x * qy;
-    if (MODE == 0 || MODE == 3) Sz += x * qz;
+    const float v = xv[0][col];
+    S0 += v * q;
+    Sx += v * qx;
+    Sy += v * qy;
+    Sz += v * qz;
+    if (TAU) {
+      const float vx = xv[TAU ? 1 : 0][col], vy = xv[TAU ? 2 : 0][col], vz = xv[TAU ? 3 : 0][col];
+      T0 += vx * qx + vy * qy + vz * qz;
+      Tx += vx * q;
+      Ty += vy * q;
+      Tz += vz * q;
+    }
   }
   __device__ void end() {
-    if (MODE == 0) {
-      o[0] += R * S0;
-      o[1] += Rx * S0 + R * Sx;
-      o[2] += Ry * S0 + R * Sy;
-      o[3] += Rz * S0 + R * Sz;
-    } else if (MODE == 1) {
-      o[0] += Rx * S0 + R * Sx;
-    } else if (MODE == 2) {
-      o[0] += Ry * S0 + R * Sy;
-    } else {
-      o[0] += Rz * S0 + R * Sz;
-    }
+    o[0] += R * S0;
+    o[1] += Rx * S0 + R * Sx;
+    o[2] += Ry * S0 + R * Sy;
+    o[3] += Rz * S0 + R * Sz;
+    if (TAU) o[TAU ? 4 : 0] += R * T0 + Rx * Tx + Ry * Ty + Rz * Tz;
   }
 };
 
@@ -564,9 +602,7 @@ struct DensMxSmem {
   double px[kBatch], py[kBatch], pz[kBatch];
 };
 
-// MODE 0: A = phi; epilogue rho and grad rho / 2 (4 components into part).
-// MODE r = 1..3 (A = d phi / d x_r, epilogue sum X_r d_r phi, the tau partial
-// of direction r) is the single-direction form of k_density_mx_tau below.
+// A = phi; epilogue rho and grad rho / 2 (4 components into part).
 // P3 (core batches only): the AO operand carries a third bf16 term (x - hi -
 // lo, 24 significant bits in all) from the core slots' side cache, and a
 // product takes the five terms hi hi, lo hi, hi lo, lo2 hi and lo lo: the AO
@@ -578,16 +614,14 @@ struct DensMxSmem {
 // is known to address global memory, and uniform table reads become scalar
 // loads; a descriptor read from device memory would leave them flat).
 // r: the block's item (after the XCD-aware remap) within the molecule's launch.
-template <int MODE, bool P3>
+template <bool P3>
 __device__ __forceinline__ void density_mx_body(const MolDev& m, int r) {
   using lds_ptr = __attribute__((address_space(3))) void*;
-  constexpr int NOUT = MODE == 0 ? 4 : 1;
-  constexpr int grp_stride = (MODE == 0 ? 4 : 3) * kBatch;  // part: [group][4][64]; tau partials: [group][3][64]
   __shared__ DensMxSmem<P3> sm;
-  const int grp = P3 ? m.core_grps[r] : (MODE == 0 && m.main_grps) ? m.main_grps[r] : r;
-  const u16* __restrict__ cache = m.cache + (size_t)MODE * kMxT;
+  const int grp = P3 ? m.core_grps[r] : m.main_grps ? m.main_grps[r] : r;
+  const u16* __restrict__ cache = m.cache;
   const size_t sstride = (size_t)m.sstride;
-  double* __restrict__ part = MODE == 0 ? m.part : m.part_tau + (MODE - 1) * kBatch;
+  double* __restrict__ part = m.part;
   const BasisView bv = m.bv;  // descriptor fields in registers, read once
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -628,7 +662,7 @@ __device__ __forceinline__ void density_mx_body(const MolDev& m, int r) {
   const u16* __restrict__ c3 = nullptr;
   if (P3) {
     // this batch's core slots in the side cache: [core slot][c][g][mu]
-    c3 = m.cache3 + ((size_t)m.core_off[b] * (m.toff / 2) + (size_t)MODE * kBatch * kTile) +
+    c3 = m.cache3 + ((size_t)m.core_off[b] * (m.toff / 2)) +
          (16 * wave + drow) * kTile + 8 * dch;
   }
   __syncthreads();
@@ -695,201 +729,44 @@ __device__ __forceinline__ void density_mx_body(const MolDev& m, int r) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) sm.X[64 * wc + 16 * c + lrow][32 * wr + 16 * r + 4 * lk + i] = acc[r][c][i];
   __syncthreads();
-  DensEpi<MODE> epi;
+  DensEpi<false> epi;
   if (wave < nt) {  // wave q = tile q of the group; lane = point
-    const int t = j0 + wave;
-    epi.load(&sm.X[kTile * wave][lane]);
-    walk_tile_f32<true>(bv, t, sm.px[lane], sm.py[lane], sm.pz[lane], epi);
+    epi.load(0, &sm.X[kTile * wave][lane]);
+    walk_tile_f32<true>(bv, j0 + wave, sm.px[lane], sm.py[lane], sm.pz[lane], epi);
   }
 #pragma unroll
-  for (int c = 0; c < NOUT; ++c) sm.red[wave][c][lane] = epi.o[c];
+  for (int c = 0; c < 4; ++c) sm.red[wave][c][lane] = epi.o[c];
   __syncthreads();
-  if (tid < NOUT * kBatch) {
+  {
     const int c = tid / kBatch, g = tid % kBatch;
     double v = 0.0;
     for (int q = 0; q < nt; ++q) v += (double)sm.red[q][c][g];
-    part[(size_t)grp * grp_stride + c * kBatch + g] = v;
+    part[(size_t)grp * 4 * kBatch + c * kBatch + g] = v;
   }
 }
-template <int MODE, bool P3>
+template <bool P3>
 __global__ __launch_bounds__(256, P3 ? 2 : 4) void k_density_mx(MolDev m) {
-  density_mx_body<MODE, P3>(m, xcd_remap(blockIdx.x, gridDim.x));
+  density_mx_body<P3>(m, xcd_remap(blockIdx.x, gridDim.x));
 }
 
-// The three tau partials in one block: per K step the three A = d_r phi
-// operands (24 fragments) and the D block (16 fragments, shared by the three
-// products) go to LDS together, so D is staged and read once instead of three
-// times and a step takes two barriers instead of six. Three accumulator sets;
-// the epilogue runs the MODE r contraction for r = 1, 2, 3 in turn through the
-// X staging area. Same indexing as k_density_mx.
-struct DensMxTauSmem {
-  union {
-    u32x4 F[(3 * kDxA + kDxB) * kDxFrag];  // one K step's fragments: A_1, A_2, A_3, D
-    float X[kGroup * kTile][kBatch + 1];   // epilogue: X_r^T [nu][g]
-  };
-  float red[kGroup][3][kBatch];
-  double px[kBatch], py[kBatch], pz[kBatch];
-};
-
-template <int R>
-__device__ __forceinline__ void dens_tau_epilogue(DensMxTauSmem& sm, const f32x4 (&acc)[2][4], const BasisView& bv,
-                                                  int j0, int nt, int wave, int lane, int wr,
-                                                  int wc, int lrow, int lk) {
-  __syncthreads();  // the previous user of the X area (fragments or X_{R-1}) is done
-#pragma unroll
-  for (int r = 0; r < 2; ++r)
-#pragma unroll
-    for (int c = 0; c < 4; ++c)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) sm.X[64 * wc + 16 * c + lrow][32 * wr + 16 * r + 4 * lk + i] = acc[r][c][i];
-  __syncthreads();
-  DensEpi<R> epi;
-  if (wave < nt) {
-    const int t = j0 + wave;
-    epi.load(&sm.X[kTile * wave][lane]);
-    walk_tile_f32<true>(bv, t, sm.px[lane], sm.py[lane], sm.pz[lane], epi);
-  }
-  sm.red[wave][R - 1][lane] = epi.o[0];
-}
-
-__global__ __launch_bounds__(256, 2) void k_density_mx_tau(MolDev m) {
-  using lds_ptr = __attribute__((address_space(3))) void*;
-  __shared__ DensMxTauSmem sm;
-  const int grp = xcd_remap(blockIdx.x, gridDim.x);
-  const u16* __restrict__ cache = m.cache + (size_t)kMxT;  // component 1 (d_x phi); d_y, d_z follow
-  const size_t sstride = (size_t)m.sstride;
-  double* __restrict__ part = m.part_tau;  // [group][3][64]
-  const BasisView bv = m.bv;
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int lrow = lane & 15, lk = lane >> 4;
-  const int wr = wave & 1, wc = wave >> 1;
-  const int b = m.grp_batch[grp];
-  const int nt = m.grp_ntiles[grp], j0 = m.grp_tile[grp];
-  const ChunkDev ch = m.chunks[m.b_chunk[b]];
-  const int it0 = m.bt_off[b], nk = ch.ntl, ld = nk * kTile;
-  if (tid < kBatch) {
-    sm.px[tid] = m.bx[b * kBatch + tid];
-    sm.py[tid] = m.by[b * kBatch + tid];
-    sm.pz[tid] = m.bz[b * kBatch + tid];
-  }
-  const int drow = lane >> 2, dch = (lane & 3) ^ ((drow >> 2) & 3);
-  const int fidx = 4 * lrow + (lk ^ ((lrow >> 2) & 3));
-  int offa[2], offb[4];
-#pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int f = wave + 4 * j;
-    offa[j] = (16 * (f >> 1) + drow) * kMxRow + (f & 1) * kTile + 8 * dch;
-  }
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int f = wave + 4 * j, c = f >> 1, q = c >> 1;
-    offb[j] = (f & 1) * ld * ld + ((j0 - ch.tile0 + (q < nt ? q : 0)) * kTile + 16 * (c & 1) + drow) * ld + 8 * dch;
-  }
-  const u16* __restrict__ Ds = m.Ds + 2 * ch.doff;
-  __syncthreads();
-  auto dma = [&](int k) {
-    const u16* a = cache + (size_t)(it0 + k) * sstride;
-#pragma unroll
-    for (int r = 0; r < 3; ++r)
-#pragma unroll
-      for (int j = 0; j < 2; ++j)
-        __builtin_amdgcn_global_load_lds(a + (size_t)r * kMxT + offa[j],
-                                         (lds_ptr)(sm.F + (r * kDxA + wave + 4 * j) * kDxFrag), 16, 0, 0);
-    const int ti = k * kTile;
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      __builtin_amdgcn_global_load_lds(Ds + offb[j] + ti, (lds_ptr)(sm.F + (3 * kDxA + wave + 4 * j) * kDxFrag), 16,
-                                       0, 0);
-  };
-
-  f32x4 acc[3][2][4];
-#pragma unroll
-  for (int d = 0; d < 3; ++d)
-#pragma unroll
-    for (int r = 0; r < 2; ++r)
-#pragma unroll
-      for (int c = 0; c < 4; ++c) acc[d][r][c] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int ncb = 2 * (nt - 2 * wc);
-  dma(0);
-  for (int k = 0; k < nk; ++k) {
-    __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this wave's fragments of step k are in LDS
-    __syncthreads();                     // ... and every other wave's
-    u32x4 a[3][2][2], bq[4][2];
-#pragma unroll
-    for (int d = 0; d < 3; ++d)
-#pragma unroll
-      for (int r = 0; r < 2; ++r)
-#pragma unroll
-        for (int h = 0; h < 2; ++h) a[d][r][h] = sm.F[(d * kDxA + (2 * wr + r) * 2 + h) * kDxFrag + fidx];
-#pragma unroll
-    for (int c = 0; c < 4; ++c)
-#pragma unroll
-      for (int h = 0; h < 2; ++h) bq[c][h] = sm.F[(3 * kDxA + (4 * wc + c) * 2 + h) * kDxFrag + fidx];
-    __syncthreads();  // every wave holds its fragments: the buffer is free
-    if (k + 1 < nk) dma(k + 1);
-#pragma unroll
-    for (int c = 0; c < 4; ++c)
-      if (c < ncb) {
-#pragma unroll
-        for (int d = 0; d < 3; ++d)
-#pragma unroll
-          for (int r = 0; r < 2; ++r)
-            acc[d][r][c] = mfma3(a[d][r][0], a[d][r][1], bq[c][0], bq[c][1], acc[d][r][c]);
-      }
-  }
-  dens_tau_epilogue<1>(sm, acc[0], bv, j0, nt, wave, lane, wr, wc, lrow, lk);
-  dens_tau_epilogue<2>(sm, acc[1], bv, j0, nt, wave, lane, wr, wc, lrow, lk);
-  dens_tau_epilogue<3>(sm, acc[2], bv, j0, nt, wave, lane, wr, wc, lrow, lk);
-  __syncthreads();
-  if (tid < 3 * kBatch) {
-    const int c = tid / kBatch, g = tid % kBatch;
-    double v = 0.0;
-    for (int q = 0; q < nt; ++q) v += (double)sm.red[q][c][g];
-    part[(size_t)grp * 3 * kBatch + c * kBatch + g] = v;
-  }
-}
-
-// Meta-GGA density in one launch: the four products Phi D and d_r Phi D share
-// one D block per K step (48 fragments: A_0..A_3, then D), so D is staged
-// once per build instead of once for rho and once for the tau partials.
-// Epilogues: rho and grad rho / 2 into part (as k_density_mx<0>), then the
-// three tau partials into part_tau (as k_density_mx_tau). Same indexing as
-// k_density_mx.
+// Meta-GGA density in one launch: the products Phi D and (d_r Phi) D share one D
+// block per K step (48 fragments: A_0..A_3, then D); one walk over the shells
+// contracts all four (DensEpi<true>) into rho, grad rho / 2 and tau. Same
+// indexing as k_density_mx. tau = sum_r x_r^T D x_r (x_r = d_r phi) is a
+// quadratic form, so for a symmetric D its products stop at the group's own
+// tiles: K steps before them count twice (the accumulators are doubled when the
+// group's first tile is reached), steps after them carry rho alone. A D that
+// the symmetry check (k_split_gather) flagged takes every step once.
+// (H2O)48 / def2-SVP / SG-2: 2.6 ms, against 5.0 with every step and a walk per
+// component.
 struct DensMxMggaSmem {
   union {
     u32x4 F[(4 * kDxA + kDxB) * kDxFrag];  // one K step's fragments: A_0..A_3, D
     float X[kGroup * kTile][kBatch + 1];
   };
-  float red[kGroup][4][kBatch];
+  float red[kGroup][5][kBatch];
   double px[kBatch], py[kBatch], pz[kBatch];
 };
-
-template <int R>
-__device__ __forceinline__ void dens_mgga_epilogue(DensMxMggaSmem& sm, const f32x4 (&acc)[2][4], const BasisView& bv,
-                                                   int j0, int nt, int wave, int lane, int wr, int wc,
-                                                   int lrow, int lk) {
-  __syncthreads();  // the previous user of the X area is done
-#pragma unroll
-  for (int r = 0; r < 2; ++r)
-#pragma unroll
-    for (int c = 0; c < 4; ++c)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) sm.X[64 * wc + 16 * c + lrow][32 * wr + 16 * r + 4 * lk + i] = acc[r][c][i];
-  __syncthreads();
-  DensEpi<R> epi;
-  if (wave < nt) {
-    const int t = j0 + wave;
-    epi.load(&sm.X[kTile * wave][lane]);
-    walk_tile_f32<true>(bv, t, sm.px[lane], sm.py[lane], sm.pz[lane], epi);
-  }
-  if (R == 0) {
-#pragma unroll
-    for (int c = 0; c < 4; ++c) sm.red[wave][c][lane] = epi.o[c];
-  } else {
-    sm.red[wave][R - 1][lane] = epi.o[0];
-  }
-}
 
 __global__ __launch_bounds__(256, 2) void k_density_mx_mgga(MolDev m) {
   using lds_ptr = __attribute__((address_space(3))) void*;
@@ -926,10 +803,15 @@ __global__ __launch_bounds__(256, 2) void k_density_mx_mgga(MolDev m) {
   }
   const u16* __restrict__ Ds = m.Ds + 2 * ch.doff;
   __syncthreads();
+  const bool sym = *m.asym != m.gen;
+  const int t0 = j0 - ch.tile0;                // the group's first tile
+  const int ktau = sym ? t0 + nt : nk;         // steps that carry tau
   auto dma = [&](int k) {
     const u16* a = cache + (size_t)(it0 + k) * sstride;
+    const int nd = k < ktau ? 4 : 1;
 #pragma unroll
     for (int r = 0; r < 4; ++r)
+      if (r < nd)
 #pragma unroll
       for (int j = 0; j < 2; ++j)
         __builtin_amdgcn_global_load_lds(a + (size_t)r * kMxT + offa[j],
@@ -951,11 +833,21 @@ __global__ __launch_bounds__(256, 2) void k_density_mx_mgga(MolDev m) {
   const int ncb = 2 * (nt - 2 * wc);
   dma(0);
   for (int k = 0; k < nk; ++k) {
+    const bool tau = k < ktau;
+    if (sym && k == t0) {
+#pragma unroll
+      for (int d = 1; d < 4; ++d)
+#pragma unroll
+        for (int r = 0; r < 2; ++r)
+#pragma unroll
+          for (int c = 0; c < 4; ++c) acc[d][r][c] *= 2.f;
+    }
     __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this wave's fragments of step k are in LDS
     __syncthreads();                     // ... and every other wave's
     u32x4 a[4][2][2], bq[4][2];
 #pragma unroll
     for (int d = 0; d < 4; ++d)
+      if (d == 0 || tau)
 #pragma unroll
       for (int r = 0; r < 2; ++r)
 #pragma unroll
@@ -971,54 +863,52 @@ __global__ __launch_bounds__(256, 2) void k_density_mx_mgga(MolDev m) {
       if (c < ncb) {
 #pragma unroll
         for (int d = 0; d < 4; ++d)
+          if (d == 0 || tau)
 #pragma unroll
           for (int r = 0; r < 2; ++r)
             acc[d][r][c] = mfma3(a[d][r][0], a[d][r][1], bq[c][0], bq[c][1], acc[d][r][c]);
       }
   }
-  dens_mgga_epilogue<0>(sm, acc[0], bv, j0, nt, wave, lane, wr, wc, lrow, lk);
-  __syncthreads();
-  if (tid < 4 * kBatch) {
-    const int c = tid / kBatch, g = tid % kBatch;
-    double v = 0.0;
-    for (int q = 0; q < nt; ++q) v += (double)sm.red[q][c][g];
-    m.part[(size_t)grp * 4 * kBatch + c * kBatch + g] = v;
+  DensEpi<true> epi;
+#pragma unroll
+  for (int d = 0; d < 4; ++d) {  // X_d -> LDS as X_d^T -> registers of the lane that holds the point
+    __syncthreads();  // the previous user of the X area is done
+#pragma unroll
+    for (int r = 0; r < 2; ++r)
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) sm.X[64 * wc + 16 * c + lrow][32 * wr + 16 * r + 4 * lk + i] = acc[d][r][c][i];
+    __syncthreads();
+    epi.load(d, &sm.X[kTile * wave][lane]);
   }
-  dens_mgga_epilogue<1>(sm, acc[1], bv, j0, nt, wave, lane, wr, wc, lrow, lk);
-  dens_mgga_epilogue<2>(sm, acc[2], bv, j0, nt, wave, lane, wr, wc, lrow, lk);
-  dens_mgga_epilogue<3>(sm, acc[3], bv, j0, nt, wave, lane, wr, wc, lrow, lk);
+  if (wave < nt) walk_tile_f32<true>(bv, j0 + wave, sm.px[lane], sm.py[lane], sm.pz[lane], epi);
+#pragma unroll
+  for (int c = 0; c < 5; ++c) sm.red[wave][c][lane] = epi.o[c];
   __syncthreads();
-  if (tid < 3 * kBatch) {
-    const int c = tid / kBatch, g = tid % kBatch;
+  for (int e = tid; e < 7 * kBatch; e += 256) {
+    const int c = e / kBatch, g = e % kBatch;
     double v = 0.0;
-    for (int q = 0; q < nt; ++q) v += (double)sm.red[q][c][g];
-    m.part_tau[(size_t)grp * 3 * kBatch + c * kBatch + g] = v;
+    for (int q = 0; q < nt; ++q) v += c < 5 ? (double)sm.red[q][c][g] : 0.0;
+    if (c < 4)
+      m.part[(size_t)grp * 4 * kBatch + c * kBatch + g] = v;
+    else  // part_tau: [group][3][64], summed over the directions in the first
+      m.part_tau[(size_t)grp * 3 * kBatch + (c - 4) * kBatch + g] = v;
   }
 }
 
-void launch_density_mx_core(hipStream_t s, int mode, int ncore_groups, const MolDev& one) {
+void launch_density_mx_core(hipStream_t s, int ncore_groups, const MolDev& one) {
   if (ncore_groups == 0) return;
-  const dim3 g(ncore_groups), b(256);
-  switch (mode) {
-    case 0: hipLaunchKernelGGL((k_density_mx<0, true>), g, b, 0, s, one); break;
-    case 1: hipLaunchKernelGGL((k_density_mx<1, true>), g, b, 0, s, one); break;
-    case 2: hipLaunchKernelGGL((k_density_mx<2, true>), g, b, 0, s, one); break;
-    case 3: hipLaunchKernelGGL((k_density_mx<3, true>), g, b, 0, s, one); break;
-    default: throw Error(CHX_ERR_ARG, "core density mode must be 0..3");
-  }
+  hipLaunchKernelGGL((k_density_mx<true>), dim3(ncore_groups), dim3(256), 0, s, one);
   CHX_HIP(hipGetLastError());
 }
 
-void launch_density_mx(hipStream_t s, int mode, int nitems, const MolDev& one) {
+void launch_density_mx(hipStream_t s, int with_tau, int nitems, const MolDev& one) {
   if (nitems == 0) return;
-  if (mode == 0)
-    hipLaunchKernelGGL((k_density_mx<0, false>), dim3(nitems), dim3(256), 0, s, one);
-  else if (mode == 4)  // the three tau partials in one launch
-    hipLaunchKernelGGL(k_density_mx_tau, dim3(nitems), dim3(256), 0, s, one);
-  else if (mode == 5)  // rho, grad rho and the tau partials in one launch
+  if (with_tau)
     hipLaunchKernelGGL(k_density_mx_mgga, dim3(nitems), dim3(256), 0, s, one);
   else
-    throw Error(CHX_ERR_ARG, "density mode must be 0 (rho, grad rho), 4 (tau partials) or 5 (both)");
+    hipLaunchKernelGGL((k_density_mx<false>), dim3(nitems), dim3(256), 0, s, one);
   CHX_HIP(hipGetLastError());
 }
 
@@ -1295,6 +1185,7 @@ __device__ __forceinline__ MolDev rebase(const char* base, const MolDev& o) {
   m.coef = rb(base, o.coef); m.bt = rb(base, o.bt);
   m.cwork = rb(base, o.cwork); m.U = rb(base, o.U);
   m.cache3 = rb(base, o.cache3);
+  m.asym = rb(base, o.asym);
   m.core_off = rb(base, o.core_off); m.core_grps = rb(base, o.core_grps); m.main_grps = rb(base, o.main_grps);
   return m;
 }
@@ -1314,7 +1205,7 @@ __device__ __forceinline__ int item_owner_from(const int* __restrict__ starts, i
   return k;
 }
 
-template <int MODE, bool P3>
+template <bool P3>
 __global__ __launch_bounds__(256, P3 ? 2 : 4) void k_density_mx_multi(const char* base, const MolDev* __restrict__ tab,
                                                                       const int* __restrict__ starts, int nmol,
                                                                       int total) {
@@ -1322,7 +1213,7 @@ __global__ __launch_bounds__(256, P3 ? 2 : 4) void k_density_mx_multi(const char
   for (int v = blockIdx.x; v < total; v += gridDim.x) {
     const int item = xcd_remap(v, total);
     k = item_owner_from(starts, nmol, item, k);
-    density_mx_body<MODE, P3>(rebase(base, tab[k]), item - starts[k]);
+    density_mx_body<P3>(rebase(base, tab[k]), item - starts[k]);
     __syncthreads();  // the next item reuses the block's LDS
   }
 }
@@ -1372,12 +1263,12 @@ void launch_stage_multi(hipStream_t s, int stage, int ncomp, const char* base, c
   if (total <= 0) return;
   switch (stage) {
     case kStageDensity: {
-      auto k = k_density_mx_multi<0, false>;
+      auto k = k_density_mx_multi<false>;
       hipLaunchKernelGGL(k, dim3(persistent_blocks(k, 256, total)), dim3(256), 0, s, base, tab, starts, nmol, total);
       break;
     }
     case kStageCore: {
-      auto k = k_density_mx_multi<0, true>;
+      auto k = k_density_mx_multi<true>;
       hipLaunchKernelGGL(k, dim3(persistent_blocks(k, 256, total)), dim3(256), 0, s, base, tab, starts, nmol, total);
       break;
     }

@@ -176,12 +176,12 @@ void build_persistent(chx_pack* p) {
   // every pointer field of a descriptor (the fields rebase() offsets), read and
   // written as addresses through memcpy
   auto fields = [](MolDev& d) {
-    return std::array<void*, 34>{
+    return std::array<void*, 35>{
         &d.grp_batch, &d.grp_tile, &d.grp_ntiles, &d.bt_off, &d.b_chunk, &d.chunks, &d.ao_of, &d.bx, &d.by, &d.bz,
         &d.bv.sh_xyz, &d.bv.sh_type, &d.bv.sh_nprim, &d.bv.sh_poff, &d.bv.p_exp, &d.bv.p_coef,
         &d.bv.tile_seg_off, &d.bv.seg, &d.bv.segrec, &d.bv.sh_atom, &d.cache, &d.Ds, &d.part, &d.part_tau,
         &d.slot_batch, &d.slot_tile, &d.coef, &d.bt, &d.cwork, &d.U, &d.cache3, &d.core_off, &d.core_grps,
-        &d.main_grps};
+        &d.main_grps, &d.asym};
   };
   auto get = [](void* f) {
     uintptr_t v;
@@ -301,8 +301,9 @@ void enqueue_lane_stages(chx_pack* p, int lane, hipStream_t s, hipEvent_t after,
   const int m0 = p->cut[lane], m1 = p->cut[lane + 1], nl = m1 - m0;
   for (int m = m0; m < m1; ++m) {
     chx_grid* g = p->grids[m];
+    g->hmol.gen = ++g->d_gen;
     launch_split_d(s, (int)g->tile_chunk.size(), g->nbasis, D[m], g->d_tile_chunk.p, g->d_chunks.p, g->d_ao_of.p,
-                   g->d_Dsplit.p, g->d_Dres.p);
+                   g->d_Dsplit.p, g->d_Dres.p, g->d_asym.p, g->hmol.gen);
   }
   if (after) CHX_HIP(hipStreamWaitEvent(s, after, 0));
   const int* st = p->d_lane_starts.p + p->lane_soff[lane];
@@ -333,16 +334,17 @@ void enqueue_lane(chx_pack* p, int lane, hipStream_t s, hipEvent_t after, hipEve
   const int m0 = p->cut[lane], m1 = p->cut[lane + 1];
   for (int m = m0; m < m1; ++m) {
     chx_grid* g = p->grids[m];
+    g->hmol.gen = ++g->d_gen;
     launch_split_d(s, (int)g->tile_chunk.size(), g->nbasis, D[m], g->d_tile_chunk.p, g->d_chunks.p, g->d_ao_of.p,
-                   g->d_Dsplit.p, g->d_Dres.p);
+                   g->d_Dsplit.p, g->d_Dres.p, g->d_asym.p, g->hmol.gen);
   }
   if (after) CHX_HIP(hipStreamWaitEvent(s, after, 0));
   for (int m = m0; m < m1; ++m) {
     chx_grid* g = p->grids[m];
     const int ng = (int)g->grp_batch.size(), ncg = (int)g->core_grps.size();
-    launch_density_mx(s, p->type >= 2 ? 5 : 0, p->type >= 2 ? ng : ng - ncg, g->hmol);
+    launch_density_mx(s, p->type >= 2, p->type >= 2 ? ng : ng - ncg, g->hmol);
     // core batches' rho and grad rho again with three-term AO operands
-    launch_density_mx_core(s, 0, (int)g->core_grps.size(), g->hmol);
+    launch_density_mx_core(s, (int)g->core_grps.size(), g->hmol);
   }
   if (dens_done) CHX_HIP(hipEventRecord(dens_done, s));
   const int nc = p->family >= 2 ? 4 : 1;
@@ -368,8 +370,9 @@ void enqueue_persistent(chx_pack* p, const double* const* D, double* const* V) {
   hipStream_t s = p->stream;
   for (int m = 0; m < n; ++m) {
     chx_grid* g = p->grids[m];
+    g->hmol.gen = ++g->d_gen;
     launch_split_d(s, (int)g->tile_chunk.size(), g->nbasis, D[m], g->d_tile_chunk.p, g->d_chunks.p, g->d_ao_of.p,
-                   g->d_Dsplit.p, g->d_Dres.p);
+                   g->d_Dsplit.p, g->d_Dres.p, g->d_asym.p, g->hmol.gen);
   }
   const int* st = p->d_starts.p;
   auto stage = [&](int k) {

@@ -81,3 +81,25 @@ def test_coarse_threshold_moves_little():
     assert g.stats()["mean_tiles"] < full.stats()["mean_tiles"]
     E6, V6 = ca.xc_build(g, xc, D)
     assert abs(E6 - E) <= 1e-4 and np.abs(V6 - V).max() <= 1e-4
+
+
+@pytest.mark.parametrize("form", [ca.CHX_PREC_FP64, ca.CHX_PREC_MIXED])
+@pytest.mark.parametrize("name", ["H", "water sto-3g", "C12"])
+def test_tau_of_a_nonsymmetric_matrix(name, form):
+    """rho and tau are quadratic forms: an antisymmetric part of D adds nothing. A symmetric D takes half of
+    tau's products, one with an antisymmetric part all of them; one with rounding-level asymmetry (products
+    like C C^T formed elsewhere) still counts as symmetric. Bounds: the forms' own rounding, 2^-16 of
+    sum |D| |d phi| |d phi| (mixed), of which tau is about 1/10 at these densities."""
+    mol, _, D = _system(name)
+    n = len(D)
+    S = np.random.default_rng(5).standard_normal((n, n)) * np.abs(D).max() * 0.05
+    g = _grid(mol, 2, form)
+    out = []
+    for M in (D, D + (S - S.T), D + 1e-16 * np.abs(D).max() * S):
+        g.getDensity([M])
+        rho, _, tau, w = g.pointDensity()
+        out.append((rho[w != 0], tau[w != 0]))
+    tol = 1e-12 if form == ca.CHX_PREC_FP64 else 2e-4
+    for k in (1, 2):
+        for a, b in zip(out[0], out[k]):
+            assert np.abs(a - b).max() <= tol * np.abs(a).max()
