@@ -134,10 +134,10 @@ void run_functional(chx_grid* g, const chx_xc* xc, bool want_e, bool want_v) {
   g->mark_end(2, e);
 }
 
-// The chunks' dense blocks of a device matrix D (FP64 form).
-void gather_d(chx_grid* g, const double* dD, DevBuf<double>& Dt) {
+// The chunks' dense blocks of a device matrix D (FP64 form); with_tau: checked for symmetry.
+void gather_d(chx_grid* g, const double* dD, DevBuf<double>& Dt, bool with_tau = false) {
   launch_gather_d(g->stream, (int)g->tile_chunk.size(), g->nbasis, dD, g->d_tile_chunk.p, g->d_chunks.p, g->d_ao_of.p,
-                  Dt.alloc_get(std::max<size_t>(1, g->dt_elems)));
+                  Dt.alloc_get(std::max<size_t>(1, g->dt_elems)), with_tau ? g->d_asym.p : nullptr, g->d_gen);
 }
 
 // Stage ids of chx_grid_kernel_times.
@@ -173,16 +173,14 @@ void density_from_device(chx_grid* g, const double* dD, int spin = 0) {
     return;
   }
   g->mark_begin(kStPermute, &e);
-  gather_d(g, dD, g->d_Dt);
+  ++g->d_gen;
+  gather_d(g, dD, g->d_Dt, g->type >= 2);
   g->mark_end(kStPermute, e);
   g->mark_begin(kStDensity, &e);
   if (g->cached) {
-    launch_density_c64(g->stream, 0, ng, g->d_grp_batch.p, g->d_grp_tile.p, g->d_grp_ntiles.p,
-                           g->d_bt_off.p, g->d_b_chunk.p, g->d_chunks.p, g->d_cache.p, g->d_Dt.p, g->d_part.p);
-    if (g->type >= 2)  // tau: three more contractions with A = d_r phi
-      for (int r = 1; r <= 3; ++r)
-        launch_density_c64(g->stream, r, ng, g->d_grp_batch.p, g->d_grp_tile.p, g->d_grp_ntiles.p,
-                           g->d_bt_off.p, g->d_b_chunk.p, g->d_chunks.p, g->d_cache.p, g->d_Dt.p, g->d_part_tau.p + (size_t)(r - 1) * kBatch);
+    launch_density_c64(g->stream, ng, g->d_grp_batch.p, g->d_grp_tile.p, g->d_grp_ntiles.p, g->d_bt_off.p,
+                       g->d_b_chunk.p, g->d_chunks.p, g->d_cache.p, g->d_Dt.p, g->d_asym.p, g->d_gen, g->d_part.p,
+                       g->type >= 2 ? g->d_part_tau.p : nullptr);
   } else {  // AO values recomputed in the kernels
     launch_density_f64(g->stream, 0, ng, g->d_grp_batch.p, g->d_grp_tile.p, g->d_grp_ntiles.p, g->d_b_chunk.p,
                          g->d_chunks.p, g->d_x.p, g->d_y.p, g->d_z.p, g->view(), g->d_Dt.p, g->d_part.p);
@@ -211,7 +209,7 @@ void fock_to_device(chx_grid* g, double* dV, int spin = 0) {
     launch_vxc_mx(g->stream, nc, g->mx_wide, (int)g->mwork.size(), g->hmol);
     g->mark_end(kStVxc, e);
     g->mark_begin(kStFinalize, &e);
-    launch_assemble_mx(g->stream, g->nbasis, g->d_rowptr.p, g->d_rows.p, g->d_ao_of.p, g->d_U.p, dV,
+    launch_assemble<float>(g->stream, g->nbasis, g->d_rowptr.p, g->d_rows.p, g->d_ao_of.p, g->d_U.p, dV,
                        g->corr_pending ? g->d_Dres.p + (size_t)spin * g->nbasis * g->nbasis : nullptr,
                        g->d_cpart.p + (size_t)spin * assemble_blocks(g->nbasis));
     g->mark_end(kStFinalize, e);
@@ -220,14 +218,15 @@ void fock_to_device(chx_grid* g, double* dV, int spin = 0) {
   if (g->cached) {
     const int nc = g->v_family >= 2 ? 4 : 1;
     g->mark_begin(kStMakeB, &e);
-    launch_make_b(g->stream, g->nbatches, g->d_bt_off.p, g->d_coef.p, g->d_cache.p, g->d_bmat.p, g->d_Mint.p,
-                  (size_t)g->npad * g->npad);
+    launch_make_b(g->stream, g->nbatches, g->d_bt_off.p, g->d_coef.p, g->d_cache.p, g->d_bmat.p);
     g->mark_end(kStMakeB, e);
     g->mark_begin(kStVxc, &e);
-    launch_vxc_c64(g->stream, nc, (int)g->cwork.size(), g->d_cwork.p, g->d_ao_of.p, g->d_cache.p, g->d_bmat.p, g->d_coef.p, g->d_Mint.p, g->npad);
+    launch_vxc_c64(g->stream, nc, (int)g->mwork.size(), g->d_mwork.p, g->d_cache.p, g->d_bmat.p, g->d_coef.p,
+                   g->d_U64.p);
     g->mark_end(kStVxc, e);
     g->mark_begin(kStFinalize, &e);
-    launch_finalize_sym(g->stream, g->nbasis, g->npad, g->d_Mint.p, dV);
+    launch_assemble<double>(g->stream, g->nbasis, g->d_rowptr.p, g->d_rows.p, g->d_ao_of.p, g->d_U64.p, dV, nullptr,
+                            nullptr);
     g->mark_end(kStFinalize, e);
     return;
   }
@@ -518,8 +517,8 @@ int chx_grid_get_density_u(chx_grid* g, const double* D, int nmats, int nspin, i
       CHX_HIP(hipMemcpyAsync(g->d_Din.p, D + m * nb2, sizeof(double) * nb2, hipMemcpyHostToDevice, g->stream));
       gather_d(g, g->d_Din.p, g->d_Dt);
       if (g->cached)
-        launch_density_c64(g->stream, 0, ng, g->d_grp_batch.p, g->d_grp_tile.p, g->d_grp_ntiles.p,
-                           g->d_bt_off.p, g->d_b_chunk.p, g->d_chunks.p, g->d_cache.p, g->d_Dt.p, part);
+        launch_density_c64(g->stream, ng, g->d_grp_batch.p, g->d_grp_tile.p, g->d_grp_ntiles.p, g->d_bt_off.p,
+                           g->d_b_chunk.p, g->d_chunks.p, g->d_cache.p, g->d_Dt.p, nullptr, 0, part, nullptr);
       else
         launch_density_f64(g->stream, 0, ng, g->d_grp_batch.p, g->d_grp_tile.p, g->d_grp_ntiles.p, g->d_b_chunk.p,
                          g->d_chunks.p, g->d_x.p, g->d_y.p, g->d_z.p, g->view(), g->d_Dt.p, part);
@@ -550,10 +549,10 @@ static void response_fock(chx_grid* g, const double* rhou, int nmats, double* F,
       launch_response_coef(g->stream, g->nbatches, rhou + (size_t)m * 4 * nslots, g->d_fx.p, g->d_w.p, g->fx_family,
                            coef);
     if (g->cached) {  // B = a phi + c . grad phi from the tables, M = Phi^T B, V = M + M^T
-      launch_make_b(g->stream, g->nbatches, g->d_bt_off.p, coef, g->d_cache.p, g->d_bmat.p, g->d_Mint.p,
-                    (size_t)g->npad * g->npad);
-      launch_vxc_c64(g->stream, 1, (int)g->cwork.size(), g->d_cwork.p, g->d_ao_of.p, g->d_cache.p, g->d_bmat.p, coef, g->d_Mint.p, g->npad);
-      launch_finalize_sym(g->stream, g->nbasis, g->npad, g->d_Mint.p, g->d_Vout.p);
+      launch_make_b(g->stream, g->nbatches, g->d_bt_off.p, coef, g->d_cache.p, g->d_bmat.p);
+      launch_vxc_c64(g->stream, 1, (int)g->mwork.size(), g->d_mwork.p, g->d_cache.p, g->d_bmat.p, coef, g->d_U64.p);
+      launch_assemble<double>(g->stream, g->nbasis, g->d_rowptr.p, g->d_rows.p, g->d_ao_of.p, g->d_U64.p, g->d_Vout.p,
+                              nullptr, nullptr);
     } else {
       launch_fill(g->stream, g->d_Mint.p, (size_t)g->npad * g->npad, 0.0);
       launch_vxc_f64(g->stream, 1, (int)g->vwork.size(), g->d_vwork.p, g->d_ao_of.p, g->d_x.p, g->d_y.p, g->d_z.p,
@@ -646,7 +645,7 @@ int chx_grid_fock_skeleton(chx_grid* g, double* F, int nspin, int nbasis) {
       for (int k = 0; k < chx::shell_size(sh.type); ++k) ao_atom[sh.ao_off + k] = sh.center;
     DevBuf<int> d_atom;
     d_atom.upload(ao_atom, g->stream);
-    launch_make_b(g->stream, g->nbatches, g->d_bt_off.p, g->d_coef.p, g->d_cache.p, g->d_bmat.p, nullptr, 0);
+    launch_make_b(g->stream, g->nbatches, g->d_bt_off.p, g->d_coef.p, g->d_cache.p, g->d_bmat.p);
     DevBuf<double> etab, qp, out;
     etab.alloc(std::max<size_t>(1, 3 * (size_t)ns * sb));
     launch_fill(g->stream, etab.p, 3 * (size_t)ns * sb, 0.0);
@@ -656,11 +655,11 @@ int chx_grid_fock_skeleton(chx_grid* g, double* F, int nspin, int nbasis) {
     launch_fill(g->stream, qp.p, 6 * pp, 0.0);
     for (int t = 0; t < 3; ++t) {
       // Q^t = (d_t Phi)^T B: the cached component t + 1 as the row operand
-      launch_vxc_c64(g->stream, 1, (int)g->cwork.size(), g->d_cwork.p, g->d_ao_of.p, g->d_cache.p + (size_t)(t + 1) * sb, g->d_bmat.p, g->d_coef.p, qp.p + t * pp,
-                     g->npad);
+      launch_prod_c64(g->stream, (int)g->pwork.size(), g->d_pwork.p, g->d_ao_of.p, g->d_cache.p + (size_t)(t + 1) * sb, g->d_bmat.p,
+                      qp.p + t * pp, g->npad);
       // P^t = Phi^T E^t: E^t in the B table's place
-      launch_vxc_c64(g->stream, 1, (int)g->cwork.size(), g->d_cwork.p, g->d_ao_of.p, g->d_cache.p, etab.p + (size_t)t * ns * sb, g->d_coef.p, qp.p + (3 + t) * pp,
-                     g->npad);
+      launch_prod_c64(g->stream, (int)g->pwork.size(), g->d_pwork.p, g->d_ao_of.p, g->d_cache.p, etab.p + (size_t)t * ns * sb,
+                      qp.p + (3 + t) * pp, g->npad);
     }
     const size_t tot = (size_t)3 * na * n * n;
     out.alloc(std::max<size_t>(1, tot));
@@ -710,7 +709,7 @@ int chx_grid_energy_hess(chx_grid* g, double* H) {
     launch_skel_rho(g->stream, ns, g->d_slot_batch.p, g->d_slot_tile.p, g->d_slot_grp.p, g->d_slot_q.p, g->d_x.p,
                     g->d_y.p, g->d_z.p, g->view(), xz1.p, xz2.p, npt, rhos.p);
     // rr[3 t + s] = (d_t Phi)^T E^s over the cached contraction
-    launch_make_b(g->stream, g->nbatches, g->d_bt_off.p, g->d_coef.p, g->d_cache.p, g->d_bmat.p, nullptr, 0);
+    launch_make_b(g->stream, g->nbatches, g->d_bt_off.p, g->d_coef.p, g->d_cache.p, g->d_bmat.p);
     etab.alloc(std::max<size_t>(1, 3 * (size_t)ns * sb));
     launch_fill(g->stream, etab.p, 3 * (size_t)ns * sb, 0.0);
     launch_skel_etab(g->stream, ns, g->d_slot_batch.p, g->d_slot_tile.p, g->d_x.p, g->d_y.p, g->d_z.p, g->view(),
@@ -719,8 +718,8 @@ int chx_grid_energy_hess(chx_grid* g, double* H) {
     launch_fill(g->stream, rr.p, 9 * pp, 0.0);
     for (int t = 0; t < 3; ++t)
       for (int u = 0; u < 3; ++u)
-        launch_vxc_c64(g->stream, 1, (int)g->cwork.size(), g->d_cwork.p, g->d_ao_of.p, g->d_cache.p + (size_t)(t + 1) * sb, etab.p + (size_t)u * ns * sb, g->d_coef.p,
-                       rr.p + (size_t)(3 * t + u) * pp, g->npad);
+        launch_prod_c64(g->stream, (int)g->pwork.size(), g->d_pwork.p, g->d_ao_of.p, g->d_cache.p + (size_t)(t + 1) * sb, etab.p + (size_t)u * ns * sb,
+                      rr.p + (size_t)(3 * t + u) * pp, g->npad);
     dH.alloc((size_t)np * np);
     launch_fill(g->stream, dH.p, (size_t)np * np, 0.0);
     launch_hess_terms(g->stream, ns, g->d_slot_batch.p, g->d_slot_tile.p, g->d_slot_grp.p, g->d_slot_q.p, g->d_x.p,
@@ -740,7 +739,7 @@ int chx_grid_energy_grad(chx_grid* g, double* grad) {
     require(g->v_nspin == 1, CHX_ERR_UNSUPPORTED, "the XC gradient is built for the closed-shell path");
     const int na = g->mol.natoms, ng = (int)g->grp_batch.size(), ns = (int)g->slot_tile.size();
     ensure_slot_groups(g);
-    launch_make_b(g->stream, g->nbatches, g->d_bt_off.p, g->d_coef.p, g->d_cache.p, g->d_bmat.p, nullptr, 0);
+    launch_make_b(g->stream, g->nbatches, g->d_bt_off.p, g->d_coef.p, g->d_cache.p, g->d_bmat.p);
     DevBuf<double> xz, dg;
     xz.alloc(std::max<size_t>(1, (size_t)ng * 2 * kGroup * kTile * kBatch));
     dg.alloc(3 * (size_t)na);

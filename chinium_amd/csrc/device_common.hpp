@@ -97,4 +97,36 @@ __device__ __forceinline__ int xcd_remap(int i, int n) {
   return x * q + (x < r ? x : r) + i / kXcd;
 }
 
+// Symmetry check of D (n x n, column-major): one 256-thread block per pair k of
+// 32 x 32 tiles (i <= j); an element further than rel sqrt(D_ii D_jj) from its
+// transpose sets *asym = gen.
+__device__ __forceinline__ void check_symmetry(int k, int n, const double* __restrict__ D, double rel,
+                                               int* __restrict__ asym, int gen) {
+  __shared__ double P[kTile][kTile + 1];
+  int j = (int)((sqrtf(8.f * (float)k + 1.f) - 1.f) * 0.5f);
+  while ((j + 1) * (j + 2) / 2 <= k) ++j;
+  while (j * (j + 1) / 2 > k) --j;
+  const int i = k - j * (j + 1) / 2;
+  for (int e = threadIdx.x; e < kTile * kTile; e += 256) {  // rows of tile j, columns of tile i
+    const int r = j * kTile + (e & 31), c = i * kTile + (e >> 5);
+    P[e >> 5][e & 31] = r < n && c < n ? D[(size_t)c * n + r] : 0.0;
+  }
+  __syncthreads();
+  bool bad = false;
+  for (int e = threadIdx.x; e < kTile * kTile; e += 256) {
+    const int r = i * kTile + (e & 31), c = j * kTile + (e >> 5);
+    if (r < n && c < n) {
+      const double u = D[(size_t)c * n + r], v = P[e & 31][e >> 5];
+      const double s = ::sqrt(::fabs(D[(size_t)r * n + r] * D[(size_t)c * n + c]));
+      bad = bad || !(::fabs(u - v) <= rel * s);
+    }
+  }
+  if (__ballot(bad) && (threadIdx.x & 63) == 0) *asym = gen;
+}
+// tile pairs of the check
+inline int symmetry_blocks(int n) {
+  const int t = (n + kTile - 1) / kTile;
+  return t * (t + 1) / 2;
+}
+
 }  // namespace chx

@@ -446,17 +446,19 @@ static void build_items(const chx_grid* g, int sup, bool upper, int len, std::ve
 }
 
 // The longest run (a power of two up to the chunk length) that still leaves
-// enough items. A run's blocks are written once (FP64 form: one atomic per
-// element), so long runs write less; but an item is a serial chain of its run's
-// K steps, which shows unless several times more items than the chip holds are
-// there. Times by run length, in us, Vxc launch and V's assembly: (H2O)16 /
-// def2-SVP / SG-1 mixed 82 + 90 (4), 84 + 40 (8), 173 + 20 (32); (H2O)4 14 + 25
-// (2), 16 + 15 (4), 69 + 10 (32); (H2O)128 2640 + 1300 (8), 2280 + 700 (32);
-// C7H16 FP64 323 (1), 179 (8), 307 (32); H2O FP64 18 (1), 260 (32).
+// enough items. A run's blocks are written once, so long runs write less; but an
+// item is a serial chain of its run's K steps, which shows unless several times
+// more items than the chip holds are there. An FP64 step is some ten times as
+// long, so runs past 4 batches do not pay there. Times by run length, in us, Vxc
+// launch and V's assembly: (H2O)16 / def2-SVP / SG-1 mixed 82 + 90 (4), 84 + 40
+// (8), 173 + 20 (32); (H2O)4 14 + 25 (2), 16 + 15 (4), 69 + 10 (32); (H2O)128
+// 2640 + 1300 (8), 2280 + 700 (32). Builds in FP64: (H2O)16 1140 (1), 977 (4),
+// 1141 (16); C18 / def2-TZVP r2SCAN 2317 (1), 2298 (4), 2665 (16); H2O 97 (1), 105 (4).
 static int default_len(const chx_grid* g, int sup, bool upper) {
   const bool mixed = g->precision == CHX_PREC_MIXED;
   for (int len = kChunkMax; len > 1; len /= 2) {
-    const long want = !mixed ? 384 : len > 8 ? 4096 : 160;
+    if (!mixed && len > 4) continue;
+    const long want = len > 8 ? 4096 : 160;
     long n = 0;
     for (size_t c = 0; c < g->chunks.size(); ++c) {
       const long ns = (g->chunks[c].ntl + sup - 1) / sup, nb = g->chunk_b0[c + 1] - g->chunk_b0[c];
@@ -498,7 +500,7 @@ static void build_mwork(chx_grid* g, int sup, int len, std::vector<RowRef>& rows
         for (int J = I; J < ng; ++J) {
           const int J0 = ch.ntl * J / ng, J1 = ch.ntl * (J + 1) / ng;
           g->mwork.push_back(MxItem{(long)g->u_elems + (J0 - I0) * kTile, I0, I1 - I0, J0, J1 - J0, g->bt_off[b], nbat,
-                                    ch.ntl, ldu});
+                                    ch.ntl, ldu, ch.tile0, b});
         }
         for (int r = I0 * kTile; r < std::min(I1 * kTile, nreal); ++r)
           rows[at[g->ao_of[a0 + r]]++] = RowRef{(long)g->u_elems + (long)(r - I0 * kTile) * (ldu + 1), a0 + r, nreal - r};
@@ -508,27 +510,39 @@ static void build_mwork(chx_grid* g, int sup, int len, std::vector<RowRef>& rows
   }
 }
 
-// Vxc work items: FP64 form over 128-AO super-tiles, mixed form over groups of
-// up to kMxTiles tiles or (wide) kMxWideTiles. Uploads them and points the descriptor at them;
-// the host vectors outlive the copies (synchronises).
+// Vxc work items of the cached tables over groups of up to kMxTiles tiles or
+// (mixed form, wide) kMxWideTiles; FP64 form: also every pair of groups for the
+// plain products. Uploads them; the host vectors outlive the copies (synchronises).
 void build_cwork(chx_grid* g) {
   hipStream_t st = g->stream;
-  if (g->precision != CHX_PREC_MIXED) {
-    build_items(g, kCacheSuper, false, g->vxc_chunk > 0 ? g->vxc_chunk : default_len(g, kCacheSuper, false), g->cwork);
-    g->d_cwork.upload(g->cwork, st);
-    CHX_HIP(hipStreamSynchronize(st));
-    return;
-  }
-  const int sup = g->mx_wide ? kMxWideTiles : kMxTiles;
+  const bool mixed = g->precision == CHX_PREC_MIXED;
+  const int sup = mixed && g->mx_wide ? kMxWideTiles : kMxTiles;
   std::vector<RowRef> rows;
   std::vector<int> rowptr;
   build_mwork(g, sup, g->vxc_chunk > 0 ? g->vxc_chunk : default_len(g, sup, true), rows, rowptr);
   g->d_mwork.upload(g->mwork, st);
   g->d_rows.upload(rows, st);
   g->d_rowptr.upload(rowptr, st);
-  g->d_U.alloc(std::max<size_t>(1, g->u_elems));
-  g->hmol.cwork = g->d_mwork.p;
-  g->hmol.U = g->d_U.p;
+  g->pwork.clear();
+  if (mixed) {
+    g->d_U64.release();
+    g->d_U.alloc(std::max<size_t>(1, g->u_elems));
+    g->hmol.cwork = g->d_mwork.p;
+    g->hmol.U = g->d_U.p;
+  } else {
+    g->d_U.release();
+    g->d_U64.alloc(std::max<size_t>(1, g->u_elems));
+    for (const MxItem& m : g->mwork) {
+      g->pwork.push_back(m);
+      if (m.I0 != m.J0) {
+        MxItem t = m;
+        std::swap(t.I0, t.J0);
+        std::swap(t.nI, t.nJ);
+        g->pwork.push_back(t);
+      }
+    }
+  }
+  g->d_pwork.upload(g->pwork, st);
   CHX_HIP(hipStreamSynchronize(st));
 }
 
@@ -654,9 +668,8 @@ void grid_plan(chx_grid* g) {
   // large bases: Vxc items over 256 x 256 blocks
   g->mx_wide = mixed && (g->vxc_shape == 1 || (g->vxc_shape < 0 && g->npad >= 1024)) ? 1 : 0;
   g->vwork.clear();
-  g->cwork.clear();
   g->mwork.clear();
-  if (mixed) g->d_Mint.release();
+  if (g->cached) g->d_Mint.release();
   else g->d_Mint.alloc((size_t)g->npad * g->npad);
   if (g->cached) {
     if (mixed) {
@@ -746,7 +759,7 @@ void grid_plan(chx_grid* g) {
   g->d_en_part.alloc(2 * (size_t)g->en_blocks);
   g->d_en.alloc(3);
   launch_fill(st, g->d_en.p, 3, 0.0);
-  if (mixed && g->type >= 2) {
+  if (g->type >= 2) {
     g->d_asym.alloc(1);
     launch_fill_u32(st, (unsigned*)g->d_asym.p, 1, 0u);
   } else {

@@ -17,9 +17,8 @@ constexpr int kTile = 32;      // AOs per screening tile
 constexpr int kGroup = 4;      // AO tiles per density work group (128 output columns)
 constexpr int kSuper = 2;      // AO tiles per Vxc super-tile (64 x 64 output block)
 constexpr int kPadAO = 128;    // nbasis is padded to a multiple of this (4 tiles)
-constexpr int kCacheSuper = 4; // tiles per Vxc super-tile in the cached path
-constexpr int kMxTiles = 4;    // tiles per Vxc group of the mixed form (128 AOs)
-constexpr int kMxWideTiles = 5;  // ... of its wide shape (160 AOs)
+constexpr int kMxTiles = 4;    // tiles per Vxc group of the cached tables (128 AOs)
+constexpr int kMxWideTiles = 5;  // ... of the mixed form's wide shape (160 AOs)
 constexpr int kChunkMax = 32;  // most consecutive batches that share one AO list
 constexpr int kCoef = 5;       // Vxc integrand coefficients per point: a, c_x, c_y, c_z, t
 constexpr double kCoreRadius = 0.3;  // bohr: points this close to a nucleus with Z > 2 are batched apart
@@ -134,11 +133,11 @@ struct VxcItem {
   int I, J, slot0, nbat, ntl, tile0, batch0, pad_;
 };
 
-// Mixed form: tiles I0 .. I0 + nI - 1 against J0 .. J0 + nJ - 1 (I0 <= J0) of a
+// Cached tables: tiles I0 .. I0 + nI - 1 against J0 .. J0 + nJ - 1 (I0 <= J0) of a
 // run (nbat batches of a chunk); the block's place u in U and its row length.
 struct MxItem {
   long u;
-  int I0, nI, J0, nJ, slot0, nbat, ntl, ldu;
+  int I0, nI, J0, nJ, slot0, nbat, ntl, ldu, tile0, batch0;
 };
 // Row of one AO in a run's blocks: element k (k < len) is V at (that AO, ao_of[a0 + k]).
 struct RowRef {
@@ -156,8 +155,9 @@ void launch_screen(hipStream_t s, int nbatches, int nshells, int nwords, const d
                    unsigned long long* alive);
 // The chunks' dense blocks of D (FP64): block r of the launch gathers the 32
 // rows of tile r from D (reference order, column-major n x n), zero for padding.
+// asym (may be null): *asym = gen when D is not symmetric to within rounding.
 void launch_gather_d(hipStream_t s, int ntiles, int n, const double* D, const int* tile_chunk, const ChunkDev* chunks,
-                     const int* ao_of, double* Dt);
+                     const int* ao_of, double* Dt, int* asym, int gen);
 void launch_pad_d(hipStream_t s, int n, int npad, const double* D, double* Dpad);
 // mode 0: rho, grad rho / 2 into part ([group][4][64]); mode r = 1..3: the tau
 // partial of direction r (part = component r - 1 of [group][3][64]).
@@ -249,15 +249,20 @@ void launch_functional_mlp(hipStream_t s, int nbatches, const int* grp_off, cons
 void launch_point_density(hipStream_t s, int nbatches, const int* grp_off, const double* part,
                           const double* part_tau, int has_tau, const double* bw, double* rho, double* sigma,
                           double* tau, double* w);
-void launch_density_c64(hipStream_t s, int mode, int ngroups, const int* grp_batch, const int* grp_tile,
-                        const int* grp_ntiles, const int* bt_off, const int* b_chunk, const ChunkDev* chunks,
-                        const double* cache, const double* Dt, double* part);
-// B = a phi + c . grad phi per slot (one component for every family); clears the nfill elements at M
+// rho, grad rho / 2 into part; part_tau (not null: meta-GGA): tau (asym / gen as launch_gather_d's)
+void launch_density_c64(hipStream_t s, int ngroups, const int* grp_batch, const int* grp_tile, const int* grp_ntiles,
+                        const int* bt_off, const int* b_chunk, const ChunkDev* chunks, const double* cache,
+                        const double* Dt, const int* asym, int gen, double* part, double* part_tau);
+// B = a phi + c . grad phi per slot (one component for every family)
 void launch_make_b(hipStream_t s, int nbatches, const int* bt_off, const double* coef, const double* cache,
-                   double* bmat, double* M, size_t nfill);
-// ncomp 4 adds the tau term, its operand t d_r phi formed from the cache and coef[4] as it is loaded
-void launch_vxc_c64(hipStream_t s, int ncomp, int nwork, const VxcItem* work, const int* ao_of, const double* cache,
-                    const double* bmat, const double* coef, double* Mint, int npad);
+                   double* bmat);
+// upper blocks of V per run into U; ncomp 4 adds the tau term, its operand t d_r
+// phi formed from the cache and coef[4] as it is loaded
+void launch_vxc_c64(hipStream_t s, int ncomp, int nwork, const MxItem* work, const double* cache, const double* bmat,
+                    const double* coef, double* U);
+// M += A^T B over every pair of groups (items with I0, J0 in any order), A component 0 at `cache`
+void launch_prod_c64(hipStream_t s, int nwork, const MxItem* work, const int* ao_of, const double* cache,
+                     const double* bmat, double* M, int npad);
 void launch_finalize_sym(hipStream_t s, int n, int npad, const double* Mint, double* V);
 // Device descriptor of one grid for the mixed-precision kernels. A kernel
 // launch covers a list of (grid, item) pairs, so one launch can serve many
@@ -341,8 +346,9 @@ void launch_split_d(hipStream_t s, int ntiles, int n, const double* D, const int
 // correction for the split of D: partial sums of V . R into cpart
 // (assemble_blocks(n) of them); launch_reduce_corr sums nparts partials into *out.
 int assemble_blocks(int n);
-void launch_assemble_mx(hipStream_t s, int n, const int* rowptr, const RowRef* rows, const int* ao_of, const float* U,
-                        double* V, const float* R, double* cpart);
+template <class T>  // float (mixed form) or double
+void launch_assemble(hipStream_t s, int n, const int* rowptr, const RowRef* rows, const int* ao_of, const T* U,
+                     double* V, const float* R, double* cpart);
 void launch_reduce_corr(hipStream_t s, int nparts, const double* cpart, double* out);
 // the packed form: per molecule of the table, en[2 slot_en] += its ncpart partials
 void launch_corr_multi(hipStream_t s, const char* base, const FnMolecule* fm, int nmol, double* en);
@@ -445,8 +451,8 @@ struct chx_grid {
   int vxc_chunk = 0;                 // batches per Vxc work item; 0 = by the item count
   int vxc_shape = -1;                // mixed form's Vxc blocks: -1 by basis size, 0 128-AO super-tiles, 1 256-AO groups
   int mx_wide = 0;                   // mixed form: Vxc over 256-AO groups (large bases)
-  std::vector<chx::VxcItem> cwork;      // FP64 form
-  std::vector<chx::MxItem> mwork;       // mixed form
+  std::vector<chx::MxItem> mwork;       // Vxc work items of the cached tables
+  std::vector<chx::MxItem> pwork;       // FP64 form: items of the plain products (skeleton derivatives)
   size_t u_elems = 0;                   // elements of the runs' blocks of V
   // mixed form: core batches (density with three-term operands)
   double core_radius = chx::kCoreRadius;  // bohr; 0 turns the core treatment off
@@ -456,11 +462,11 @@ struct chx_grid {
   chx::DevBuf<int> d_core_off, d_core_grps, d_main_grps, d_slot_core;
   chx::DevBuf<double> d_cache, d_bmat, d_Mint;
   chx::DevBuf<int> d_slot_batch, d_slot_tile;
-  chx::DevBuf<chx::VxcItem> d_cwork;
-  chx::DevBuf<chx::MxItem> d_mwork;
+  chx::DevBuf<chx::MxItem> d_mwork, d_pwork;
   chx::DevBuf<chx::RowRef> d_rows;
   chx::DevBuf<int> d_rowptr;
   chx::DevBuf<float> d_U;
+  chx::DevBuf<double> d_U64;
   chx::DevBuf<int> d_asym;              // number of the last build whose D was not symmetric
   int d_gen = 0;                        // builds counted
   double flops_build = 0, mean_tiles = 0;

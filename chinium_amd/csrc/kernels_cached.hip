@@ -3,17 +3,25 @@
 // phi and grad phi do not change between SCF iterations, so they are computed
 // once per grid (at Grid::getAO, as the reference caches its AO tables,
 // src/Grid/Grid.cpp:22-33) for every (batch, 32-AO tile of its list) slot and kept in
-// HBM (~80 KB per slot: 4.4 GB at (H2O)16/def2-SVP/SG-2). Each iteration then
-// streams them through two MFMA contractions:
-//   density: X = Phi_b D_b (A = phi tiles, B = D blocks, both staged in LDS,
-//            double-buffered, next tile prefetched into registers), then
-//            rho = sum X phi and grad rho / 2 = sum X grad phi from the cache;
-//   Vxc:     M_IJ = Phi_I^T B_J over 128-AO super-tiles, B = a phi + c . grad phi
-//            built once per iteration by k_make_b; V = M + M^T at finalisation.
+// HBM (~80 KB per slot). Each iteration then streams them through two MFMA
+// contractions:
+//   density: X = Phi_b D_b, then rho = sum X phi and grad rho / 2 = sum X grad phi
+//            from the cache;
+//   Vxc:     V_IJ = Phi_I^T B_J + B_I^T Phi_J over groups of up to 128 of the
+//            list's AOs, B = a phi + c . grad phi built once per iteration by
+//            k_make_b, summed over the runs by k_assemble.
 // Meta-GGA adds tau = 1/2 sum_r (d_r Phi D) . d_r phi (three more density
-// contractions) and sum_r (d_r Phi)^T T_r to M (three more K components).
-// Layouts: cache[slot][c][g][32] (c = phi, d/dx, d/dy, d/dz), bmat[slot][NC][g][32].
+// products) and sum_r (d_r Phi)^T T_r to V.
+// Layouts: cache[slot][c][g][32] (c = phi, d/dx, d/dy, d/dz), bmat[slot][g][32].
+//
+// A v_mfma_f64_16x16x4 holds its SIMD for 64 cycles and takes 512 bytes per
+// operand, so a wave that owns 64 x 64 (or 64 x 32) results needs 8 to 12 bytes
+// per cycle: the waves read their operands straight from the caches in operand
+// order (rows of 128 bytes), with no LDS stage and no barrier, the next loads in
+// flight while the products of the current ones run.
 #include <hip/hip_runtime.h>
+
+#include <type_traits>
 
 #include "device_common.hpp"
 #include "internal.hpp"
@@ -22,9 +30,6 @@ namespace chx {
 
 constexpr int kSlotAO = 4 * kBatch * kTile;  // doubles per cached slot
 constexpr int kSlotB = kBatch * kTile;
-constexpr int kSupC = 4;                    // tiles per Vxc super-tile (128 AOs)
-constexpr int kSupCAO = kSupC * kTile;
-constexpr int kHalf = 32;                   // points per Vxc LDS stage
 
 // ---------------------------------------------------------------------------
 // AO cache: one block per slot.
@@ -76,149 +81,156 @@ void launch_ao_cache(hipStream_t s, int nslots, const int* slot_batch, const int
 }
 
 // ---------------------------------------------------------------------------
-// Density from the cache. Block = (batch, group of <= 4 tiles of its list as output
-// columns), 8 waves: wave w owns rows g = 16(w%4)..+15 and output columns
-// 64(w/4)..+63 (two tiles). K loop over the list's tiles: phi tile
-// [g][mu] and D block [mu][nu] double-buffered in LDS, the next K step
-// prefetched into registers while the MFMAs of the current one run.
-struct DensCSmem {
-  double A[2][kBatch][kTile + 1];
-  double B[2][kTile][kGroup * kTile];
-  double red[2][4][kBatch];
-};
-
-// MODE 0: A = phi, epilogue rho and grad rho / 2 (4 components into part).
-// MODE r = 1..3: A = d phi / d x_r, epilogue sum X_r d_r phi into part (one
-// component: the tau partial of direction r).
-template <int MODE>
-__global__ __launch_bounds__(512) void k_density_c64(const int* __restrict__ grp_batch, const int* __restrict__ grp_tile,
-                                                     const int* __restrict__ grp_ntiles, const int* __restrict__ bt_off,
-                                                     const int* __restrict__ b_chunk, const ChunkDev* __restrict__ chunks,
-                                                     const double* __restrict__ cache, const double* __restrict__ Dt,
-                                                     double* __restrict__ part, int grp_stride) {
-  constexpr int NOUT = MODE == 0 ? 4 : 1;
-  __shared__ DensCSmem sm;
+// Density from the cache. Block = (batch, group of <= 4 tiles of its list as
+// output columns). A wave owns one tile's 32 columns of X = Phi D: all 64 points
+// (4 waves), or with TAU 32 points of all four products Phi D, (d_r Phi) D (8
+// waves). K runs over the list's tiles in 8-AO pieces: lane (lk, lrow) holds AOs
+// 2 lk, 2 lk + 1 of point lrow (one 16-byte load, 64 contiguous bytes per
+// point), and rows 2 lk, 2 lk + 1 of D, so both see the same order of K.
+// tau = sum_r x_r^T D x_r (x_r = d_r phi) is a quadratic form: for a symmetric D
+// (asym != gen) the wave's tau products run over the tiles up to its own, those
+// before it counted twice (accumulators doubled when it is reached).
+// C18 / def2-TZVP / SG-3: 4.6 ms (7.6 in four launches with LDS stages).
+template <bool TAU>
+__global__ __launch_bounds__(TAU ? 512 : 256, 2) void k_density_c64(
+    const int* __restrict__ grp_batch, const int* __restrict__ grp_tile, const int* __restrict__ grp_ntiles,
+    const int* __restrict__ bt_off, const int* __restrict__ b_chunk, const ChunkDev* __restrict__ chunks,
+    const double* __restrict__ cache, const double* __restrict__ Dt, const int* __restrict__ asym, int gen,
+    double* __restrict__ part, double* __restrict__ part_tau) {
+  constexpr int NC = TAU ? 4 : 1, NR = TAU ? 2 : 4, NOUT = TAU ? 5 : 4;
+  __shared__ double red[kGroup][NOUT][kBatch];
   const int grp = blockIdx.x;
   const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform, keeps branches scalar
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lrow = lane & 15, lk = lane >> 4;
-  const int wr = wave & 3, wc = wave >> 2;  // row block, column half
-  const int b = grp_batch[grp];
-  const int nt = grp_ntiles[grp];
+  const int q = TAU ? wave >> 1 : wave, row0 = TAU ? 32 * (wave & 1) : 0;  // the wave's tile of the group, first point
+  const int b = grp_batch[grp], nt = grp_ntiles[grp];
   const ChunkDev ch = chunks[b_chunk[b]];
-  const int ld = ch.ntl * kTile, j0 = grp_tile[grp] - ch.tile0;  // j0: the group's first tile in the chunk
-  const int it0 = bt_off[b], it1 = it0 + ch.ntl;
-  const double* __restrict__ Dc = Dt + ch.doff + j0 * kTile;
-
-  double2 ra[2], rb[4];
-  auto load = [&](int it) {
-    const double2* src = reinterpret_cast<const double2*>(cache + (size_t)it * kSlotAO + MODE * kSlotB);
+  const int nk = ch.ntl, ld = nk * kTile, it0 = bt_off[b], tq = grp_tile[grp] - ch.tile0 + q;  // the tile in the list
+  if (q < nt) {
+    const bool sym = TAU && *asym != gen;
+    const double* __restrict__ A0 = cache + (size_t)it0 * kSlotAO + (row0 + lrow) * kTile + 2 * lk;
+    const double* __restrict__ D0 = Dt + ch.doff + (size_t)(2 * lk) * ld + tq * kTile + lrow;
+    dbl4 acc[NC][NR][2];
 #pragma unroll
-    for (int j = 0; j < 2; ++j) ra[j] = src[tid + 512 * j];
-    const double* __restrict__ Drow = Dc + (size_t)(it - it0) * kTile * ld;
+    for (int d = 0; d < NC; ++d)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int e = 2 * (tid + 512 * j);
-      const int r = e / (kGroup * kTile), cc = e % (kGroup * kTile), q = cc / kTile;
-      rb[j] = (q < nt) ? *reinterpret_cast<const double2*>(Drow + (size_t)r * ld + cc) : double2{0.0, 0.0};
-    }
-  };
-  auto store = [&](int buf) {
+      for (int r = 0; r < NR; ++r)
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int e = 2 * (tid + 512 * j);
-      sm.A[buf][e / kTile][e % kTile] = ra[j].x;
-      sm.A[buf][e / kTile][e % kTile + 1] = ra[j].y;
-    }
+        for (int h = 0; h < 2; ++h) acc[d][r][h] = dbl4{0, 0, 0, 0};
+    // pieces [p0, p1) of K: AOs 8 (p % 4).. of tile p / 4; every load is unconditional (a branch around
+    // one makes the compiler wait for all that are in flight)
+    auto run = [&](auto with_tau, int p0, int p1) {
+      constexpr int ND = decltype(with_tau)::value ? NC : 1;
+      if (p0 >= p1) return;
+      double2 a[2][ND][NR];
+      double bb[2][2][2];  // [buffer][row of the pair][half]
+      auto load = [&](int p, int buf) {
+        const int k = p >> 2, o = 8 * (p & 3);
+        const double* __restrict__ pa = A0 + (size_t)k * kSlotAO + o;
+        const double* __restrict__ pd = D0 + (size_t)(k * kTile + o) * ld;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int e = 2 * (tid + 512 * j);
-      *reinterpret_cast<double2*>(&sm.B[buf][e / (kGroup * kTile)][e % (kGroup * kTile)]) = rb[j];
-    }
-  };
-
-  dbl4 acc[4];
+        for (int d = 0; d < ND; ++d)
 #pragma unroll
-  for (int c = 0; c < 4; ++c) acc[c] = dbl4{0, 0, 0, 0};
-  const int ncb = min(4, max(0, 2 * nt - 4 * wc));  // valid column blocks of this wave
-  if (it0 < it1) load(it0);
-  int buf = 0;
-  for (int it = it0; it < it1; ++it) {
-    store(buf);
-    __syncthreads();
-    if (it + 1 < it1) load(it + 1);
+          for (int r = 0; r < NR; ++r)
+            a[buf][d][r] = *reinterpret_cast<const double2*>(pa + d * kSlotB + 16 * r * kTile);
 #pragma unroll
-    for (int ks = 0; ks < kTile / 4; ++ks) {
-      const double a = sm.A[buf][16 * wr + lrow][4 * ks + lk];
-      // columns of absent tiles hold zeros in LDS, so every wave runs all four
+        for (int e = 0; e < 2; ++e)
 #pragma unroll
-      for (int cb = 0; cb < 4; ++cb) acc[cb] = mfma_f64(a, sm.B[buf][4 * ks + lk][64 * wc + 16 * cb + lrow], acc[cb]);
-    }
-    buf ^= 1;
-  }
-
-  // Epilogue: X[g = 16wr + 4r + lk][nu = 16h + lrow] of tile q = 2wc + cb/2, against phi and grad phi.
-  double s[4][4];
+          for (int h = 0; h < 2; ++h) bb[buf][e][h] = pd[(size_t)e * ld + 16 * h];
+      };
+      auto step = [&](int buf) {
 #pragma unroll
-  for (int c = 0; c < 4; ++c)
+        for (int d = 0; d < ND; ++d)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) s[c][r] = 0.0;
+          for (int r = 0; r < NR; ++r)
 #pragma unroll
-  for (int cb = 0; cb < 4; ++cb) {
-    if (cb < ncb) {
-      const int q = 2 * wc + cb / 2, h = cb % 2;
-      const double* src = cache + (size_t)(it0 + j0 + q) * kSlotAO;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int g = 16 * wr + 4 * r + lk;
-        const double x = acc[cb][r];
-#pragma unroll
-        for (int c = 0; c < NOUT; ++c)
-          s[c][r] += x * src[((size_t)(MODE == 0 ? c : MODE) * kBatch + g) * kTile + 16 * h + lrow];
+            for (int h = 0; h < 2; ++h) {
+              acc[d][r][h] = mfma_f64(a[buf][d][r].x, bb[buf][0][h], acc[d][r][h]);
+              acc[d][r][h] = mfma_f64(a[buf][d][r].y, bb[buf][1][h], acc[d][r][h]);
+            }
+      };
+      load(p0, 0);
+      for (int p = p0; p < p1; p += 2) {  // whole tiles: an even number of pieces
+        load(p + 1, 1);
+        __builtin_amdgcn_sched_barrier(0);  // the loads go out before the products that they run beside
+        step(0);
+        load(min(p + 2, p1 - 1), 0);
+        __builtin_amdgcn_sched_barrier(0);
+        step(1);
       }
+    };
+    if (sym) {
+      run(std::true_type{}, 0, 4 * tq);
+#pragma unroll
+      for (int d = 1; d < NC; ++d)
+#pragma unroll
+        for (int r = 0; r < NR; ++r)
+#pragma unroll
+          for (int h = 0; h < 2; ++h) acc[d][r][h] *= 2.0;
+      run(std::true_type{}, 4 * tq, 4 * tq + 4);
+      run(std::false_type{}, 4 * tq + 4, 4 * nk);
+    } else {
+      run(std::true_type{}, 0, 4 * nk);
+    }
+    // X[g = row0 + 16 r + 4 i + lk][nu = 16 h + lrow] of the wave's tile, against phi and grad phi;
+    // sums over the tile's columns (the 16 lanes of a row)
+    const double* __restrict__ src = cache + (size_t)(it0 + tq) * kSlotAO + (row0 + lk) * kTile + lrow;
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      double f[2][4][4];
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int d = 0; d < 4; ++d) f[h][i][d] = src[d * kSlotB + (16 * r + 4 * i) * kTile + 16 * h];
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int c = 0; c < NOUT; ++c) {
+          double v = 0.0;
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            if (c < 4) v += acc[0][r][h][i] * f[h][i][c & 3];
+            if (c == 4) {
+#pragma unroll
+              for (int d = 1; d < NC; ++d) v += acc[d][r][h][i] * f[h][i][d];
+            }
+          }
+          v += __shfl_xor(v, 1, 64);
+          v += __shfl_xor(v, 2, 64);
+          v += __shfl_xor(v, 4, 64);
+          v += __shfl_xor(v, 8, 64);
+          if (lrow == 4 * i + (c & 3)) red[q][c][row0 + 16 * r + 4 * i + lk] = v;
+        }
     }
   }
-#pragma unroll
-  for (int c = 0; c < NOUT; ++c)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      double v = s[c][r];
-      v += __shfl_xor(v, 1, 64);
-      v += __shfl_xor(v, 2, 64);
-      v += __shfl_xor(v, 4, 64);
-      v += __shfl_xor(v, 8, 64);
-      s[c][r] = v;
-    }
-  double out = 0;
-#pragma unroll
-  for (int c = 0; c < NOUT; ++c)
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-      if (lrow == 4 * c + r) out = s[c][r];
-  const int c = lrow >> 2, r = lrow & 3;
-  if (c < NOUT) sm.red[wc][c][16 * wr + 4 * r + lk] = out;
+  // the sums over the group's tiles
   __syncthreads();
-  if (tid < NOUT * kBatch) {
-    const int cc = tid / kBatch, g = tid % kBatch;
-    part[(size_t)grp * grp_stride + cc * kBatch + g] = sm.red[0][cc][g] + sm.red[1][cc][g];
+  for (int e = tid; e < (TAU ? 7 : 4) * kBatch; e += TAU ? 512 : 256) {
+    const int c = e / kBatch, g = e % kBatch;
+    double v = 0.0;
+    if (c < NOUT)
+      for (int t = 0; t < nt; ++t) v += red[t][c][g];
+    if (c < 4)
+      part[(size_t)grp * 4 * kBatch + c * kBatch + g] = v;
+    else  // part_tau: [group][3][64], summed over the directions in the first
+      part_tau[(size_t)grp * 3 * kBatch + (c - 4) * kBatch + g] = v;
   }
 }
 
-void launch_density_c64(hipStream_t s, int mode, int ngroups, const int* grp_batch, const int* grp_tile,
-                        const int* grp_ntiles, const int* bt_off, const int* b_chunk, const ChunkDev* chunks,
-                        const double* cache, const double* Dt, double* part) {
+void launch_density_c64(hipStream_t s, int ngroups, const int* grp_batch, const int* grp_tile, const int* grp_ntiles,
+                        const int* bt_off, const int* b_chunk, const ChunkDev* chunks, const double* cache,
+                        const double* Dt, const int* asym, int gen, double* part, double* part_tau) {
   if (ngroups == 0) return;
-  const int stride = (mode == 0 ? 4 : 3) * kBatch;  // part: [group][4][64]; tau partials: [group][3][64]
-#define CHX_DC64(M)                                                                                        \
-  hipLaunchKernelGGL(k_density_c64<M>, dim3(ngroups), dim3(512), 0, s, grp_batch, grp_tile, grp_ntiles,    \
-                     bt_off, b_chunk, chunks, cache, Dt, part, stride);
-  switch (mode) {
-    case 0: CHX_DC64(0); break;
-    case 1: CHX_DC64(1); break;
-    case 2: CHX_DC64(2); break;
-    default: CHX_DC64(3); break;
-  }
-#undef CHX_DC64
+  if (part_tau)
+    hipLaunchKernelGGL(k_density_c64<true>, dim3(ngroups), dim3(512), 0, s, grp_batch, grp_tile, grp_ntiles, bt_off,
+                       b_chunk, chunks, cache, Dt, asym, gen, part, part_tau);
+  else
+    hipLaunchKernelGGL(k_density_c64<false>, dim3(ngroups), dim3(256), 0, s, grp_batch, grp_tile, grp_ntiles, bt_off,
+                       b_chunk, chunks, cache, Dt, asym, gen, part, part_tau);
   CHX_HIP(hipGetLastError());
 }
 
@@ -227,17 +239,9 @@ void launch_density_c64(hipStream_t s, int mode, int ngroups, const int* grp_bat
 // one component per slot for every family: the meta-GGA operand
 // T_r = t d_r phi (t = w v_tau / 4, so that V = M + M^T carries
 // (1/2) w v_tau grad phi_mu . grad phi_nu) is formed from the cached d_r phi
-// while the Vxc kernel loads it, instead of being stored. The blocks past the
-// batches clear M for the Vxc launch that follows.
-constexpr int kFillBlock = 4096;
+// while the Vxc kernel loads it, instead of being stored.
 __global__ __launch_bounds__(256) void k_make_b(const int* __restrict__ bt_off, const double* __restrict__ coef,
-                                                const double* __restrict__ cache, double* __restrict__ bmat,
-                                                int nbatches, double* __restrict__ M, size_t nfill) {
-  if ((int)blockIdx.x >= nbatches) {
-    const size_t e0 = (size_t)(blockIdx.x - nbatches) * kFillBlock;
-    for (size_t i = e0 + threadIdx.x; i < e0 + kFillBlock && i < nfill; i += 256) M[i] = 0.0;
-    return;
-  }
+                                                const double* __restrict__ cache, double* __restrict__ bmat) {
   __shared__ double ca[kBatch], cx[kBatch], cy[kBatch], cz[kBatch];
   const int b = blockIdx.x, tid = threadIdx.x;
   if (tid < kBatch) {
@@ -260,111 +264,178 @@ __global__ __launch_bounds__(256) void k_make_b(const int* __restrict__ bt_off, 
 }
 
 void launch_make_b(hipStream_t s, int nbatches, const int* bt_off, const double* coef, const double* cache,
-                   double* bmat, double* M, size_t nfill) {
-  const unsigned nb = (unsigned)(nbatches + (nfill + kFillBlock - 1) / kFillBlock);
-  if (nb == 0) return;
-  hipLaunchKernelGGL(k_make_b, dim3(nb), dim3(256), 0, s, bt_off, coef, cache, bmat, nbatches, M, nfill);
+                   double* bmat) {
+  if (nbatches == 0) return;
+  hipLaunchKernelGGL(k_make_b, dim3(nbatches), dim3(256), 0, s, bt_off, coef, cache, bmat);
   CHX_HIP(hipGetLastError());
 }
 
 // ---------------------------------------------------------------------------
-// Vxc from the cache: M_IJ += sum_g phi_I[g]^T B_J[g] over the work item's
-// batches, I and J super-tiles of the chunk's AO list, 32 points per LDS stage (double-buffered), 8 waves: wave w owns rows
-// mu = 16w..16w+15 of the 128 x 128 block. One atomic add per element per item.
-struct VxcCSmem {
-  double P[2][kHalf][kSupCAO + 1];
-  double Bt[2][kHalf][kSupCAO + 1];
-};
-
-// NC = 1: M = phi^T B. NC = 4 (meta-GGA): also sum_r (d_r phi)^T T_r, each
-// component streamed as further K stages, T_r = t d_r phi formed from the
-// cached d_r phi and the point's t = coef[4] as it is loaded.
-template <int NC>
-__global__ __launch_bounds__(512) void k_vxc_c64(const VxcItem* __restrict__ work, const int* __restrict__ ao_of,
-                                                 const double* __restrict__ cache, const double* __restrict__ bmat,
-                                                 const double* __restrict__ coef, double* __restrict__ Mint,
-                                                 int npad) {
-  __shared__ VxcCSmem sm;
-  const VxcItem wk = work[blockIdx.x];
-  const int I = wk.I, J = wk.J;
+// Contractions over the points, C_IJ = sum_g A_I[g]^T B_J[g], for groups I and J
+// of up to 4 of a chunk's tiles over a run of its batches. 4 waves in a 2 x 2
+// grid, each owning half of the row and of the column blocks (up to 64 x 64).
+// Passes over the batch's 64 points, 4 points per product, lane (lk, lrow) point
+// lk and AO lrow of either operand:
+//   KIND 0: V of one run, upper blocks I0 <= J0: phi^T B, and for I < J B^T phi
+//           into the same accumulators; I = J is symmetrised through LDS;
+//   KIND 1: the same with the meta-GGA passes (d_r phi)^T (t d_r phi) first (t =
+//           coef[4] of the point; twice t for I < J, the term is symmetric);
+//   KIND 2: A^T B alone for any (I, J), added to M by FP64 atomics.
+// KIND 0 and 1 store the block once into U (see k_assemble). C18 / def2-TZVP
+// r2SCAN: 2.6 ms (9.6 with both triangles, LDS stages and atomics into M).
+constexpr int kSymStrip = 32;  // columns of the diagonal block transposed at a time
+template <int KIND>
+__global__ __launch_bounds__(256, 2) void k_vxc_c64(const MxItem* __restrict__ work, const double* __restrict__ cache,
+                                                    const double* __restrict__ bmat, const double* __restrict__ coef,
+                                                    const int* __restrict__ ao_of, double* __restrict__ out,
+                                                    int npad) {
+  const MxItem wk = work[blockIdx.x];
+  const bool diag = wk.I0 == wk.J0;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lrow = lane & 15, lk = lane >> 4;
-  // Per stage and operand: 4 tiles x 32 points x 32 AOs; thread t moves the
-  // double2 at element 2 (t + 512 j) of tile j.
-  double2 rp[kSupC], rq[kSupC];
-  const int r0 = 2 * tid;  // element within a tile's 32 x 32 block
-  auto load = [&](int k) {  // stage k -> (batch, half, component)
-    const int it = k / (2 * NC), h = (k / NC) % 2, c = k % NC;
-    const int b = wk.batch0 + it, s0 = wk.slot0 + it * wk.ntl;
-    const int g = h * kHalf + r0 / kTile, mu = r0 % kTile;
-    const double t = c ? coef[kCoef * ((size_t)b * kBatch + g) + 4] : 0.0;
+  const int nr = wk.nI, nc = wk.nJ, r0 = nr * (wave & 1), c0 = nc * (wave >> 1);  // the wave's row and column blocks
+  const int ntau = KIND == 1 ? 3 : 0, npass = ntau + (KIND == 2 || diag ? 1 : 2);
+  dbl4 acc[4][4];
 #pragma unroll
-    for (int j = 0; j < kSupC; ++j) {
-      const int si = I * kSupC + j < wk.ntl ? s0 + I * kSupC + j : -1;
-      const int sj = J * kSupC + j < wk.ntl ? s0 + J * kSupC + j : -1;
-      rp[j] = si >= 0 ? *reinterpret_cast<const double2*>(cache + (size_t)si * kSlotAO + (size_t)c * kSlotB + g * kTile + mu)
-                      : double2{0.0, 0.0};
-      if (sj < 0) {
-        rq[j] = double2{0.0, 0.0};
-      } else if (c == 0) {
-        rq[j] = *reinterpret_cast<const double2*>(bmat + (size_t)sj * kSlotB + g * kTile + mu);
-      } else {
-        const double2 d = *reinterpret_cast<const double2*>(cache + (size_t)sj * kSlotAO + (size_t)c * kSlotB +
-                                                             g * kTile + mu);
-        rq[j] = double2{t * d.x, t * d.y};
+  for (int r = 0; r < 4; ++r)
+#pragma unroll
+    for (int c = 0; c < 4; ++c) acc[r][c] = dbl4{0, 0, 0, 0};
+  double a[2][2][4], bb[2][2][4], tt[2][2];  // [buffer][4-point step of the pair][block]
+  const int lo = lk * kTile + lrow;
+  auto load = [&](int k, int buf) {  // piece k: 8 points of one pass of one batch
+    const int p8 = k & 7, pass = (k >> 3) % npass, it = (k >> 3) / npass;
+    const size_t s0 = (size_t)wk.slot0 + (size_t)it * wk.ntl;
+    const bool tau = pass < ntau, swap = pass > ntau;
+    const double* __restrict__ pa = (swap ? bmat + (s0 + wk.I0) * kSlotB
+                                          : cache + (s0 + wk.I0) * kSlotAO + (tau ? pass + 1 : 0) * kSlotB) +
+                                    8 * p8 * kTile + lo;
+    const double* __restrict__ pb = (tau    ? cache + (s0 + wk.J0) * kSlotAO + (pass + 1) * kSlotB
+                                     : swap ? cache + (s0 + wk.J0) * kSlotAO
+                                            : bmat + (s0 + wk.J0) * kSlotB) +
+                                    8 * p8 * kTile + lo;
+    const int sa = swap ? kSlotB : kSlotAO, sb = tau || swap ? kSlotAO : kSlotB;
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      double t = 1.0;  // (non-tau passes load one too)
+      if (KIND == 1) t = coef[kCoef * ((size_t)(wk.batch0 + it) * kBatch + 8 * p8 + 4 * e + lk) + 4];
+      if (KIND == 1) tt[buf][e] = t;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {  // past the group: its last block again (a branch would wait for all loads)
+        const int q = r0 + min(r, nr - 1);
+        a[buf][e][r] = pa[(size_t)(q >> 1) * sa + (q & 1) * 16 + 4 * e * kTile];
+      }
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const int q = c0 + min(c, nc - 1);
+        bb[buf][e][c] = pb[(size_t)(q >> 1) * sb + (q & 1) * 16 + 4 * e * kTile];
       }
     }
   };
-  auto store = [&](int buf) {
-    const int g = r0 / kTile, m = r0 % kTile;
+  auto step = [&](int k, int buf) {
+    double scale = 1.0;
 #pragma unroll
-    for (int j = 0; j < kSupC; ++j) {
-      const int col = j * kTile + m;
-      sm.P[buf][g][col] = rp[j].x;
-      sm.P[buf][g][col + 1] = rp[j].y;
-      sm.Bt[buf][g][col] = rq[j].x;
-      sm.Bt[buf][g][col + 1] = rq[j].y;
+    for (int e = 0; e < 2; ++e) {
+      if (KIND == 1) scale = (k >> 3) % npass < ntau ? (diag ? 1.0 : 2.0) * tt[buf][e] : 1.0;
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        if (c < nc) {
+          const double v = KIND == 1 ? scale * bb[buf][e][c] : bb[buf][e][c];
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (r < nr) acc[r][c] = mfma_f64(a[buf][e][r], v, acc[r][c]);
+        }
     }
   };
-  dbl4 acc[8];
-#pragma unroll
-  for (int cb = 0; cb < 8; ++cb) acc[cb] = dbl4{0, 0, 0, 0};
-  const int nstage = wk.nbat * (kBatch / kHalf) * NC;
-  if (nstage > 0) load(0);
-  int buf = 0;
-  for (int k = 0; k < nstage; ++k) {
-    store(buf);
-    __syncthreads();
-    if (k + 1 < nstage) load(k + 1);
-#pragma unroll
-    for (int ks = 0; ks < kHalf / 4; ++ks) {
-      const int g = 4 * ks + lk;
-      const double a = sm.P[buf][g][16 * wave + lrow];
-#pragma unroll
-      for (int cb = 0; cb < 8; ++cb) acc[cb] = mfma_f64(a, sm.Bt[buf][g][16 * cb + lrow], acc[cb]);
-    }
-    buf ^= 1;
+  const int n8 = wk.nbat * npass * 8;  // even
+  load(0, 0);
+  for (int k = 0; k < n8; k += 2) {
+    load(k + 1, 1);
+    __builtin_amdgcn_sched_barrier(0);  // the loads go out before the products that they run beside
+    step(k, 0);
+    load(min(k + 2, n8 - 1), 0);
+    __builtin_amdgcn_sched_barrier(0);
+    step(k + 1, 1);
   }
-  const int nrow = wk.ntl * kTile;
-  const int* __restrict__ ao = ao_of + (size_t)wk.tile0 * kTile;
+  // C layout: acc[r][c][i] = C[row 16 (r0 + r) + 4 i + lk][column 16 (c0 + c) + lrow]
+  if (KIND == 2) {
+    const int* __restrict__ ao = ao_of + (size_t)wk.tile0 * kTile;
 #pragma unroll
-  for (int cb = 0; cb < 8; ++cb)
+    for (int r = 0; r < 4; ++r)
+      if (r < nr) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int lr = I * kSupCAO + 16 * wave + 4 * r + lk, lc = J * kSupCAO + 16 * cb + lrow;
-      const int mu = lr < nrow ? ao[lr] : -1, nu = lc < nrow ? ao[lc] : -1;
-      if (mu >= 0 && nu >= 0) unsafeAtomicAdd(&Mint[(size_t)mu * npad + nu], acc[cb][r]);
-    }
+        for (int i = 0; i < 4; ++i) {
+          const int mu = ao[wk.I0 * kTile + 16 * (r0 + r) + 4 * i + lk];
+#pragma unroll
+          for (int c = 0; c < 4; ++c)
+            if (c < nc) {
+              const int nu = ao[wk.J0 * kTile + 16 * (c0 + c) + lrow];
+              if (mu >= 0 && nu >= 0) unsafeAtomicAdd(&out[(size_t)mu * npad + nu], acc[r][c][i]);
+            }
+        }
+      }
+    return;
+  }
+  double* __restrict__ U = out + wk.u;
+  const int ld = wk.ldu;
+  if (!diag) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if (r < nr) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+          if (c < nc) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+              U[(size_t)(16 * (r0 + r) + 4 * i + lk) * ld + 16 * (c0 + c) + lrow] = acc[r][c][i];
+          }
+      }
+    return;
+  }
+  __shared__ double T[kSymStrip][4 * kTile + 4];
+  for (int s = 0; s < 2 * nc; s += kSymStrip / 16) {  // U = M + M^T, 32 rows at a time
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+      if (c < nc && c0 + c >= s && c0 + c < s + kSymStrip / 16) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (r < nr) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) T[16 * (c0 + c - s) + lrow][16 * (r0 + r) + 4 * i + lk] = acc[r][c][i];
+          }
+      }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if (r < nr && r0 + r >= s && r0 + r < s + kSymStrip / 16) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+          if (c < nc) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              const int row = 16 * (r0 + r) + 4 * i + lk, col = 16 * (c0 + c) + lrow;
+              U[(size_t)row * ld + col] = acc[r][c][i] + T[row - 16 * s][col];
+            }
+          }
+      }
+  }
 }
 
-void launch_vxc_c64(hipStream_t s, int ncomp, int nwork, const VxcItem* work, const int* ao_of, const double* cache,
-                    const double* bmat, const double* coef, double* Mint, int npad) {
+void launch_vxc_c64(hipStream_t s, int ncomp, int nwork, const MxItem* work, const double* cache, const double* bmat,
+                    const double* coef, double* U) {
   if (nwork == 0) return;
   if (ncomp == 4)
-    hipLaunchKernelGGL(k_vxc_c64<4>, dim3(nwork), dim3(512), 0, s, work, ao_of, cache, bmat, coef, Mint, npad);
+    hipLaunchKernelGGL(k_vxc_c64<1>, dim3(nwork), dim3(256), 0, s, work, cache, bmat, coef, nullptr, U, 0);
   else
-    hipLaunchKernelGGL(k_vxc_c64<1>, dim3(nwork), dim3(512), 0, s, work, ao_of, cache, bmat, coef, Mint, npad);
+    hipLaunchKernelGGL(k_vxc_c64<0>, dim3(nwork), dim3(256), 0, s, work, cache, bmat, coef, nullptr, U, 0);
+  CHX_HIP(hipGetLastError());
+}
+
+void launch_prod_c64(hipStream_t s, int nwork, const MxItem* work, const int* ao_of, const double* cache,
+                     const double* bmat, double* M, int npad) {
+  if (nwork == 0) return;
+  hipLaunchKernelGGL(k_vxc_c64<2>, dim3(nwork), dim3(256), 0, s, work, cache, bmat, nullptr, ao_of, M, npad);
   CHX_HIP(hipGetLastError());
 }
 

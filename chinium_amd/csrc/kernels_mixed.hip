@@ -173,7 +173,7 @@ void launch_ao_cache_mx(hipStream_t s, int nslots, const int* slot_batch, const 
 // included), at D's own position. The products see hi + lo; sum V . R, with V
 // the potential of this density, is the first-order energy of the remainder
 // (dE/dD = V), which the energy takes back when the potential is built
-// (k_assemble_mx). With asym (meta-GGA) the last blocks compare D with D^T: an
+// (k_assemble). With asym (meta-GGA) the last blocks compare D with D^T: an
 // element more than 1e-12 sqrt(D_ii D_jj) off (products of FP64 rounding stay far
 // below, as this does below the split) sets *asym = gen, this build's number.
 // One launch: small molecules (and packs of them) are bound by the launches.
@@ -186,27 +186,7 @@ __global__ __launch_bounds__(256) void k_split_gather(int n, const double* __res
                                                       int* __restrict__ asym, int gen) {
   const int t = blockIdx.x;
   if (t >= ntiles + nrest) {  // 32 x 32 tile pair (i <= j) of the symmetry check
-    __shared__ double P[kTile][kTile + 1];
-    const int k = t - ntiles - nrest;
-    int j = (int)((sqrtf(8.f * (float)k + 1.f) - 1.f) * 0.5f);
-    while ((j + 1) * (j + 2) / 2 <= k) ++j;
-    while (j * (j + 1) / 2 > k) --j;
-    const int i = k - j * (j + 1) / 2;
-    for (int e = threadIdx.x; e < kTile * kTile; e += 256) {  // rows of tile j, columns of tile i
-      const int r = j * kTile + (e & 31), c = i * kTile + (e >> 5);
-      P[e >> 5][e & 31] = r < n && c < n ? D[(size_t)c * n + r] : 0.0;
-    }
-    __syncthreads();
-    bool bad = false;
-    for (int e = threadIdx.x; e < kTile * kTile; e += 256) {
-      const int r = i * kTile + (e & 31), c = j * kTile + (e >> 5);
-      if (r < n && c < n) {
-        const double u = D[(size_t)c * n + r], v = P[e & 31][e >> 5];
-        const double s = ::sqrt(::fabs(D[(size_t)r * n + r] * D[(size_t)c * n + c]));
-        bad = bad || !(::fabs(u - v) <= 1e-12 * s);
-      }
-    }
-    if (__ballot(bad) && (threadIdx.x & 63) == 0) *asym = gen;
+    check_symmetry(t - ntiles - nrest, n, D, 1e-12, asym, gen);
     return;
   }
   if (t >= ntiles) {
@@ -249,8 +229,8 @@ __global__ __launch_bounds__(256) void k_split_gather(int n, const double* __res
 void launch_split_d(hipStream_t s, int ntiles, int n, const double* D, const int* tile_chunk, const ChunkDev* chunks,
                     const int* ao_of, unsigned short* Ds, float* R, int* asym, int gen) {
   const long n2 = (long)n * n;
-  const int nrest = (int)((n2 + kRestBlock - 1) / kRestBlock), nt = (n + kTile - 1) / kTile;
-  const unsigned nb = (unsigned)(ntiles + nrest + (asym ? nt * (nt + 1) / 2 : 0));
+  const int nrest = (int)((n2 + kRestBlock - 1) / kRestBlock);
+  const unsigned nb = (unsigned)(ntiles + nrest + (asym ? symmetry_blocks(n) : 0));
   hipLaunchKernelGGL(k_split_gather, dim3(nb), dim3(256), 0, s, n, D, tile_chunk, chunks, ao_of, Ds, ntiles, n2, R, nrest,
                      asym, gen);
   CHX_HIP(hipGetLastError());
@@ -286,11 +266,11 @@ static int asm_copies(int n) { return n <= kAsmLds / 16 ? 16 : 1; }
 static int asm_ranges(int n) { return (n + kAsmLds / asm_copies(n) - 1) / (kAsmLds / asm_copies(n)); }
 int assemble_blocks(int n) { return n * asm_ranges(n); }
 
-template <int COPIES>
-__global__ __launch_bounds__(kAsmThreads) void k_assemble_mx(int n, const int* __restrict__ rowptr,
+template <int COPIES, class T>
+__global__ __launch_bounds__(kAsmThreads) void k_assemble(int n, const int* __restrict__ rowptr,
                                                              const RowRef* __restrict__ rows,
                                                              const int* __restrict__ ao_of,
-                                                             const float* __restrict__ U, double* __restrict__ V,
+                                                             const T* __restrict__ U, double* __restrict__ V,
                                                              const float* __restrict__ R,
                                                              double* __restrict__ cpart) {
   extern __shared__ double asum[];
@@ -316,7 +296,7 @@ __global__ __launch_bounds__(kAsmThreads) void k_assemble_mx(int n, const int* _
     }
     for (int k = lane; k < len; k += 64) {
       int nu[kAsmUnroll];
-      float v[kAsmUnroll];
+      T v[kAsmUnroll];
 #pragma unroll
       for (int q = 0; q < kAsmUnroll; ++q) {  // clamped, not skipped: the loads go out together
         const int kk = min(k, max(r[q].len - 1, 0));
@@ -351,18 +331,23 @@ __global__ __launch_bounds__(kAsmThreads) void k_assemble_mx(int n, const int* _
   }
 }
 
-void launch_assemble_mx(hipStream_t s, int n, const int* rowptr, const RowRef* rows, const int* ao_of, const float* U,
-                        double* V, const float* R, double* cpart) {
+template <class T>
+void launch_assemble(hipStream_t s, int n, const int* rowptr, const RowRef* rows, const int* ao_of, const T* U,
+                     double* V, const float* R, double* cpart) {
   if (n == 0) return;
   const int copies = asm_copies(n);
   const dim3 grid(n, asm_ranges(n));
   const size_t lds = (size_t)std::min(n, kAsmLds / copies) * copies * sizeof(double);
   if (copies == 16)
-    hipLaunchKernelGGL(k_assemble_mx<16>, grid, dim3(kAsmThreads), lds, s, n, rowptr, rows, ao_of, U, V, R, cpart);
+    hipLaunchKernelGGL((k_assemble<16, T>), grid, dim3(kAsmThreads), lds, s, n, rowptr, rows, ao_of, U, V, R, cpart);
   else
-    hipLaunchKernelGGL(k_assemble_mx<1>, grid, dim3(kAsmThreads), lds, s, n, rowptr, rows, ao_of, U, V, R, cpart);
+    hipLaunchKernelGGL((k_assemble<1, T>), grid, dim3(kAsmThreads), lds, s, n, rowptr, rows, ao_of, U, V, R, cpart);
   CHX_HIP(hipGetLastError());
 }
+template void launch_assemble<float>(hipStream_t, int, const int*, const RowRef*, const int*, const float*, double*,
+                                     const float*, double*);
+template void launch_assemble<double>(hipStream_t, int, const int*, const RowRef*, const int*, const double*, double*,
+                                      const float*, double*);
 
 __global__ __launch_bounds__(256) void k_reduce_corr(int nparts, const double* __restrict__ cpart,
                                                      double* __restrict__ out) {
@@ -1015,7 +1000,7 @@ void launch_make_b_mx(hipStream_t s, int ncomp, const MolDev& one) {
 // room for two blocks per CU).
 // The result is stored once per run, in FP32 like the accumulators (row-major,
 // the row panel of group I from column I0 on), and summed in FP64 by
-// k_assemble_mx.
+// k_assemble.
 template <int MT>
 struct VxcMxSmem {
   u32x4 F[2][8 * MT * kDxFrag];  // step k in buffer k & 1: row group's fragments, then the column group's
