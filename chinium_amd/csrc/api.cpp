@@ -1266,7 +1266,7 @@ int chx_mlp_create(unsigned long long seed, chx_mlp** out) {
       m->P.alloc(kMlpParams);
       m->Prun.alloc(kMlpParams);
       m->Pinf.alloc(kMlpParams);
-      m->G.alloc(kMlpParams);
+      m->Gpart.alloc((size_t)kMlpGradBlocks * (kMlpParams + 1));
       m->M.alloc(kMlpParams);
       m->V.alloc(kMlpParams);
       m->loss.alloc(1);
@@ -1274,7 +1274,6 @@ int chx_mlp_create(unsigned long long seed, chx_mlp** out) {
       std::vector<float> P;
       mlp_init(seed, P);
       mlp_upload_params(m, P.data());
-      CHX_HIP(hipMemsetAsync(m->G.p, 0, sizeof(float) * kMlpParams, m->stream));
       CHX_HIP(hipMemsetAsync(m->M.p, 0, sizeof(float) * kMlpParams, m->stream));
       CHX_HIP(hipMemsetAsync(m->V.p, 0, sizeof(float) * kMlpParams, m->stream));
       CHX_HIP(hipStreamSynchronize(m->stream));
@@ -1406,27 +1405,30 @@ int chx_mlp_train(chx_mlp* m, int epochs, long batch, double lr, double lr_final
     require(m && epochs >= 0 && batch > 0 && lr > 0 && lr_final >= 0, CHX_ERR_ARG, "bad arguments");
     require(m->ndata > 0, CHX_ERR_STATE, "no training set (chx_mlp_set_data)");
     const long n = m->ndata;
-    const long nb = (n + batch - 1) / batch;
-    const long total = (long)epochs * nb;
+    const long nbatch = (n + batch - 1) / batch;
+    const long total = (long)epochs * nbatch;
     long it = 0;
+    float* losspart = m->Gpart.p + (size_t)kMlpGradBlocks * kMlpParams;
     for (int ep = 0; ep < epochs; ++ep) {
       launch_fill_u32(m->stream, (unsigned*)m->loss.p, 1, 0u);  // 0.0f
-      for (long b = 0; b < nb; ++b, ++it) {
+      for (long b = 0; b < nbatch; ++b, ++it) {
         const long s0 = b * batch, s1 = std::min(n, s0 + batch);
         const double csum = m->cprefix[s1] - m->cprefix[s0];
         if (!(csum > 0)) continue;
         const double cosw = 0.5 * (1.0 + std::cos(M_PI * (double)it / (double)std::max<long>(1, total)));
         const double lr_t = lr_final + (lr - lr_final) * cosw;
-        launch_mlp_grad(m->stream, s1 - s0, m->U.p + 3 * s0, m->T.p + s0, m->C.p ? m->C.p + s0 : nullptr,
-                        (float)(1.0 / csum), m->Prun.p, m->G.p, m->loss.p, 512);
+        const int nb = launch_mlp_grad(m->stream, s1 - s0, m->U.p + 3 * s0, m->T.p + s0, m->C.p ? m->C.p + s0 : nullptr,
+                                       (float)(1.0 / csum), m->P.p, m->Gpart.p, losspart);
         m->step += 1;
-        launch_mlp_adam(m->stream, m->P.p, m->G.p, m->M.p, m->V.p, m->Prun.p, m->Pinf.p, (float)lr_t, m->step);
+        launch_mlp_adam(m->stream, nb, m->Gpart.p, losspart, m->P.p, m->M.p, m->V.p, m->loss.p, (float)lr_t,
+                        m->step);
       }
       float l = 0.f;
       CHX_HIP(hipMemcpyAsync(&l, m->loss.p, sizeof(float), hipMemcpyDeviceToHost, m->stream));
       CHX_HIP(hipStreamSynchronize(m->stream));
-      if (epoch_loss) epoch_loss[ep] = (double)l / (double)nb;
+      if (epoch_loss) epoch_loss[ep] = (double)l / (double)nbatch;
     }
+    launch_mlp_pack(m->stream, m->P.p, m->Prun.p, m->Pinf.p);
     launch_mlp_pack_mx(m->stream, m->P.p, m->Wpk.p);
     CHX_HIP(hipStreamSynchronize(m->stream));
   });
@@ -1448,12 +1450,13 @@ int chx_mlp_loss_grad(chx_mlp* m, long n, const float* U, const float* T, const 
       for (long i = 0; i < n; ++i) csum += C[i];
     }
     require(csum > 0, CHX_ERR_ARG, "sample weights sum to zero");
-    DevBuf<float> dG;
+    DevBuf<float> dG, dP;
     dG.alloc(kMlpParams);
-    launch_fill_u32(m->stream, (unsigned*)dG.p, kMlpParams, 0u);
+    dP.alloc((size_t)kMlpGradBlocks * (kMlpParams + 1));
+    float* lp = dP.p + (size_t)kMlpGradBlocks * kMlpParams;
     launch_fill_u32(m->stream, (unsigned*)m->loss.p, 1, 0u);
-    launch_mlp_grad(m->stream, n, dU.p, dT.p, C ? dC.p : nullptr, (float)(1.0 / csum), m->Prun.p, dG.p, m->loss.p,
-                    512);
+    const int nb = launch_mlp_grad(m->stream, n, dU.p, dT.p, C ? dC.p : nullptr, (float)(1.0 / csum), m->P.p, dP.p, lp);
+    launch_mlp_reduce(m->stream, nb, dP.p, lp, dG.p, m->loss.p);
     float l = 0.f;
     CHX_HIP(hipMemcpyAsync(G, dG.p, sizeof(float) * kMlpParams, hipMemcpyDeviceToHost, m->stream));
     CHX_HIP(hipMemcpyAsync(&l, m->loss.p, sizeof(float), hipMemcpyDeviceToHost, m->stream));

@@ -232,10 +232,15 @@ void launch_mlp_forward(hipStream_t s, long n, const float* U, const float* R, c
                         float* dF);
 constexpr int kMlpPacked = 4 * 4 * 2 * 2 * 64 * 4;  // u32 words of the packed split-BF16 (hi, lo) MFMA weight fragments
 void launch_mlp_pack_mx(hipStream_t s, const float* P, unsigned* Wpk);
-void launch_mlp_grad(hipStream_t s, long n, const float* U, const float* T, const float* C, float cs, const float* R,
-                     float* G, float* loss, int max_blocks);
-void launch_mlp_adam(hipStream_t s, float* P, float* G, float* M, float* V, float* Prun, float* Pinf, float lr,
-                     int step);
+// Gradient and loss as per-block sums (at most kMlpGradBlocks blocks; returns
+// their number): Gpart[block][kMlpParams], losspart[block].
+constexpr int kMlpGradBlocks = 256;
+int launch_mlp_grad(hipStream_t s, long n, const float* U, const float* T, const float* C, float cs, const float* P,
+                    float* Gpart, float* losspart);
+// their sums: one Adam step on P, or the gradient to G; the loss is added to *loss
+void launch_mlp_adam(hipStream_t s, int nparts, const float* Gpart, const float* losspart, float* P, float* M,
+                     float* V, float* loss, float lr, int step);
+void launch_mlp_reduce(hipStream_t s, int nparts, const float* Gpart, const float* losspart, float* G, float* loss);
 void launch_mlp_features(hipStream_t s, long n, const double* rho, const double* sigma, const double* tau,
                          const int* codes, int ncodes, float* t, float* F);
 void launch_mlp_eval(hipStream_t s, long n, const float* R, const unsigned* Wpk, const MlpBox& box, const int* codes,
@@ -388,7 +393,8 @@ struct chx_mol {
 
 struct chx_mlp {
   hipStream_t stream = nullptr;
-  chx::DevBuf<float> P, Prun, Pinf, G, M, V, loss;  // canonical, run (FP32), run (BF16-rounded); Adam state
+  chx::DevBuf<float> P, Prun, Pinf, M, V, loss;  // canonical, run (FP32), run (BF16-rounded); Adam state
+  chx::DevBuf<float> Gpart;                      // per-block gradients and losses (kMlpGradBlocks of each)
   chx::DevBuf<unsigned> Wpk;                         // packed BF16 MFMA fragments of the inference weights
   chx::DevBuf<float> U, T, C;                        // training set: inputs, targets, sample weights
   std::vector<double> cprefix;                       // prefix sums of C (minibatch normalisation)

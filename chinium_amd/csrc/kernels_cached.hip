@@ -282,7 +282,7 @@ void launch_make_b(hipStream_t s, int nbatches, const int* bt_off, const double*
 //           coef[4] of the point; twice t for I < J, the term is symmetric);
 //   KIND 2: A^T B alone for any (I, J), added to M by FP64 atomics.
 // KIND 0 and 1 store the block once into U (see k_assemble). C18 / def2-TZVP
-// r2SCAN: 2.6 ms (9.6 with both triangles, LDS stages and atomics into M).
+// r2SCAN: 4.3 ms (9.6 with both triangles, LDS stages and atomics into M).
 constexpr int kSymStrip = 32;  // columns of the diagonal block transposed at a time
 template <int KIND>
 __global__ __launch_bounds__(256, 2) void k_vxc_c64(const MxItem* __restrict__ work, const double* __restrict__ cache,

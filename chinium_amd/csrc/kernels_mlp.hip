@@ -12,10 +12,11 @@
 // (src/ExchangeCorrelation.cpp:86-163), whose result this replaces.
 //
 // Network: 3 -> 64 -> 64 -> 64 -> 1, tanh hidden units, linear output. One
-// wave handles 64 samples (lane = sample). Training runs the network per lane
-// in FP32 with the weights uniform across the wave, read through the constant
-// address space (scalar loads) from a run copy that holds W2 transposed, so
-// that every weight row a loop walks is contiguous. Inference (Evaluate and
+// wave handles 64 samples (lane = sample); the raw forward pass runs the network
+// per lane in FP32 with the weights uniform across the wave, read through the
+// constant address space (scalar loads) from a run copy that holds W2 transposed,
+// so that every weight row a loop walks is contiguous. Training runs forward and
+// backward as FP32 MFMA products over 64 samples per block. Inference (Evaluate and
 // point evaluation) runs the three hidden products and the two backward ones
 // as transposed split-BF16 MFMA GEMMs over the wave's 64 points.
 #include "internal.hpp"
@@ -401,178 +402,256 @@ __global__ void k_mlp_pack_mx(const float* __restrict__ P, unsigned short* __res
 }
 
 // Loss L = cs sum_i C_i (y_i - T_i)^2 over the samples [0, n) (C_i = 1 when C
-// is null) and its gradient with respect to the canonical parameters, added
-// to G (and L to *loss). A block takes chunks of 64 samples. Per chunk, each
-// lane runs its sample's forward pass and layer deltas, and lane t then
-// reduces row t of every weight gradient over the chunk's samples
-// (dW = D A^T). Activations are held sample-major [sample][unit], deltas
-// unit-major [unit][sample], both with a 65-float pitch, so the per-lane and
-// the per-row accesses are conflict-free. The rows accumulate in registers
-// over the block's chunks and are added to G once.
-__global__ __launch_bounds__(64) void k_mlp_grad(long n, const float* __restrict__ U, const float* __restrict__ T,
-                                                 const float* __restrict__ C, float cs, const float* R,
-                                                 float* __restrict__ G, float* __restrict__ loss) {
-  __shared__ float A1[kLanes][kMlpH + 1];  // layer-1 activations, [sample][unit]
-  __shared__ float A2[kLanes][kMlpH + 1];  // layer-2 activations, [sample][unit]
-  __shared__ float D[kMlpH][kLanes + 1];   // h3, then d3, d2, d1: [unit][sample]
-  __shared__ float Us[kLanes][4];
-  __shared__ float gs[kLanes];
-  const int lane = threadIdx.x;
-  float gW2[kMlpH], gW3[kMlpH];
+// is null) and its gradient with respect to the canonical parameters P: block b
+// writes its samples' sums to Gpart[b] and losspart[b] (k_mlp_update adds them up).
+//
+// A block of 4 waves takes 64 samples at a time; every layer is a product on
+// v_mfma_f32_16x16x4_f32 (FP32 operands and sums, as the per-lane loops it
+// replaces): Z = W H (units x samples), dW = D H^T, and W^T D. Wave w owns the
+// units 16 w..+15 of a layer's result: lane (g = lane / 16, c = lane % 16) holds
+// units 16 w + 4 g + r at samples 16 nt + c. The K order of every product is 16
+// ks + 4 g + e (step 4 ks + e, lane group g), so an operand is read four steps at
+// a time as 16 bytes along K: activations and deltas lie in LDS both [sample]
+// [unit] (K = units) and [unit][sample] (K = samples), with a pitch of 68 floats
+// that spreads a wave's 16-byte reads over the banks; the weights of the wave's
+// units stay in registers. One wave per 64 samples (the per-lane network) left
+// most of the chip idle: 23.5 us for a minibatch of 16384 (500 before), the update 7.6.
+constexpr int kGp = 68;
+struct MlpGradSmem {
+  float Hs1[kLanes][kGp], Hu1[kMlpH][kGp];  // layer-1 activations [sample][unit], [unit][sample]
+  float Hs2[kLanes][kGp], Hu2[kMlpH][kGp];
+  float Ds[kLanes][kGp], Du[kMlpH][kGp];    // deltas of the layer at hand
+  float U[kLanes][4];
+  float y[4][kLanes];
+};
+
+// acc[nt] += sum_k A[m][k] B[k][n] over 64 K values: a (4 ks + e) the wave's A
+// operand, B read from rows[n = 16 nt + c][k].
+__device__ __forceinline__ void mlp_gemm(const float (&a)[16], const float (*rows)[kGp], int g, int c,
+                                         f32x4_t (&acc)[4]) {
 #pragma unroll
-  for (int j = 0; j < kMlpH; ++j) gW2[j] = gW3[j] = 0.f;
-  float gW1[3] = {0.f, 0.f, 0.f}, gb1 = 0.f, gb2 = 0.f, gb3 = 0.f, gw4 = 0.f, gb4 = 0.f, lsum = 0.f;
+  for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+    for (int nt = 0; nt < 4; ++nt) {
+      const f32x4_t b = *reinterpret_cast<const f32x4_t*>(&rows[16 * nt + c][16 * ks + 4 * g]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[nt] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[4 * ks + e], b[e], acc[nt], 0, 0, 0);
+    }
+}
+
+__global__ __launch_bounds__(256) void k_mlp_grad(long n, const float* __restrict__ U, const float* __restrict__ T,
+                                                  const float* __restrict__ C, float cs, const float* __restrict__ P,
+                                                  float* __restrict__ Gpart, float* __restrict__ losspart) {
+  __shared__ __attribute__((aligned(16))) MlpGradSmem sm;
+  const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, c = lane & 15;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int u0 = 16 * w + 4 * g;  // the lane's first unit
+  // operands of the wave's 16 rows: W2, W3 (row 16 w + c) and their transposes (column 16 w + c)
+  float a2[16], a3[16], t2[16], t3[16];
+#pragma unroll
+  for (int q = 0; q < 16; ++q) {
+    const int k = 16 * (q >> 2) + 4 * g + (q & 3);
+    a2[q] = P[kMlpW2 + kMlpH * (16 * w + c) + k];
+    a3[q] = P[kMlpW3 + kMlpH * (16 * w + c) + k];
+    t2[q] = P[kMlpW2 + kMlpH * k + 16 * w + c];
+    t3[q] = P[kMlpW3 + kMlpH * k + 16 * w + c];
+  }
+  float w1[4][3], b1[4], b2[4], b3[4], w4[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+#pragma unroll
+    for (int k = 0; k < 3; ++k) w1[r][k] = P[kMlpW1 + 3 * (u0 + r) + k];
+    b1[r] = P[kMlpB1 + u0 + r];
+    b2[r] = P[kMlpB2 + u0 + r];
+    b3[r] = P[kMlpB3 + u0 + r];
+    w4[r] = P[kMlpW4 + u0 + r];
+  }
+  const float b4 = P[kMlpB4];
+  f32x4_t gW2[4], gW3[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) gW2[j] = gW3[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  float gW1[4][3] = {}, gb1[4] = {}, gb2[4] = {}, gb3[4] = {}, gw4[4] = {}, gb4 = 0.f, lsum = 0.f;
+  // a layer's result at the lane's units and samples, into both layouts
+  auto put = [&](float (*Sm)[kGp], float (*Um)[kGp], const f32x4_t (&v)[4]) {
+#pragma unroll
+    for (int nt = 0; nt < 4; ++nt) {
+      *reinterpret_cast<f32x4_t*>(&Sm[16 * nt + c][u0]) = v[nt];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) Um[u0 + r][16 * nt + c] = v[nt][r];
+    }
+  };
+  // dW (rows 16 w.., 64 columns) += D H^T over the chunk's samples
+  auto outer = [&](const float (*Um)[kGp], f32x4_t (&dW)[4]) {
+    float a[16];
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      const f32x4_t v = *reinterpret_cast<const f32x4_t*>(&sm.Du[16 * w + c][16 * ks + 4 * g]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) a[4 * ks + e] = v[e];
+    }
+    mlp_gemm(a, Um, g, c, dW);
+  };
   const long nchunks = (n + kLanes - 1) / kLanes;
-  for (long c = blockIdx.x; c < nchunks; c += gridDim.x) {
-    const long i = c * kLanes + lane;
-    const bool live = i < n;
-    const long ic = live ? i : n - 1;
-    const float u[3] = {U[3 * ic], U[3 * ic + 1], U[3 * ic + 2]};
+  for (long ch = blockIdx.x; ch < nchunks; ch += gridDim.x) {
     __syncthreads();  // the previous chunk's readers are done
-    Us[lane][0] = u[0];
-    Us[lane][1] = u[1];
-    Us[lane][2] = u[2];
-    // forward, own sample
-    float z2[kMlpH];
-#pragma unroll
-    for (int q = 0; q < kMlpH; ++q) z2[q] = ldp(R, kMlpB2 + q);
-    for (int j = 0; j < kMlpH; ++j) {
-      const float aj = ::tanhf(ldp(R, kMlpB1 + j) + ldp(R, kMlpW1 + 3 * j) * u[0] +
-                               ldp(R, kMlpW1 + 3 * j + 1) * u[1] + ldp(R, kMlpW1 + 3 * j + 2) * u[2]);
-      A1[lane][j] = aj;
-#pragma unroll
-      for (int q = 0; q < kMlpH; ++q) z2[q] += ldp(R, kMlpW2 + kMlpH * j + q) * aj;
+    if (tid < 3 * kLanes) {
+      const long i = ch * kLanes + tid / 3;
+      sm.U[tid / 3][tid % 3] = U[3 * (i < n ? i : n - 1) + tid % 3];
     }
-#pragma unroll
-    for (int q = 0; q < kMlpH; ++q) {
-      z2[q] = ::tanhf(z2[q]);
-      A2[lane][q] = z2[q];
-    }
-    float y = ldp(R, kMlpB4);
-    for (int q = 0; q < kMlpH; ++q) {
-      float z = ldp(R, kMlpB3 + q);
-#pragma unroll
-      for (int j = 0; j < kMlpH; ++j) z += ldp(R, kMlpW3 + kMlpH * q + j) * z2[j];
-      const float h = ::tanhf(z);
-      D[q][lane] = h;
-      y += ldp(R, kMlpW4 + q) * h;
-    }
-    const float cw = live ? cs * (C ? C[ic] : 1.f) : 0.f;
-    const float e = live ? y - T[ic] : 0.f;
-    lsum += cw * e * e;
-    const float g = 2.f * cw * e;  // dL/dy
-    gs[lane] = g;
     __syncthreads();
-    // w4, b4: row `lane` of h3 against dL/dy
-    {
-      float t = 0.f, b = 0.f;
-      for (int q = 0; q < kLanes; ++q) {
-        t += gs[q] * D[lane][q];
-        b += gs[q];
+    f32x4_t h1[4], h2[4], h3[4], d[4];
+    float us[4][3];
+#pragma unroll
+    for (int nt = 0; nt < 4; ++nt) {
+#pragma unroll
+      for (int k = 0; k < 3; ++k) us[nt][k] = sm.U[16 * nt + c][k];
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        h1[nt][r] = ::tanhf(b1[r] + w1[r][0] * us[nt][0] + w1[r][1] * us[nt][1] + w1[r][2] * us[nt][2]);
+    }
+    put(sm.Hs1, sm.Hu1, h1);
+    __syncthreads();
+#pragma unroll
+    for (int nt = 0; nt < 4; ++nt) h2[nt] = f32x4_t{b2[0], b2[1], b2[2], b2[3]};
+    mlp_gemm(a2, sm.Hs1, g, c, h2);
+#pragma unroll
+    for (int nt = 0; nt < 4; ++nt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) h2[nt][r] = ::tanhf(h2[nt][r]);
+    put(sm.Hs2, sm.Hu2, h2);
+    __syncthreads();
+#pragma unroll
+    for (int nt = 0; nt < 4; ++nt) h3[nt] = f32x4_t{b3[0], b3[1], b3[2], b3[3]};
+    mlp_gemm(a3, sm.Hs2, g, c, h3);
+#pragma unroll
+    for (int nt = 0; nt < 4; ++nt) {
+      float y = 0.f;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        h3[nt][r] = ::tanhf(h3[nt][r]);
+        y += w4[r] * h3[nt][r];
       }
-      gw4 += t;
-      gb4 += b;  // every lane holds the same sum; lane 0 adds it to G
+      y += __shfl_xor(y, 16);
+      y += __shfl_xor(y, 32);
+      if (g == 0) sm.y[w][16 * nt + c] = y;
     }
     __syncthreads();
-    // d3, own column
 #pragma unroll
-    for (int q = 0; q < kMlpH; ++q) {
-      const float h = D[q][lane];
-      D[q][lane] = g * ldp(R, kMlpW4 + q) * (1.f - h * h);
-    }
-    __syncthreads();
-    // row `lane` of dW3 = d3 a2^T, db3
-    for (int q = 0; q < kLanes; ++q) {
-      const float d = D[lane][q];
-      gb3 += d;
+    for (int nt = 0; nt < 4; ++nt) {
+      const int s = 16 * nt + c;
+      const long i = ch * kLanes + s;
+      const bool live = i < n;
+      const float y = b4 + ((sm.y[0][s] + sm.y[1][s]) + (sm.y[2][s] + sm.y[3][s]));
+      const float cw = live ? cs * (C ? C[i] : 1.f) : 0.f, e = live ? y - T[i] : 0.f;
+      const float gy = 2.f * cw * e;  // dL/dy
+      lsum += cw * e * e;
+      gb4 += gy;
 #pragma unroll
-      for (int j = 0; j < kMlpH; ++j) gW3[j] += d * A2[q][j];
-    }
-    __syncthreads();
-    // d2 = (W3^T d3)(1 - a2^2), own column
-    {
-      float acc[kMlpH];
-#pragma unroll
-      for (int j = 0; j < kMlpH; ++j) acc[j] = 0.f;
-      for (int q = 0; q < kMlpH; ++q) {
-        const float d3 = D[q][lane];
-#pragma unroll
-        for (int j = 0; j < kMlpH; ++j) acc[j] += ldp(R, kMlpW3 + kMlpH * q + j) * d3;
-      }
-#pragma unroll
-      for (int j = 0; j < kMlpH; ++j) {
-        const float b = A2[lane][j];
-        D[j][lane] = acc[j] * (1.f - b * b);
+      for (int r = 0; r < 4; ++r) {
+        gw4[r] += gy * h3[nt][r];
+        d[nt][r] = gy * w4[r] * (1.f - h3[nt][r] * h3[nt][r]);
+        gb3[r] += d[nt][r];
       }
     }
+    put(sm.Ds, sm.Du, d);
     __syncthreads();
-    // row `lane` of dW2 = d2 a1^T, db2
-    for (int q = 0; q < kLanes; ++q) {
-      const float d = D[lane][q];
-      gb2 += d;
+    outer(sm.Hu2, gW3);
 #pragma unroll
-      for (int j = 0; j < kMlpH; ++j) gW2[j] += d * A1[q][j];
-    }
-    __syncthreads();
-    // d1 = (W2^T d2)(1 - a1^2), own column
-    {
-      float d2[kMlpH];
+    for (int nt = 0; nt < 4; ++nt) d[nt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    mlp_gemm(t3, sm.Ds, g, c, d);
 #pragma unroll
-      for (int j = 0; j < kMlpH; ++j) d2[j] = D[j][lane];
-      for (int k = 0; k < kMlpH; ++k) {
-        float t = 0.f;
+    for (int nt = 0; nt < 4; ++nt)
 #pragma unroll
-        for (int j = 0; j < kMlpH; ++j) t += ldp(R, kMlpW2 + kMlpH * k + j) * d2[j];
-        const float a = A1[lane][k];
-        D[k][lane] = t * (1.f - a * a);
+      for (int r = 0; r < 4; ++r) {
+        d[nt][r] *= 1.f - h2[nt][r] * h2[nt][r];
+        gb2[r] += d[nt][r];
       }
-    }
+    __syncthreads();  // layer 3's deltas are read
+    put(sm.Ds, sm.Du, d);
     __syncthreads();
-    // row `lane` of dW1 = d1 u^T, db1
-    for (int q = 0; q < kLanes; ++q) {
-      const float d = D[lane][q];
-      gb1 += d;
-      gW1[0] += d * Us[q][0];
-      gW1[1] += d * Us[q][1];
-      gW1[2] += d * Us[q][2];
+    outer(sm.Hu1, gW2);
+#pragma unroll
+    for (int nt = 0; nt < 4; ++nt) d[nt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    mlp_gemm(t2, sm.Ds, g, c, d);
+#pragma unroll
+    for (int nt = 0; nt < 4; ++nt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float d1 = d[nt][r] * (1.f - h1[nt][r] * h1[nt][r]);
+        gb1[r] += d1;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) gW1[r][k] += d1 * us[nt][k];
+      }
+  }
+  float* __restrict__ G = Gpart + (size_t)blockIdx.x * kMlpParams;
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      G[kMlpW2 + kMlpH * (u0 + r) + 16 * j + c] = gW2[j][r];
+      G[kMlpW3 + kMlpH * (u0 + r) + 16 * j + c] = gW3[j][r];
+    }
+  auto sum16 = [](float v) {  // over the 16 lanes of a group: the samples
+    for (int o = 1; o < 16; o <<= 1) v += __shfl_xor(v, o);
+    return v;
+  };
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const float s1 = sum16(gb1[r]), s2 = sum16(gb2[r]), s3 = sum16(gb3[r]), s4 = sum16(gw4[r]);
+    const float q0 = sum16(gW1[r][0]), q1 = sum16(gW1[r][1]), q2 = sum16(gW1[r][2]);
+    if (c == 0) {
+      G[kMlpB1 + u0 + r] = s1;
+      G[kMlpB2 + u0 + r] = s2;
+      G[kMlpB3 + u0 + r] = s3;
+      G[kMlpW4 + u0 + r] = s4;
+      G[kMlpW1 + 3 * (u0 + r)] = q0;
+      G[kMlpW1 + 3 * (u0 + r) + 1] = q1;
+      G[kMlpW1 + 3 * (u0 + r) + 2] = q2;
     }
   }
-  // canonical layout: W[out][in], row `lane` of each matrix
-#pragma unroll
-  for (int j = 0; j < kMlpH; ++j) {
-    atomicAdd(&G[kMlpW2 + kMlpH * lane + j], gW2[j]);
-    atomicAdd(&G[kMlpW3 + kMlpH * lane + j], gW3[j]);
-  }
-  atomicAdd(&G[kMlpW1 + 3 * lane], gW1[0]);
-  atomicAdd(&G[kMlpW1 + 3 * lane + 1], gW1[1]);
-  atomicAdd(&G[kMlpW1 + 3 * lane + 2], gW1[2]);
-  atomicAdd(&G[kMlpB1 + lane], gb1);
-  atomicAdd(&G[kMlpB2 + lane], gb2);
-  atomicAdd(&G[kMlpB3 + lane], gb3);
-  atomicAdd(&G[kMlpW4 + lane], gw4);
-  for (int o = 32; o > 0; o >>= 1) lsum += __shfl_xor(lsum, o);
-  if (lane == 0) {
-    atomicAdd(&G[kMlpB4], gb4);
-    atomicAdd(loss, lsum);
+  gb4 = sum16(gb4);  // the same in every group
+  lsum = sum16(lsum);
+  if (tid == 0) {
+    G[kMlpB4] = gb4;
+    losspart[blockIdx.x] = lsum;
   }
 }
 
-// Adam (Kingma and Ba, ICLR 2015) on the canonical FP32 weights; clears the
-// gradient and refreshes both run copies.
-__global__ void k_mlp_adam(float* __restrict__ P, float* __restrict__ G, float* __restrict__ M,
-                           float* __restrict__ V, float* __restrict__ Prun, float* __restrict__ Pinf, float lr, float b1,
-                           float b2, float eps, float c1, float c2) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= kMlpParams) return;
-  const float g = G[k];
-  const float m = b1 * M[k] + (1.f - b1) * g, v = b2 * V[k] + (1.f - b2) * g * g;
-  M[k] = m;
-  V[k] = v;
-  const float p = P[k] - lr * (m / c1) / (::sqrtf(v / c2) + eps);
-  P[k] = p;
-  G[k] = 0.f;
-  Prun[run_index(k)] = p;
-  Pinf[run_index(k)] = bf16_round(p);
+// The gradient and loss from the blocks' sums, 64 parameters per block, 16
+// partial sums each; ADAM: one step of Adam (Kingma and Ba, ICLR 2015) on the
+// canonical FP32 weights, else the gradient goes to G. *loss gets the loss added.
+template <bool ADAM>
+__global__ __launch_bounds__(1024) void k_mlp_update(int nparts, const float* __restrict__ Gpart,
+                                                     const float* __restrict__ losspart, float* __restrict__ P,
+                                                     float* __restrict__ G, float* __restrict__ M,
+                                                     float* __restrict__ V, float* __restrict__ loss, float lr,
+                                                     float b1, float b2, float eps, float c1, float c2) {
+  __shared__ float red[16][64];
+  const int p = threadIdx.x & 63, s = threadIdx.x >> 6, k = blockIdx.x * 64 + p;
+  float t = 0.f;
+  if (k < kMlpParams)
+    for (int b = s; b < nparts; b += 16) t += Gpart[(size_t)b * kMlpParams + k];
+  red[s][p] = t;
+  __syncthreads();
+  if (s == 0 && k < kMlpParams) {
+    float g = 0.f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) g += red[i][p];
+    if (ADAM) {
+      const float m = b1 * M[k] + (1.f - b1) * g, v = b2 * V[k] + (1.f - b2) * g * g;
+      M[k] = m;
+      V[k] = v;
+      P[k] -= lr * (m / c1) / (::sqrtf(v / c2) + eps);
+    } else {
+      G[k] = g;
+    }
+  }
+  if (blockIdx.x == 0 && s == 1) {
+    float l = 0.f;
+    for (int b = p; b < nparts; b += 64) l += losspart[b];
+    for (int o = 32; o > 0; o >>= 1) l += __shfl_xor(l, o);
+    if (p == 0) *loss += l;
+  }
 }
 
 // Training samples: descriptors t (n x 3) and target F = e_xc / e_x^unif of
@@ -719,21 +798,28 @@ void launch_mlp_pack_mx(hipStream_t st, const float* P, unsigned* Wpk) {
   CHX_HIP(hipGetLastError());
 }
 
-void launch_mlp_grad(hipStream_t st, long n, const float* U, const float* T, const float* C, float cs, const float* R,
-                     float* G, float* loss, int max_blocks) {
-  if (n <= 0) return;
+int launch_mlp_grad(hipStream_t st, long n, const float* U, const float* T, const float* C, float cs, const float* P,
+                    float* Gpart, float* losspart) {
+  if (n <= 0) return 0;
   const long nchunks = (n + kLanes - 1) / kLanes;
-  const unsigned nb = (unsigned)(nchunks < max_blocks ? nchunks : max_blocks);
-  hipLaunchKernelGGL(k_mlp_grad, dim3(nb), dim3(kLanes), 0, st, n, U, T, C, cs, R, G, loss);
+  const int nb = (int)(nchunks < kMlpGradBlocks ? nchunks : kMlpGradBlocks);
+  hipLaunchKernelGGL(k_mlp_grad, dim3(nb), dim3(256), 0, st, n, U, T, C, cs, P, Gpart, losspart);
+  CHX_HIP(hipGetLastError());
+  return nb;
+}
+
+void launch_mlp_adam(hipStream_t st, int nparts, const float* Gpart, const float* losspart, float* P, float* M,
+                     float* V, float* loss, float lr, int step) {
+  const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
+  const float c1 = 1.f - std::pow(b1, (float)step), c2 = 1.f - std::pow(b2, (float)step);
+  hipLaunchKernelGGL(k_mlp_update<true>, dim3((kMlpParams + 63) / 64), dim3(1024), 0, st, nparts, Gpart, losspart, P,
+                     nullptr, M, V, loss, lr, b1, b2, eps, c1, c2);
   CHX_HIP(hipGetLastError());
 }
 
-void launch_mlp_adam(hipStream_t st, float* P, float* G, float* M, float* V, float* Prun, float* Pinf, float lr,
-                     int step) {
-  const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
-  const float c1 = 1.f - std::pow(b1, (float)step), c2 = 1.f - std::pow(b2, (float)step);
-  hipLaunchKernelGGL(k_mlp_adam, dim3((kMlpParams + 255) / 256), dim3(256), 0, st, P, G, M, V, Prun, Pinf, lr, b1, b2,
-                     eps, c1, c2);
+void launch_mlp_reduce(hipStream_t st, int nparts, const float* Gpart, const float* losspart, float* G, float* loss) {
+  hipLaunchKernelGGL(k_mlp_update<false>, dim3((kMlpParams + 63) / 64), dim3(1024), 0, st, nparts, Gpart, losspart,
+                     nullptr, G, nullptr, nullptr, loss, 0.f, 0.f, 0.f, 0.f, 1.f, 1.f);
   CHX_HIP(hipGetLastError());
 }
 

@@ -74,6 +74,23 @@ def test_loss_gradient_against_oracle(n, weighted):
     assert eg <= 1e-4
 
 
+@pytest.mark.parametrize("n", [15, 63, 65, 16384, 16385])
+def test_loss_gradient_at_block_edges(n):
+    """64 samples per pass of a block, 256 blocks: one short, one over, and a repeated call (the blocks' sums
+    are added in a fixed order, so it gives the same bits)."""
+    s = Surrogate(4)
+    s.params = _rand_params(6)
+    rng = np.random.default_rng(n)
+    U = rng.uniform(-1, 1, (n, 3)).astype(np.float32)
+    T = rng.uniform(0.8, 1.7, n).astype(np.float32)
+    L, G = s.loss_grad(U, T, None)
+    Lo, Go = ol.mlp_loss_grad(s.params.astype(np.float64), U.astype(np.float64), T.astype(np.float64), None)
+    assert abs(L - Lo) <= 1e-5 * Lo
+    assert np.abs(G - Go).max() <= 1e-4 * np.abs(Go).max()
+    L2, G2 = s.loss_grad(U, T, None)
+    assert L2 == L and np.array_equal(G, G2)
+
+
 @pytest.mark.parametrize("base", [(), (1, 7)])
 def test_eval_points_and_fallback(base):
     s = Surrogate(6, base=base)
