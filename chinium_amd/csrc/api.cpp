@@ -578,6 +578,32 @@ int chx_grid_fock_u(chx_grid* g, double* F, int nmats, int nspin, int nbasis) {
   });
 }
 
+// Workspace of one derivative call, kept on the grid for the next one (until it
+// is planned again) unless it is larger than kWsKeep: hipMalloc and hipFree of
+// these buffers on every call cost more than the kernels of a small system, and
+// now and then 10 ms and more.
+struct Workspace {
+  static constexpr size_t kWsKeep = (size_t)1 << 30;  // bytes
+  chx_grid* g;
+  size_t used = 0;
+  // total: doubles of all takes, each rounded up by round()
+  Workspace(chx_grid* grid, size_t total) : g(grid) {
+    if (g->d_ws.n < total) g->d_ws.alloc(total);
+  }
+  ~Workspace() {
+    if (g->d_ws.n * sizeof(double) > kWsKeep) g->d_ws.release();
+  }
+  Workspace(const Workspace&) = delete;
+  Workspace& operator=(const Workspace&) = delete;
+  static size_t round(size_t n) { return (std::max<size_t>(n, 1) + 31) / 32 * 32; }  // 256 bytes
+  double* take(size_t n) {
+    double* p = g->d_ws.p + used;
+    used += round(n);
+    require(used <= g->d_ws.n, CHX_ERR_STATE, "workspace overrun");
+    return p;
+  }
+};
+
 // slot -> (density group, column tile in the group), for the per-slot epilogues
 static void ensure_slot_groups(chx_grid* g) {
   const int ng = (int)g->grp_batch.size(), ns = (int)g->slot_tile.size();
@@ -740,15 +766,14 @@ int chx_grid_energy_grad(chx_grid* g, double* grad) {
     const int na = g->mol.natoms, ng = (int)g->grp_batch.size(), ns = (int)g->slot_tile.size();
     ensure_slot_groups(g);
     launch_make_b(g->stream, g->nbatches, g->d_bt_off.p, g->d_coef.p, g->d_cache.p, g->d_bmat.p);
-    DevBuf<double> xz, dg;
-    xz.alloc(std::max<size_t>(1, (size_t)ng * 2 * kGroup * kTile * kBatch));
-    dg.alloc(3 * (size_t)na);
-    launch_fill(g->stream, dg.p, 3 * (size_t)na, 0.0);
+    const size_t nxz = (size_t)ng * 2 * kGroup * kTile * kBatch, n3 = 3 * (size_t)na;
+    Workspace ws(g, Workspace::round(nxz) + Workspace::round(kGradCopies * n3) + Workspace::round(n3));
+    double *xz = ws.take(nxz), *gpart = ws.take(kGradCopies * n3), *dg = ws.take(n3);
     launch_xgrad_xz(g->stream, ng, g->d_grp_batch.p, g->d_grp_tile.p, g->d_grp_ntiles.p, g->d_bt_off.p, g->d_b_chunk.p,
-                    g->d_chunks.p, g->d_cache.p, g->d_bmat.p, g->d_Dskel_t.p, 0, -1, xz.p);
+                    g->d_chunks.p, g->d_cache.p, g->d_bmat.p, g->d_Dskel_t.p, 0, -1, xz);
     launch_xgrad_epi(g->stream, ns, g->d_slot_batch.p, g->d_slot_tile.p, g->d_slot_grp.p, g->d_slot_q.p, g->d_x.p,
-                     g->d_y.p, g->d_z.p, g->view(), g->d_coef.p, xz.p, dg.p);
-    CHX_HIP(hipMemcpyAsync(grad, dg.p, sizeof(double) * 3 * na, hipMemcpyDeviceToHost, g->stream));
+                     g->d_y.p, g->d_z.p, g->view(), g->d_coef.p, xz, na, gpart, dg);
+    CHX_HIP(hipMemcpyAsync(grad, dg, sizeof(double) * n3, hipMemcpyDeviceToHost, g->stream));
     CHX_HIP(hipStreamSynchronize(g->stream));
   });
 }

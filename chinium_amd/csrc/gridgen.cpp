@@ -567,6 +567,7 @@ void set_vxc_shape(chx_grid* g, int shape) {
 // Screening and work plans (Grid::getAO counterpart).
 void grid_plan(chx_grid* g) {
   hipStream_t st = g->stream;
+  g->d_ws.release();
   const int nb = g->nbatches, nsh = (int)g->sh_type.size(), nwords = (nsh + 63) / 64;
   std::vector<double> reach2(nsh);
   for (int s = 0; s < nsh; ++s) {

@@ -303,13 +303,15 @@ struct MolDev {
 constexpr int kMxMaxTiles = 512;  // basis size the mixed form takes (npad <= 16384)
 constexpr int kMxMaxChunk = 128;  // batches per Vxc work item in the mixed form
 
-// XC nuclear gradient (kernels_grad.hip), FP64 cached form.
+// XC nuclear gradient (kernels_grad.hip), FP64 cached form. gpart: kGradCopies
+// partial gradients of 3 natoms.
+constexpr int kGradCopies = 64;
 void launch_xgrad_xz(hipStream_t s, int ngroups, const int* grp_batch, const int* grp_tile, const int* grp_ntiles,
                      const int* bt_off, const int* b_chunk, const ChunkDev* chunks, const double* cache,
                      const double* bmat, const double* Dt, int c1, int c2, double* xz);
 void launch_xgrad_epi(hipStream_t s, int nslots, const int* slot_batch, const int* slot_tile, const int* slot_grp,
                       const int* slot_q, const double* bx, const double* by, const double* bz, BasisView bv,
-                      const double* coef, const double* xz, double* grad);
+                      const double* coef, const double* xz, int natoms, double* gpart, double* grad);
 // skeleton density derivatives (rho, grad rho per nuclear coordinate) into
 // rhos[3 atom + t][npt points][4], accumulated (clear it first)
 // Skeleton Fock derivative: E^t = a d_t phi + (c . grad) d_t phi per slot into
@@ -475,6 +477,7 @@ struct chx_grid {
   chx::DevBuf<double> d_U64;
   chx::DevBuf<int> d_asym;              // number of the last build whose D was not symmetric
   int d_gen = 0;                        // builds counted
+  chx::DevBuf<double> d_ws;             // derivative calls' workspace (Workspace in api.cpp)
   double flops_build = 0, mean_tiles = 0;
   std::vector<double> batch_work;  // g_b n_b^2 per batch (points x kept AOs squared)
   double core_flops = 0;           // the core batches' three-term (rho, grad rho) launch: 2 sum g_b n_b^2

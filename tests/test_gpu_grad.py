@@ -59,6 +59,20 @@ def test_water_cluster_gradient():
     assert np.abs(G - Go).max() <= G_TOL
 
 
+@pytest.mark.parametrize("nw,basis", [(2, "cc-pvdz"), (3, "def2-svp"), (6, "def2-svp")])
+def test_gradient_by_tiles_per_group(nw, basis):
+    """2 and 3 column tiles in a density group, and a second, short group (5 tiles)."""
+    Z, X = wl.water_cluster_angstrom(nw, 6.0, 20 + nw)
+    xyz = X * ca.ANGSTROM_TO_BOHR
+    mol = ca.Molecule(Z, xyz, basis)
+    D, S = wl.workload_density(mol, 5 * nw, 3)
+    grid, G = _gpu_grad(mol, "SG-1", "PBE", D)
+    orc = ol.OracleSystem(Z, xyz, "SG-1", basis)
+    orc.set_functional("PBE")
+    orc.get_ao()
+    assert np.abs(G - orc.xc_grad(D)).max() <= G_TOL
+
+
 def test_gradient_protocol():
     w = wl.build_workload("h2o_ccpvdz_sg1_pbe")
     mol = ca.Molecule(w["Z"], w["xyz_bohr"], w["basis"])
