@@ -504,25 +504,71 @@ int chx_grid_get_density_skeleton(chx_grid* g, const double* D, int nspin, int n
   });
 }
 
+// Workspace of one derivative call, kept on the grid for the next one (until it
+// is planned again) unless it is larger than kWsKeep: hipMalloc and hipFree of
+// these buffers on every call cost more than the kernels of a small system, and
+// now and then 10 ms and more.
+struct Workspace {
+  static constexpr size_t kWsKeep = (size_t)1 << 30;  // bytes
+  chx_grid* g;
+  size_t used = 0;
+  // total: doubles of all takes, each rounded up by round()
+  Workspace(chx_grid* grid, size_t total) : g(grid) {
+    require(!g->ws_live, CHX_ERR_STATE, "the grid's workspace is in use");
+    if (g->d_ws.n < total) g->d_ws.alloc(total);
+    g->ws_live = true;
+  }
+  ~Workspace() {
+    g->ws_live = false;
+    if (g->d_ws.n * sizeof(double) > kWsKeep) g->d_ws.release();
+  }
+  Workspace(const Workspace&) = delete;
+  Workspace& operator=(const Workspace&) = delete;
+  static size_t round(size_t n) { return (std::max<size_t>(n, 1) + 31) / 32 * 32; }  // 256 bytes
+  double* take(size_t n) {
+    double* p = g->d_ws.p + used;
+    used += round(n);
+    require(used <= g->d_ws.n, CHX_ERR_STATE, "workspace overrun");
+    return p;
+  }
+};
+
+// Matrices that one set of launches takes together, `per` doubles of workspace
+// each: as many as fit into a quarter of what a workspace may keep (their kernels
+// are a few microseconds each for small systems, and large systems fill the chip
+// with one).
+static int matrices_at_once(size_t per, int nmats) {
+  const size_t fit = Workspace::kWsKeep / sizeof(double) / 4 / std::max<size_t>(per, 1);
+  return (int)std::max<size_t>(1, std::min<size_t>({fit, (size_t)nmats, (size_t)1024}));
+}
+
 int chx_grid_get_density_u(chx_grid* g, const double* D, int nmats, int nspin, int nbasis) {
   return guard([&] {
     check_dm_args(g, nspin, nbasis, 2);
     require(D != nullptr && nmats >= 1, CHX_ERR_ARG, "bad perturbed density matrices");
     require(g->precision == CHX_PREC_FP64, CHX_ERR_UNSUPPORTED, "the response path is built for the FP64 form");
     const size_t nslots = (size_t)g->nbatches * kBatch, nb2 = (size_t)nbasis * nbasis;
-    const int ng = (int)g->grp_batch.size();
-    double* part = g->d_part_u.alloc_get(std::max<size_t>(1, (size_t)ng * 4 * kBatch));
-    double* rhou = g->d_rhou.alloc_get(std::max<size_t>(1, (size_t)nspin * nmats * 4 * nslots));
-    for (int m = 0; m < nspin * nmats; ++m) {  // rho^x and grad rho^x of each matrix ([spin][mat]), per point
-      CHX_HIP(hipMemcpyAsync(g->d_Din.p, D + m * nb2, sizeof(double) * nb2, hipMemcpyHostToDevice, g->stream));
-      gather_d(g, g->d_Din.p, g->d_Dt);
+    const int ng = (int)g->grp_batch.size(), ntot = nspin * nmats;
+    double* rhou = g->d_rhou.alloc_get(std::max<size_t>(1, (size_t)ntot * 4 * nslots));
+    // rho^x and grad rho^x of each matrix ([spin][mat]), per point
+    const size_t sP = (size_t)ng * 4 * kBatch, sD = g->dt_elems;
+    const size_t rP = Workspace::round(sP), rD = Workspace::round(sD), rI = Workspace::round(nb2);
+    const int mb = g->cached ? matrices_at_once(rP + rD + rI, ntot) : 1;
+    Workspace ws(g, rI * mb + rP * mb + (mb > 1 ? rD * mb : 0));
+    double *Din = ws.take(rI * mb), *part = ws.take(rP * mb);
+    double* Dt = mb > 1 ? ws.take(rD * mb) : g->d_Dt.alloc_get(std::max<size_t>(1, sD));
+    for (int m = 0; m < ntot; m += mb) {
+      const int k = std::min(mb, ntot - m);
+      CHX_HIP(hipMemcpyAsync(Din, D + m * nb2, sizeof(double) * nb2 * k, hipMemcpyHostToDevice, g->stream));
+      launch_gather_d(g->stream, (int)g->tile_chunk.size(), nbasis, Din, g->d_tile_chunk.p, g->d_chunks.p,
+                      g->d_ao_of.p, Dt, nullptr, 0, k, sD);
       if (g->cached)
         launch_density_c64(g->stream, ng, g->d_grp_batch.p, g->d_grp_tile.p, g->d_grp_ntiles.p, g->d_bt_off.p,
-                           g->d_b_chunk.p, g->d_chunks.p, g->d_cache.p, g->d_Dt.p, nullptr, 0, part, nullptr);
+                           g->d_b_chunk.p, g->d_chunks.p, g->d_cache.p, Dt, nullptr, 0, part, nullptr, k, sD, sP);
       else
         launch_density_f64(g->stream, 0, ng, g->d_grp_batch.p, g->d_grp_tile.p, g->d_grp_ntiles.p, g->d_b_chunk.p,
-                         g->d_chunks.p, g->d_x.p, g->d_y.p, g->d_z.p, g->view(), g->d_Dt.p, part);
-      launch_point_rho(g->stream, g->nbatches, g->d_grp_off.p, part, rhou + (size_t)m * 4 * nslots);
+                           g->d_chunks.p, g->d_x.p, g->d_y.p, g->d_z.p, g->view(), Dt, part);
+      launch_point_rho(g->stream, g->nbatches, g->d_grp_off.p, part, rhou + (size_t)m * 4 * nslots, k, sP);
     }
     CHX_HIP(hipStreamSynchronize(g->stream));
     g->nmats_u = nmats;
@@ -535,31 +581,42 @@ int chx_grid_get_density_u(chx_grid* g, const double* D, int nmats, int nspin, i
 // (and spin, nspin = 2) the response coefficients (k_response_coef /
 // k_response_coef_pol), then the ground-state Vxc pipeline on them
 // (B = a phi + c . grad phi, M = Phi^T B, V = M + M^T), V to F (host,
-// [spin][mat]).
+// [spin][mat]). With the AO tables in HBM several matrices go through each
+// launch: (H2O)2 / def2-SVP / SG-1, 18 perturbations: 4 launches instead of 72.
 static void response_fock(chx_grid* g, const double* rhou, int nmats, double* F, int nspin = 1) {
   const size_t nslots = (size_t)g->nbatches * kBatch, nb2 = (size_t)g->nbasis * g->nbasis;
+  const int ntot = nspin * nmats;
   g->vout_ready = false;  // d_Vout stages the response matrices
-  double* coef = g->d_coef_u.alloc_get(std::max<size_t>(kCoef, kCoef * nslots));
-  for (int m = 0; m < nspin * nmats; ++m) {
-    if (nspin == 2)  // output m = spin u, perturbation m % nmats (both spins' rho^x enter)
-      launch_response_coef_pol(g->stream, g->nbatches, rhou + (size_t)(m % nmats) * 4 * nslots,
-                               rhou + (size_t)(nmats + m % nmats) * 4 * nslots, g->d_fx.p, g->d_w.p, g->fx_family,
-                               m / nmats, coef);
+  const size_t sC = kCoef * nslots, sB = g->slot_tile.size() * (size_t)kBatch * kTile, sU = g->u_elems;
+  const size_t rC = Workspace::round(sC), rB = Workspace::round(sB), rU = Workspace::round(sU);
+  const size_t rV = Workspace::round(nb2);
+  const int mb = g->cached ? matrices_at_once(rC + rB + rU + rV, ntot) : 1;
+  Workspace ws(g, rC * mb + (mb > 1 ? (rB + rU + rV) * mb : 0));
+  double *coef = ws.take(rC * mb), *bmat = g->d_bmat.p, *U = g->d_U64.p, *V = g->d_Vout.p;
+  if (mb > 1) {
+    bmat = ws.take(rB * mb);
+    U = ws.take(rU * mb);
+    V = ws.take(rV * mb);
+  }
+  for (int m = 0; m < ntot; m += mb) {
+    const int k = std::min(mb, ntot - m);
+    if (nspin == 2)
+      launch_response_coef_pol(g->stream, g->nbatches, rhou, g->d_fx.p, g->d_w.p, g->fx_family, m, k, nmats, coef);
     else
       launch_response_coef(g->stream, g->nbatches, rhou + (size_t)m * 4 * nslots, g->d_fx.p, g->d_w.p, g->fx_family,
-                           coef);
+                           k, coef);
     if (g->cached) {  // B = a phi + c . grad phi from the tables, M = Phi^T B, V = M + M^T
-      launch_make_b(g->stream, g->nbatches, g->d_bt_off.p, coef, g->d_cache.p, g->d_bmat.p);
-      launch_vxc_c64(g->stream, 1, (int)g->mwork.size(), g->d_mwork.p, g->d_cache.p, g->d_bmat.p, coef, g->d_U64.p);
-      launch_assemble<double>(g->stream, g->nbasis, g->d_rowptr.p, g->d_rows.p, g->d_ao_of.p, g->d_U64.p, g->d_Vout.p,
-                              nullptr, nullptr);
+      launch_make_b(g->stream, g->nbatches, g->d_bt_off.p, coef, g->d_cache.p, bmat, k, sC, sB);
+      launch_vxc_c64(g->stream, 1, (int)g->mwork.size(), g->d_mwork.p, g->d_cache.p, bmat, coef, U, k, sB, sU);
+      launch_assemble<double>(g->stream, g->nbasis, g->d_rowptr.p, g->d_rows.p, g->d_ao_of.p, U, V, nullptr, nullptr,
+                              k, sU);
     } else {
       launch_fill(g->stream, g->d_Mint.p, (size_t)g->npad * g->npad, 0.0);
       launch_vxc_f64(g->stream, 1, (int)g->vwork.size(), g->d_vwork.p, g->d_ao_of.p, g->d_x.p, g->d_y.p, g->d_z.p,
                      coef, g->view(), g->d_Mint.p, g->npad);
-      launch_finalize_sym(g->stream, g->nbasis, g->npad, g->d_Mint.p, g->d_Vout.p);
+      launch_finalize_sym(g->stream, g->nbasis, g->npad, g->d_Mint.p, V);
     }
-    CHX_HIP(hipMemcpyAsync(F + m * nb2, g->d_Vout.p, sizeof(double) * nb2, hipMemcpyDeviceToHost, g->stream));
+    CHX_HIP(hipMemcpyAsync(F + m * nb2, V, sizeof(double) * nb2 * k, hipMemcpyDeviceToHost, g->stream));
   }
   CHX_HIP(hipStreamSynchronize(g->stream));
 }
@@ -578,33 +635,7 @@ int chx_grid_fock_u(chx_grid* g, double* F, int nmats, int nspin, int nbasis) {
   });
 }
 
-// Workspace of one derivative call, kept on the grid for the next one (until it
-// is planned again) unless it is larger than kWsKeep: hipMalloc and hipFree of
-// these buffers on every call cost more than the kernels of a small system, and
-// now and then 10 ms and more.
-struct Workspace {
-  static constexpr size_t kWsKeep = (size_t)1 << 30;  // bytes
-  chx_grid* g;
-  size_t used = 0;
-  // total: doubles of all takes, each rounded up by round()
-  Workspace(chx_grid* grid, size_t total) : g(grid) {
-    if (g->d_ws.n < total) g->d_ws.alloc(total);
-  }
-  ~Workspace() {
-    if (g->d_ws.n * sizeof(double) > kWsKeep) g->d_ws.release();
-  }
-  Workspace(const Workspace&) = delete;
-  Workspace& operator=(const Workspace&) = delete;
-  static size_t round(size_t n) { return (std::max<size_t>(n, 1) + 31) / 32 * 32; }  // 256 bytes
-  double* take(size_t n) {
-    double* p = g->d_ws.p + used;
-    used += round(n);
-    require(used <= g->d_ws.n, CHX_ERR_STATE, "workspace overrun");
-    return p;
-  }
-};
-
-// slot -> (density group, column tile in the group), for the per-slot epilogues
+// slot -> (density group, column tile in the group) for the per-slot epilogues, AO -> atom
 static void ensure_slot_groups(chx_grid* g) {
   const int ng = (int)g->grp_batch.size(), ns = (int)g->slot_tile.size();
   if (g->slot_grp.size() == (size_t)ns) return;
@@ -617,6 +648,10 @@ static void ensure_slot_groups(chx_grid* g) {
       g->slot_q[s0 + q] = q;
     }
   }
+  std::vector<int> ao_atom(g->npad, -1);
+  for (const chx::ShellH& sh : g->mol.shells)
+    for (int k = 0; k < chx::shell_size(sh.type); ++k) ao_atom[sh.ao_off + k] = sh.center;
+  g->d_ao_atom.upload(ao_atom, g->stream);
   g->d_slot_grp.upload(g->slot_grp, g->stream);
   g->d_slot_q.upload(g->slot_q, g->stream);
 }
@@ -635,18 +670,19 @@ int chx_grid_fock_s(chx_grid* g, double* F, int nspin, int nbasis) {
     const long npt = (long)g->nbatches * kBatch;
     ensure_slot_groups(g);
     // per point and nuclear coordinate: rho^{A,t}, grad rho^{A,t}
-    const size_t nxz = std::max<size_t>(1, (size_t)ng * 2 * kGroup * kTile * kBatch);
-    DevBuf<double> xz1, xz2;
-    xz1.alloc(nxz);
-    xz2.alloc(nxz);
+    const size_t nxz = (size_t)ng * 2 * kGroup * kTile * kBatch;
     double* rhos = g->d_rhou.alloc_get(std::max<size_t>(1, (size_t)3 * na * 4 * npt));
     launch_fill(g->stream, rhos, (size_t)3 * na * 4 * npt, 0.0);
-    launch_xgrad_xz(g->stream, ng, g->d_grp_batch.p, g->d_grp_tile.p, g->d_grp_ntiles.p, g->d_bt_off.p,
-                    g->d_b_chunk.p, g->d_chunks.p, g->d_cache.p, g->d_bmat.p, g->d_Dskel_t.p, 0, 1, xz1.p);
-    launch_xgrad_xz(g->stream, ng, g->d_grp_batch.p, g->d_grp_tile.p, g->d_grp_ntiles.p, g->d_bt_off.p,
-                    g->d_b_chunk.p, g->d_chunks.p, g->d_cache.p, g->d_bmat.p, g->d_Dskel_t.p, 2, 3, xz2.p);
-    launch_skel_rho(g->stream, ns, g->d_slot_batch.p, g->d_slot_tile.p, g->d_slot_grp.p, g->d_slot_q.p, g->d_x.p,
-                    g->d_y.p, g->d_z.p, g->view(), xz1.p, xz2.p, npt, rhos);
+    {
+      Workspace ws(g, 2 * Workspace::round(nxz));
+      double *xz1 = ws.take(nxz), *xz2 = ws.take(nxz);
+      launch_xgrad_xz(g->stream, ng, g->d_grp_batch.p, g->d_grp_tile.p, g->d_grp_ntiles.p, g->d_bt_off.p,
+                      g->d_b_chunk.p, g->d_chunks.p, g->d_cache.p, g->d_bmat.p, g->d_Dskel_t.p, 0, 1, xz1);
+      launch_xgrad_xz(g->stream, ng, g->d_grp_batch.p, g->d_grp_tile.p, g->d_grp_ntiles.p, g->d_bt_off.p,
+                      g->d_b_chunk.p, g->d_chunks.p, g->d_cache.p, g->d_bmat.p, g->d_Dskel_t.p, 2, 3, xz2);
+      launch_skel_rho(g->stream, ns, g->d_slot_batch.p, g->d_slot_tile.p, g->d_slot_grp.p, g->d_slot_q.p, g->d_x.p,
+                      g->d_y.p, g->d_z.p, g->view(), xz1, xz2, npt, rhos);
+    }
     g->nmats_u = 0;  // rhou now holds the skeleton densities, not getDensityU's
     response_fock(g, rhos, 3 * na, F);
   });
@@ -665,32 +701,23 @@ int chx_grid_fock_skeleton(chx_grid* g, double* F, int nspin, int nbasis) {
             "the skeleton Fock derivative is built for the FP64 form with the AO tables in HBM");
     const int na = g->mol.natoms, ns = (int)g->slot_tile.size(), n = g->nbasis;
     const size_t pp = (size_t)g->npad * g->npad, sb = (size_t)kBatch * kTile;
-    // atom of each AO, reference order
-    std::vector<int> ao_atom(n, 0);
-    for (const chx::ShellH& sh : g->mol.shells)
-      for (int k = 0; k < chx::shell_size(sh.type); ++k) ao_atom[sh.ao_off + k] = sh.center;
-    DevBuf<int> d_atom;
-    d_atom.upload(ao_atom, g->stream);
+    ensure_slot_groups(g);
     launch_make_b(g->stream, g->nbatches, g->d_bt_off.p, g->d_coef.p, g->d_cache.p, g->d_bmat.p);
-    DevBuf<double> etab, qp, out;
-    etab.alloc(std::max<size_t>(1, 3 * (size_t)ns * sb));
-    launch_fill(g->stream, etab.p, 3 * (size_t)ns * sb, 0.0);
+    const size_t net = 3 * (size_t)ns * sb, tot = (size_t)3 * na * n * n;
+    Workspace ws(g, Workspace::round(net) + Workspace::round(6 * pp) + Workspace::round(tot));
+    double *etab = ws.take(net), *qp = ws.take(6 * pp), *out = ws.take(tot);
+    launch_fill(g->stream, etab, net, 0.0);
     launch_skel_etab(g->stream, ns, g->d_slot_batch.p, g->d_slot_tile.p, g->d_x.p, g->d_y.p, g->d_z.p, g->view(),
-                     g->d_coef.p, etab.p);
-    qp.alloc(6 * pp);
-    launch_fill(g->stream, qp.p, 6 * pp, 0.0);
-    for (int t = 0; t < 3; ++t) {
-      // Q^t = (d_t Phi)^T B: the cached component t + 1 as the row operand
-      launch_prod_c64(g->stream, (int)g->pwork.size(), g->d_pwork.p, g->d_ao_of.p, g->d_cache.p + (size_t)(t + 1) * sb, g->d_bmat.p,
-                      qp.p + t * pp, g->npad);
-      // P^t = Phi^T E^t: E^t in the B table's place
-      launch_prod_c64(g->stream, (int)g->pwork.size(), g->d_pwork.p, g->d_ao_of.p, g->d_cache.p, etab.p + (size_t)t * ns * sb,
-                      qp.p + (3 + t) * pp, g->npad);
-    }
-    const size_t tot = (size_t)3 * na * n * n;
-    out.alloc(std::max<size_t>(1, tot));
-    launch_fock_skel_fin(g->stream, n, g->npad, na, qp.p, d_atom.p, out.p);
-    CHX_HIP(hipMemcpyAsync(F, out.p, sizeof(double) * tot, hipMemcpyDeviceToHost, g->stream));
+                     g->d_coef.p, etab);
+    launch_fill(g->stream, qp, 6 * pp, 0.0);
+    // Q^t = (d_t Phi)^T B: the cached component t + 1 as the row operand
+    launch_prod_c64(g->stream, (int)g->pwork.size(), g->d_pwork.p, g->d_ao_of.p, g->d_cache.p + sb, g->d_bmat.p, qp,
+                    g->npad, 3, ProdBatch{1, sb, 0, pp});
+    // P^t = Phi^T E^t: E^t in the B table's place
+    launch_prod_c64(g->stream, (int)g->pwork.size(), g->d_pwork.p, g->d_ao_of.p, g->d_cache.p, etab, qp + 3 * pp,
+                    g->npad, 3, ProdBatch{3, 0, (size_t)ns * sb, pp});
+    launch_fock_skel_fin(g->stream, n, g->npad, na, qp, g->d_ao_atom.p, out);
+    CHX_HIP(hipMemcpyAsync(F, out, sizeof(double) * tot, hipMemcpyDeviceToHost, g->stream));
     CHX_HIP(hipStreamSynchronize(g->stream));
   });
 }
@@ -715,43 +742,32 @@ int chx_grid_energy_hess(chx_grid* g, double* H) {
     const long npt = (long)g->nbatches * kBatch;
     const size_t pp = (size_t)g->npad * g->npad, sb = (size_t)kBatch * kTile;
     ensure_slot_groups(g);
-    // atom of each AO (-1: padding)
-    std::vector<int> ao_atom(g->npad, -1);
-    for (const chx::ShellH& sh : g->mol.shells)
-      for (int k = 0; k < chx::shell_size(sh.type); ++k) ao_atom[sh.ao_off + k] = sh.center;
-    DevBuf<int> d_atom;
-    d_atom.upload(ao_atom, g->stream);
+    const size_t nxz = (size_t)ng * 2 * kGroup * kTile * kBatch, nrho = (size_t)np * 4 * npt, net = 3 * (size_t)ns * sb;
+    const size_t nhp = hess_part_elems(npt, np), nh = (size_t)np * np;
+    Workspace ws(g, 2 * Workspace::round(nxz) + Workspace::round(nrho) + Workspace::round(net) +
+                        Workspace::round(9 * pp) + Workspace::round(nhp) + Workspace::round(nh));
+    double *xz1 = ws.take(nxz), *xz2 = ws.take(nxz), *rhos = ws.take(nrho), *etab = ws.take(net), *rr = ws.take(9 * pp);
+    double *hpart = ws.take(nhp), *dH = ws.take(nh);
     // X = D phi, Y^x = D d_x phi (xz1); Y^y, Y^z (xz2); first-order skeleton densities
-    const size_t nxz = std::max<size_t>(1, (size_t)ng * 2 * kGroup * kTile * kBatch);
-    DevBuf<double> xz1, xz2, rhos, etab, rr, dH;
-    xz1.alloc(nxz);
-    xz2.alloc(nxz);
     launch_xgrad_xz(g->stream, ng, g->d_grp_batch.p, g->d_grp_tile.p, g->d_grp_ntiles.p, g->d_bt_off.p,
-                    g->d_b_chunk.p, g->d_chunks.p, g->d_cache.p, g->d_bmat.p, g->d_Dskel_t.p, 0, 1, xz1.p);
+                    g->d_b_chunk.p, g->d_chunks.p, g->d_cache.p, g->d_bmat.p, g->d_Dskel_t.p, 0, 1, xz1);
     launch_xgrad_xz(g->stream, ng, g->d_grp_batch.p, g->d_grp_tile.p, g->d_grp_ntiles.p, g->d_bt_off.p,
-                    g->d_b_chunk.p, g->d_chunks.p, g->d_cache.p, g->d_bmat.p, g->d_Dskel_t.p, 2, 3, xz2.p);
-    rhos.alloc(std::max<size_t>(1, (size_t)np * 4 * npt));
-    launch_fill(g->stream, rhos.p, (size_t)np * 4 * npt, 0.0);
+                    g->d_b_chunk.p, g->d_chunks.p, g->d_cache.p, g->d_bmat.p, g->d_Dskel_t.p, 2, 3, xz2);
+    launch_fill(g->stream, rhos, nrho, 0.0);
     launch_skel_rho(g->stream, ns, g->d_slot_batch.p, g->d_slot_tile.p, g->d_slot_grp.p, g->d_slot_q.p, g->d_x.p,
-                    g->d_y.p, g->d_z.p, g->view(), xz1.p, xz2.p, npt, rhos.p);
+                    g->d_y.p, g->d_z.p, g->view(), xz1, xz2, npt, rhos);
     // rr[3 t + s] = (d_t Phi)^T E^s over the cached contraction
     launch_make_b(g->stream, g->nbatches, g->d_bt_off.p, g->d_coef.p, g->d_cache.p, g->d_bmat.p);
-    etab.alloc(std::max<size_t>(1, 3 * (size_t)ns * sb));
-    launch_fill(g->stream, etab.p, 3 * (size_t)ns * sb, 0.0);
+    launch_fill(g->stream, etab, net, 0.0);
     launch_skel_etab(g->stream, ns, g->d_slot_batch.p, g->d_slot_tile.p, g->d_x.p, g->d_y.p, g->d_z.p, g->view(),
-                     g->d_coef.p, etab.p);
-    rr.alloc(9 * pp);
-    launch_fill(g->stream, rr.p, 9 * pp, 0.0);
-    for (int t = 0; t < 3; ++t)
-      for (int u = 0; u < 3; ++u)
-        launch_prod_c64(g->stream, (int)g->pwork.size(), g->d_pwork.p, g->d_ao_of.p, g->d_cache.p + (size_t)(t + 1) * sb, etab.p + (size_t)u * ns * sb,
-                      rr.p + (size_t)(3 * t + u) * pp, g->npad);
-    dH.alloc((size_t)np * np);
-    launch_fill(g->stream, dH.p, (size_t)np * np, 0.0);
+                     g->d_coef.p, etab);
+    launch_fill(g->stream, rr, 9 * pp, 0.0);
+    launch_prod_c64(g->stream, (int)g->pwork.size(), g->d_pwork.p, g->d_ao_of.p, g->d_cache.p + sb, etab, rr, g->npad,
+                    9, ProdBatch{3, sb, (size_t)ns * sb, pp});
     launch_hess_terms(g->stream, ns, g->d_slot_batch.p, g->d_slot_tile.p, g->d_slot_grp.p, g->d_slot_q.p, g->d_x.p,
-                      g->d_y.p, g->d_z.p, g->view(), g->d_coef.p, xz1.p, xz2.p, npt, rhos.p, g->d_fx.p, g->d_w.p,
-                      g->fx_family, g->npad, g->d_Dskel.p, rr.p, d_atom.p, np, dH.p);
-    CHX_HIP(hipMemcpyAsync(H, dH.p, sizeof(double) * np * np, hipMemcpyDeviceToHost, g->stream));
+                      g->d_y.p, g->d_z.p, g->view(), g->d_coef.p, xz1, xz2, npt, rhos, g->d_fx.p, g->d_w.p,
+                      g->fx_family, g->npad, g->d_Dskel.p, rr, g->d_ao_atom.p, np, hpart, dH);
+    CHX_HIP(hipMemcpyAsync(H, dH, sizeof(double) * nh, hipMemcpyDeviceToHost, g->stream));
     CHX_HIP(hipStreamSynchronize(g->stream));
   });
 }

@@ -157,7 +157,7 @@ void launch_screen(hipStream_t s, int nbatches, int nshells, int nwords, const d
 // rows of tile r from D (reference order, column-major n x n), zero for padding.
 // asym (may be null): *asym = gen when D is not symmetric to within rounding.
 void launch_gather_d(hipStream_t s, int ntiles, int n, const double* D, const int* tile_chunk, const ChunkDev* chunks,
-                     const int* ao_of, double* Dt, int* asym, int gen);
+                     const int* ao_of, double* Dt, int* asym, int gen, int nmat = 1, size_t sO = 0);
 void launch_pad_d(hipStream_t s, int n, int npad, const double* D, double* Dpad);
 // mode 0: rho, grad rho / 2 into part ([group][4][64]); mode r = 1..3: the tau
 // partial of direction r (part = component r - 1 of [group][3][64]).
@@ -193,15 +193,17 @@ constexpr int kFx = 8;  // per slot: v2rho2, v2rhosigma, v2sigma2, v_sigma, grad
 constexpr int kFxPol = 24;
 void launch_functional_fpol(hipStream_t s, int nbatches, const int* grp_off, const double* part, const double* part_b,
                             const int* codes, int ncodes, int family, double* fx);
-void launch_response_coef_pol(hipStream_t s, int nbatches, const double* rhou_a, const double* rhou_b,
-                              const double* fx, const double* bw, int family, int spin, double* coef);
+// outputs m0 .. m0 + nmat - 1 of [spin][perturbation] (nper perturbations)
+void launch_response_coef_pol(hipStream_t s, int nbatches, const double* rhou, const double* fx, const double* bw,
+                              int family, int m0, int nmat, int nper, double* coef);
 void launch_eval_functional_fpol(hipStream_t s, long n, const int* codes, int ncodes, const double* rho,
                                  const double* sigma, double* v2rho2, double* v2rhosigma, double* v2sigma2);
 void launch_functional_f(hipStream_t s, int nbatches, const int* grp_off, const double* part, const int* codes,
                          int ncodes, int family, double* fx);
-void launch_point_rho(hipStream_t s, int nbatches, const int* grp_off, const double* part, double* rhou);
+void launch_point_rho(hipStream_t s, int nbatches, const int* grp_off, const double* part, double* rhou, int nmat,
+                      size_t sP);
 void launch_response_coef(hipStream_t s, int nbatches, const double* rhou, const double* fx, const double* bw,
-                          int family, double* coef);
+                          int family, int nmat, double* coef);
 void launch_eval_functional_f(hipStream_t s, long n, const int* codes, int ncodes, const double* rho,
                               const double* sigma, double* v2rho2, double* v2rhosigma, double* v2sigma2);
 // spin-polarised (nspin = 2) functional, LDA/GGA and r2SCAN (part_tau / part_tau_b: meta-GGA)
@@ -254,20 +256,28 @@ void launch_functional_mlp(hipStream_t s, int nbatches, const int* grp_off, cons
 void launch_point_density(hipStream_t s, int nbatches, const int* grp_off, const double* part,
                           const double* part_tau, int has_tau, const double* bw, double* rho, double* sigma,
                           double* tau, double* w);
+// (the launches below: nmat matrices of one launch, s*: doubles from one matrix's
+// operand or result to the next one's; tau and ncomp 4 take one)
 // rho, grad rho / 2 into part; part_tau (not null: meta-GGA): tau (asym / gen as launch_gather_d's)
 void launch_density_c64(hipStream_t s, int ngroups, const int* grp_batch, const int* grp_tile, const int* grp_ntiles,
                         const int* bt_off, const int* b_chunk, const ChunkDev* chunks, const double* cache,
-                        const double* Dt, const int* asym, int gen, double* part, double* part_tau);
+                        const double* Dt, const int* asym, int gen, double* part, double* part_tau, int nmat = 1,
+                        size_t sD = 0, size_t sP = 0);
 // B = a phi + c . grad phi per slot (one component for every family)
 void launch_make_b(hipStream_t s, int nbatches, const int* bt_off, const double* coef, const double* cache,
-                   double* bmat);
+                   double* bmat, int nmat = 1, size_t sC = 0, size_t sB = 0);
 // upper blocks of V per run into U; ncomp 4 adds the tau term, its operand t d_r
 // phi formed from the cache and coef[4] as it is loaded
 void launch_vxc_c64(hipStream_t s, int ncomp, int nwork, const MxItem* work, const double* cache, const double* bmat,
-                    const double* coef, double* U);
-// M += A^T B over every pair of groups (items with I0, J0 in any order), A component 0 at `cache`
+                    const double* coef, double* U, int nmat = 1, size_t sB = 0, size_t sU = 0);
+// M += A^T B over every pair of groups (items with I0, J0 in any order), A component 0 at `cache`.
+// nmat products: A = cache + (m / nb) sA, B = bmat + (m % nb) sB, M + m sO.
+struct ProdBatch {
+  int nb = 1;
+  size_t sA = 0, sB = 0, sO = 0;
+};
 void launch_prod_c64(hipStream_t s, int nwork, const MxItem* work, const int* ao_of, const double* cache,
-                     const double* bmat, double* M, int npad);
+                     const double* bmat, double* M, int npad, int nmat, const ProdBatch& pb);
 void launch_finalize_sym(hipStream_t s, int n, int npad, const double* Mint, double* V);
 // Device descriptor of one grid for the mixed-precision kernels. A kernel
 // launch covers a list of (grid, item) pairs, so one launch can serve many
@@ -321,7 +331,7 @@ void launch_skel_etab(hipStream_t s, int nslots, const int* slot_batch, const in
                       const double* by, const double* bz, BasisView bv, const double* coef, double* etab);
 void launch_fock_skel_fin(hipStream_t s, int n, int npad, int natoms, const double* qp,
                           const int* ao_atom, double* F);
-// XC energy Hessian terms added to H (np x np, np = 3 natoms; clear it first):
+// XC energy Hessian terms into H (np x np, np = 3 natoms):
 // the per-slot diagonal-atom term (AO third derivatives, X and Y^r from xz1 /
 // xz2), the f_xc term of the first-order skeleton densities rhos, and the D
 // term from rr[3 t + s] = (d_t Phi)^T E^s (npad^2 each, internal order).
@@ -329,7 +339,8 @@ void launch_hess_terms(hipStream_t s, int nslots, const int* slot_batch, const i
                        const int* slot_q, const double* bx, const double* by, const double* bz, BasisView bv,
                        const double* coef, const double* xz1, const double* xz2, long npt, const double* rhos,
                        const double* fx, const double* bw, int family, int npad, const double* Dint,
-                       const double* rr, const int* atom, int np, double* H);
+                       const double* rr, const int* atom, int np, double* hpart, double* H);
+size_t hess_part_elems(long npt, int np);  // doubles of hpart (partial sums)
 void launch_skel_rho(hipStream_t s, int nslots, const int* slot_batch, const int* slot_tile, const int* slot_grp,
                      const int* slot_q, const double* bx, const double* by, const double* bz, BasisView bv,
                      const double* xz1, const double* xz2, long npt, double* rhos);
@@ -355,7 +366,7 @@ void launch_split_d(hipStream_t s, int ntiles, int n, const double* D, const int
 int assemble_blocks(int n);
 template <class T>  // float (mixed form) or double
 void launch_assemble(hipStream_t s, int n, const int* rowptr, const RowRef* rows, const int* ao_of, const T* U,
-                     double* V, const float* R, double* cpart);
+                     double* V, const float* R, double* cpart, int nmat = 1, size_t sU = 0);
 void launch_reduce_corr(hipStream_t s, int nparts, const double* cpart, double* out);
 // the packed form: per molecule of the table, en[2 slot_en] += its ncpart partials
 void launch_corr_multi(hipStream_t s, const char* base, const FnMolecule* fm, int nmol, double* en);
@@ -478,6 +489,8 @@ struct chx_grid {
   chx::DevBuf<int> d_asym;              // number of the last build whose D was not symmetric
   int d_gen = 0;                        // builds counted
   chx::DevBuf<double> d_ws;             // derivative calls' workspace (Workspace in api.cpp)
+  bool ws_live = false;
+  chx::DevBuf<int> d_ao_atom;           // atom of each AO (-1: padding), with the slot tables below
   double flops_build = 0, mean_tiles = 0;
   std::vector<double> batch_work;  // g_b n_b^2 per batch (points x kept AOs squared)
   double core_flops = 0;           // the core batches' three-term (rho, grad rho) launch: 2 sum g_b n_b^2
@@ -520,7 +533,7 @@ struct chx_grid {
   bool have_skeleton = false;
   bool have_density = false, have_eval = false, have_v = false;
   // response path: f_xc at the ground-state density, perturbed densities
-  chx::DevBuf<double> d_fx, d_part_u, d_rhou, d_coef_u;
+  chx::DevBuf<double> d_fx, d_rhou;
   int fx_family = -1;  // family of the f_xc on the grid (-1: none)
   int fx_nspin = 1;    // spin count of that f_xc (2: kFxPol values per slot)
   int nmats_u = 0;     // perturbed densities held in d_rhou (per spin)

@@ -131,7 +131,9 @@ __global__ __launch_bounds__(256) void k_gather_d(int n, const double* __restric
                                                   const int* __restrict__ tile_chunk,
                                                   const ChunkDev* __restrict__ chunks, const int* __restrict__ ao_of,
                                                   double* __restrict__ Dt, int ntiles, int* __restrict__ asym,
-                                                  int gen) {
+                                                  int gen, size_t sO) {
+  D += (size_t)blockIdx.y * n * n;  // the matrix of the launch
+  Dt += blockIdx.y * sO;
   const int t = blockIdx.x;
   if (t >= ntiles) {  // 1e-13: above the rounding of a product formed in FP64, below what tau shows
     check_symmetry(t - ntiles, n, D, 1e-13, asym, gen);
@@ -156,10 +158,10 @@ __global__ __launch_bounds__(256) void k_gather_d(int n, const double* __restric
 }
 
 void launch_gather_d(hipStream_t s, int ntiles, int n, const double* D, const int* tile_chunk, const ChunkDev* chunks,
-                     const int* ao_of, double* Dt, int* asym, int gen) {
+                     const int* ao_of, double* Dt, int* asym, int gen, int nmat, size_t sO) {
   if (ntiles == 0) return;
-  hipLaunchKernelGGL(k_gather_d, dim3(ntiles + (asym ? symmetry_blocks(n) : 0)), dim3(256), 0, s, n, D, tile_chunk,
-                     chunks, ao_of, Dt, ntiles, asym, gen);
+  hipLaunchKernelGGL(k_gather_d, dim3(ntiles + (asym ? symmetry_blocks(n) : 0), nmat), dim3(256), 0, s, n, D,
+                     tile_chunk, chunks, ao_of, Dt, ntiles, asym, gen, sO);
   CHX_HIP(hipGetLastError());
 }
 
@@ -670,7 +672,10 @@ __global__ __launch_bounds__(256) void k_functional_f(int nslots, const int* __r
 
 // rho^x and grad rho^x of one perturbed density matrix, per slot, from its partials.
 __global__ __launch_bounds__(256) void k_point_rho(int nslots, const int* __restrict__ grp_off,
-                                                   const double* __restrict__ part, double* __restrict__ rhou) {
+                                                   const double* __restrict__ part, size_t sP,
+                                                   double* __restrict__ rhou) {
+  part += blockIdx.y * sP;  // the matrix of the launch
+  rhou += 4 * (size_t)nslots * blockIdx.y;
   const int slot = blockIdx.x * 256 + threadIdx.x;
   if (slot >= nslots) return;
   const int b = slot / kBatch, g = slot % kBatch;
@@ -696,6 +701,8 @@ __global__ __launch_bounds__(256) void k_point_rho(int nslots, const int* __rest
 __global__ __launch_bounds__(256) void k_response_coef(int nslots, const double* __restrict__ rhou,
                                                        const double* __restrict__ fx, const double* __restrict__ bw,
                                                        int family, double* __restrict__ coef) {
+  rhou += 4 * (size_t)nslots * blockIdx.y;  // the matrix of the launch
+  coef += kCoef * (size_t)nslots * blockIdx.y;
   const int slot = blockIdx.x * 256 + threadIdx.x;
   if (slot >= nslots) return;
   const double* f = fx + (size_t)kFx * slot;
@@ -775,11 +782,14 @@ __global__ __launch_bounds__(256) void k_functional_fpol(int nslots, const int* 
 //   c = w (2 dv_sigma_uu grad rho_u + dv_sigma_ab grad rho_o + 2 v_sigma_uu grad rho^x_u
 //          + v_sigma_ab grad rho^x_o)
 // (the derivative of the polarised ground-state potential along D^x).
-__global__ __launch_bounds__(256) void k_response_coef_pol(int nslots, const double* __restrict__ rhou_a,
-                                                           const double* __restrict__ rhou_b,
+__global__ __launch_bounds__(256) void k_response_coef_pol(int nslots, const double* __restrict__ rhou,
                                                            const double* __restrict__ fx,
-                                                           const double* __restrict__ bw, int family, int spin,
+                                                           const double* __restrict__ bw, int family, int m0, int nper,
                                                            double* __restrict__ coef) {
+  const int m = m0 + blockIdx.y, spin = m / nper;  // output [spin][perturbation]: both spins' rho^x enter
+  const double* __restrict__ rhou_a = rhou + 4 * (size_t)nslots * (m % nper);
+  const double* __restrict__ rhou_b = rhou_a + 4 * (size_t)nslots * nper;
+  coef += kCoef * (size_t)nslots * blockIdx.y;
   const int slot = blockIdx.x * 256 + threadIdx.x;
   if (slot >= nslots) return;
   const double* f = fx + (size_t)kFxPol * slot;
@@ -855,12 +865,12 @@ void launch_functional_fpol(hipStream_t s, int nbatches, const int* grp_off, con
   CHX_HIP(hipGetLastError());
 }
 
-void launch_response_coef_pol(hipStream_t s, int nbatches, const double* rhou_a, const double* rhou_b,
-                              const double* fx, const double* bw, int family, int spin, double* coef) {
+void launch_response_coef_pol(hipStream_t s, int nbatches, const double* rhou, const double* fx, const double* bw,
+                              int family, int m0, int nmat, int nper, double* coef) {
   const int nslots = nbatches * kBatch;
   if (nslots == 0) return;
-  hipLaunchKernelGGL(k_response_coef_pol, dim3((nslots + 255) / 256), dim3(256), 0, s, nslots, rhou_a, rhou_b, fx, bw,
-                     family, spin, coef);
+  hipLaunchKernelGGL(k_response_coef_pol, dim3((nslots + 255) / 256, nmat), dim3(256), 0, s, nslots, rhou, fx, bw,
+                     family, m0, nper, coef);
   CHX_HIP(hipGetLastError());
 }
 
@@ -891,18 +901,20 @@ void launch_functional_f(hipStream_t s, int nbatches, const int* grp_off, const 
   CHX_HIP(hipGetLastError());
 }
 
-void launch_point_rho(hipStream_t s, int nbatches, const int* grp_off, const double* part, double* rhou) {
+void launch_point_rho(hipStream_t s, int nbatches, const int* grp_off, const double* part, double* rhou, int nmat,
+                      size_t sP) {
   const int nslots = nbatches * kBatch;
   if (nslots == 0) return;
-  hipLaunchKernelGGL(k_point_rho, dim3((nslots + 255) / 256), dim3(256), 0, s, nslots, grp_off, part, rhou);
+  hipLaunchKernelGGL(k_point_rho, dim3((nslots + 255) / 256, nmat), dim3(256), 0, s, nslots, grp_off, part, sP, rhou);
   CHX_HIP(hipGetLastError());
 }
 
 void launch_response_coef(hipStream_t s, int nbatches, const double* rhou, const double* fx, const double* bw,
-                          int family, double* coef) {
+                          int family, int nmat, double* coef) {
   const int nslots = nbatches * kBatch;
   if (nslots == 0) return;
-  hipLaunchKernelGGL(k_response_coef, dim3((nslots + 255) / 256), dim3(256), 0, s, nslots, rhou, fx, bw, family, coef);
+  hipLaunchKernelGGL(k_response_coef, dim3((nslots + 255) / 256, nmat), dim3(256), 0, s, nslots, rhou, fx, bw, family,
+                     coef);
   CHX_HIP(hipGetLastError());
 }
 

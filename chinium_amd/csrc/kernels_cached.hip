@@ -95,8 +95,10 @@ template <bool TAU>
 __global__ __launch_bounds__(TAU ? 512 : 256, 2) void k_density_c64(
     const int* __restrict__ grp_batch, const int* __restrict__ grp_tile, const int* __restrict__ grp_ntiles,
     const int* __restrict__ bt_off, const int* __restrict__ b_chunk, const ChunkDev* __restrict__ chunks,
-    const double* __restrict__ cache, const double* __restrict__ Dt, const int* __restrict__ asym, int gen,
-    double* __restrict__ part, double* __restrict__ part_tau) {
+    const double* __restrict__ cache, const double* __restrict__ Dt, size_t sD, const int* __restrict__ asym, int gen,
+    double* __restrict__ part, size_t sP, double* __restrict__ part_tau) {
+  Dt += blockIdx.y * sD;
+  part += blockIdx.y * sP;
   constexpr int NC = TAU ? 4 : 1, NR = TAU ? 2 : 4, NOUT = TAU ? 5 : 4;
   __shared__ double red[kGroup][NOUT][kBatch];
   const int grp = blockIdx.x;
@@ -223,14 +225,15 @@ __global__ __launch_bounds__(TAU ? 512 : 256, 2) void k_density_c64(
 
 void launch_density_c64(hipStream_t s, int ngroups, const int* grp_batch, const int* grp_tile, const int* grp_ntiles,
                         const int* bt_off, const int* b_chunk, const ChunkDev* chunks, const double* cache,
-                        const double* Dt, const int* asym, int gen, double* part, double* part_tau) {
+                        const double* Dt, const int* asym, int gen, double* part, double* part_tau, int nmat,
+                        size_t sD, size_t sP) {
   if (ngroups == 0) return;
   if (part_tau)
-    hipLaunchKernelGGL(k_density_c64<true>, dim3(ngroups), dim3(512), 0, s, grp_batch, grp_tile, grp_ntiles, bt_off,
-                       b_chunk, chunks, cache, Dt, asym, gen, part, part_tau);
+    hipLaunchKernelGGL(k_density_c64<true>, dim3(ngroups, nmat), dim3(512), 0, s, grp_batch, grp_tile, grp_ntiles,
+                       bt_off, b_chunk, chunks, cache, Dt, sD, asym, gen, part, sP, part_tau);
   else
-    hipLaunchKernelGGL(k_density_c64<false>, dim3(ngroups), dim3(256), 0, s, grp_batch, grp_tile, grp_ntiles, bt_off,
-                       b_chunk, chunks, cache, Dt, asym, gen, part, part_tau);
+    hipLaunchKernelGGL(k_density_c64<false>, dim3(ngroups, nmat), dim3(256), 0, s, grp_batch, grp_tile, grp_ntiles,
+                       bt_off, b_chunk, chunks, cache, Dt, sD, asym, gen, part, sP, part_tau);
   CHX_HIP(hipGetLastError());
 }
 
@@ -241,7 +244,10 @@ void launch_density_c64(hipStream_t s, int ngroups, const int* grp_batch, const 
 // (1/2) w v_tau grad phi_mu . grad phi_nu) is formed from the cached d_r phi
 // while the Vxc kernel loads it, instead of being stored.
 __global__ __launch_bounds__(256) void k_make_b(const int* __restrict__ bt_off, const double* __restrict__ coef,
-                                                const double* __restrict__ cache, double* __restrict__ bmat) {
+                                                size_t sC, const double* __restrict__ cache,
+                                                double* __restrict__ bmat, size_t sB) {
+  coef += blockIdx.y * sC;  // the matrix of the launch
+  bmat += blockIdx.y * sB;
   __shared__ double ca[kBatch], cx[kBatch], cy[kBatch], cz[kBatch];
   const int b = blockIdx.x, tid = threadIdx.x;
   if (tid < kBatch) {
@@ -264,9 +270,9 @@ __global__ __launch_bounds__(256) void k_make_b(const int* __restrict__ bt_off, 
 }
 
 void launch_make_b(hipStream_t s, int nbatches, const int* bt_off, const double* coef, const double* cache,
-                   double* bmat) {
+                   double* bmat, int nmat, size_t sC, size_t sB) {
   if (nbatches == 0) return;
-  hipLaunchKernelGGL(k_make_b, dim3(nbatches), dim3(256), 0, s, bt_off, coef, cache, bmat);
+  hipLaunchKernelGGL(k_make_b, dim3(nbatches, nmat), dim3(256), 0, s, bt_off, coef, sC, cache, bmat, sB);
   CHX_HIP(hipGetLastError());
 }
 
@@ -288,7 +294,10 @@ template <int KIND>
 __global__ __launch_bounds__(256, 2) void k_vxc_c64(const MxItem* __restrict__ work, const double* __restrict__ cache,
                                                     const double* __restrict__ bmat, const double* __restrict__ coef,
                                                     const int* __restrict__ ao_of, double* __restrict__ out,
-                                                    int npad) {
+                                                    int npad, ProdBatch pb) {
+  cache += (blockIdx.y / pb.nb) * pb.sA;  // the matrix of the launch
+  bmat += (blockIdx.y % pb.nb) * pb.sB;
+  out += blockIdx.y * pb.sO;
   const MxItem wk = work[blockIdx.x];
   const bool diag = wk.I0 == wk.J0;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -310,7 +319,7 @@ __global__ __launch_bounds__(256, 2) void k_vxc_c64(const MxItem* __restrict__ w
     const double* __restrict__ pa = (swap ? bmat + (s0 + wk.I0) * kSlotB
                                           : cache + (s0 + wk.I0) * kSlotAO + (tau ? pass + 1 : 0) * kSlotB) +
                                     8 * p8 * kTile + lo;
-    const double* __restrict__ pb = (tau    ? cache + (s0 + wk.J0) * kSlotAO + (pass + 1) * kSlotB
+    const double* __restrict__ pB = (tau    ? cache + (s0 + wk.J0) * kSlotAO + (pass + 1) * kSlotB
                                      : swap ? cache + (s0 + wk.J0) * kSlotAO
                                             : bmat + (s0 + wk.J0) * kSlotB) +
                                     8 * p8 * kTile + lo;
@@ -328,7 +337,7 @@ __global__ __launch_bounds__(256, 2) void k_vxc_c64(const MxItem* __restrict__ w
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
         const int q = c0 + min(c, nc - 1);
-        bb[buf][e][c] = pb[(size_t)(q >> 1) * sb + (q & 1) * 16 + 4 * e * kTile];
+        bb[buf][e][c] = pB[(size_t)(q >> 1) * sb + (q & 1) * 16 + 4 * e * kTile];
       }
     }
   };
@@ -423,19 +432,20 @@ __global__ __launch_bounds__(256, 2) void k_vxc_c64(const MxItem* __restrict__ w
 }
 
 void launch_vxc_c64(hipStream_t s, int ncomp, int nwork, const MxItem* work, const double* cache, const double* bmat,
-                    const double* coef, double* U) {
+                    const double* coef, double* U, int nmat, size_t sB, size_t sU) {
   if (nwork == 0) return;
+  const ProdBatch pb{nmat, 0, sB, sU};
   if (ncomp == 4)
-    hipLaunchKernelGGL(k_vxc_c64<1>, dim3(nwork), dim3(256), 0, s, work, cache, bmat, coef, nullptr, U, 0);
+    hipLaunchKernelGGL(k_vxc_c64<1>, dim3(nwork), dim3(256), 0, s, work, cache, bmat, coef, nullptr, U, 0, pb);
   else
-    hipLaunchKernelGGL(k_vxc_c64<0>, dim3(nwork), dim3(256), 0, s, work, cache, bmat, coef, nullptr, U, 0);
+    hipLaunchKernelGGL(k_vxc_c64<0>, dim3(nwork, nmat), dim3(256), 0, s, work, cache, bmat, coef, nullptr, U, 0, pb);
   CHX_HIP(hipGetLastError());
 }
 
 void launch_prod_c64(hipStream_t s, int nwork, const MxItem* work, const int* ao_of, const double* cache,
-                     const double* bmat, double* M, int npad) {
+                     const double* bmat, double* M, int npad, int nmat, const ProdBatch& pb) {
   if (nwork == 0) return;
-  hipLaunchKernelGGL(k_vxc_c64<2>, dim3(nwork), dim3(256), 0, s, work, cache, bmat, nullptr, ao_of, M, npad);
+  hipLaunchKernelGGL(k_vxc_c64<2>, dim3(nwork, nmat), dim3(256), 0, s, work, cache, bmat, nullptr, ao_of, M, npad, pb);
   CHX_HIP(hipGetLastError());
 }
 

@@ -213,7 +213,7 @@ __device__ __forceinline__ void xgrad_shell(double x, double y, double z, double
 // One wave per slot (batch, tile), lane = point; the three sums of consecutive
 // shells of one atom are reduced over the wave and added to gpart[copy][atom][t]
 // (scaled by -2; the block's number picks one of kGradCopies copies, which
-// k_sum_copies adds up). All waves adding every shell to one copy waited for each
+// k_sum_parts adds up). All waves adding every shell to one copy waited for each
 // other's FP64 atomics: (H2O)8 / def2-SVP / SG-2 1.54 ms, now 0.17.
 __global__ __launch_bounds__(256) void k_xgrad_epi(int nslots, const int* __restrict__ slot_batch,
                                                    const int* __restrict__ slot_tile, const int* __restrict__ slot_grp,
@@ -281,14 +281,23 @@ __global__ __launch_bounds__(256) void k_xgrad_epi(int nslots, const int* __rest
   flush();
 }
 
-// out[i] = sum over the kGradCopies copies of part[copy][i]
-__global__ __launch_bounds__(256) void k_sum_copies(int n, const double* __restrict__ part, double* __restrict__ out) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= n) return;
+// out[i] = sum of part[k][i] over nparts parts in a fixed order, 64 elements per
+// block, 16 partial sums each.
+__global__ __launch_bounds__(1024) void k_sum_parts(int n, int nparts, const double* __restrict__ part,
+                                                    double* __restrict__ out) {
+  __shared__ double red[16][64];
+  const int e = threadIdx.x & 63, s = threadIdx.x >> 6, i = blockIdx.x * 64 + e;
   double v = 0.0;
-#pragma unroll 8
-  for (int c = 0; c < kGradCopies; ++c) v += part[(size_t)c * n + i];
-  out[i] = v;
+  if (i < n) {
+#pragma unroll 4
+    for (int k = s; k < nparts; k += 16) v += part[(size_t)k * n + i];
+  }
+  red[s][e] = v;
+  __syncthreads();
+  if (s == 0 && i < n) {
+    for (int k = 1; k < 16; ++k) v += red[k][e];
+    out[i] = v;
+  }
 }
 
 void launch_xgrad_epi(hipStream_t s, int nslots, const int* slot_batch, const int* slot_tile, const int* slot_grp,
@@ -300,7 +309,7 @@ void launch_xgrad_epi(hipStream_t s, int nslots, const int* slot_batch, const in
   if (nslots > 0)
     hipLaunchKernelGGL(k_xgrad_epi, dim3((nslots + 3) / 4), dim3(256), 0, s, nslots, slot_batch, slot_tile, slot_grp,
                        slot_q, bx, by, bz, bv, coef, xz, n3, gpart);
-  hipLaunchKernelGGL(k_sum_copies, dim3((n3 + 255) / 256), dim3(256), 0, s, n3, gpart, grad);
+  hipLaunchKernelGGL(k_sum_parts, dim3((n3 + 63) / 64), dim3(1024), 0, s, n3, kGradCopies, gpart, grad);
   CHX_HIP(hipGetLastError());
 }
 
@@ -597,14 +606,14 @@ __device__ __forceinline__ void hess3_shell(double x, double y, double z, double
 }
 
 // One wave per slot, lane = point: H3 summed over the wave per run of one
-// atom's shells and added to H[3 A + t][3 A + u] (np = 3 natoms).
+// atom's shells and added to hpart[copy][A][tu] (kGradCopies copies, as in k_xgrad_epi).
 __global__ __launch_bounds__(256) void k_hess_diag(int nslots, const int* __restrict__ slot_batch,
                                                    const int* __restrict__ slot_tile, const int* __restrict__ slot_grp,
                                                    const int* __restrict__ slot_q, const double* __restrict__ bx,
                                                    const double* __restrict__ by, const double* __restrict__ bz,
                                                    BasisView bv, const double* __restrict__ coef,
                                                    const double* __restrict__ xz1, const double* __restrict__ xz2,
-                                                   int np, double* __restrict__ H) {
+                                                   int natoms, double* __restrict__ hpart) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = threadIdx.x & 63;
   const int slot = blockIdx.x * 4 + wave;
   if (slot >= nslots) return;
@@ -616,9 +625,9 @@ __global__ __launch_bounds__(256) void k_hess_diag(int nslots, const int* __rest
   const size_t col0 = (size_t)slot_grp[slot] * 2 * kGCols * kBatch + (size_t)slot_q[slot] * kTile * kBatch + g;
   const double* X1 = xz1 + col0;
   const double* X2 = xz2 + col0;
+  double* __restrict__ H = hpart + (size_t)(blockIdx.x % kGradCopies) * 6 * natoms;
   double acc[6] = {0, 0, 0, 0, 0, 0};
   int atom = -1;
-  const int pt[6] = {0, 0, 0, 1, 1, 2}, pu[6] = {0, 1, 2, 1, 2, 2};
   auto flush = [&]() {
     if (atom < 0) return;
 #pragma unroll
@@ -626,11 +635,7 @@ __global__ __launch_bounds__(256) void k_hess_diag(int nslots, const int* __rest
       double v = acc[k];
       for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
       acc[k] = 0.0;
-      if (g == 0) {
-        const int r0 = 3 * atom + pt[k], r1 = 3 * atom + pu[k];
-        unsafeAtomicAdd(&H[(size_t)r0 * np + r1], v);
-        if (r0 != r1) unsafeAtomicAdd(&H[(size_t)r1 * np + r0], v);
-      }
+      if (g == 0) unsafeAtomicAdd(&H[6 * atom + k], v);
     }
   };
   const int s0 = bv.tile_seg_off[t], s1 = bv.tile_seg_off[t + 1];
@@ -680,31 +685,67 @@ __global__ __launch_bounds__(256) void k_hess_diag(int nslots, const int* __rest
   flush();
 }
 
-// H1: block (16 a's x 16 b's, chunk of points), thread (a, b); the response
-// coefficients of rho^a (rhos[a][p][0..3]) with fx (v2rho2, v2rhosigma,
-// v2sigma2, v_sigma, grad rho) contracted with (2 rho^b, grad rho^b).
+// H1 of a 16 x 16 block (a's x b's) over the points [z chunk, (z + 1) chunk): with
+// the response coefficients of (rho^a, grad rho^a) (rhos[a][p][0..3]) under fx
+// (v2rho2, v2rhosigma, v2sigma2, v_sigma, grad rho) it is a product over K = 4
+// components x points, one v_mfma_f64_16x16x4 per point: lane (k = lane / 16, i =
+// lane % 16) forms component k of coordinate a = i's coefficients and reads
+// component k of rho^b for b = i. The block's 4 waves take a quarter of the points
+// each and store their sum in hpart[z]; k_sum_parts adds the chunks. (H2O)2 /
+// def2-SVP / SG-1: 36 us (2120 with one thread per (a, b) walking 4096 points).
 __global__ __launch_bounds__(256) void k_hess_fx(long npt, int np, const double* __restrict__ rhos,
                                                  const double* __restrict__ fx, const double* __restrict__ bw,
-                                                 int family, long chunk, double* __restrict__ H) {
-  const int a = blockIdx.x * 16 + (threadIdx.x >> 4), b = blockIdx.y * 16 + (threadIdx.x & 15);
-  if (a >= np || b >= np) return;
-  const long p0 = (long)blockIdx.z * chunk, p1 = p0 + chunk < npt ? p0 + chunk : npt;
-  double e = 0.0;
-  for (long p = p0; p < p1; ++p) {
-    const double w = bw[p];
-    if (w == 0.0) continue;
-    const double* f = fx + (size_t)kFx * p;
-    const double* u = rhos + ((size_t)a * npt + p) * 4;
-    const double* v = rhos + ((size_t)b * npt + p) * 4;
-    const double sx = 2.0 * (f[4] * u[1] + f[5] * u[2] + f[6] * u[3]);
-    double t = w * (f[0] * u[0] + f[1] * sx) * v[0];  // 2 c0 rho^b
-    if (family >= 1) {
-      const double q = 2.0 * w * (f[1] * u[0] + f[2] * sx), r = 2.0 * w * f[3];
-      t += (q * f[4] + r * u[1]) * v[1] + (q * f[5] + r * u[2]) * v[2] + (q * f[6] + r * u[3]) * v[3];
+                                                 int family, long chunk, double* __restrict__ hpart) {
+  __shared__ double red[4][256];
+  const int lane = threadIdx.x & 63, i = lane & 15, k = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int a = min((int)blockIdx.x * 16 + i, np - 1), b = min((int)blockIdx.y * 16 + i, np - 1);
+  const double* __restrict__ U = rhos + (size_t)a * npt * 4;
+  const double* __restrict__ V = rhos + (size_t)b * npt * 4 + k;
+  const long per = chunk / 4, p0 = (long)blockIdx.z * chunk + wave * per, p1 = min(p0 + per, npt);
+  dbl4 acc = {0, 0, 0, 0};
+  for (long p = p0; p < p1; p += 4) {  // npt and chunk / 4 are multiples of 4
+    double2 u0[4], u1[4];
+    double v[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      u0[q] = *reinterpret_cast<const double2*>(U + 4 * (p + q));
+      u1[q] = *reinterpret_cast<const double2*>(U + 4 * (p + q) + 2);
+      v[q] = V[4 * (p + q)];
     }
-    e += t;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const double w = bw[p + q];
+      const double* __restrict__ f = fx + (size_t)kFx * (p + q);
+      const double sx = 2.0 * (f[4] * u0[q].y + f[5] * u1[q].x + f[6] * u1[q].y);
+      const double gk = k == 1 ? f[4] : k == 2 ? f[5] : f[6], uk = k == 1 ? u0[q].y : k == 2 ? u1[q].x : u1[q].y;
+      double c;
+      if (k == 0) c = w * (f[0] * u0[q].x + f[1] * sx);  // 2 c0
+      else c = family >= 1 ? 2.0 * w * (f[1] * u0[q].x + f[2] * sx) * gk + 2.0 * w * f[3] * uk : 0.0;
+      const bool live = w != 0.0;  // (padding: its table entries do not enter)
+      acc = mfma_f64(live ? c : 0.0, live ? v[q] : 0.0, acc);
+    }
   }
-  unsafeAtomicAdd(&H[(size_t)a * np + b], e);
+#pragma unroll
+  for (int r = 0; r < 4; ++r) red[wave][16 * (4 * r + k) + i] = acc[r];  // [a][b]
+  __syncthreads();
+  const int e = threadIdx.x, ra = blockIdx.x * 16 + (e >> 4), rb = blockIdx.y * 16 + (e & 15);
+  if (ra < np && rb < np)
+    hpart[((size_t)blockIdx.z * np + ra) * np + rb] = (red[0][e] + red[1][e]) + (red[2][e] + red[3][e]);
+}
+
+// H += the atoms' own blocks (xx, xy, xz, yy, yz, zz of each), summed over the copies.
+__global__ __launch_bounds__(64) void k_hess_diag_add(int natoms, int np, const double* __restrict__ hpart,
+                                                      double* __restrict__ H) {
+  const int e = blockIdx.x * 64 + threadIdx.x;
+  if (e >= 6 * natoms) return;
+  double v = 0.0;
+#pragma unroll 8
+  for (int c = 0; c < kGradCopies; ++c) v += hpart[(size_t)c * 6 * natoms + e];
+  const int k = e % 6, t = k < 3 ? 0 : k < 5 ? 1 : 2, u = k < 3 ? k : k < 5 ? k - 2 : 2;
+  const size_t r0 = 3 * (e / 6) + t, r1 = 3 * (e / 6) + u;
+  H[r0 * np + r1] += v;
+  if (r0 != r1) H[r1 * np + r0] += v;
 }
 
 // H2: one thread per element (mu, nu) of D (npad^2, zero padded), nine products
@@ -729,17 +770,35 @@ __global__ void k_hess_dk(int npad, int np, const double* __restrict__ Dint, con
   }
 }
 
+// Points per chunk of k_hess_fx: about 2048 blocks, at least 64 points each.
+static long hess_fx_chunk(long npt, int np) {
+  const long tiles = (long)((np + 15) / 16) * ((np + 15) / 16), nz = std::max<long>(1, 2048 / tiles);
+  return std::max<long>(64, ((npt + nz - 1) / nz + 63) / 64 * 64);
+}
+
+size_t hess_part_elems(long npt, int np) {
+  const long chunk = hess_fx_chunk(npt, np);
+  return std::max<size_t>((size_t)((npt + chunk - 1) / chunk) * np * np, (size_t)kGradCopies * 2 * np);
+}
+
 void launch_hess_terms(hipStream_t s, int nslots, const int* slot_batch, const int* slot_tile, const int* slot_grp,
                        const int* slot_q, const double* bx, const double* by, const double* bz, BasisView bv,
                        const double* coef, const double* xz1, const double* xz2, long npt, const double* rhos,
                        const double* fx, const double* bw, int family, int npad, const double* Dint,
-                       const double* rr, const int* atom, int np, double* H) {
+                       const double* rr, const int* atom, int np, double* hpart, double* H) {
+  if (np == 0) return;
+  const long chunk = hess_fx_chunk(npt, np);
+  const unsigned nz = (unsigned)((npt + chunk - 1) / chunk);
+  if (nz > 0)
+    hipLaunchKernelGGL(k_hess_fx, dim3((np + 15) / 16, (np + 15) / 16, nz), dim3(256), 0, s, npt, np, rhos, fx, bw,
+                       family, chunk, hpart);
+  hipLaunchKernelGGL(k_sum_parts, dim3((np * np + 63) / 64), dim3(1024), 0, s, np * np, (int)nz, hpart, H);
+  const int na = np / 3;
+  launch_fill(s, hpart, (size_t)kGradCopies * 6 * na, 0.0);
   if (nslots > 0)
     hipLaunchKernelGGL(k_hess_diag, dim3((nslots + 3) / 4), dim3(256), 0, s, nslots, slot_batch, slot_tile, slot_grp,
-                       slot_q, bx, by, bz, bv, coef, xz1, xz2, np, H);
-  const long chunk = 4096;
-  const dim3 gf((np + 15) / 16, (np + 15) / 16, (unsigned)((npt + chunk - 1) / chunk));
-  if (npt > 0) hipLaunchKernelGGL(k_hess_fx, gf, dim3(256), 0, s, npt, np, rhos, fx, bw, family, chunk, H);
+                       slot_q, bx, by, bz, bv, coef, xz1, xz2, na, hpart);
+  hipLaunchKernelGGL(k_hess_diag_add, dim3((6 * na + 63) / 64), dim3(64), 0, s, na, np, hpart, H);
   const size_t pp = (size_t)npad * npad;
   const unsigned blocks = (unsigned)std::min<size_t>((pp + 255) / 256, 65536);
   hipLaunchKernelGGL(k_hess_dk, dim3(blocks), dim3(256), 0, s, npad, np, Dint, rr, atom, H);

@@ -272,8 +272,10 @@ __global__ __launch_bounds__(kAsmThreads) void k_assemble(int n, const int* __re
                                                              const int* __restrict__ ao_of,
                                                              const T* __restrict__ U, double* __restrict__ V,
                                                              const float* __restrict__ R,
-                                                             double* __restrict__ cpart) {
+                                                             double* __restrict__ cpart, size_t sU) {
   extern __shared__ double asum[];
+  U += blockIdx.z * sU;  // the matrix of the launch
+  V += (size_t)blockIdx.z * n * n;
   constexpr int kCols = kAsmLds / COPIES, kWaves = kAsmThreads / 64;
   const int mu = blockIdx.x, c0 = blockIdx.y * kCols, w = min(kCols, n - c0), tid = threadIdx.x;
   if (c0 + w <= mu) {  // below the diagonal: the block of row nu writes it
@@ -333,21 +335,21 @@ __global__ __launch_bounds__(kAsmThreads) void k_assemble(int n, const int* __re
 
 template <class T>
 void launch_assemble(hipStream_t s, int n, const int* rowptr, const RowRef* rows, const int* ao_of, const T* U,
-                     double* V, const float* R, double* cpart) {
+                     double* V, const float* R, double* cpart, int nmat, size_t sU) {
   if (n == 0) return;
   const int copies = asm_copies(n);
-  const dim3 grid(n, asm_ranges(n));
+  const dim3 grid(n, asm_ranges(n), nmat);
   const size_t lds = (size_t)std::min(n, kAsmLds / copies) * copies * sizeof(double);
   if (copies == 16)
-    hipLaunchKernelGGL((k_assemble<16, T>), grid, dim3(kAsmThreads), lds, s, n, rowptr, rows, ao_of, U, V, R, cpart);
+    hipLaunchKernelGGL((k_assemble<16, T>), grid, dim3(kAsmThreads), lds, s, n, rowptr, rows, ao_of, U, V, R, cpart, sU);
   else
-    hipLaunchKernelGGL((k_assemble<1, T>), grid, dim3(kAsmThreads), lds, s, n, rowptr, rows, ao_of, U, V, R, cpart);
+    hipLaunchKernelGGL((k_assemble<1, T>), grid, dim3(kAsmThreads), lds, s, n, rowptr, rows, ao_of, U, V, R, cpart, sU);
   CHX_HIP(hipGetLastError());
 }
 template void launch_assemble<float>(hipStream_t, int, const int*, const RowRef*, const int*, const float*, double*,
-                                     const float*, double*);
+                                     const float*, double*, int, size_t);
 template void launch_assemble<double>(hipStream_t, int, const int*, const RowRef*, const int*, const double*, double*,
-                                      const float*, double*);
+                                      const float*, double*, int, size_t);
 
 __global__ __launch_bounds__(256) void k_reduce_corr(int nparts, const double* __restrict__ cpart,
                                                      double* __restrict__ out) {

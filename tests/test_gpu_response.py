@@ -103,6 +103,23 @@ def test_water_cluster_response():
     assert abs(E - Eo) <= 1e-10 and np.abs(V - Vo).max() <= 1e-9
 
 
+@pytest.mark.parametrize("nmats", [2, 300])
+def test_perturbations_together_and_alone(nmats):
+    """Several matrices go through one launch (300: more than one set of launches, the last one short): each
+    is what it is by itself, to the bit (the same kernels, sums in a fixed order)."""
+    w, mol, D = _h2o()
+    rng = np.random.default_rng(12)
+    Dxs = []
+    for _ in range(nmats):
+        A = rng.standard_normal(D.shape)
+        Dxs.append(0.1 * (A + A.T))
+    grid, xc, Fs = _response(mol, "SG-1", "PBE", D, Dxs, 1)
+    for m in sorted({0, 1, nmats // 2, nmats - 2, nmats - 1}):
+        grid.getDensityU([[Dxs[m]]])
+        (F,), = grid.getFockU()
+        assert np.array_equal(F, Fs[m]), m
+
+
 def test_response_protocol_errors():
     w, mol, D = _h2o()
     grid = ca.Grid(mol, "SG-1", 1, 0)
