@@ -14,7 +14,7 @@
 #include <fstream>
 #include <numeric>
 #include <sstream>
-#include <unordered_map>
+#include <type_traits>
 
 #include "internal.hpp"
 
@@ -119,61 +119,108 @@ Radial read_grid_file(const std::string& path) {
   return R;
 }
 
-// Nuclei with Z > 2 in a uniform hash of 1-bohr cells, to find the nucleus
-// (if any) within r <= 0.5 bohr of a point by looking at 27 cells.
-struct HeavyHash {
-  std::unordered_map<uint64_t, std::vector<int>> cells;
-  const std::vector<double>* xyz = nullptr;
-  static uint64_t key(long ix, long iy, long iz) {
-    return ((uint64_t)(ix & 0x1fffff) << 42) | ((uint64_t)(iy & 0x1fffff) << 21) | (uint64_t)(iz & 0x1fffff);
+// Nuclei with Z > 2 by cells of at least 1 bohr over their bounding box, to find
+// the nucleus (if any) within r <= 1 bohr of a point. A cell lists the nuclei of
+// the 27 cells around it, so that a point reads one cell (mostly an empty one): a
+// hash table asked for 27 keys per point took half of a geometry step's host time.
+struct HeavyCells {
+  const std::vector<double>& xyz;
+  double lo[3] = {0, 0, 0}, h = 1 + 1e-6;  // the edge: 1 bohr and a margin for rounding
+  long n[3] = {0, 0, 0};
+  std::vector<int> start, atoms;  // cell c: atoms[start[c]] .. atoms[start[c + 1]]
+  HeavyCells(const chx_mol& m) : xyz(m.xyz) {
+    std::vector<int> heavy;
+    double hi[3] = {0, 0, 0};
+    for (int a = 0; a < m.natoms; ++a) {
+      const double* c = &xyz[3 * a];
+      if (m.Z[a] <= 2 || !(std::fabs(c[0]) + std::fabs(c[1]) + std::fabs(c[2]) < 1e100)) continue;
+      for (int d = 0; d < 3; ++d) {
+        lo[d] = heavy.empty() ? c[d] : std::min(lo[d], c[d]);
+        hi[d] = heavy.empty() ? c[d] : std::max(hi[d], c[d]);
+      }
+      heavy.push_back(a);
+    }
+    if (heavy.empty()) return;
+    auto cells = [&] {
+      double c = 1;
+      for (int d = 0; d < 3; ++d) c *= std::floor((hi[d] - lo[d]) / h) + 4;
+      return c;
+    };
+    while (cells() > 1 << 21) h *= 2;
+    for (int d = 0; d < 3; ++d) {
+      lo[d] -= 2 * h;  // so that no nucleus is in an outermost cell
+      n[d] = (long)std::floor((hi[d] - lo[d]) / h) + 2;
+    }
+    std::vector<int> count((size_t)(n[0] * n[1] * n[2]) + 1, 0);
+    auto each = [&](auto&& f) {  // the cells around each nucleus
+      for (int d = 0; d < 27; ++d)
+        for (int a : heavy) {
+          long c[3];
+          for (int k = 0; k < 3; ++k) c[k] = (long)std::floor((xyz[3 * a + k] - lo[k]) / h);
+          f(((c[0] + d / 9 - 1) * n[1] + c[1] + d / 3 % 3 - 1) * n[2] + c[2] + d % 3 - 1, a);
+        }
+    };
+    each([&](long c, int) { ++count[c + 1]; });
+    for (size_t c = 1; c < count.size(); ++c) count[c] += count[c - 1];
+    start = count;
+    atoms.resize(start.back());
+    each([&](long c, int a) { atoms[count[c]++] = a; });
   }
-  HeavyHash(const chx_mol& m) : xyz(&m.xyz) {
-    for (int a = 0; a < m.natoms; ++a)
-      if (m.Z[a] > 2)
-        cells[key((long)std::floor(m.xyz[3 * a]), (long)std::floor(m.xyz[3 * a + 1]), (long)std::floor(m.xyz[3 * a + 2]))]
-            .push_back(a);
+  long cell(double x, double y, double z) const {  // -1: outside
+    const double c[3] = {std::floor((x - lo[0]) / h), std::floor((y - lo[1]) / h), std::floor((z - lo[2]) / h)};
+    for (int d = 0; d < 3; ++d)
+      if (!(c[d] >= 0 && c[d] < (double)n[d])) return -1;
+    return ((long)c[0] * n[1] + (long)c[1]) * n[2] + (long)c[2];
   }
   // a heavy atom within sqrt(r2) of (x, y, z), sqrt(r2) <= 1; -1 if none
   int near(double x, double y, double z, double r2) const {
-    if (cells.empty()) return -1;
-    const long ix = (long)std::floor(x), iy = (long)std::floor(y), iz = (long)std::floor(z);
-    for (long dx = -1; dx <= 1; ++dx)
-      for (long dy = -1; dy <= 1; ++dy)
-        for (long dz = -1; dz <= 1; ++dz) {
-          auto it = cells.find(key(ix + dx, iy + dy, iz + dz));
-          if (it == cells.end()) continue;
-          for (int a : it->second) {
-            const double ex = x - (*xyz)[3 * a], ey = y - (*xyz)[3 * a + 1], ez = z - (*xyz)[3 * a + 2];
-            if (ex * ex + ey * ey + ez * ez < r2) return a;
-          }
-        }
+    if (atoms.empty()) return -1;
+    const long c = cell(x, y, z);
+    if (c < 0) return -1;
+    for (int k = start[c]; k < start[c + 1]; ++k) {
+      const int a = atoms[k];
+      const double ex = x - xyz[3 * a], ey = y - xyz[3 * a + 1], ez = z - xyz[3 * a + 2];
+      if (ex * ex + ey * ey + ez * ez < r2) return a;
+    }
     return -1;
   }
 };
 
-// Recursive bisection into batches of exactly kBatch points (one remainder).
-void bisect(const std::vector<double>& x, const std::vector<double>& y, const std::vector<double>& z,
-            std::vector<long>& idx, long lo, long hi, std::vector<std::pair<long, long>>& out) {
+// Recursive bisection into batches of exactly kBatch points (one remainder). The
+// coordinates move with the points: through an index every comparison missed the caches.
+struct BisPoint {
+  double c[3];
+  long i;
+};
+
+void bisect(std::vector<BisPoint>& p, long lo, long hi, std::vector<std::pair<long, long>>& out) {
   const long n = hi - lo;
   if (n <= kBatch) {
     out.push_back({lo, hi});
     return;
   }
   double mn[3] = {1e300, 1e300, 1e300}, mx[3] = {-1e300, -1e300, -1e300};
-  for (long i = lo; i < hi; ++i) {
-    const double c[3] = {x[idx[i]], y[idx[i]], z[idx[i]]};
-    for (int d = 0; d < 3; ++d) { mn[d] = std::min(mn[d], c[d]); mx[d] = std::max(mx[d], c[d]); }
-  }
+  for (long i = lo; i < hi; ++i)
+    for (int d = 0; d < 3; ++d) {
+      mn[d] = std::min(mn[d], p[i].c[d]);
+      mx[d] = std::max(mx[d], p[i].c[d]);
+    }
   int ax = 0;
   for (int d = 1; d < 3; ++d)
     if (mx[d] - mn[d] > mx[ax] - mn[ax]) ax = d;
-  const std::vector<double>& key = ax == 0 ? x : (ax == 1 ? y : z);
   const long nb = (n + kBatch - 1) / kBatch;
   const long left = kBatch * (nb / 2);
-  std::nth_element(idx.begin() + lo, idx.begin() + lo + left, idx.begin() + hi,
-                   [&](long a, long b) { return key[a] < key[b] || (key[a] == key[b] && a < b); });
-  bisect(x, y, z, idx, lo, lo + left, out);
-  bisect(x, y, z, idx, lo + left, hi, out);
+  auto split = [&](auto axis) {
+    constexpr int d = decltype(axis)::value;
+    std::nth_element(p.begin() + lo, p.begin() + lo + left, p.begin() + hi, [](const BisPoint& a, const BisPoint& b) {
+      return a.c[d] < b.c[d] || (a.c[d] == b.c[d] && a.i < b.i);
+    });
+  };
+  if (ax == 0) split(std::integral_constant<int, 0>{});
+  else if (ax == 1) split(std::integral_constant<int, 1>{});
+  else split(std::integral_constant<int, 2>{});
+  bisect(p, lo, lo + left, out);
+  bisect(p, lo + left, hi, out);
 }
 
 }  // namespace
@@ -197,10 +244,12 @@ void grid_build(chx_grid* g, const std::string& grid_name, const std::string& da
   // ---- atom-centred points in generation order (atom -> shell -> angular point)
   std::vector<double> px, py, pz, pw;
   std::vector<int> owner;
+  std::vector<Radial> radial(37);  // one file per element
   for (int a = 0; a < nat; ++a) {
     const int Z = m.Z[a];
     if (Z < 1 || Z > 36) throw Error(CHX_ERR_ARG, "unsupported element");
-    const Radial R = read_grid_file(data_root + "/Grids/" + grid_name + "/" + kElemNames[Z] + ".grid");
+    Radial& R = radial[Z];
+    if (R.r.empty()) R = read_grid_file(data_root + "/Grids/" + grid_name + "/" + kElemNames[Z] + ".grid");
     const double* c = &m.xyz[3 * a];
     for (size_t s = 0; s < R.r.size(); ++s) {
       const auto& L = lebedev(R.nang[s]);
@@ -236,36 +285,34 @@ void grid_build(chx_grid* g, const std::string& grid_name, const std::string& da
     CHX_HIP(hipStreamSynchronize(g->stream));
   }
   // ---- drop exactly-zero weights, batch the rest spatially
-  std::vector<long> keep;
-  keep.reserve(G);
-  for (long i = 0; i < G; ++i)
-    if (pw[i] != 0.0) keep.push_back(i);
   // The points within kCoreRadius of a nucleus with Z > 2 (atomic cores, where
   // the density is largest) are batched apart, per atom, so that the mixed
   // form's three-term core treatment covers few batches; the rest is bisected
   // as one set. Only the batch membership depends on this.
+  std::vector<BisPoint> keep;
   std::vector<std::pair<long, long>> parts;
   {
     const double rc2 = kCoreRadius * kCoreRadius;
-    const HeavyHash hh(m);
+    const HeavyCells hc(m);
     std::vector<std::vector<long>> core(nat);
-    std::vector<long> rest;
-    rest.reserve(keep.size());
-    for (long i : keep) {  // any nucleus with Z > 2, not only the point's own atom's
-      const int a = hh.near(px[i], py[i], pz[i], rc2);
+    std::vector<BisPoint> rest;
+    rest.reserve(G);
+    for (long i = 0; i < G; ++i) {  // any nucleus with Z > 2, not only the point's own atom's
+      if (pw[i] == 0.0) continue;
+      const int a = hc.near(px[i], py[i], pz[i], rc2);
       if (a >= 0) core[a].push_back(i);
-      else rest.push_back(i);
+      else rest.push_back({{px[i], py[i], pz[i]}, i});
     }
-    keep.clear();
     std::vector<long> seg = {0};
+    keep.reserve(G);
     for (int a = 0; a < nat; ++a) {
-      keep.insert(keep.end(), core[a].begin(), core[a].end());
+      for (long i : core[a]) keep.push_back({{px[i], py[i], pz[i]}, i});
       seg.push_back((long)keep.size());
     }
     keep.insert(keep.end(), rest.begin(), rest.end());
     seg.push_back((long)keep.size());
     for (size_t k = 0; k + 1 < seg.size(); ++k)
-      if (seg[k + 1] > seg[k]) bisect(px, py, pz, keep, seg[k], seg[k + 1], parts);
+      if (seg[k + 1] > seg[k]) bisect(keep, seg[k], seg[k + 1], parts);
   }
   g->npoints = (long)keep.size();
   g->nbatches = (int)parts.size();
@@ -276,10 +323,10 @@ void grid_build(chx_grid* g, const std::string& grid_name, const std::string& da
     const long lo = parts[b].first, n = parts[b].second - parts[b].first;
     g->batch_n[b] = (int)n;
     for (int k = 0; k < kBatch; ++k) {
-      const long src = keep[lo + (k < n ? k : 0)];
+      const BisPoint& p = keep[lo + (k < n ? k : 0)];
       const size_t s = (size_t)b * kBatch + k;
-      g->hx[s] = px[src]; g->hy[s] = py[src]; g->hz[s] = pz[src];
-      g->hw[s] = k < n ? pw[src] : 0.0;
+      g->hx[s] = p.c[0]; g->hy[s] = p.c[1]; g->hz[s] = p.c[2];
+      g->hw[s] = k < n ? pw[p.i] : 0.0;
     }
   }
   // ---- shells in the reference's AO order
@@ -570,9 +617,21 @@ void grid_plan(chx_grid* g) {
   g->d_ws.release();
   const int nb = g->nbatches, nsh = (int)g->sh_type.size(), nwords = (nsh + 63) / 64;
   std::vector<double> reach2(nsh);
+  std::vector<int> kinds;  // one shell of each kind (atoms of an element repeat theirs)
   for (int s = 0; s < nsh; ++s) {
-    const double r = shell_reach(g->sh_type[s], g->sh_nprim[s], &g->p_exp[g->sh_poff[s]], &g->p_coef[g->sh_poff[s]],
-                                 g->screen_thr);
+    const int np = g->sh_nprim[s];
+    const double *e = &g->p_exp[g->sh_poff[s]], *c = &g->p_coef[g->sh_poff[s]];
+    auto same = [&](int k) {
+      return g->sh_type[k] == g->sh_type[s] && g->sh_nprim[k] == np && std::equal(e, e + np, &g->p_exp[g->sh_poff[k]]) &&
+             std::equal(c, c + np, &g->p_coef[g->sh_poff[k]]);
+    };
+    const auto it = std::find_if(kinds.begin(), kinds.end(), same);
+    if (it != kinds.end()) {
+      reach2[s] = reach2[*it];
+      continue;
+    }
+    kinds.push_back(s);
+    const double r = shell_reach(g->sh_type[s], np, e, c, g->screen_thr);
     reach2[s] = r * r;
   }
   std::vector<unsigned long long> alive((size_t)nb * nwords, 0ull);
@@ -690,13 +749,13 @@ void grid_plan(chx_grid* g) {
       g->core_flops = 0.0;
       int ncore_slots = 0;
       if (g->core_radius > 0) {
-        const double r2c = g->core_radius * g->core_radius;  // <= 1 bohr: the hash's reach
-        const HeavyHash hh(g->mol);
+        const double r2c = g->core_radius * g->core_radius;  // <= 1 bohr: the cells' reach
+        const HeavyCells hc(g->mol);
         for (int b = 0; b < nb; ++b) {
           bool core = false;
           for (int q = 0; q < g->batch_n[b] && !core; ++q) {
             const size_t p = (size_t)b * kBatch + q;
-            core = hh.near(g->hx[p], g->hy[p], g->hz[p], r2c) >= 0;
+            core = hc.near(g->hx[p], g->hy[p], g->hz[p], r2c) >= 0;
           }
           if (!core) {
             for (int k = g->grp_off[b]; k < g->grp_off[b + 1]; ++k) g->main_grps.push_back(k);
