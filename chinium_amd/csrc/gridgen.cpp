@@ -14,7 +14,6 @@
 #include <fstream>
 #include <numeric>
 #include <sstream>
-#include <type_traits>
 
 #include "internal.hpp"
 
@@ -186,41 +185,28 @@ struct HeavyCells {
   }
 };
 
-// Recursive bisection into batches of exactly kBatch points (one remainder). The
-// coordinates move with the points: through an index every comparison missed the caches.
-struct BisPoint {
-  double c[3];
-  long i;
-};
-
-void bisect(std::vector<BisPoint>& p, long lo, long hi, std::vector<std::pair<long, long>>& out) {
-  const long n = hi - lo;
-  if (n <= kBatch) {
-    out.push_back({lo, hi});
-    return;
-  }
-  double mn[3] = {1e300, 1e300, 1e300}, mx[3] = {-1e300, -1e300, -1e300};
-  for (long i = lo; i < hi; ++i)
-    for (int d = 0; d < 3; ++d) {
-      mn[d] = std::min(mn[d], p[i].c[d]);
-      mx[d] = std::max(mx[d], p[i].c[d]);
-    }
-  int ax = 0;
-  for (int d = 1; d < 3; ++d)
-    if (mx[d] - mn[d] > mx[ax] - mn[ax]) ax = d;
-  const long nb = (n + kBatch - 1) / kBatch;
-  const long left = kBatch * (nb / 2);
-  auto split = [&](auto axis) {
-    constexpr int d = decltype(axis)::value;
-    std::nth_element(p.begin() + lo, p.begin() + lo + left, p.begin() + hi, [](const BisPoint& a, const BisPoint& b) {
-      return a.c[d] < b.c[d] || (a.c[d] == b.c[d] && a.i < b.i);
-    });
+// Recursive bisection into batches of exactly kBatch points (one remainder): what
+// goes to the left depends on the numbers of points only, so all levels' segments
+// are known before any point has moved. levels: first segment of each level, and the end.
+void bisect_plan(const std::vector<long>& sets, std::vector<BisSeg>& segs, std::vector<int>& levels,
+                 std::vector<int2>& batches) {
+  std::vector<BisSeg> cur;
+  auto add = [&](std::vector<BisSeg>& v, long lo, long n) {
+    if (n > 0) v.push_back(BisSeg{(int)lo, (int)n, n <= kBatch ? 0 : kBatch * (int)((n + kBatch - 1) / kBatch / 2)});
   };
-  if (ax == 0) split(std::integral_constant<int, 0>{});
-  else if (ax == 1) split(std::integral_constant<int, 1>{});
-  else split(std::integral_constant<int, 2>{});
-  bisect(p, lo, lo + left, out);
-  bisect(p, lo + left, hi, out);
+  for (size_t k = 0; k + 1 < sets.size(); ++k) add(cur, sets[k], sets[k + 1] - sets[k]);
+  levels.assign(1, 0);
+  while (std::any_of(cur.begin(), cur.end(), [](const BisSeg& s) { return s.left > 0; })) {
+    segs.insert(segs.end(), cur.begin(), cur.end());
+    levels.push_back((int)segs.size());
+    std::vector<BisSeg> next;
+    for (const BisSeg& s : cur) {
+      add(next, s.lo, s.left ? s.left : s.n);
+      if (s.left) add(next, s.lo + s.left, s.n - s.left);
+    }
+    cur.swap(next);
+  }
+  for (const BisSeg& s : cur) batches.push_back(make_int2(s.lo, s.n));
 }
 
 }  // namespace
@@ -263,24 +249,29 @@ void grid_build(chx_grid* g, const std::string& grid_name, const std::string& da
     }
   }
   const long G = (long)px.size();
+  if (G > (1l << 30)) throw Error(CHX_ERR_UNSUPPORTED, "more than 2^30 grid points");
   // ---- Becke weights on the device (FP64); the data files are all read by now
   ensure_stream(g);
+  DevBuf<double> dx, dy, dz, dw;
   {
-    std::vector<double> inv(nat * (size_t)nat, 0.0);
+    const int ld = becke_ld(nat);
+    std::vector<double2> rab((size_t)nat * ld, make_double2(1.0, 1.0));
     for (int b = 0; b < nat; ++b)
       for (int c = 0; c < nat; ++c) {
         if (b == c) continue;
         const double dx = m.xyz[3 * b] - m.xyz[3 * c], dy = m.xyz[3 * b + 1] - m.xyz[3 * c + 1],
                      dz = m.xyz[3 * b + 2] - m.xyz[3 * c + 2];
-        inv[(size_t)b * nat + c] = std::sqrt(dx * dx + dy * dy + dz * dz);
+        const double R = std::sqrt(dx * dx + dy * dy + dz * dz);
+        rab[(size_t)b * ld + c] = make_double2(R, 1.0 / R);
       }
-    DevBuf<double> dx, dy, dz, dw, dxyz, dinv;
+    DevBuf<double> dxyz;
+    DevBuf<double2> drab;
     DevBuf<int> down;
     dx.upload(px, g->stream); dy.upload(py, g->stream); dz.upload(pz, g->stream); dw.upload(pw, g->stream);
     down.upload(owner, g->stream);
     dxyz.upload(m.xyz, g->stream);
-    dinv.upload(inv, g->stream);
-    launch_becke(g->stream, G, dx.p, dy.p, dz.p, dw.p, down.p, nat, dxyz.p, dinv.p);
+    drab.upload(rab, g->stream);
+    launch_becke(g->stream, G, dx.p, dy.p, dz.p, dw.p, down.p, nat, dxyz.p, drab.p, ld);
     CHX_HIP(hipMemcpyAsync(pw.data(), dw.p, sizeof(double) * G, hipMemcpyDeviceToHost, g->stream));
     CHX_HIP(hipStreamSynchronize(g->stream));
   }
@@ -289,45 +280,63 @@ void grid_build(chx_grid* g, const std::string& grid_name, const std::string& da
   // the density is largest) are batched apart, per atom, so that the mixed
   // form's three-term core treatment covers few batches; the rest is bisected
   // as one set. Only the batch membership depends on this.
-  std::vector<BisPoint> keep;
-  std::vector<std::pair<long, long>> parts;
+  std::vector<int> keep;
+  std::vector<long> sets = {0};
   {
     const double rc2 = kCoreRadius * kCoreRadius;
     const HeavyCells hc(m);
-    std::vector<std::vector<long>> core(nat);
-    std::vector<BisPoint> rest;
+    std::vector<std::vector<int>> core(nat);
+    std::vector<int> rest;
     rest.reserve(G);
     for (long i = 0; i < G; ++i) {  // any nucleus with Z > 2, not only the point's own atom's
       if (pw[i] == 0.0) continue;
       const int a = hc.near(px[i], py[i], pz[i], rc2);
-      if (a >= 0) core[a].push_back(i);
-      else rest.push_back({{px[i], py[i], pz[i]}, i});
+      (a >= 0 ? core[a] : rest).push_back((int)i);
     }
-    std::vector<long> seg = {0};
     keep.reserve(G);
     for (int a = 0; a < nat; ++a) {
-      for (long i : core[a]) keep.push_back({{px[i], py[i], pz[i]}, i});
-      seg.push_back((long)keep.size());
+      keep.insert(keep.end(), core[a].begin(), core[a].end());
+      sets.push_back((long)keep.size());
     }
     keep.insert(keep.end(), rest.begin(), rest.end());
-    seg.push_back((long)keep.size());
-    for (size_t k = 0; k + 1 < seg.size(); ++k)
-      if (seg[k + 1] > seg[k]) bisect(keep, seg[k], seg[k + 1], parts);
+    sets.push_back((long)keep.size());
   }
+  std::vector<BisSeg> segs;
+  std::vector<int> levels;
+  std::vector<int2> batches;
+  bisect_plan(sets, segs, levels, batches);
   g->npoints = (long)keep.size();
-  g->nbatches = (int)parts.size();
+  g->nbatches = (int)batches.size();
   const size_t nslots = (size_t)g->nbatches * kBatch;
   g->hx.assign(nslots, 0); g->hy.assign(nslots, 0); g->hz.assign(nslots, 0); g->hw.assign(nslots, 0);
   g->batch_n.assign(g->nbatches, 0);
-  for (int b = 0; b < g->nbatches; ++b) {
-    const long lo = parts[b].first, n = parts[b].second - parts[b].first;
-    g->batch_n[b] = (int)n;
-    for (int k = 0; k < kBatch; ++k) {
-      const BisPoint& p = keep[lo + (k < n ? k : 0)];
-      const size_t s = (size_t)b * kBatch + k;
-      g->hx[s] = p.c[0]; g->hy[s] = p.c[1]; g->hz[s] = p.c[2];
-      g->hw[s] = k < n ? pw[p.i] : 0.0;
+  for (int b = 0; b < g->nbatches; ++b) g->batch_n[b] = batches[b].y;
+  g->d_x.alloc(nslots); g->d_y.alloc(nslots); g->d_z.alloc(nslots); g->d_w.alloc(nslots);
+  if (nslots) {
+    const long n = g->npoints;
+    DevBuf<double> pts[2];
+    DevBuf<int> ids[2], didx;
+    DevBuf<BisSeg> dsegs;
+    DevBuf<int2> dbat;
+    for (int k = 0; k < 2; ++k) {
+      pts[k].alloc(3 * (size_t)n);
+      ids[k].alloc(n);
     }
+    didx.upload(keep, g->stream);
+    dsegs.upload(segs, g->stream);
+    dbat.upload(batches, g->stream);
+    double* pp[2] = {pts[0].p, pts[1].p};
+    int* ip[2] = {ids[0].p, ids[1].p};
+    launch_bisect(g->stream, n, didx.p, dx.p, dy.p, dz.p, levels, dsegs.p, pp, ip);
+    const size_t nl = levels.size() - 1;
+    launch_batch_slots(g->stream, g->nbatches, dbat.p, pp[nl & 1], nl ? ip[nl & 1] : didx.p, n, dw.p, g->d_x.p,
+                       g->d_y.p, g->d_z.p, g->d_w.p);
+    const size_t bytes = sizeof(double) * nslots;
+    CHX_HIP(hipMemcpyAsync(g->hx.data(), g->d_x.p, bytes, hipMemcpyDeviceToHost, g->stream));
+    CHX_HIP(hipMemcpyAsync(g->hy.data(), g->d_y.p, bytes, hipMemcpyDeviceToHost, g->stream));
+    CHX_HIP(hipMemcpyAsync(g->hz.data(), g->d_z.p, bytes, hipMemcpyDeviceToHost, g->stream));
+    CHX_HIP(hipMemcpyAsync(g->hw.data(), g->d_w.p, bytes, hipMemcpyDeviceToHost, g->stream));
+    CHX_HIP(hipStreamSynchronize(g->stream));
   }
   // ---- shells in the reference's AO order
   g->nbasis = m.nbasis;
@@ -355,7 +364,6 @@ void grid_build(chx_grid* g, const std::string& grid_name, const std::string& da
   g->d_sh_xyz.upload(g->sh_xyz, st); g->d_sh_type.upload(g->sh_type, st); g->d_sh_nprim.upload(g->sh_nprim, st);
   g->d_sh_atom.upload(g->sh_atom, st);
   g->d_sh_poff.upload(g->sh_poff, st); g->d_p_exp.upload(g->p_exp, st); g->d_p_coef.upload(g->p_coef, st);
-  g->d_x.upload(g->hx, st); g->d_y.upload(g->hy, st); g->d_z.upload(g->hz, st); g->d_w.upload(g->hw, st);
   g->d_bn.upload(g->batch_n, st);
   CHX_HIP(hipStreamSynchronize(st));
   g->ao_ready = false;

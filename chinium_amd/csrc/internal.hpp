@@ -145,9 +145,20 @@ struct RowRef {
   int a0, len;
 };
 
-// Launchers (kernels.hip).
+// Grid set-up (kernels_grid.hip). rab: (R, 1 / R) of every pair of atoms, rows of
+// becke_ld(natoms), the rest of a row (1, 1).
+int becke_ld(int natoms);
 void launch_becke(hipStream_t s, long npts, const double* px, const double* py, const double* pz, double* w,
-                  const int* owner, int natoms, const double* atom_xyz, const double* inv_rab);
+                  const int* owner, int natoms, const double* atom_xyz, const double2* rab, int ld);
+struct BisSeg { int lo, n, left; };  // points [lo, lo + n), the first `left` to go to the left half (0: a batch)
+// Bisects the n points of the indexes idx level by level (segments levels[l] ..
+// levels[l + 1] of segs); points and indexes end in pts / ids[levels.size() - 1
+// odd or even] (without levels: pts[0] and idx).
+void launch_bisect(hipStream_t s, long n, const int* idx, const double* px, const double* py, const double* pz,
+                   const std::vector<int>& levels, const BisSeg* segs, double* pts[2], int* ids[2]);
+void launch_batch_slots(hipStream_t s, int nbatches, const int2* batch, const double* pts, const int* idx, long stride,
+                        const double* w, double* bx, double* by, double* bz, double* bw);
+// Launchers (kernels.hip).
 // alive: per batch nwords 64-bit words, bit k of word w set when shell 64 w + k
 // comes closer than its reach (reach2: squared) to one of the batch's points
 void launch_screen(hipStream_t s, int nbatches, int nshells, int nwords, const double* bx, const double* by,

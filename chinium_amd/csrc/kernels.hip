@@ -24,46 +24,6 @@
 namespace chx {
 
 // ---------------------------------------------------------------------------
-// Becke partition (GridGeneration.cpp:136-153): w *= P_owner / sum_B P_B,
-// P_B = prod_{C != B} s(mu_BC), s = (1 - p(p(p(mu))))/2, p(m) = 1.5m - 0.5m^3.
-__global__ __launch_bounds__(256) void k_becke(long npts, const double* __restrict__ px, const double* __restrict__ py,
-                                               const double* __restrict__ pz, double* __restrict__ w,
-                                               const int* __restrict__ owner, int natoms,
-                                               const double* __restrict__ axyz, const double* __restrict__ inv_rab) {
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= npts) return;
-  const double x = px[i], y = py[i], z = pz[i];
-  const int me = owner[i];
-  double total = 0, mine = 0;
-  for (int b = 0; b < natoms; ++b) {
-    const double dxb = x - axyz[3 * b], dyb = y - axyz[3 * b + 1], dzb = z - axyz[3 * b + 2];
-    const double rb = ::sqrt(dxb * dxb + dyb * dyb + dzb * dzb);
-    double pb = 1.0;
-    for (int c = 0; c < natoms && pb != 0.0; ++c) {
-      if (c == b) continue;
-      const double dxc = x - axyz[3 * c], dyc = y - axyz[3 * c + 1], dzc = z - axyz[3 * c + 2];
-      const double rc = ::sqrt(dxc * dxc + dyc * dyc + dzc * dzc);
-      double m = (rb - rc) / inv_rab[b * natoms + c];  // inv_rab holds R_BC (division as in s_p_mu)
-      m = 1.5 * m - 0.5 * m * m * m;
-      m = 1.5 * m - 0.5 * m * m * m;
-      m = 1.5 * m - 0.5 * m * m * m;
-      pb *= 0.5 * (1.0 - m);
-    }
-    total += pb;
-    if (b == me) mine = pb;
-  }
-  w[i] *= mine / total;
-}
-
-void launch_becke(hipStream_t s, long npts, const double* px, const double* py, const double* pz, double* w,
-                  const int* owner, int natoms, const double* atom_xyz, const double* inv_rab) {
-  if (npts == 0) return;
-  const int blocks = (int)((npts + 255) / 256);
-  hipLaunchKernelGGL(k_becke, dim3(blocks), dim3(256), 0, s, npts, px, py, pz, w, owner, natoms, atom_xyz, inv_rab);
-  CHX_HIP(hipGetLastError());
-}
-
-// ---------------------------------------------------------------------------
 // AO screening: one block per batch. A shell is alive when its centre comes
 // closer to one of the batch's points than the shell's reach, the distance
 // beyond which neither |phi| nor |grad phi| of any of its components exceeds
