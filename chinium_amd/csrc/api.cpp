@@ -156,15 +156,16 @@ void density_from_device(chx_grid* g, const double* dD, int spin = 0) {
                    g->d_Dsplit.p, g->d_Dres.p + (size_t)spin * g->nbasis * g->nbasis, g->d_asym.p, g->hmol.gen);
     g->mark_end(kStPermute, e);
     g->mark_begin(kStDensity, &e);
-    // meta-GGA: rho, grad rho and the tau partials (A = d_r phi) in one launch that stages D once
-    // (rho, grad rho alone: the core batches' groups are left to the core launch)
-    launch_density_mx(g->stream, g->type >= 2, g->type >= 2 ? ng : ng - ncg, g->hmol);
+    // meta-GGA: rho, grad rho and the tau partials (A = d_r phi) in one launch that stages D once,
+    // then the core batches' rho and grad rho with three-term AO operands, over their partials (tau
+    // keeps two terms: near the nuclei its error is far below rho's effect on E_xc). rho, grad rho
+    // alone: the core groups and the others in one launch, or in two to be timed apart.
+    const bool tau = g->type >= 2, apart = g->profile && ncg;
+    launch_density_mx(g->stream, tau, tau ? ng : ng - ncg, apart ? 0 : ncg, g->hmol);
     g->mark_end(kStDensity, e);
-    // core batches' rho and grad rho with three-term AO operands (meta-GGA: overwriting their
-    // partials; tau keeps two terms: near the nuclei its error is far below rho's effect on E_xc)
-    if (ncg) {
+    if (apart) {
       g->mark_begin(kStCore, &e);
-      launch_density_mx_core(g->stream, ncg, g->hmol);
+      launch_density_mx(g->stream, 0, 0, ncg, g->hmol);
       g->mark_end(kStCore, e);
     }
     g->have_density = true;

@@ -453,7 +453,7 @@ static void build_chunks(chx_grid* g, int nwords, const std::vector<unsigned lon
       ++b1;
     }
     // the list, packed: shells in AO order, one that does not fit a tile continues in the next
-    ChunkDev ch{(long)g->dt_elems, (int)g->tile_chunk.size(), 0};
+    ChunkDev ch{(long)g->dt_elems, (int)g->tile_chunk.size(), 0, b0, b1 - b0};
     int col = kTile;
     for (int s = 0; s < nsh; ++s) {
       if (!(cur[s >> 6] >> (s & 63) & 1ull)) continue;
@@ -701,8 +701,9 @@ void grid_plan(chx_grid* g) {
     r.col = sg.w;
     if (k > 0 && sg.w > 0 && g->sh_atom[g->seg[k - 1].x] == g->sh_atom[sh]) r.meta |= kSegSame;
     for (int p = 0; p < np && p < kSegPrim; ++p) {
-      r.e[p] = (float)g->p_exp[po + p];
-      r.c[p] = (float)g->p_coef[po + p];
+      r.p[p][0] = (float)(-1.4426950408889634 * g->p_exp[po + p]);
+      r.p[p][1] = (float)g->p_coef[po + p];
+      r.p[p][2] = (float)(g->p_exp[po + p] * g->p_coef[po + p]);
     }
   }
   g->d_segrec.upload(rec, st);

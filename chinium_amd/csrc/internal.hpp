@@ -89,17 +89,21 @@ template <class T> struct DevBuf {
   }
 };
 
-// One shell segment of a tile with everything its evaluation reads, so that a
-// wave fetches it with two scalar loads (mixed-precision form).
+// One shell segment of a tile with everything its evaluation reads (mixed-precision
+// form): the scalar unit fetches the first 80 bytes, which hold up to kSegInline
+// primitives, and the rest only where a shell has more. A primitive is (-a log2 e,
+// c, a c), so that exp(-a r^2) is one product and the hardware's exp2.
 constexpr int kSegPrim = 12;  // primitives per record
+constexpr int kSegInline = 4;
 constexpr int kSegSame = 1 << 15;  // meta: the same centre as the record before (in the tile)
 struct SegRec {
   double ax, ay, az;  // shell centre
   int meta;           // type & 0xff | nprim << 8 | first component << 16 | count << 24
   int col;            // AO offset in the tile
-  float e[kSegPrim], c[kSegPrim];
+  float p[kSegPrim][3];
+  float pad[4];
 };
-static_assert(sizeof(SegRec) == 128, "segment record is two 64-byte scalar loads");
+static_assert(sizeof(SegRec) == 192, "records start on 64-byte lines");
 
 // Kernel-side view of the basis. Tiles are the chunks' own: every chunk of
 // batches (see ChunkDev) holds the AOs alive in it, packed in 32-AO tiles, and
@@ -126,6 +130,7 @@ struct BasisView {
 struct ChunkDev {
   long doff;
   int tile0, ntl;
+  int b0, nb;  // its batches b0 .. b0 + nb - 1
 };
 // A Vxc work item: the block (I, J) of super-tiles of one chunk over nbat of
 // its batches; slot0 is the first batch's first slot.
@@ -385,9 +390,8 @@ void launch_bf16_check(hipStream_t s, unsigned n, unsigned* bad);
 void launch_fill_u32(hipStream_t s, unsigned* p, size_t n, unsigned v);
 // One launch over the grid `one` (descriptor by value): density work groups,
 // B^T slot blocks, Vxc work items. Density: rho, grad rho; with_tau: tau too.
-void launch_density_mx(hipStream_t s, int with_tau, int nitems, const MolDev& one);
-// the core groups' rho, grad rho (again) with three-term operands
-void launch_density_mx_core(hipStream_t s, int ncore_groups, const MolDev& one);
+// ncore_groups: the core groups' rho, grad rho with three-term operands too (GGA: in the same launch)
+void launch_density_mx(hipStream_t s, int with_tau, int nitems, int ncore_groups, const MolDev& one);
 // B^T of every slot for ncomp components
 void launch_make_b_mx(hipStream_t s, int ncomp, const MolDev& one);
 // wide: groups of up to kMxWideTiles tiles instead of kMxTiles

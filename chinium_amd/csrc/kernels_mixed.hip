@@ -435,35 +435,53 @@ __device__ __forceinline__ void emit_shell_f32(float x, float y, float z, int fi
   }
 }
 
-// R = sum_p c_p exp(-a_p r^2) and sum_p a_p c_p exp(-a_p r^2) over NP primitives.
-template <int NP>
-__device__ __forceinline__ void radial_f32(const SegRec& rec, float r2, float& A0, float& A1) {
-#pragma unroll
-  for (int p = 0; p < NP; ++p) {
-    const float e = rec.c[p] * __expf(-rec.e[p] * r2);
-    A0 += e;
-    A1 += rec.e[p] * e;
-  }
-}
-
 // One wave walks one tile at 64 points, lane = point. Every segment record
 // comes in through scalar loads and the shell loop is uniform across the
 // wave: no divergence, no LDS, no block barrier. The offset from the centre
 // is taken in FP64 (points and centres are tens of bohr apart, the offsets
-// that matter are small), everything after it in FP32 with the hardware exp.
+// that matter are small), everything after it in FP32 with the hardware exp2.
 // The basis tables are read through the constant address space: they never
 // change while a kernel runs, and so are always read with scalar loads (a
 // kernel that also issues LDS DMA loads would otherwise get vector loads).
-
-__device__ __forceinline__ SegRec load_segrec(const SegRec* recs, int k) {
-  using cvec = const __attribute__((address_space(4))) u32x4;
-  static_assert(sizeof(SegRec) == 8 * sizeof(u32x4), "SegRec is 128 bytes");
-  u32x4 w[8];
+using cvec4 = const __attribute__((address_space(4))) u32x4;
+struct SegHead {  // the first 80 bytes of a record
+  double ax, ay, az;
+  int meta, col;
+  float p[kSegInline][3];
+};
+__device__ __forceinline__ SegHead load_seghead(const SegRec* recs, int k) {
+  static_assert(sizeof(SegHead) == 5 * sizeof(u32x4) && offsetof(SegRec, p) == offsetof(SegHead, p), "record layout");
+  u32x4 w[5];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) w[i] = ((cvec*)(recs + k))[i];
-  SegRec r;
-  __builtin_memcpy(&r, w, sizeof(SegRec));
+  for (int i = 0; i < 5; ++i) w[i] = ((cvec4*)(recs + k))[i];
+  SegHead r;
+  __builtin_memcpy(&r, w, sizeof(SegHead));
   return r;
+}
+
+// R = sum_p c_p exp(-a_p r^2) and sum_p a_p c_p exp(-a_p r^2) over NP primitives
+template <int NP>
+__device__ __forceinline__ void radial_f32(const SegHead& h, const SegRec* rec, float r2, float& A0, float& A1) {
+  A0 = A1 = 0.f;
+  auto add = [&](float e, float c, float ec) {
+    const float v = __builtin_amdgcn_exp2f(e * r2);
+    A0 += c * v;
+    A1 += ec * v;
+  };
+#pragma unroll
+  for (int i = 0; i < (NP < kSegInline ? NP : kSegInline); ++i) add(h.p[i][0], h.p[i][1], h.p[i][2]);
+  if (NP > kSegInline) {
+    constexpr int kMore = NP > kSegInline ? (3 * (NP - kSegInline) + 3) / 4 : 1;
+    u32x4 w[kMore];
+#pragma unroll
+    for (int i = 0; i < kMore; ++i) w[i] = ((cvec4*)rec)[5 + i];
+#pragma unroll
+    for (int i = kSegInline; i < NP; ++i) {
+      const int o = 3 * (i - kSegInline);
+      add(__uint_as_float(w[o / 4][o % 4]), __uint_as_float(w[(o + 1) / 4][(o + 1) % 4]),
+          __uint_as_float(w[(o + 2) / 4][(o + 2) % 4]));
+    }
+  }
 }
 
 // PREFETCH: the next record is loaded while the current one is evaluated
@@ -473,15 +491,15 @@ __device__ __forceinline__ void walk_tile_f32(const BasisView& bv, int t, double
   using cint = const __attribute__((address_space(4))) int;
   const int s0 = ((cint*)bv.tile_seg_off)[t], s1 = ((cint*)bv.tile_seg_off)[t + 1];
   float x = 0.f, y = 0.f, z = 0.f, r2 = 0.f;
-  SegRec nxt;
-  if (PREFETCH && s0 < s1) nxt = load_segrec(bv.segrec, s0);
+  SegHead nxt;
+  if (PREFETCH && s0 < s1) nxt = load_seghead(bv.segrec, s0);
   for (int k = s0; k < s1; ++k) {
-    SegRec rec;
+    SegHead rec;
     if (PREFETCH) {
       rec = nxt;
-      nxt = load_segrec(bv.segrec, k + 1 < s1 ? k + 1 : k);
+      nxt = load_seghead(bv.segrec, k + 1 < s1 ? k + 1 : k);
     } else {
-      rec = load_segrec(bv.segrec, k);
+      rec = load_seghead(bv.segrec, k);
     }
     if (!(rec.meta & kSegSame)) {  // a new centre (the shells of an atom follow each other)
       x = (float)(px - rec.ax);
@@ -489,17 +507,22 @@ __device__ __forceinline__ void walk_tile_f32(const BasisView& bv, int t, double
       z = (float)(pz - rec.az);
       r2 = x * x + y * y + z * z;
     }
-    float A0 = 0.f, A1 = 0.f;
-    switch ((rec.meta >> 8) & 0x7f) {  // primitive count: straight-line code per count
-      case 1: radial_f32<1>(rec, r2, A0, A1); break;
-      case 2: radial_f32<2>(rec, r2, A0, A1); break;
-      case 3: radial_f32<3>(rec, r2, A0, A1); break;
-      case 4: radial_f32<4>(rec, r2, A0, A1); break;
-      case 5: radial_f32<5>(rec, r2, A0, A1); break;
-      case 6: radial_f32<6>(rec, r2, A0, A1); break;
-      case 7: radial_f32<7>(rec, r2, A0, A1); break;
-      case 8: radial_f32<8>(rec, r2, A0, A1); break;
-      default: radial_f32<kSegPrim>(rec, r2, A0, A1); break;  // unused slots hold c = 0
+    float A0, A1;
+    const SegRec* rp = bv.segrec + k;
+    const int np = (rec.meta >> 8) & 0x7f;
+    if (np == 1) {  // primitive count: straight-line code per count
+      radial_f32<1>(rec, rp, r2, A0, A1);
+    } else {
+      switch (np) {
+        case 2: radial_f32<2>(rec, rp, r2, A0, A1); break;
+        case 3: radial_f32<3>(rec, rp, r2, A0, A1); break;
+        case 4: radial_f32<4>(rec, rp, r2, A0, A1); break;
+        case 5: radial_f32<5>(rec, rp, r2, A0, A1); break;
+        case 6: radial_f32<6>(rec, rp, r2, A0, A1); break;
+        case 7: radial_f32<7>(rec, rp, r2, A0, A1); break;
+        case 8: radial_f32<8>(rec, rp, r2, A0, A1); break;
+        default: radial_f32<kSegPrim>(rec, rp, r2, A0, A1); break;  // unused slots hold c = 0
+      }
     }
     // R = A0, grad R = -2 r A1
     op.begin(A0, -2.f * x * A1, -2.f * y * A1, -2.f * z * A1);
@@ -522,15 +545,16 @@ __device__ __forceinline__ void walk_tile_f32(const BasisView& bv, int t, double
 // walk, not the MFMAs, is most of a GGA density on lists of a few hundred AOs).
 // X is held in registers (uniform column index: no memory access).
 typedef float f32x32 __attribute__((ext_vector_type(32)));
+constexpr int kXPitch = kBatch + 4;  // of X^T in LDS: 16-byte rows that 16 lanes write without bank conflicts
 template <bool TAU>
 struct DensEpi {
   f32x32 xv[TAU ? 4 : 1];
   float o[TAU ? 5 : 4] = {};
   float R, Rx, Ry, Rz, S0, Sx, Sy, Sz, T0, Tx, Ty, Tz;
-  // xq: X^T of this tile at this lane's point, xq[col * (kBatch + 1)]
+  // xq: X^T of this tile at this lane's point, xq[col * kXPitch]
   __device__ void load(int d, const float* xq) {
 #pragma unroll
-    for (int c = 0; c < kTile; ++c) xv[d][c] = xq[c * (kBatch + 1)];
+    for (int c = 0; c < kTile; ++c) xv[d][c] = xq[c * kXPitch];
   }
   __device__ void begin(float a, float ax, float ay, float az) {
     R = a; Rx = ax; Ry = ay; Rz = az;
@@ -579,11 +603,10 @@ constexpr int kDxFrag = 64;  // u32x4 per fragment
 constexpr int kDxA = 8;      // A fragments per step: [row block][hl]
 constexpr int kDxB = 16;     // D fragments per step: [column block][hl]
 constexpr int kDxA3 = 4;     // P3: third-term A fragments per step: [row block]
-template <bool P3>
 struct DensMxSmem {
   union {
-    u32x4 F[(kDxA + kDxB + (P3 ? kDxA3 : 0)) * kDxFrag];  // one K step's fragments
-    float X[kGroup * kTile][kBatch + 1];                          // epilogue: X^T [nu][g]
+    u32x4 F[(kDxA + kDxB + kDxA3) * kDxFrag];  // one K step's fragments
+    float X[kGroup * kTile][kXPitch];          // epilogue: X^T [nu][g]
   };
   float red[kGroup][4][kBatch];
   double px[kBatch], py[kBatch], pz[kBatch];
@@ -602,9 +625,8 @@ struct DensMxSmem {
 // loads; a descriptor read from device memory would leave them flat).
 // r: the block's item (after the XCD-aware remap) within the molecule's launch.
 template <bool P3>
-__device__ __forceinline__ void density_mx_body(const MolDev& m, int r) {
+__device__ __forceinline__ void density_mx_body(const MolDev& m, int r, DensMxSmem& sm) {
   using lds_ptr = __attribute__((address_space(3))) void*;
-  __shared__ DensMxSmem<P3> sm;
   const int grp = P3 ? m.core_grps[r] : m.main_grps ? m.main_grps[r] : r;
   const u16* __restrict__ cache = m.cache;
   const size_t sstride = (size_t)m.sstride;
@@ -713,8 +735,7 @@ __device__ __forceinline__ void density_mx_body(const MolDev& m, int r) {
   for (int r = 0; r < 2; ++r)
 #pragma unroll
     for (int c = 0; c < 4; ++c)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) sm.X[64 * wc + 16 * c + lrow][32 * wr + 16 * r + 4 * lk + i] = acc[r][c][i];
+      *reinterpret_cast<f32x4*>(&sm.X[64 * wc + 16 * c + lrow][32 * wr + 16 * r + 4 * lk]) = acc[r][c];
   __syncthreads();
   DensEpi<false> epi;
   if (wave < nt) {  // wave q = tile q of the group; lane = point
@@ -731,9 +752,12 @@ __device__ __forceinline__ void density_mx_body(const MolDev& m, int r) {
     part[(size_t)grp * 4 * kBatch + c * kBatch + g] = v;
   }
 }
-template <bool P3>
-__global__ __launch_bounds__(256, P3 ? 2 : 4) void k_density_mx(MolDev m) {
-  density_mx_body<P3>(m, xcd_remap(blockIdx.x, gridDim.x));
+// The first ncore blocks take the core groups (their products are longer), the
+// others the rest: one launch, since the core batches alone leave the chip half empty.
+__global__ __launch_bounds__(256, 4) void k_density_mx(MolDev m, int ncore) {
+  __shared__ DensMxSmem sm;
+  if ((int)blockIdx.x < ncore) density_mx_body<true>(m, xcd_remap(blockIdx.x, ncore), sm);
+  else density_mx_body<false>(m, xcd_remap(blockIdx.x - ncore, gridDim.x - ncore), sm);
 }
 
 // Meta-GGA density in one launch: the products Phi D and (d_r Phi) D share one D
@@ -749,7 +773,7 @@ __global__ __launch_bounds__(256, P3 ? 2 : 4) void k_density_mx(MolDev m) {
 struct DensMxMggaSmem {
   union {
     u32x4 F[(4 * kDxA + kDxB) * kDxFrag];  // one K step's fragments: A_0..A_3, D
-    float X[kGroup * kTile][kBatch + 1];
+    float X[kGroup * kTile][kXPitch];
   };
   float red[kGroup][5][kBatch];
   double px[kBatch], py[kBatch], pz[kBatch];
@@ -864,8 +888,7 @@ __global__ __launch_bounds__(256, 2) void k_density_mx_mgga(MolDev m) {
     for (int r = 0; r < 2; ++r)
 #pragma unroll
       for (int c = 0; c < 4; ++c)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) sm.X[64 * wc + 16 * c + lrow][32 * wr + 16 * r + 4 * lk + i] = acc[d][r][c][i];
+        *reinterpret_cast<f32x4*>(&sm.X[64 * wc + 16 * c + lrow][32 * wr + 16 * r + 4 * lk]) = acc[d][r][c];
     __syncthreads();
     epi.load(d, &sm.X[kTile * wave][lane]);
   }
@@ -884,18 +907,13 @@ __global__ __launch_bounds__(256, 2) void k_density_mx_mgga(MolDev m) {
   }
 }
 
-void launch_density_mx_core(hipStream_t s, int ncore_groups, const MolDev& one) {
-  if (ncore_groups == 0) return;
-  hipLaunchKernelGGL((k_density_mx<true>), dim3(ncore_groups), dim3(256), 0, s, one);
-  CHX_HIP(hipGetLastError());
-}
-
-void launch_density_mx(hipStream_t s, int with_tau, int nitems, const MolDev& one) {
-  if (nitems == 0) return;
-  if (with_tau)
+void launch_density_mx(hipStream_t s, int with_tau, int nitems, int ncore_groups, const MolDev& one) {
+  if (with_tau && nitems > 0) {
     hipLaunchKernelGGL(k_density_mx_mgga, dim3(nitems), dim3(256), 0, s, one);
-  else
-    hipLaunchKernelGGL((k_density_mx<false>), dim3(nitems), dim3(256), 0, s, one);
+    nitems = 0;  // the core groups come after it
+  }
+  if (nitems + ncore_groups > 0)
+    hipLaunchKernelGGL(k_density_mx, dim3(nitems + ncore_groups), dim3(256), 0, s, one, ncore_groups);
   CHX_HIP(hipGetLastError());
 }
 
@@ -904,66 +922,72 @@ void launch_density_mx(hipStream_t s, int with_tau, int nitems, const MolDev& on
 // recomputed in FP32:
 //   Bt[slot][0][hl][nu][g] = split(a phi + c . grad phi),
 //   meta-GGA (NC = 4) adds Bt[slot][r][hl][nu][g] = split(t d_r phi), t = w v_tau / 4.
-// Each lane stores its point's values straight into the slot's [c][hl][nu][g]
-// block (for each AO, the wave's 64 lanes write one contiguous 128-byte row);
-// columns past the tile's last AO are written as zeros. No LDS stage and no
-// barrier, so occupancy is set by registers alone.
+// Neighbouring lanes exchange halves, so that an AO's two rows of 128 bytes in
+// the slot's [c][hl][nu][g] block go out in one store of the wave; columns past
+// the tile's last AO are written as zeros. No LDS stage and no barrier, so
+// occupancy is set by registers alone. Bound by the walk's instructions and the
+// waits for its records ((H2O)128 / def2-SVP / SG-2: 1.8 ms for 4 GB; the stores
+// alone take 0.8).
 template <int NC>
 struct MakeB {
-  u16* sv;  // this lane's column of the [c][hl][nu][g] block
+  u16* sv;       // where this lane's pairs go in the [c][hl][nu][g] block
+  unsigned sel;  // byte selection of its pairs
   float ca, cx, cy, cz, ct, R, Rx, Ry, Rz, s1;
   __device__ void begin(float a, float ax, float ay, float az) {
     R = a; Rx = ax; Ry = ay; Rz = az;
     s1 = ca * a + cx * ax + cy * ay + cz * az;  // (a + c . grad) R
   }
-  __device__ void comp(int col, float q, float qx, float qy, float qz) {
+  __device__ void put(int c, int col, float v) {
     u16 hi, lo;
-    split_bf(q * s1 + R * (cx * qx + cy * qy + cz * qz), hi, lo);  // a phi + c . grad phi
-    sv[col * kBatch] = hi;
-    sv[kTile * kBatch + col * kBatch] = lo;
+    split_bf(v, hi, lo);
+    const int own = hi | (int)lo << 16, other = __builtin_amdgcn_mov_dpp(own, 0xb1, 0xf, 0xf, true);  // lane ^ 1
+    *reinterpret_cast<unsigned*>(sv + c * kMxT + col * kBatch) = __builtin_amdgcn_perm(other, own, sel);
+  }
+  __device__ void comp(int col, float q, float qx, float qy, float qz) {
+    put(0, col, q * s1 + R * (cx * qx + cy * qy + cz * qz));  // a phi + c . grad phi
     if (NC == 4) {
-      split_bf(ct * (Rx * q + R * qx), hi, lo);
-      sv[kMxT + col * kBatch] = hi;
-      sv[kMxT + kTile * kBatch + col * kBatch] = lo;
-      split_bf(ct * (Ry * q + R * qy), hi, lo);
-      sv[2 * kMxT + col * kBatch] = hi;
-      sv[2 * kMxT + kTile * kBatch + col * kBatch] = lo;
-      split_bf(ct * (Rz * q + R * qz), hi, lo);
-      sv[3 * kMxT + col * kBatch] = hi;
-      sv[3 * kMxT + kTile * kBatch + col * kBatch] = lo;
+      put(1, col, ct * (Rx * q + R * qx));
+      put(2, col, ct * (Ry * q + R * qy));
+      put(3, col, ct * (Rz * q + R * qz));
     }
   }
   __device__ void end() {}
 };
 
 template <int NC>
-__device__ __forceinline__ void make_b_slot(const MolDev& m, int slot, int g) {
-  if (slot >= m.nslots) return;
-  u16* __restrict__ col0 = m.bt + (size_t)slot * NC * kMxT + g;  // [c][hl][nu][g], this lane's point
+__device__ __forceinline__ void make_b_slot(const MolDev& m, int item, int g) {
+  if (item >= m.nslots) return;
   const BasisView bv = m.bv;  // descriptor fields in registers, read once
-  const int b = m.slot_batch[slot], t = m.slot_tile[slot];
+  int slot = item, b = m.slot_batch[item], t = m.slot_tile[item];
+  if (NC == 1) {  // a chunk's items tile by tile, so that the waves that run together read the same records
+    const ChunkDev ch = m.chunks[m.b_chunk[b]];
+    const int local = (b - ch.b0) * ch.ntl + t - ch.tile0, q = local / ch.nb;
+    b = ch.b0 + local - q * ch.nb;
+    t = ch.tile0 + q;
+    slot = item - local + (b - ch.b0) * ch.ntl + q;
+  }
   const size_t p = (size_t)b * kBatch + g;
-  const double* __restrict__ coef = m.coef;
+  const double* __restrict__ coef = m.coef + kCoef * p;
   MakeB<NC> op;
-  op.sv = col0;
-  op.ca = (float)coef[kCoef * p];
-  op.cx = (float)coef[kCoef * p + 1];
-  op.cy = (float)coef[kCoef * p + 2];
-  op.cz = (float)coef[kCoef * p + 3];
-  op.ct = (float)coef[kCoef * p + 4];
+  // even lanes store the hi parts of points g, g + 1, odd lanes the lo parts of g - 1, g
+  op.sv = m.bt + (size_t)slot * NC * kMxT + (g & 1) * (kTile * kBatch) + (g & ~1);
+  op.sel = g & 1 ? 0x03020706u : 0x05040100u;
+  op.ca = (float)coef[0];
+  op.cx = (float)coef[1];
+  op.cy = (float)coef[2];
+  op.cz = (float)coef[3];
+  op.ct = (float)coef[4];
   walk_tile_f32<true>(bv, t, m.bx[p], m.by[p], m.bz[p], op);
-  // zeros past the tile's last AO (segments hold (shell, first component, count, local offset))
+  // zeros past the tile's last AO (its segments are in column order)
+  const int s1 = bv.tile_seg_off[t + 1];
   int nao = 0;
-  for (int k = bv.tile_seg_off[t]; k < bv.tile_seg_off[t + 1]; ++k) {
-    const int4 sg = bv.seg[k];
-    nao = max(nao, sg.w + sg.z);
+  if (s1 > bv.tile_seg_off[t]) {
+    const int4 sg = bv.seg[s1 - 1];  // (shell, first component, count, local offset)
+    nao = sg.w + sg.z;
   }
   for (int col = nao; col < kTile; ++col)
 #pragma unroll
-    for (int c = 0; c < NC; ++c) {
-      col0[c * kMxT + col * kBatch] = 0;
-      col0[c * kMxT + kTile * kBatch + col * kBatch] = 0;
-    }
+    for (int c = 0; c < NC; ++c) *reinterpret_cast<unsigned*>(op.sv + c * kMxT + col * kBatch) = 0u;
 }
 template <int NC>
 __global__ __launch_bounds__(NC == 4 ? 64 : 256) void k_make_b_mx(MolDev m) {
@@ -1193,14 +1217,15 @@ __device__ __forceinline__ int item_owner_from(const int* __restrict__ starts, i
 }
 
 template <bool P3>
-__global__ __launch_bounds__(256, P3 ? 2 : 4) void k_density_mx_multi(const char* base, const MolDev* __restrict__ tab,
+__global__ __launch_bounds__(256, 4) void k_density_mx_multi(const char* base, const MolDev* __restrict__ tab,
                                                                       const int* __restrict__ starts, int nmol,
                                                                       int total) {
+  __shared__ DensMxSmem sm;
   int k = -1;
   for (int v = blockIdx.x; v < total; v += gridDim.x) {
     const int item = xcd_remap(v, total);
     k = item_owner_from(starts, nmol, item, k);
-    density_mx_body<P3>(rebase(base, tab[k]), item - starts[k]);
+    density_mx_body<P3>(rebase(base, tab[k]), item - starts[k], sm);
     __syncthreads();  // the next item reuses the block's LDS
   }
 }

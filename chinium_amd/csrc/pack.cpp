@@ -342,9 +342,7 @@ void enqueue_lane(chx_pack* p, int lane, hipStream_t s, hipEvent_t after, hipEve
   for (int m = m0; m < m1; ++m) {
     chx_grid* g = p->grids[m];
     const int ng = (int)g->grp_batch.size(), ncg = (int)g->core_grps.size();
-    launch_density_mx(s, p->type >= 2, p->type >= 2 ? ng : ng - ncg, g->hmol);
-    // core batches' rho and grad rho again with three-term AO operands
-    launch_density_mx_core(s, (int)g->core_grps.size(), g->hmol);
+    launch_density_mx(s, p->type >= 2, p->type >= 2 ? ng : ng - ncg, ncg, g->hmol);
   }
   if (dens_done) CHX_HIP(hipEventRecord(dens_done, s));
   const int nc = p->family >= 2 ? 4 : 1;
