@@ -140,6 +140,44 @@ void gather_d(chx_grid* g, const double* dD, DevBuf<double>& Dt, bool with_tau =
                   Dt.alloc_get(std::max<size_t>(1, g->dt_elems)), with_tau ? g->d_asym.p : nullptr, g->d_gen);
 }
 
+// Workspace of one call (derivatives, both spins together), kept on the grid for the next one (until it
+// is planned again) unless it is larger than kWsKeep: hipMalloc and hipFree of
+// these buffers on every call cost more than the kernels of a small system, and
+// now and then 10 ms and more.
+struct Workspace {
+  static constexpr size_t kWsKeep = (size_t)1 << 30;  // bytes
+  chx_grid* g;
+  size_t used = 0;
+  // total: doubles of all takes, each rounded up by round()
+  Workspace(chx_grid* grid, size_t total) : g(grid) {
+    require(!g->ws_live, CHX_ERR_STATE, "the grid's workspace is in use");
+    if (g->d_ws.n < total) g->d_ws.alloc(total);
+    g->ws_live = true;
+  }
+  ~Workspace() {
+    g->ws_live = false;
+    if (g->d_ws.n * sizeof(double) > kWsKeep) g->d_ws.release();
+  }
+  Workspace(const Workspace&) = delete;
+  Workspace& operator=(const Workspace&) = delete;
+  static size_t round(size_t n) { return (std::max<size_t>(n, 1) + 31) / 32 * 32; }  // 256 bytes
+  double* take(size_t n) {
+    double* p = g->d_ws.p + used;
+    used += round(n);
+    require(used <= g->d_ws.n, CHX_ERR_STATE, "workspace overrun");
+    return p;
+  }
+};
+
+// Matrices that one set of launches takes together, `per` doubles of workspace
+// each: as many as fit into half of what a workspace may keep (their kernels
+// are a few microseconds each for small systems, and large systems fill the chip
+// with one).
+int matrices_at_once(size_t per, int nmats) {
+  const size_t fit = Workspace::kWsKeep / sizeof(double) / 2 / std::max<size_t>(per, 1);
+  return (int)std::max<size_t>(1, std::min<size_t>({fit, (size_t)nmats, (size_t)1024}));
+}
+
 // Stage ids of chx_grid_kernel_times.
 enum { kStPermute = 0, kStDensity = 1, kStFunctional = 2, kStVxc = 3, kStFinalize = 4, kStMakeB = 5, kStCore = 6 };
 
@@ -248,10 +286,38 @@ void check_dm_args(const chx_grid* g, int nspin, int nbasis, int max_spin = 1) {
   require(nbasis == g->nbasis, CHX_ERR_ARG, "density matrix size does not match the basis");
 }
 
+// FP64 form, LDA and GGA: the two spins' B tables and runs' blocks fit a kept workspace.
+bool spins_together(const chx_grid* g, int family) {
+  const size_t per = g->slot_tile.size() * (size_t)kBatch * kTile + g->u_elems + g->dt_elems;
+  return g->precision == CHX_PREC_FP64 && g->cached && family < 2 && 2 * sizeof(double) * per < Workspace::kWsKeep;
+}
+
 // Density of one or two spin matrices at dD (device, back to back): beta first,
 // its partials kept in d_part_b, then alpha in d_part (GridDensity.cpp:12-31
 // per spin index).
 void density_spin(chx_grid* g, const double* dD, int nspin) {
+  if (nspin == 2 && spins_together(g, g->type)) {  // FP64, rho and grad rho: both spins in one set of launches
+    hipEvent_t e = nullptr;
+    const size_t sD = g->dt_elems;
+    g->corr_pending = g->corr_done = g->vout_ready = false;
+    g->d_part_b.alloc(g->d_part.n);
+    ++g->d_gen;
+    Workspace ws(g, Workspace::round(2 * sD));
+    double* Dt = ws.take(2 * sD);
+    g->mark_begin(kStPermute, &e);
+    launch_gather_d(g->stream, (int)g->tile_chunk.size(), g->nbasis, dD, g->d_tile_chunk.p, g->d_chunks.p, g->d_ao_of.p,
+                    Dt, nullptr, 0, 2, sD);
+    g->mark_end(kStPermute, e);
+    g->mark_begin(kStDensity, &e);
+    launch_density_c64(g->stream, (int)g->grp_batch.size(), g->d_grp_batch.p, g->d_grp_tile.p, g->d_grp_ntiles.p,
+                       g->d_bt_off.p, g->d_b_chunk.p, g->d_chunks.p, g->d_cache.p, Dt, nullptr, 0, g->d_part.p, nullptr,
+                       2, sD, 0, g->d_part_b.p);
+    g->mark_end(kStDensity, e);
+    g->have_density = true;
+    g->have_eval = g->have_v = false;
+    g->nspin = nspin;
+    return;
+  }
   if (nspin == 2) {
     density_from_device(g, dD + (size_t)g->nbasis * g->nbasis, 1);
     g->d_part_b.alloc(g->d_part.n);
@@ -273,6 +339,23 @@ void density_spin(chx_grid* g, const double* dD, int nspin) {
 // sum_s V_s . (D_s - hi - lo), into d_en[2].
 void fock_spin(chx_grid* g, double* dV, int nspin) {
   require(nspin == g->v_nspin, CHX_ERR_ARG, "Fock spin count differs from the evaluated density's");
+  if (nspin == 2 && spins_together(g, g->v_family)) {
+    hipEvent_t e = nullptr;
+    const size_t sB = Workspace::round(g->slot_tile.size() * (size_t)kBatch * kTile), sU = Workspace::round(g->u_elems);
+    Workspace ws(g, 2 * (sB + sU));
+    double *bmat = ws.take(2 * sB), *U = ws.take(2 * sU);
+    g->mark_begin(kStMakeB, &e);
+    launch_make_b(g->stream, g->nbatches, g->d_bt_off.p, g->d_coef.p, g->d_cache.p, bmat, 2, 0, sB, g->d_coef_b.p);
+    g->mark_end(kStMakeB, e);
+    g->mark_begin(kStVxc, &e);
+    launch_vxc_c64(g->stream, 1, (int)g->mwork.size(), g->d_mwork.p, g->d_cache.p, bmat, nullptr, U, 2, sB, sU);
+    g->mark_end(kStVxc, e);
+    g->mark_begin(kStFinalize, &e);
+    launch_assemble<double>(g->stream, g->nbasis, g->d_rowptr.p, g->d_rows.p, g->d_ao_of.p, U, dV, nullptr, nullptr, 2,
+                            sU);
+    g->mark_end(kStFinalize, e);
+    return;
+  }
   fock_to_device(g, dV, 0);
   if (nspin == 2) {
     const size_t nc = g->d_coef.n, nb2 = (size_t)g->nbasis * g->nbasis;
@@ -503,44 +586,6 @@ int chx_grid_get_density_skeleton(chx_grid* g, const double* D, int nspin, int n
     gather_d(g, g->d_Din.p, g->d_Dskel_t);
     g->have_skeleton = true;
   });
-}
-
-// Workspace of one derivative call, kept on the grid for the next one (until it
-// is planned again) unless it is larger than kWsKeep: hipMalloc and hipFree of
-// these buffers on every call cost more than the kernels of a small system, and
-// now and then 10 ms and more.
-struct Workspace {
-  static constexpr size_t kWsKeep = (size_t)1 << 30;  // bytes
-  chx_grid* g;
-  size_t used = 0;
-  // total: doubles of all takes, each rounded up by round()
-  Workspace(chx_grid* grid, size_t total) : g(grid) {
-    require(!g->ws_live, CHX_ERR_STATE, "the grid's workspace is in use");
-    if (g->d_ws.n < total) g->d_ws.alloc(total);
-    g->ws_live = true;
-  }
-  ~Workspace() {
-    g->ws_live = false;
-    if (g->d_ws.n * sizeof(double) > kWsKeep) g->d_ws.release();
-  }
-  Workspace(const Workspace&) = delete;
-  Workspace& operator=(const Workspace&) = delete;
-  static size_t round(size_t n) { return (std::max<size_t>(n, 1) + 31) / 32 * 32; }  // 256 bytes
-  double* take(size_t n) {
-    double* p = g->d_ws.p + used;
-    used += round(n);
-    require(used <= g->d_ws.n, CHX_ERR_STATE, "workspace overrun");
-    return p;
-  }
-};
-
-// Matrices that one set of launches takes together, `per` doubles of workspace
-// each: as many as fit into a quarter of what a workspace may keep (their kernels
-// are a few microseconds each for small systems, and large systems fill the chip
-// with one).
-static int matrices_at_once(size_t per, int nmats) {
-  const size_t fit = Workspace::kWsKeep / sizeof(double) / 4 / std::max<size_t>(per, 1);
-  return (int)std::max<size_t>(1, std::min<size_t>({fit, (size_t)nmats, (size_t)1024}));
 }
 
 int chx_grid_get_density_u(chx_grid* g, const double* D, int nmats, int nspin, int nbasis) {

@@ -273,15 +273,16 @@ void launch_point_density(hipStream_t s, int nbatches, const int* grp_off, const
                           const double* part_tau, int has_tau, const double* bw, double* rho, double* sigma,
                           double* tau, double* w);
 // (the launches below: nmat matrices of one launch, s*: doubles from one matrix's
-// operand or result to the next one's; tau and ncomp 4 take one)
+// operand or result to the next one's; part1, coef1: the second one's (not null), of
+// two; tau and ncomp 4 take one)
 // rho, grad rho / 2 into part; part_tau (not null: meta-GGA): tau (asym / gen as launch_gather_d's)
 void launch_density_c64(hipStream_t s, int ngroups, const int* grp_batch, const int* grp_tile, const int* grp_ntiles,
                         const int* bt_off, const int* b_chunk, const ChunkDev* chunks, const double* cache,
                         const double* Dt, const int* asym, int gen, double* part, double* part_tau, int nmat = 1,
-                        size_t sD = 0, size_t sP = 0);
+                        size_t sD = 0, size_t sP = 0, double* part1 = nullptr);
 // B = a phi + c . grad phi per slot (one component for every family)
 void launch_make_b(hipStream_t s, int nbatches, const int* bt_off, const double* coef, const double* cache,
-                   double* bmat, int nmat = 1, size_t sC = 0, size_t sB = 0);
+                   double* bmat, int nmat = 1, size_t sC = 0, size_t sB = 0, const double* coef1 = nullptr);
 // upper blocks of V per run into U; ncomp 4 adds the tau term, its operand t d_r
 // phi formed from the cache and coef[4] as it is loaded
 void launch_vxc_c64(hipStream_t s, int ncomp, int nwork, const MxItem* work, const double* cache, const double* bmat,

@@ -91,16 +91,21 @@ void launch_ao_cache(hipStream_t s, int nslots, const int* slot_batch, const int
 // (asym != gen) the wave's tau products run over the tiles up to its own, those
 // before it counted twice (accumulators doubled when it is reached).
 // C18 / def2-TZVP / SG-3: 4.6 ms (7.6 in four launches with LDS stages).
-template <bool TAU>
+// NM = 2: two matrices (spins, perturbations) against the same phi, which is then
+// read once for both, the epilogue's grad phi too. Radical C7 / UKS, def2-SVP /
+// SG-2: 0.26 ms for both spins, 0.29 in two launches.
+template <bool TAU, int NM>
 __global__ __launch_bounds__(TAU ? 512 : 256, 2) void k_density_c64(
     const int* __restrict__ grp_batch, const int* __restrict__ grp_tile, const int* __restrict__ grp_ntiles,
     const int* __restrict__ bt_off, const int* __restrict__ b_chunk, const ChunkDev* __restrict__ chunks,
     const double* __restrict__ cache, const double* __restrict__ Dt, size_t sD, const int* __restrict__ asym, int gen,
-    double* __restrict__ part, size_t sP, double* __restrict__ part_tau) {
-  Dt += blockIdx.y * sD;
-  part += blockIdx.y * sP;
+    double* __restrict__ part, size_t sP, double* __restrict__ part1, double* __restrict__ part_tau) {
+  static_assert(!TAU || NM == 1, "tau takes one matrix");
   constexpr int NC = TAU ? 4 : 1, NR = TAU ? 2 : 4, NOUT = TAU ? 5 : 4;
-  __shared__ double red[kGroup][NOUT][kBatch];
+  __shared__ double red[kGroup][NM * NOUT][kBatch];
+  Dt += blockIdx.y * NM * sD;
+  part += blockIdx.y * NM * sP;
+  if (!part1) part1 = part + sP;
   const int grp = blockIdx.x;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -113,9 +118,9 @@ __global__ __launch_bounds__(TAU ? 512 : 256, 2) void k_density_c64(
     const bool sym = TAU && *asym != gen;
     const double* __restrict__ A0 = cache + (size_t)it0 * kSlotAO + (row0 + lrow) * kTile + 2 * lk;
     const double* __restrict__ D0 = Dt + ch.doff + (size_t)(2 * lk) * ld + tq * kTile + lrow;
-    dbl4 acc[NC][NR][2];
+    dbl4 acc[NC * NM][NR][2];
 #pragma unroll
-    for (int d = 0; d < NC; ++d)
+    for (int d = 0; d < NC * NM; ++d)
 #pragma unroll
       for (int r = 0; r < NR; ++r)
 #pragma unroll
@@ -126,7 +131,7 @@ __global__ __launch_bounds__(TAU ? 512 : 256, 2) void k_density_c64(
       constexpr int ND = decltype(with_tau)::value ? NC : 1;
       if (p0 >= p1) return;
       double2 a[2][ND][NR];
-      double bb[2][2][2];  // [buffer][row of the pair][half]
+      double bb[2][NM][2][2];  // [buffer][matrix][row of the pair][half]
       auto load = [&](int p, int buf) {
         const int k = p >> 2, o = 8 * (p & 3);
         const double* __restrict__ pa = A0 + (size_t)k * kSlotAO + o;
@@ -137,19 +142,22 @@ __global__ __launch_bounds__(TAU ? 512 : 256, 2) void k_density_c64(
           for (int r = 0; r < NR; ++r)
             a[buf][d][r] = *reinterpret_cast<const double2*>(pa + d * kSlotB + 16 * r * kTile);
 #pragma unroll
-        for (int e = 0; e < 2; ++e)
+        for (int m = 0; m < NM; ++m)
 #pragma unroll
-          for (int h = 0; h < 2; ++h) bb[buf][e][h] = pd[(size_t)e * ld + 16 * h];
+          for (int e = 0; e < 2; ++e)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) bb[buf][m][e][h] = pd[m * sD + (size_t)e * ld + 16 * h];
       };
       auto step = [&](int buf) {
 #pragma unroll
-        for (int d = 0; d < ND; ++d)
+        for (int d = 0; d < ND * NM; ++d)  // component d, or (one component) matrix d
 #pragma unroll
           for (int r = 0; r < NR; ++r)
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
-              acc[d][r][h] = mfma_f64(a[buf][d][r].x, bb[buf][0][h], acc[d][r][h]);
-              acc[d][r][h] = mfma_f64(a[buf][d][r].y, bb[buf][1][h], acc[d][r][h]);
+              const double2 x = a[buf][NM == 1 ? d : 0][r];
+              acc[d][r][h] = mfma_f64(x.x, bb[buf][NM == 1 ? 0 : d][0][h], acc[d][r][h]);
+              acc[d][r][h] = mfma_f64(x.y, bb[buf][NM == 1 ? 0 : d][1][h], acc[d][r][h]);
             }
       };
       load(p0, 0);
@@ -191,12 +199,13 @@ __global__ __launch_bounds__(TAU ? 512 : 256, 2) void k_density_c64(
 #pragma unroll
       for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int c = 0; c < NOUT; ++c) {
+        for (int c = 0; c < NM * NOUT; ++c) {
+          const int m = NM == 1 ? 0 : c / NOUT, o = c % NOUT;
           double v = 0.0;
 #pragma unroll
           for (int h = 0; h < 2; ++h) {
-            if (c < 4) v += acc[0][r][h][i] * f[h][i][c & 3];
-            if (c == 4) {
+            if (o < 4) v += acc[m][r][h][i] * f[h][i][o & 3];
+            if (o == 4) {
 #pragma unroll
               for (int d = 1; d < NC; ++d) v += acc[d][r][h][i] * f[h][i][d];
             }
@@ -205,19 +214,21 @@ __global__ __launch_bounds__(TAU ? 512 : 256, 2) void k_density_c64(
           v += __shfl_xor(v, 2, 64);
           v += __shfl_xor(v, 4, 64);
           v += __shfl_xor(v, 8, 64);
-          if (lrow == 4 * i + (c & 3)) red[q][c][row0 + 16 * r + 4 * i + lk] = v;
+          if (lrow == 4 * i + (o & 3)) red[q][c][row0 + 16 * r + 4 * i + lk] = v;
         }
     }
   }
   // the sums over the group's tiles
   __syncthreads();
-  for (int e = tid; e < (TAU ? 7 : 4) * kBatch; e += TAU ? 512 : 256) {
+  for (int e = tid; e < (TAU ? 7 : 4 * NM) * kBatch; e += TAU ? 512 : 256) {
     const int c = e / kBatch, g = e % kBatch;
     double v = 0.0;
-    if (c < NOUT)
+    if (c < NM * NOUT)
       for (int t = 0; t < nt; ++t) v += red[t][c][g];
     if (c < 4)
       part[(size_t)grp * 4 * kBatch + c * kBatch + g] = v;
+    else if (NM == 2)
+      part1[(size_t)grp * 4 * kBatch + (c - 4) * kBatch + g] = v;
     else  // part_tau: [group][3][64], summed over the directions in the first
       part_tau[(size_t)grp * 3 * kBatch + (c - 4) * kBatch + g] = v;
   }
@@ -226,14 +237,19 @@ __global__ __launch_bounds__(TAU ? 512 : 256, 2) void k_density_c64(
 void launch_density_c64(hipStream_t s, int ngroups, const int* grp_batch, const int* grp_tile, const int* grp_ntiles,
                         const int* bt_off, const int* b_chunk, const ChunkDev* chunks, const double* cache,
                         const double* Dt, const int* asym, int gen, double* part, double* part_tau, int nmat,
-                        size_t sD, size_t sP) {
+                        size_t sD, size_t sP, double* part1) {
   if (ngroups == 0) return;
+  const int pairs = part_tau ? 0 : nmat / 2, done = 2 * pairs;
+  if (pairs)
+    hipLaunchKernelGGL((k_density_c64<false, 2>), dim3(ngroups, pairs), dim3(256), 0, s, grp_batch, grp_tile,
+                       grp_ntiles, bt_off, b_chunk, chunks, cache, Dt, sD, asym, gen, part, sP, part1, nullptr);
   if (part_tau)
-    hipLaunchKernelGGL(k_density_c64<true>, dim3(ngroups, nmat), dim3(512), 0, s, grp_batch, grp_tile, grp_ntiles,
-                       bt_off, b_chunk, chunks, cache, Dt, sD, asym, gen, part, sP, part_tau);
-  else
-    hipLaunchKernelGGL(k_density_c64<false>, dim3(ngroups, nmat), dim3(256), 0, s, grp_batch, grp_tile, grp_ntiles,
-                       bt_off, b_chunk, chunks, cache, Dt, sD, asym, gen, part, sP, part_tau);
+    hipLaunchKernelGGL((k_density_c64<true, 1>), dim3(ngroups), dim3(512), 0, s, grp_batch, grp_tile, grp_ntiles,
+                       bt_off, b_chunk, chunks, cache, Dt, sD, asym, gen, part, sP, nullptr, part_tau);
+  else if (done < nmat)
+    hipLaunchKernelGGL((k_density_c64<false, 1>), dim3(ngroups), dim3(256), 0, s, grp_batch, grp_tile, grp_ntiles,
+                       bt_off, b_chunk, chunks, cache, Dt + done * sD, sD, asym, gen, part + done * sP, sP, nullptr,
+                       nullptr);
   CHX_HIP(hipGetLastError());
 }
 
@@ -243,36 +259,39 @@ void launch_density_c64(hipStream_t s, int ngroups, const int* grp_batch, const 
 // T_r = t d_r phi (t = w v_tau / 4, so that V = M + M^T carries
 // (1/2) w v_tau grad phi_mu . grad phi_nu) is formed from the cached d_r phi
 // while the Vxc kernel loads it, instead of being stored.
+// kMakeBMat matrices at a time read phi and grad phi once for all of them.
+constexpr int kMakeBMat = 4;
 __global__ __launch_bounds__(256) void k_make_b(const int* __restrict__ bt_off, const double* __restrict__ coef,
-                                                size_t sC, const double* __restrict__ cache,
-                                                double* __restrict__ bmat, size_t sB) {
-  coef += blockIdx.y * sC;  // the matrix of the launch
-  bmat += blockIdx.y * sB;
-  __shared__ double ca[kBatch], cx[kBatch], cy[kBatch], cz[kBatch];
-  const int b = blockIdx.x, tid = threadIdx.x;
-  if (tid < kBatch) {
-    const size_t slot = (size_t)b * kBatch + tid;
-    ca[tid] = coef[kCoef * slot];
-    cx[tid] = coef[kCoef * slot + 1];
-    cy[tid] = coef[kCoef * slot + 2];
-    cz[tid] = coef[kCoef * slot + 3];
+                                                size_t sC, const double* __restrict__ coef1,
+                                                const double* __restrict__ cache, double* __restrict__ bmat,
+                                                size_t sB, int nmat) {
+  __shared__ double cf[kMakeBMat][4][kBatch];
+  const int b = blockIdx.x, tid = threadIdx.x, m0 = blockIdx.y * kMakeBMat, nm = min(kMakeBMat, nmat - m0);
+  for (int e = tid; e < nm * 4 * kBatch; e += 256) {
+    const int m = e / (4 * kBatch), c = (e / kBatch) % 4, g = e % kBatch;
+    const double* __restrict__ src = coef1 && m0 + m == 1 ? coef1 : coef + (m0 + m) * sC;
+    cf[m][c][g] = src[kCoef * ((size_t)b * kBatch + g) + c];
   }
   __syncthreads();
+  bmat += m0 * sB;
   for (int it = bt_off[b]; it < bt_off[b + 1]; ++it) {
     const double* src = cache + (size_t)it * kSlotAO;
     double* dst = bmat + (size_t)it * kSlotB;
     for (int e = tid; e < kSlotB; e += 256) {
       const int g = e / kTile;
-      const double dx = src[kSlotB + e], dy = src[2 * kSlotB + e], dz = src[3 * kSlotB + e];
-      dst[e] = ca[g] * src[e] + cx[g] * dx + cy[g] * dy + cz[g] * dz;
+      const double v = src[e], dx = src[kSlotB + e], dy = src[2 * kSlotB + e], dz = src[3 * kSlotB + e];
+#pragma unroll
+      for (int m = 0; m < kMakeBMat; ++m)
+        if (m < nm) dst[m * sB + e] = cf[m][0][g] * v + cf[m][1][g] * dx + cf[m][2][g] * dy + cf[m][3][g] * dz;
     }
   }
 }
 
 void launch_make_b(hipStream_t s, int nbatches, const int* bt_off, const double* coef, const double* cache,
-                   double* bmat, int nmat, size_t sC, size_t sB) {
+                   double* bmat, int nmat, size_t sC, size_t sB, const double* coef1) {
   if (nbatches == 0) return;
-  hipLaunchKernelGGL(k_make_b, dim3(nbatches, nmat), dim3(256), 0, s, bt_off, coef, sC, cache, bmat, sB);
+  hipLaunchKernelGGL(k_make_b, dim3(nbatches, (nmat + kMakeBMat - 1) / kMakeBMat), dim3(256), 0, s, bt_off, coef, sC,
+                     coef1, cache, bmat, sB, nmat);
   CHX_HIP(hipGetLastError());
 }
 
@@ -295,10 +314,17 @@ __global__ __launch_bounds__(256, 2) void k_vxc_c64(const MxItem* __restrict__ w
                                                     const double* __restrict__ bmat, const double* __restrict__ coef,
                                                     const int* __restrict__ ao_of, double* __restrict__ out,
                                                     int npad, ProdBatch pb) {
-  cache += (blockIdx.y / pb.nb) * pb.sA;  // the matrix of the launch
-  bmat += (blockIdx.y % pb.nb) * pb.sB;
-  out += blockIdx.y * pb.sO;
-  const MxItem wk = work[blockIdx.x];
+  int item = blockIdx.x;
+  if (gridDim.y > 1) {  // an item's matrices side by side on one XCD: they share the operand A
+    const int nm = gridDim.y, full = gridDim.x / 8 * 8, lin = blockIdx.y * gridDim.x + blockIdx.x;
+    const int r = lin - full * nm, rest = gridDim.x - full;
+    const int mat = r < 0 ? lin / 8 % nm : r / rest;
+    item = r < 0 ? lin / (8 * nm) * 8 + lin % 8 : full + r % rest;
+    cache += (mat / pb.nb) * pb.sA;
+    bmat += (mat % pb.nb) * pb.sB;
+    out += mat * pb.sO;
+  }
+  const MxItem wk = work[item];
   const bool diag = wk.I0 == wk.J0;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
