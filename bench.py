@@ -224,14 +224,14 @@ def main():
     st = chosen["stats"]
     flops_build = st["flops_per_build"]
     ms_step = chosen["ms"]
-    names64 = {"density": ("k_density_c64<0..3>" if nc == 4 else "k_density_c64<0>") if plain and plain["cached"]
-               else "k_density_f64",
-               "vxc": ("k_vxc_c64<%d>" % nc) if plain and plain["cached"] else "k_vxc_f64",
-               "density_launches": 4 if nc == 4 else 1}
-    vxc_mx = chosen["grid"].vxcKernel() + "<%d>" % nc
+    cached64 = plain and plain["cached"]
+    names64 = {"density": ("k_density_c64<%s, 1>" % ("true" if nc == 4 else "false")) if cached64 else "k_density_f64",
+               "vxc": ("k_vxc_c64<%d>" % (nc == 4)) if cached64 else "k_vxc_f64",
+               "density_launches": 4 if nc == 4 and not cached64 else 1}
+    vxc_mx = chosen["grid"].vxcKernel() + "<%d, %d>" % (nc, 5 if chosen["grid"].vxcShape() == 1 else 4)
     # the density stage: one launch (meta-GGA: rho, grad rho and tau fused, every group; LDA / GGA: the
-    # groups of the other batches); the core batches' three-term launch is timed on its own
-    namesmx = {"density": "k_density_mx_mgga" if nc == 4 else "k_density_mx<0>",
+    # groups of the other batches); the core batches' three-term groups are timed in a launch of their own
+    namesmx = {"density": "k_density_mx_mgga" if nc == 4 else "k_density_mx",
                "vxc": vxc_mx, "density_launches": 1}
 
     out = {
@@ -260,8 +260,8 @@ def main():
                         "memory (PCIe included); not the value",
         "speedup_vs_plain_fp64": round(plain["ms"] / ms_step, 3) if plain else None,
         "autotune": {"vxc_shape": chosen["tuned"][0], "vxc_chunk": chosen["tuned"][1],
-                     "shapes": {"0": "128 x 128 blocks over 128-AO super-tile pairs",
-                                "1": "256 x 256 blocks over 8-tile groups of each chunk's AO list"},
+                     "shapes": {"0": "pairs of groups of up to 4 tiles (128 AOs) of each chunk's AO list",
+                                "1": "pairs of groups of up to 5 tiles (160 AOs) of each chunk's AO list"},
                      "ms": {"%d/%d" % k: round(v, 4) for k, v in chosen["tuned"][2].items()}}
         if chosen["tuned"] else None,
         "tflops": round(flops_build / (ms_step * 1e-3) / 1e12, 3),

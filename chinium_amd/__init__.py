@@ -356,7 +356,7 @@ class Grid:
         return c.value, dict(zip((8, 16, 32, 128), list(ms)))
 
     def autotuneTiles(self, xc, D_ptr, V_ptr, reps=3):
-        """Mixed form: times both Vxc block shapes (0: 128-AO super-tiles, 1: 256-AO groups) at
+        """Mixed form: times both Vxc block shapes (0: groups of 4 tiles of 32 AOs, 1: of 5) at
         each work-item length, keeps the fastest; returns (shape, chunk, {(shape, chunk): ms})."""
         sh, c = ctypes.c_int(), ctypes.c_int()
         ms = (ctypes.c_float * 8)()
@@ -495,8 +495,9 @@ class Grid:
         return {k: (float(ms[i]), int(n[i])) for i, k in enumerate(self.STAGES)}
 
     def vxcKernel(self):
-        """Name of the kernel the mixed form runs for the Vxc contraction (the block shape in use)."""
-        return "k_vxc_mx_wide" if self.vxcShape() == 1 else "k_vxc_mx"
+        """Name of the kernel the mixed form runs for the Vxc contraction; its template arguments are the
+        operand components (1, meta-GGA 4) and the tiles per group (4, or 5 for shape 1)."""
+        return "k_vxc_mx"
 
     def stats(self):
         nb, npnt, mt, fl = ctypes.c_long(), ctypes.c_long(), ctypes.c_double(), ctypes.c_double()
@@ -717,7 +718,7 @@ class Pack:
         return c.value, dict(zip((8, 16, 32, 128), list(ms)))
 
     def vxcWideFrom(self):
-        """The autotuned Vxc shape threshold: 256-AO groups for npad >= it (-1: none)."""
+        """The autotuned Vxc shape threshold: groups of 5 tiles for npad >= it (-1: none)."""
         v = ctypes.c_int()
         _check(lib().chx_pack_vxc_wide_from(self.h, ctypes.byref(v)))
         return v.value

@@ -610,8 +610,8 @@ void set_vxc_chunk(chx_grid* g, int chunk) {
   build_cwork(g);
 }
 
-// Vxc block shape of the mixed form (-1: 256-AO groups from npad 1024
-// on, 128-AO super-tiles below; 0, 1: either), rebuilding the work items.
+// Vxc block shape of the mixed form (-1: groups of up to 5 tiles from npad 1024
+// on, of up to 4 below; 0, 1: either), rebuilding the work items.
 void set_vxc_shape(chx_grid* g, int shape) {
   g->vxc_shape = shape;
   if (!g->ao_ready || g->precision != CHX_PREC_MIXED) return;
@@ -734,7 +734,7 @@ void grid_plan(chx_grid* g) {
     throw Error(CHX_ERR_DEVICE, "the mixed-precision form needs " + std::to_string(cache_bytes / 1e9) +
                                     " GB of device memory for its AO cache");
   g->cached = mixed || g->cache_mode == 1 || (g->cache_mode == -1 && cache_bytes < 0.8 * (double)free_b);
-  // large bases: Vxc items over 256 x 256 blocks
+  // large bases: Vxc items over groups of up to 5 tiles
   g->mx_wide = mixed && (g->vxc_shape == 1 || (g->vxc_shape < 0 && g->npad >= 1024)) ? 1 : 0;
   g->vwork.clear();
   g->mwork.clear();

@@ -484,8 +484,8 @@ struct chx_grid {
   int cache_mode = -1;               // -1 automatic, 0 never, 1 always
   std::vector<int> slot_batch, slot_tile;
   int vxc_chunk = 0;                 // batches per Vxc work item; 0 = by the item count
-  int vxc_shape = -1;                // mixed form's Vxc blocks: -1 by basis size, 0 128-AO super-tiles, 1 256-AO groups
-  int mx_wide = 0;                   // mixed form: Vxc over 256-AO groups (large bases)
+  int vxc_shape = -1;                // mixed form's Vxc groups: -1 by basis size, 0 up to 4 tiles, 1 up to 5
+  int mx_wide = 0;                   // mixed form: Vxc over groups of up to 5 tiles (large bases)
   std::vector<chx::MxItem> mwork;       // Vxc work items of the cached tables
   std::vector<chx::MxItem> pwork;       // FP64 form: items of the plain products (skeleton derivatives)
   size_t u_elems = 0;                   // elements of the runs' blocks of V

@@ -53,7 +53,7 @@ struct chx_pack {
   std::vector<unsigned long> gen;  // each grid's plan generation when the lanes and graph were built
   std::vector<double> h_en;
   int lanes = 16;
-  int wide_from = -2;    // Vxc shape of the last autotune: 256-AO groups for npad >= wide_from (-1: none; -2: not tuned)
+  int wide_from = -2;    // Vxc shape of the last autotune: groups of 5 tiles for npad >= wide_from (-1: none; -2: not tuned)
   std::vector<int> cut;  // lane k holds molecules [cut[k], cut[k + 1])
   std::vector<hipStream_t> lane_st;
   std::vector<hipEvent_t> ev_dens, ev_done;
@@ -201,7 +201,7 @@ void build_persistent(chx_pack* p) {
     }
   p->mol_base = (const char*)base;
   p->mol_tab.upload(mols, p->stream);
-  // per stage: density (the groups outside the core batches), core groups, B^T slots, Vxc items of 128-AO molecules, Vxc items of 256-AO molecules
+  // per stage: density (the groups outside the core batches), core groups, B^T slots, Vxc items over groups of 4 tiles, over groups of 5
   std::vector<int> starts(5 * (size_t)(n + 1), 0);
   p->totals.assign(5, 0);
   for (int m = 0; m < n; ++m) {
@@ -543,8 +543,8 @@ int chx_pack_autotune(chx_pack* p, const chx_xc* xc, const double* const* D_dev,
       }
     }
     for (chx_grid* g : p->grids) set_vxc_chunk(g, cand[best]);
-    // then the Vxc tile shape per molecule, by a basis-size threshold: 256-AO groups for
-    // npad >= T, 128-AO super-tiles below (T = 0: all groups; -1: none)
+    // then the Vxc tile shape per molecule, by a basis-size threshold: groups of 5 tiles for
+    // npad >= T, of 4 below (T = 0: 5 for all; -1: none)
     static const int thr[] = {-1, 1024, 512, 0};
     int best_thr = -1;
     float best_thr_ms = 0.f;

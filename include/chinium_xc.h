@@ -221,8 +221,8 @@ int chx_grid_set_screening(chx_grid* g, double threshold);
  * ms_out[4] the times. Needs the AO tables in HBM (cached or mixed form). */
 int chx_grid_autotune(chx_grid* g, const chx_xc* xc, const double* D_dev, double* V_dev, int reps, int* chunk_out,
                       float* ms_out);
-/* Mixed form's Vxc block shape (no reference counterpart): 0 = 128 x 128
- * blocks, 1 = 256 x 256 blocks of each batch chunk's AO list; -1 (default) = 1
+/* Mixed form's Vxc block shape (no reference counterpart): groups of up to 4
+ * (0) or 5 (1) tiles of 32 AOs of each batch chunk's list; -1 (default) = 1
  * from npad 1024 on, else 0. chx_grid_vxc_shape reports the shape in use. */
 int chx_grid_set_vxc_shape(chx_grid* g, int shape);
 /* Vxc work-item length in batches (0: by the number of items, at most 128; an
@@ -353,7 +353,7 @@ int chx_pack_set_graph(chx_pack* p, int enable);
 /* Autotuner: times `reps` builds for each Vxc work-item length (8, 16, 32,
  * 128 batches), keeps the fastest (chunk_out gets it, ms_out[4] the times);
  * then the Vxc tile shape per molecule (chx_grid_set_vxc_shape) by a
- * basis-size threshold T (256-AO union groups for npad >= T: none, 1024, 512,
+ * basis-size threshold T (groups of 5 tiles for npad >= T: none, 1024, 512,
  * all), keeps the fastest; then the form and lanes (per-molecule kernels or
  * per-lane stage launches on 4, 8 or 16 lanes, or persistent stages; the last
  * two for LDA/GGA), keeps the fastest. */
