@@ -1,5 +1,6 @@
 // C ABI of the XC path (include/chinium_xc.h). Every entry point catches
 // exceptions and returns a status; the message is kept per host thread.
+#include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -681,10 +682,11 @@ int chx_grid_fock_u(chx_grid* g, double* F, int nmats, int nspin, int nbasis) {
   });
 }
 
-// slot -> (density group, column tile in the group) for the per-slot epilogues, AO -> atom
+// slot -> (density group, column tile in the group) for the per-slot epilogues, AO -> atom (which the
+// skeleton calls read for every AO, also where no shell is alive and there is no slot)
 static void ensure_slot_groups(chx_grid* g) {
   const int ng = (int)g->grp_batch.size(), ns = (int)g->slot_tile.size();
-  if (g->slot_grp.size() == (size_t)ns) return;
+  if (g->slot_tables) return;
   g->slot_grp.assign(ns, 0);
   g->slot_q.assign(ns, 0);
   for (int k = 0; k < ng; ++k) {
@@ -700,6 +702,8 @@ static void ensure_slot_groups(chx_grid* g) {
   g->d_ao_atom.upload(ao_atom, g->stream);
   g->d_slot_grp.upload(g->slot_grp, g->stream);
   g->d_slot_q.upload(g->slot_q, g->stream);
+  CHX_HIP(hipStreamSynchronize(g->stream));  // ao_atom goes out of scope
+  g->slot_tables = true;
 }
 
 int chx_grid_fock_s(chx_grid* g, double* F, int nspin, int nbasis) {

@@ -863,8 +863,7 @@ void grid_plan(chx_grid* g) {
   ++g->plan_gen;
   g->have_density = g->have_eval = g->have_v = g->have_skeleton = false;
   g->corr_pending = g->corr_done = g->vout_ready = false;
-  g->slot_grp.clear();
-  g->slot_q.clear();
+  g->slot_tables = false;
 }
 
 }  // namespace chx

@@ -507,6 +507,7 @@ struct chx_grid {
   chx::DevBuf<double> d_ws;             // derivative calls' workspace (Workspace in api.cpp)
   bool ws_live = false;
   chx::DevBuf<int> d_ao_atom;           // atom of each AO (-1: padding), with the slot tables below
+  bool slot_tables = false;             // ... of this plan are on the device
   double flops_build = 0, mean_tiles = 0;
   std::vector<double> batch_work;  // g_b n_b^2 per batch (points x kept AOs squared)
   double core_flops = 0;           // the core batches' three-term (rho, grad rho) launch: 2 sum g_b n_b^2

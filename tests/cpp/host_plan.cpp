@@ -1,0 +1,231 @@
+// Host-only checks of the library's planning and call code (gridgen.cpp, api.cpp): the HIP runtime and
+// the kernel launches are replaced by the ones below, so that a plan, a call's arguments and what happens
+// when memory runs out can be looked at without a GPU. Device memory is host memory under a byte budget;
+// a launch checks that the tables it would read are there and returns.
+//   host_plan <check> <data root>; exit status 0 when it holds.
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <map>
+#include <string>
+#include <vector>
+
+#include "internal.hpp"
+
+// ---- the runtime ---------------------------------------------------------------------------------
+namespace fake {
+size_t budget = (size_t)64 << 30, used = 0;
+std::map<char*, size_t> live;  // base -> bytes
+hipError_t last = hipSuccess;
+hipError_t done(hipError_t e) { return e == hipSuccess ? e : last = e; }
+// p lies in a live allocation with at least n bytes behind it
+bool at(const void* p, size_t n = 1) {
+  auto it = live.upper_bound((char*)p);
+  if (p == nullptr || it == live.begin()) return false;
+  --it;
+  return (char*)p + n <= it->first + it->second;
+}
+int failed = 0;
+void check(bool ok, const char* what) {
+  if (ok) return;
+  ++failed;
+  std::printf("FAILED: %s\n", what);
+}
+}  // namespace fake
+#define CHECK(x) fake::check((x), #x)
+
+extern "C" {
+hipError_t hipMalloc(void** p, size_t n) {
+  if (fake::used + n > fake::budget) return fake::done(hipErrorOutOfMemory);
+  *p = std::calloc(n ? n : 1, 1);
+  fake::live[(char*)*p] = n;
+  fake::used += n;
+  return hipSuccess;
+}
+hipError_t hipFree(void* p) {
+  auto it = fake::live.find((char*)p);
+  if (it == fake::live.end()) return hipSuccess;
+  fake::used -= it->second;
+  fake::live.erase(it);
+  std::free(p);
+  return hipSuccess;
+}
+hipError_t hipMemGetInfo(size_t* f, size_t* t) {
+  *f = fake::budget - fake::used;
+  *t = fake::budget;
+  return hipSuccess;
+}
+hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) {
+  std::memcpy(d, s, n);
+  return hipSuccess;
+}
+hipError_t hipGetLastError() {
+  const hipError_t e = fake::last;
+  fake::last = hipSuccess;
+  return e;
+}
+const char* hipGetErrorString(hipError_t) { return "out of memory"; }
+hipError_t hipGetDeviceCount(int* n) { return *n = 1, hipSuccess; }
+hipError_t hipGetDevice(int* d) { return *d = 0, hipSuccess; }
+hipError_t hipStreamCreate(hipStream_t* s) { return *s = nullptr, hipSuccess; }
+hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+}
+
+// ---- the launches ----------------------------------------------------------------------------------
+namespace chx {
+using fake::at;
+static void launched() { CHX_HIP(hipGetLastError()); }
+std::vector<std::pair<std::string, const void*>> nulls;
+int becke_ld(int natoms) { return natoms; }
+void launch_becke(hipStream_t, long, const double*, const double*, const double*, double*, const int*, int,
+                  const double*, const double2*, int) {}
+void launch_bisect(hipStream_t, long n, const int* idx, const double* px, const double* py, const double* pz,
+                   const std::vector<int>& levels, const BisSeg*, double* pts[2], int* ids[2]) {
+  for (int k = 0; k < 2; ++k)  // in the points' own order
+    for (long i = 0; i < n; ++i) {
+      pts[k][i] = px[idx[i]];
+      pts[k][n + i] = py[idx[i]];
+      pts[k][2 * n + i] = pz[idx[i]];
+      ids[k][i] = idx[i];
+    }
+}
+void launch_batch_slots(hipStream_t, int nb, const int2* batch, const double* pts, const int* idx, long stride,
+                        const double* w, double* bx, double* by, double* bz, double* bw) {
+  for (int b = 0; b < nb; ++b)
+    for (int k = 0; k < kBatch; ++k) {
+      const int p = batch[b].x + (k < batch[b].y ? k : 0), s = b * kBatch + k;
+      bx[s] = pts[p];
+      by[s] = pts[stride + p];
+      bz[s] = pts[2 * stride + p];
+      bw[s] = k < batch[b].y ? w[idx[p]] : 0.0;
+    }
+}
+void launch_screen(hipStream_t, int nb, int nsh, int nwords, const double* bx, const double* by, const double* bz,
+                   const int* bn, const double* sh, const double* reach2, unsigned long long* alive) {
+  for (int b = 0; b < nb; ++b)
+    for (int s = 0; s < nsh; ++s)
+      for (int k = 0; k < bn[b]; ++k) {
+        const double x = bx[b * kBatch + k] - sh[3 * s], y = by[b * kBatch + k] - sh[3 * s + 1],
+                     z = bz[b * kBatch + k] - sh[3 * s + 2];
+        if (x * x + y * y + z * z < reach2[s]) alive[(size_t)b * nwords + (s >> 6)] |= 1ull << (s & 63);
+      }
+}
+void launch_fill(hipStream_t, double* p, size_t n, double) { CHECK(n == 0 || at(p, n * sizeof(double))); launched(); }
+void launch_fill_u32(hipStream_t, unsigned* p, size_t n, unsigned) { CHECK(n == 0 || at(p, n * 4)); launched(); }
+void launch_ao_cache(hipStream_t, int, const int*, const int*, const double*, const double*, const double*, BasisView,
+                     double*) { launched(); }
+void launch_ao_cache_mx(hipStream_t, int, const int*, const int*, const double*, const double*, const double*,
+                        BasisView, int, int, unsigned short*, const int*, unsigned short*) { launched(); }
+void launch_gather_d(hipStream_t, int, int, const double*, const int*, const ChunkDev*, const int*, double* Dt, int*,
+                     int, int, size_t) { CHECK(at(Dt)); launched(); }
+void launch_pad_d(hipStream_t, int, int npad, const double*, double* D) {
+  CHECK(at(D, sizeof(double) * npad * npad));
+  launched();
+}
+void launch_density_c64(hipStream_t, int, const int*, const int*, const int*, const int*, const int*, const ChunkDev*,
+                        const double*, const double*, const int*, int, double* part, double*, int, size_t, size_t,
+                        double*) { CHECK(at(part)); launched(); }
+void launch_functional(hipStream_t, int, const int* off, const double*, const double*, const double*, const int*, int,
+                       int, int, int, double*, double*, double*, int) { CHECK(at(off)); launched(); }
+void launch_functional_f(hipStream_t, int, const int*, const double*, const int*, int, int, double*) { launched(); }
+void launch_reduce_en(hipStream_t, int, const double*, double* en) { CHECK(at(en)); launched(); }
+void launch_make_b(hipStream_t, int, const int*, const double*, const double*, double* b, int, size_t, size_t,
+                   const double*) { CHECK(at(b)); launched(); }
+void launch_vxc_c64(hipStream_t, int, int nwork, const MxItem*, const double*, const double*, const double*, double* U,
+                    int, size_t, size_t) { CHECK(nwork == 0 || at(U)); launched(); }
+int assemble_blocks(int n) { return n; }
+template <class T>
+void launch_assemble(hipStream_t, int n, const int* rowptr, const RowRef* rows, const int*, const T* U, double* V,
+                     const float*, double*, int, size_t) {
+  CHECK(at(rowptr, 4 * (n + 1)) && at(V, sizeof(double) * n * n));
+  for (int e = 0; e < rowptr[n]; ++e) CHECK(at(U + rows[e].u, sizeof(T) * rows[e].len));
+  launched();
+}
+template void launch_assemble<float>(hipStream_t, int, const int*, const RowRef*, const int*, const float*, double*,
+                                     const float*, double*, int, size_t);
+template void launch_assemble<double>(hipStream_t, int, const int*, const RowRef*, const int*, const double*, double*,
+                                      const float*, double*, int, size_t);
+void launch_xgrad_xz(hipStream_t, int, const int*, const int*, const int*, const int*, const int*, const ChunkDev*,
+                     const double*, const double*, const double*, int, int, double*) { launched(); }
+void launch_skel_rho(hipStream_t, int, const int*, const int*, const int*, const int*, const double*, const double*,
+                     const double*, BasisView, const double*, const double*, long, double*) { launched(); }
+void launch_skel_etab(hipStream_t, int, const int*, const int*, const double*, const double*, const double*, BasisView,
+                      const double*, double*) { launched(); }
+void launch_prod_c64(hipStream_t, int, const MxItem*, const int*, const double*, const double*, double*, int, int,
+                     const ProdBatch&) { launched(); }
+void launch_fock_skel_fin(hipStream_t, int n, int, int, const double*, const int* ao_atom, double*) {
+  CHECK(at(ao_atom, sizeof(int) * n));  // read for every AO
+  launched();
+}
+size_t hess_part_elems(long, int np) { return (size_t)np * np; }
+void launch_hess_terms(hipStream_t, int, const int*, const int*, const int*, const int*, const double*, const double*,
+                       const double*, BasisView, const double*, const double*, const double*, long, const double*,
+                       const double*, const double*, int, int npad, const double*, const double*, const int* atom, int,
+                       double*, double*) {
+  CHECK(at(atom, sizeof(int) * npad));  // read for every AO and padding column
+  launched();
+}
+}  // namespace chx
+
+// ---- the checks --------------------------------------------------------------------------------------
+namespace {
+std::string root;
+
+// nat hydrogens 2 bohr apart with nsh s shells each (exponents 0.1 .. 1: everything overlaps everything), SG-1
+chx_grid* grid(int nat, int nsh, double expo = 0.1) {
+  std::vector<int> Z(nat, 1);
+  std::vector<double> xyz(3 * nat, 0.0);
+  for (int a = 0; a < nat; ++a) xyz[3 * a] = 2.0 * a;
+  chx_mol* m;
+  chx_grid* g;
+  CHECK(chx_mol_create(nat, Z.data(), xyz.data(), &m) == CHX_OK);
+  for (int a = 0; a < nat; ++a)
+    for (int k = 0; k < nsh; ++k) {
+      const double e = expo * (1 + 9.0 * k / nsh), c = 1;
+      CHECK(chx_mol_add_shell(m, a, 0, 1, &e, &c) == CHX_OK);
+    }
+  if (chx_grid_create(m, "SG-1", root.c_str(), 1, 0, &g) != CHX_OK) {
+    std::printf("%s\n", chx_last_error());
+    std::exit(2);
+  }
+  chx_mol_destroy(m);
+  return g;
+}
+chx_xc* functional(int code) {
+  chx_xc* xc;
+  CHECK(chx_xc_create(1, &code, 1, &xc) == CHX_OK);
+  return xc;
+}
+
+// Skeleton calls on a plan whose threshold leaves no shell alive.
+void empty_lists() {
+  chx_grid* g = grid(2, 3);
+  const int n = 6;
+  chx_xc* xc = functional(1);
+  std::vector<double> D(n * n, 0.1), F(6 * n * n), H(36);
+  for (double thr : {1e6, 1e-14}) {  // the second plan has slots
+    CHECK(chx_grid_set_screening(g, thr) == CHX_OK);
+    CHECK(chx_grid_get_ao(g, 0, 0) == CHX_OK);
+    CHECK((g->slot_tile.size() == 0) == (thr > 1));
+    CHECK(chx_grid_get_density(g, D.data(), 1, n) == CHX_OK);
+    CHECK(chx_xc_evaluate(xc, g, "ev") == CHX_OK);
+    CHECK(chx_grid_fock(g, F.data(), 1, n) == CHX_OK);
+    CHECK(chx_xc_evaluate(xc, g, "f") == CHX_OK);
+    CHECK(chx_grid_get_density_skeleton(g, D.data(), 1, n) == CHX_OK);
+    CHECK(chx_grid_fock_skeleton(g, F.data(), 1, n) == CHX_OK);
+    CHECK(chx_grid_energy_hess(g, H.data()) == CHX_OK);
+  }
+  chx_xc_destroy(xc);
+  chx_grid_destroy(g);
+}
+}  // namespace
+
+int main(int argc, char** argv) {
+  const std::map<std::string, void (*)()> checks = {{"empty_lists", empty_lists}};
+  if (argc != 3 || !checks.count(argv[1])) return 2;
+  root = argv[2];
+  checks.at(argv[1])();
+  std::printf("%s: %s\n", argv[1], fake::failed ? "failed" : "ok");
+  return fake::failed != 0;
+}

@@ -103,3 +103,20 @@ def test_tau_of_a_nonsymmetric_matrix(name, form):
     for k in (1, 2):
         for a, b in zip(out[0], out[k]):
             assert np.abs(a - b).max() <= tol * np.abs(a).max()
+
+
+@pytest.mark.parametrize("form,cache", [(ca.CHX_PREC_FP64, 1), (ca.CHX_PREC_FP64, 0), (ca.CHX_PREC_MIXED, -1)])
+def test_no_shell_alive(form, cache):
+    """A threshold above every value leaves empty lists: no electrons, no potential, zero derivatives."""
+    mol, _, D = _system("water sto-3g")
+    xc = ca.ExchangeCorrelation()
+    xc.Read("PBE")
+    g = _grid(mol, 1, form, cache, thr=1e6)
+    E, V = ca.xc_build(g, xc, D)
+    assert g.stats()["mean_tiles"] == 0 and E == 0 and not V.any() and g.getNumElectrons() == 0
+    if form == ca.CHX_PREC_FP64 and cache:
+        xc.Evaluate("f", g)
+        g.getDensitySkeleton([D])
+        assert not g.getEnergyGrad().any()
+        assert not any(F.any() for F in g.getFockSkeleton()[0])
+        assert not g.getEnergyHess().any()
