@@ -26,7 +26,9 @@ int chx_lebedev_rule_impl(int n, double* xyzw);
 namespace chx {
 
 void hip_check(hipError_t e, const char* what) {
-  if (e != hipSuccess) throw Error(CHX_ERR_DEVICE, std::string(what) + ": " + hipGetErrorString(e));
+  if (e == hipSuccess) return;
+  (void)hipGetLastError();  // reported here: not once more by the next launch's check
+  throw Error(CHX_ERR_DEVICE, std::string(what) + ": " + hipGetErrorString(e));
 }
 }  // namespace chx
 

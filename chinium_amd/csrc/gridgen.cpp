@@ -575,18 +575,21 @@ void build_cwork(chx_grid* g) {
   std::vector<RowRef> rows;
   std::vector<int> rowptr;
   build_mwork(g, sup, g->vxc_chunk > 0 ? g->vxc_chunk : default_len(g, sup, true), rows, rowptr);
+  if (mixed) {
+    g->d_U64.release();
+    g->d_U.alloc(std::max<size_t>(1, g->u_elems));
+  } else {
+    g->d_U.release();
+    g->d_U64.alloc(std::max<size_t>(1, g->u_elems));
+  }
   g->d_mwork.upload(g->mwork, st);
   g->d_rows.upload(rows, st);
   g->d_rowptr.upload(rowptr, st);
   g->pwork.clear();
   if (mixed) {
-    g->d_U64.release();
-    g->d_U.alloc(std::max<size_t>(1, g->u_elems));
     g->hmol.cwork = g->d_mwork.p;
     g->hmol.U = g->d_U.p;
   } else {
-    g->d_U.release();
-    g->d_U64.alloc(std::max<size_t>(1, g->u_elems));
     for (const MxItem& m : g->mwork) {
       g->pwork.push_back(m);
       if (m.I0 != m.J0) {
@@ -601,26 +604,59 @@ void build_cwork(chx_grid* g) {
   CHX_HIP(hipStreamSynchronize(st));
 }
 
-// Rebuilds the Vxc work items for another chunk length (autotuning) without
-// touching the AO tables.
-void set_vxc_chunk(chx_grid* g, int chunk) {
+// After a failure half way: no plan and nothing that was made with it, for this
+// grid's calls and for a pack that holds it.
+static void drop_plan(chx_grid* g) {
+  ++g->plan_gen;
+  g->ao_ready = g->have_density = g->have_eval = g->have_v = g->have_skeleton = g->slot_tables = false;
+  g->corr_pending = g->corr_done = g->vout_ready = false;
+  g->fx_family = -1;
+  g->nmats_u = 0;
+}
+
+// Mixed form: Vxc over groups of up to kMxWideTiles tiles. -1: from npad 1024 on.
+static int wide_groups(const chx_grid* g) {
+  return g->precision == CHX_PREC_MIXED && (g->vxc_shape == 1 || (g->vxc_shape < 0 && g->npad >= 1024)) ? 1 : 0;
+}
+
+// Rebuilds the Vxc work items for another run length or group size without touching
+// the AO tables. Where the new runs' blocks cannot be allocated the call fails and the
+// former ones, which fitted, are made again; should that fail too, the plan is dropped.
+static void rebuild_runs(chx_grid* g, int chunk, int shape) {
+  const int was_chunk = g->vxc_chunk, was_shape = g->vxc_shape;
   g->vxc_chunk = chunk;
+  g->vxc_shape = shape;
   if (!g->ao_ready || !g->cached) return;
   ++g->plan_gen;
-  build_cwork(g);
+  auto rebuild = [&] {
+    g->mx_wide = wide_groups(g);
+    build_cwork(g);
+  };
+  try {
+    rebuild();
+  } catch (...) {
+    g->vxc_chunk = was_chunk;
+    g->vxc_shape = was_shape;
+    try {
+      rebuild();
+    } catch (...) {
+      drop_plan(g);
+    }
+    throw;
+  }
 }
+
+void set_vxc_chunk(chx_grid* g, int chunk) { rebuild_runs(g, chunk, g->vxc_shape); }
 
 // Vxc block shape of the mixed form (-1: groups of up to 5 tiles from npad 1024
 // on, of up to 4 below; 0, 1: either), rebuilding the work items.
 void set_vxc_shape(chx_grid* g, int shape) {
-  g->vxc_shape = shape;
-  if (!g->ao_ready || g->precision != CHX_PREC_MIXED) return;
-  g->mx_wide = (shape == 1 || (shape < 0 && g->npad >= 1024)) ? 1 : 0;
-  set_vxc_chunk(g, g->vxc_chunk);
+  if (g->precision != CHX_PREC_MIXED) g->vxc_shape = shape;
+  else rebuild_runs(g, g->vxc_chunk, shape);
 }
 
 // Screening and work plans (Grid::getAO counterpart).
-void grid_plan(chx_grid* g) {
+static void make_plan(chx_grid* g) {
   hipStream_t st = g->stream;
   g->d_ws.release();
   const int nb = g->nbatches, nsh = (int)g->sh_type.size(), nwords = (nsh + 63) / 64;
@@ -735,7 +771,7 @@ void grid_plan(chx_grid* g) {
                                     " GB of device memory for its AO cache");
   g->cached = mixed || g->cache_mode == 1 || (g->cache_mode == -1 && cache_bytes < 0.8 * (double)free_b);
   // large bases: Vxc items over groups of up to 5 tiles
-  g->mx_wide = mixed && (g->vxc_shape == 1 || (g->vxc_shape < 0 && g->npad >= 1024)) ? 1 : 0;
+  g->mx_wide = wide_groups(g);
   g->vwork.clear();
   g->mwork.clear();
   if (g->cached) g->d_Mint.release();
@@ -864,6 +900,15 @@ void grid_plan(chx_grid* g) {
   g->have_density = g->have_eval = g->have_v = g->have_skeleton = false;
   g->corr_pending = g->corr_done = g->vout_ready = false;
   g->slot_tables = false;
+}
+
+void grid_plan(chx_grid* g) {
+  try {
+    make_plan(g);
+  } catch (...) {
+    drop_plan(g);
+    throw;
+  }
 }
 
 }  // namespace chx

@@ -51,7 +51,7 @@ hipError_t hipFree(void* p) {
   return hipSuccess;
 }
 hipError_t hipMemGetInfo(size_t* f, size_t* t) {
-  *f = fake::budget - fake::used;
+  *f = fake::budget > fake::used ? fake::budget - fake::used : 0;
   *t = fake::budget;
   return hipSuccess;
 }
@@ -130,6 +130,15 @@ void launch_functional(hipStream_t, int, const int* off, const double*, const do
                        int, int, int, double*, double*, double*, int) { CHECK(at(off)); launched(); }
 void launch_functional_f(hipStream_t, int, const int*, const double*, const int*, int, int, double*) { launched(); }
 void launch_reduce_en(hipStream_t, int, const double*, double* en) { CHECK(at(en)); launched(); }
+void launch_split_d(hipStream_t, int, int, const double*, const int*, const ChunkDev*, const int*, unsigned short* Ds,
+                    float* R, int*, int) { CHECK(at(Ds) && at(R)); launched(); }
+void launch_density_mx(hipStream_t, int, int, int, const MolDev& m) { CHECK(at(m.part)); launched(); }
+void launch_make_b_mx(hipStream_t, int, const MolDev& m) { CHECK(at(m.bt)); launched(); }
+void launch_vxc_mx(hipStream_t, int, int, int nitems, const MolDev& m) {
+  for (int k = 0; k < nitems; ++k) CHECK(at(m.cwork + k, sizeof(MxItem)) && at(m.U + m.cwork[k].u));
+  launched();
+}
+void launch_reduce_corr(hipStream_t, int, const double*, double* out) { CHECK(at(out)); launched(); }
 void launch_make_b(hipStream_t, int, const int*, const double*, const double*, double* b, int, size_t, size_t,
                    const double*) { CHECK(at(b)); launched(); }
 void launch_vxc_c64(hipStream_t, int, int nwork, const MxItem*, const double*, const double*, const double*, double* U,
@@ -219,10 +228,64 @@ void empty_lists() {
   chx_xc_destroy(xc);
   chx_grid_destroy(g);
 }
+
+int build(chx_grid* g, const chx_xc* xc, const std::vector<double>& D, std::vector<double>& F) {
+  int rc = chx_grid_get_density(g, D.data(), 1, g->nbasis);
+  if (rc == CHX_OK) rc = chx_xc_evaluate(xc, g, "ev");
+  if (rc == CHX_OK) rc = chx_grid_fock(g, F.data(), 1, g->nbasis);
+  return rc;
+}
+
+// Run lengths and plans that do not fit: the call fails, and what was there before stays usable or is
+// known to be gone (no call reaches a freed table).
+void failed_plans() {
+  const size_t all = fake::budget;
+  for (int form : {CHX_PREC_FP64, CHX_PREC_MIXED}) {
+    chx_grid* g = grid(1, 300);
+    chx_xc* xc = functional(1);
+    const int n = g->nbasis;
+    std::vector<double> D((size_t)n * n, 0.1), F((size_t)n * n);
+    CHECK(chx_grid_set_precision(g, form) == CHX_OK && chx_grid_get_ao(g, 0, 0) == CHX_OK && g->cached);
+    CHECK(chx_grid_set_vxc_chunk(g, 4) == CHX_OK);
+    CHECK(build(g, xc, D, F) == CHX_OK);
+    const size_t u = g->u_elems, per = form == CHX_PREC_FP64 ? sizeof(double) : sizeof(float);
+    // shorter runs: more blocks than there is room for
+    fake::budget = fake::used + u * per;
+    const unsigned long gen = g->plan_gen;
+    CHECK(chx_grid_set_vxc_chunk(g, 1) == CHX_ERR_DEVICE);
+    CHECK(g->ao_ready && g->plan_gen != gen && g->vxc_chunk == 4 && g->u_elems == u);
+    CHECK(fake::at(form == CHX_PREC_FP64 ? (void*)g->d_U64.p : (void*)g->d_U.p, u * per));
+    if (form == CHX_PREC_MIXED) CHECK(g->hmol.U == g->d_U.p && g->hmol.cwork == g->d_mwork.p);
+    CHECK(chx_grid_fock(g, F.data(), 1, n) == CHX_OK && build(g, xc, D, F) == CHX_OK);
+    // no room for any: the plan is gone, and getAO makes another of it
+    fake::budget = 0;
+    CHECK(chx_grid_set_vxc_chunk(g, 1) == CHX_ERR_DEVICE);
+    CHECK(!g->ao_ready && g->vxc_chunk == 4);
+    CHECK(chx_grid_fock(g, F.data(), 1, n) == CHX_ERR_STATE && build(g, xc, D, F) == CHX_ERR_STATE);
+    fake::budget = all;
+    CHECK(chx_grid_get_ao(g, 0, 0) == CHX_OK && build(g, xc, D, F) == CHX_OK && g->u_elems == u);
+    // a plan that fails half way
+    CHECK(chx_grid_set_type(g, 2) == CHX_OK);
+    fake::budget = fake::used;
+    CHECK(chx_grid_get_ao(g, 0, 0) != CHX_OK);
+    CHECK(chx_grid_fock(g, F.data(), 1, n) == CHX_ERR_STATE && build(g, xc, D, F) == CHX_ERR_STATE);
+    fake::budget = all;
+    CHECK(chx_grid_get_ao(g, 0, 0) == CHX_OK && build(g, xc, D, F) == CHX_OK);
+    if (form == CHX_PREC_MIXED) {  // the other group size
+      CHECK(chx_grid_set_vxc_shape(g, 0) == CHX_OK && chx_grid_set_vxc_chunk(g, 1) == CHX_OK);
+      fake::budget = 0;
+      CHECK(chx_grid_set_vxc_shape(g, 1) == CHX_ERR_DEVICE || g->d_U.p);
+      CHECK(chx_grid_fock(g, F.data(), 1, n) == (g->ao_ready ? CHX_OK : CHX_ERR_STATE));
+      fake::budget = all;
+    }
+    chx_xc_destroy(xc);
+    chx_grid_destroy(g);
+  }
+}
 }  // namespace
 
 int main(int argc, char** argv) {
-  const std::map<std::string, void (*)()> checks = {{"empty_lists", empty_lists}};
+  const std::map<std::string, void (*)()> checks = {{"empty_lists", empty_lists}, {"failed_plans", failed_plans}};
   if (argc != 3 || !checks.count(argv[1])) return 2;
   root = argv[2];
   checks.at(argv[1])();
