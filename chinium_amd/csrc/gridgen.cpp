@@ -376,7 +376,8 @@ void grid_build(chx_grid* g, const std::string& grid_name, const std::string& da
 // (the components' angular parts are at most 1 and their derivatives at most l
 // on the unit sphere). Every term falls beyond sqrt((l + 1) / (2 a_min)), so
 // the last crossing is bisected there, or searched below when the threshold is
-// that coarse. A zero threshold keeps a shell until its exponentials underflow.
+// that coarse. A zero threshold keeps a shell until its exponentials underflow; a
+// shell with an exponent that does not decay is kept everywhere.
 static double shell_reach(int type, int np, const double* e, const double* c, double thr) {
   const int l = std::abs(type);
   auto bound = [&](double r) {
@@ -391,6 +392,7 @@ static double shell_reach(int type, int np, const double* e, const double* c, do
   };
   double amin = e[0];
   for (int p = 1; p < np; ++p) amin = std::min(amin, e[p]);
+  if (!(amin > 0)) return HUGE_VAL;
   double lo = std::sqrt((l + 1) / (2 * amin)), hi = lo + std::sqrt(800 / amin);
   if (bound(lo) > thr) {
     for (int k = 0; k < 100; ++k) {

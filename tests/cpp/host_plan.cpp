@@ -3,10 +3,13 @@
 // when memory runs out can be looked at without a GPU. Device memory is host memory under a byte budget;
 // a launch checks that the tables it would read are there and returns.
 //   host_plan <check> <data root>; exit status 0 when it holds.
+#include <algorithm>
+#include <cmath>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
 #include <map>
+#include <random>
 #include <string>
 #include <vector>
 
@@ -282,10 +285,70 @@ void failed_plans() {
     chx_grid_destroy(g);
   }
 }
+
+// A shell is in the list of every batch in which one of its components or their derivatives exceeds the
+// threshold: contractions of steep and diffuse primitives of either sign, coarse thresholds, exponents of 0.
+void reaches() {
+  std::mt19937 rng(3);
+  auto uni = [&](double a, double b) { return a + (b - a) * (rng() / 4294967296.0); };
+  for (int trial = 0; trial < 60; ++trial) {
+    chx_mol* m;
+    chx_grid* g;
+    const int Z = 1;
+    const double at[3] = {0, 0, 0};
+    CHECK(chx_mol_create(1, &Z, at, &m) == CHX_OK);
+    static const int types[] = {0, 1, -2, -3};
+    std::vector<std::vector<double>> e, c;
+    for (int k = 0; k < 12; ++k) {
+      const int np = 1 + rng() % 4;
+      std::vector<double> ee, cc;
+      for (int p = 0; p < np; ++p) {
+        ee.push_back(trial % 6 == 5 && p == 0 ? (k % 2 ? 0.0 : -1e-4) : std::pow(10.0, uni(-2, 6)));
+        cc.push_back(uni(-1, 1) * std::pow(10.0, uni(-2, 2)));
+      }
+      CHECK(chx_mol_add_shell(m, 0, types[k % 4], np, ee.data(), cc.data()) == CHX_OK);
+      e.push_back(ee);
+      c.push_back(cc);
+    }
+    CHECK(chx_grid_create(m, "SG-1", root.c_str(), 1, 0, &g) == CHX_OK);
+    for (double thr : {0.0, 1e-14, 1e-6, 1e-3, 0.1, 1.0, 30.0}) {
+      CHECK(chx_grid_set_screening(g, thr) == CHX_OK && chx_grid_get_ao(g, 0, 0) == CHX_OK);
+      int missing = 0;
+      for (int k = 0; k < 12; ++k)
+        for (int b = 0; b < g->nbatches; ++b) {
+          const chx::ChunkDev& ch = g->chunks[g->b_chunk[b]];
+          bool listed = false;
+          for (int i = 0; i < ch.ntl * chx::kTile; ++i) listed |= g->ao_of[ch.tile0 * chx::kTile + i] == g->sh_ao[k];
+          if (listed) continue;
+          for (int i = 0; i < g->batch_n[b]; ++i) {
+            const double x = g->hx[b * chx::kBatch + i], y = g->hy[b * chx::kBatch + i], z = g->hz[b * chx::kBatch + i];
+            double A = 0, A1 = 0;
+            for (size_t p = 0; p < e[k].size(); ++p) {
+              const double t = c[k][p] * std::exp(-e[k][p] * (x * x + y * y + z * z));
+              A += t;
+              A1 -= 2 * e[k][p] * t;
+            }
+            // one component of the type and its gradient
+            const double q[4] = {1, x, std::sqrt(3.0) * x * y, z * (z * z - 1.5 * (x * x + y * y))};
+            const double dx[4] = {0, 1, std::sqrt(3.0) * y, -3 * x * z}, dz[4] = {0, 0, 0, 3 * z * z - 1.5 * (x * x + y * y)};
+            const int t = k % 4;
+            const double v = std::max({std::fabs(A * q[t]), std::fabs(A1 * x * q[t] + A * dx[t]),
+                                       std::fabs(A1 * z * q[t] + A * dz[t])});
+            missing += v > thr * (1 + 1e-12);
+          }
+        }
+      if (missing) std::printf("trial %d threshold %g: %d values above it left out\n", trial, thr, missing);
+      CHECK(missing == 0);
+    }
+    chx_grid_destroy(g);
+    chx_mol_destroy(m);
+  }
+}
 }  // namespace
 
 int main(int argc, char** argv) {
-  const std::map<std::string, void (*)()> checks = {{"empty_lists", empty_lists}, {"failed_plans", failed_plans}};
+  const std::map<std::string, void (*)()> checks = {
+      {"empty_lists", empty_lists}, {"failed_plans", failed_plans}, {"reaches", reaches}};
   if (argc != 3 || !checks.count(argv[1])) return 2;
   root = argv[2];
   checks.at(argv[1])();
