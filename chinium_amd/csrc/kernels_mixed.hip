@@ -252,7 +252,8 @@ __device__ __forceinline__ double block_sum_d(double v) {
 // and V[nu][mu] (reference order), and with R the partial sum of V . R over them.
 // 16 waves; a run's row is contiguous in U, kAsmUnroll rows are in flight per
 // wave. Up to kAsmLds / 16 = 512 AOs each wave has a copy of the sums (COPIES =
-// 16), so that a plain LDS read-add-write does; larger rows share one (COPIES = 1)
+// 16), so that a plain LDS read-add-write does, its rows ordered by wave-scope
+// fences (which cost no instruction); larger rows share one (COPIES = 1)
 // through ds_add_f64, which is the bound there, some 130 cycles per wave: fewer
 // waves with copies are slower still. (H2O)16: 48 us against 86 shared; (H2O)48:
 // 250 us shared against 363 with 4 waves; (H2O)128 700 us against 1430 with 2.
@@ -296,7 +297,8 @@ __global__ __launch_bounds__(kAsmThreads) void k_assemble(int n, const int* __re
       if (e + q >= e1) r[q].len = 0;
       len = max(len, r[q].len);
     }
-    for (int k = lane; k < len; k += 64) {
+    for (int k0 = 0; k0 < len; k0 += 64) {  // every lane to the end: the fences below are for the whole wave
+      const int k = k0 + lane;
       int nu[kAsmUnroll];
       T v[kAsmUnroll];
 #pragma unroll
@@ -307,13 +309,18 @@ __global__ __launch_bounds__(kAsmThreads) void k_assemble(int n, const int* __re
         if (k >= r[q].len) nu[q] = -1;
       }
 #pragma unroll
-      for (int q = 0; q < kAsmUnroll; ++q)
+      for (int q = 0; q < kAsmUnroll; ++q) {
         if (nu[q] >= 0 && nu[q] < w) {
           if (COPIES == 1)
             __hip_atomic_fetch_add(&sum[nu[q]], (double)v[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
           else
             sum[nu[q]] += (double)v[q];
         }
+        if (COPIES > 1) {  // a row's columns differ, two rows' may not: one row's sums before the next one's
+          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+          __builtin_amdgcn_wave_barrier();
+        }
+      }
     }
   }
   __syncthreads();
