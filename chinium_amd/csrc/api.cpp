@@ -253,7 +253,7 @@ void fock_to_device(chx_grid* g, double* dV, int spin = 0) {
     g->mark_begin(kStFinalize, &e);
     launch_assemble<float>(g->stream, g->nbasis, g->d_rowptr.p, g->d_rows.p, g->d_ao_of.p, g->d_U.p, dV,
                        g->corr_pending ? g->d_Dres.p + (size_t)spin * g->nbasis * g->nbasis : nullptr,
-                       g->d_cpart.p + (size_t)spin * assemble_blocks(g->nbasis));
+                       g->d_cpart.p + (size_t)spin * assemble_blocks(g->nbasis), 1, g->u_elems);
     g->mark_end(kStFinalize, e);
     return;
   }
@@ -268,7 +268,7 @@ void fock_to_device(chx_grid* g, double* dV, int spin = 0) {
     g->mark_end(kStVxc, e);
     g->mark_begin(kStFinalize, &e);
     launch_assemble<double>(g->stream, g->nbasis, g->d_rowptr.p, g->d_rows.p, g->d_ao_of.p, g->d_U64.p, dV, nullptr,
-                            nullptr);
+                            nullptr, 1, 0);
     g->mark_end(kStFinalize, e);
     return;
   }

@@ -507,9 +507,12 @@ static void build_items(const chx_grid* g, int sup, bool upper, int len, std::ve
 // item is a serial chain of its run's K steps, which shows unless several times
 // more items than the chip holds are there. An FP64 step is some ten times as
 // long, so runs past 4 batches do not pay there. Times by run length, in us, Vxc
-// launch and V's assembly: (H2O)16 / def2-SVP / SG-1 mixed 82 + 90 (4), 84 + 40
-// (8), 173 + 20 (32); (H2O)4 14 + 25 (2), 16 + 15 (4), 69 + 10 (32); (H2O)128
-// 2640 + 1300 (8), 2280 + 700 (32). Builds in FP64: (H2O)16 1140 (1), 977 (4),
+// launch and V's assembly, mixed form, GGA, def2-SVP: (H2O)16 / SG-2 197 + 101 (4),
+// 189 + 57 (8), 210 + 38 (16), 261 + 29 (32); (H2O)4 / SG-1 15 + 15 (2), 17 + 12 (4),
+// 71 + 9 (32); (H2O)128 / SG-2 3578 + 1549 (8), 3508 + 1012 (16), 3548 + 774 (32).
+// A meta-GGA step is four times as long and would take shorter runs in the largest
+// systems: (H2O)48 / SG-2 r2SCAN 2951 + 587 (4), 3214 + 330 (8), 3689 + 201 (the rule).
+// Builds in FP64: (H2O)16 1140 (1), 977 (4),
 // 1141 (16); C18 / def2-TZVP r2SCAN 2317 (1), 2298 (4), 2665 (16); H2O 97 (1), 105 (4).
 static int default_len(const chx_grid* g, int sup, bool upper) {
   const bool mixed = g->precision == CHX_PREC_MIXED;
@@ -579,7 +582,7 @@ void build_cwork(chx_grid* g) {
   build_mwork(g, sup, g->vxc_chunk > 0 ? g->vxc_chunk : default_len(g, sup, true), rows, rowptr);
   if (mixed) {
     g->d_U64.release();
-    g->d_U.alloc(std::max<size_t>(1, g->u_elems));
+    g->d_U.alloc(std::max<size_t>(1, 2 * g->u_elems));
   } else {
     g->d_U.release();
     g->d_U64.alloc(std::max<size_t>(1, g->u_elems));
@@ -591,6 +594,7 @@ void build_cwork(chx_grid* g) {
   if (mixed) {
     g->hmol.cwork = g->d_mwork.p;
     g->hmol.U = g->d_U.p;
+    g->hmol.uplane = (long)g->u_elems;
   } else {
     for (const MxItem& m : g->mwork) {
       g->pwork.push_back(m);

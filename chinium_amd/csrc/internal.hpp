@@ -315,7 +315,8 @@ struct MolDev {
   const double* coef;           // Vxc integrand coefficients per point
   unsigned short* bt;           // B^T per slot
   const MxItem* cwork;          // Vxc work items
-  float* U;                     // the runs' blocks of V (upper)
+  float* U;                     // the runs' blocks of V (upper): Phi_I^T B_J, and uplane on, B_I^T Phi_J
+  long uplane;
   // core batches (points within the core radius of a nucleus with Z > 2): their
   // density runs with the AO operands split in three bf16 terms; cache3 holds
   // the third term of their slots' AOg blocks [core slot][c][g][mu],
@@ -377,13 +378,14 @@ void launch_ao_cache_mx(hipStream_t s, int nslots, const int* slot_batch, const 
 // not symmetric to within rounding
 void launch_split_d(hipStream_t s, int ntiles, int n, const double* D, const int* tile_chunk, const ChunkDev* chunks,
                     const int* ao_of, unsigned short* Ds, float* R, int* asym, int gen);
-// V (reference order) from the runs' blocks U and, with R, the first-order energy
+// V (reference order) from the runs' blocks U (float: the two products, sU elements
+// apart; double: their sum, nmat matrices sU elements apart) and, with R, the first-order energy
 // correction for the split of D: partial sums of V . R into cpart
 // (assemble_blocks(n) of them); launch_reduce_corr sums nparts partials into *out.
 int assemble_blocks(int n);
 template <class T>  // float (mixed form) or double
 void launch_assemble(hipStream_t s, int n, const int* rowptr, const RowRef* rows, const int* ao_of, const T* U,
-                     double* V, const float* R, double* cpart, int nmat = 1, size_t sU = 0);
+                     double* V, const float* R, double* cpart, int nmat, size_t sU);
 void launch_reduce_corr(hipStream_t s, int nparts, const double* cpart, double* out);
 // the packed form: per molecule of the table, en[2 slot_en] += its ncpart partials
 void launch_corr_multi(hipStream_t s, const char* base, const FnMolecule* fm, int nmol, double* en);
@@ -488,7 +490,7 @@ struct chx_grid {
   int mx_wide = 0;                   // mixed form: Vxc over groups of up to 5 tiles (large bases)
   std::vector<chx::MxItem> mwork;       // Vxc work items of the cached tables
   std::vector<chx::MxItem> pwork;       // FP64 form: items of the plain products (skeleton derivatives)
-  size_t u_elems = 0;                   // elements of the runs' blocks of V
+  size_t u_elems = 0;                   // elements of the runs' blocks of V (mixed form: of either product's)
   // mixed form: core batches (density with three-term operands)
   double core_radius = chx::kCoreRadius;  // bohr; 0 turns the core treatment off
   int ncore_batches = 0;

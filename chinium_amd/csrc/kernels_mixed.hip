@@ -255,8 +255,11 @@ __device__ __forceinline__ double block_sum_d(double v) {
 // 16), so that a plain LDS read-add-write does, its rows ordered by wave-scope
 // fences (which cost no instruction); larger rows share one (COPIES = 1)
 // through ds_add_f64, which is the bound there, some 130 cycles per wave: fewer
-// waves with copies are slower still. (H2O)16: 48 us against 86 shared; (H2O)48:
-// 250 us shared against 363 with 4 waves; (H2O)128 700 us against 1430 with 2.
+// waves with copies are slower still. With one FP32 block per run: (H2O)16 48 us
+// against 86 shared; (H2O)48 250 us shared against 363 with 4 waves; (H2O)128 700 us
+// against 1430 with 2. With both products of a run, added here in FP64 (def2-SVP /
+// SG-2): (H2O)16 57 us (48 with one FP32 sum), (H2O)48 157 to 201 (157 to 163),
+// (H2O)128 0.79 ms (0.62).
 // The FP64 atomics to HBM that all this replaces, one per element of M and run
 // at about 40 G/s, took most of the Vxc launch. kAsmLds sums per block: larger
 // bases take several column ranges (grid y).
@@ -275,7 +278,8 @@ __global__ __launch_bounds__(kAsmThreads) void k_assemble(int n, const int* __re
                                                              const float* __restrict__ R,
                                                              double* __restrict__ cpart, size_t sU) {
   extern __shared__ double asum[];
-  U += blockIdx.z * sU;  // the matrix of the launch
+  constexpr bool kTwo = sizeof(T) == 4;  // both products in FP32, the second sU elements on
+  if (!kTwo) U += blockIdx.z * sU;       // the matrix of the launch
   V += (size_t)blockIdx.z * n * n;
   constexpr int kCols = kAsmLds / COPIES, kWaves = kAsmThreads / 64;
   const int mu = blockIdx.x, c0 = blockIdx.y * kCols, w = min(kCols, n - c0), tid = threadIdx.x;
@@ -300,21 +304,23 @@ __global__ __launch_bounds__(kAsmThreads) void k_assemble(int n, const int* __re
     for (int k0 = 0; k0 < len; k0 += 64) {  // every lane to the end: the fences below are for the whole wave
       const int k = k0 + lane;
       int nu[kAsmUnroll];
-      T v[kAsmUnroll];
+      T v[kAsmUnroll], v2[kAsmUnroll];
 #pragma unroll
       for (int q = 0; q < kAsmUnroll; ++q) {  // clamped, not skipped: the loads go out together
         const int kk = min(k, max(r[q].len - 1, 0));
         nu[q] = ao_of[r[q].a0 + kk] - c0;
         v[q] = U[r[q].u + kk];
+        if (kTwo) v2[q] = U[sU + r[q].u + kk];
         if (k >= r[q].len) nu[q] = -1;
       }
 #pragma unroll
       for (int q = 0; q < kAsmUnroll; ++q) {
+        const double x = kTwo ? (double)v[q] + (double)v2[q] : (double)v[q];
         if (nu[q] >= 0 && nu[q] < w) {
           if (COPIES == 1)
-            __hip_atomic_fetch_add(&sum[nu[q]], (double)v[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            __hip_atomic_fetch_add(&sum[nu[q]], x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
           else
-            sum[nu[q]] += (double)v[q];
+            sum[nu[q]] += x;
         }
         if (COPIES > 1) {  // a row's columns differ, two rows' may not: one row's sums before the next one's
           __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
@@ -1017,11 +1023,12 @@ void launch_make_b_mx(hipStream_t s, int ncomp, const MolDev& one) {
 // Vxc: one block of one run's V, U_IJ = sum_g Phi_I^T B_J + B_I^T Phi_J over
 // the run's batches, for groups I <= J of at most MT of the chunk's tiles (the
 // groups of a list are equal to within a tile, so no block is mostly padding).
-// For I < J both products go into the same accumulators (second pass: the
-// operands swap roles), so only the upper blocks are formed; for I = J one
-// product M is formed and U = M + M^T through LDS at the end. The tau part
-// (NC = 4) is symmetric, M_tau = sum_r (d_r Phi)^T (t d_r Phi): its steps run
-// first and once, doubled for I < J.
+// Only the upper blocks are formed. For I < J the two products follow each other
+// (second pass: the operands swap roles); for I = J there is one product M, and M^T
+// comes from it through LDS at the end. Both go to U as they are, in FP32 like the
+// accumulators, and k_assemble adds them in FP64. The tau part (NC = 4) is symmetric,
+// M_tau = sum_r (d_r Phi)^T (t d_r Phi): its steps run first and once, doubled for
+// I < J.
 // A K step is 32 points of one component: the row group's and the column
 // group's operands, hi and lo, fragments of 1 KB (16 rows of 64 bytes) that the
 // waves' DMA loads bring straight into LDS, coalesced and swizzled as in the
@@ -1031,9 +1038,12 @@ void launch_make_b_mx(hipStream_t s, int ncomp, const MolDev& one) {
 // in a 2 x 2 grid, each owning half of the row and of the column blocks (up to
 // MT x MT fragments of 16 x 16; MT = 5 is the largest whose two buffers leave
 // room for two blocks per CU).
-// The result is stored once per run, in FP32 like the accumulators (row-major,
-// the row panel of group I from column I0 on), and summed in FP64 by
-// k_assemble.
+// Either product is stored once per run, row-major, the row panel of group I from
+// column I0 on, the second one uplane elements after the first. One accumulator for
+// both and one store, which adds them in FP32, took (H2O)16 / def2-SVP / SG-2 from
+// 190 to 175 us and (H2O)128 from 3.6 to 3.5 ms: their bytes. A second set of
+// accumulators, their FP64 sum stored at the end, is as slow (188 us; with MT = 5 it
+// does not fit the registers).
 template <int MT>
 struct VxcMxSmem {
   u32x4 F[2][8 * MT * kDxFrag];  // step k in buffer k & 1: row group's fragments, then the column group's
@@ -1088,42 +1098,44 @@ __device__ __forceinline__ void vxc_mx_body(const MolDev& m, int item) {
     }
   };
   f32x4 acc[MT][MT];
-#pragma unroll
-  for (int r = 0; r < MT; ++r)
-#pragma unroll
-    for (int c = 0; c < MT; ++c) acc[r][c] = f32x4{0.f, 0.f, 0.f, 0.f};
-  dma(0, 0);
-  for (int k = 0; k < nstage; ++k) {
-    if (NC == 4 && k == ntau && !diag) {  // 2 M_tau
-#pragma unroll
-      for (int r = 0; r < MT; ++r)
-#pragma unroll
-        for (int c = 0; c < MT; ++c) acc[r][c] *= 2.f;
-    }
-    __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this wave's fragments of step k are in LDS
-    __syncthreads();                     // ... and every other wave's, and step k - 1's buffer is read
-    if (k + 1 < nstage) dma(k + 1, (k + 1) & 1);
-    const u32x4* F = sm.F[k & 1];
-    u32x4 a[MT][2];
-#pragma unroll
-    for (int r = 0; r < MT; ++r)
-      if (r < nI) {
-#pragma unroll
-        for (int hh = 0; hh < 2; ++hh) a[r][hh] = F[((r0 + r) * 2 + hh) * kDxFrag + fidx];
-      }
-#pragma unroll
-    for (int c = 0; c < MT; ++c)
-      if (c < nc) {
-        const u32x4* Fc = F + (2 * RB + (c0 + c) * 2) * kDxFrag + fidx;
-        const u32x4 bh = Fc[0], bl = Fc[kDxFrag];
-#pragma unroll
-        for (int r = 0; r < MT; ++r)
-          if (r < nI) acc[r][c] = mfma3(a[r][0], a[r][1], bh, bl, acc[r][c]);
-      }
-  }
   float* __restrict__ U = m.U + wk.u;
   const int ld = wk.ldu;
-  if (!diag) {
+  dma(0, 0);
+  for (int pass = 0, k = 0; k < nstage; ++pass) {  // the products of the run, one after the other
+    const int kend = pass == 0 ? kswap : nstage;
+#pragma unroll
+    for (int r = 0; r < MT; ++r)
+#pragma unroll
+      for (int c = 0; c < MT; ++c) acc[r][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (; k < kend; ++k) {
+      if (NC == 4 && k == ntau && !diag) {  // 2 M_tau
+#pragma unroll
+        for (int r = 0; r < MT; ++r)
+#pragma unroll
+          for (int c = 0; c < MT; ++c) acc[r][c] *= 2.f;
+      }
+      __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this wave's fragments of step k are in LDS
+      __syncthreads();                     // ... and every other wave's, and step k - 1's buffer is read
+      if (k + 1 < nstage) dma(k + 1, (k + 1) & 1);
+      const u32x4* F = sm.F[k & 1];
+      u32x4 a[MT][2];
+#pragma unroll
+      for (int r = 0; r < MT; ++r)
+        if (r < nI) {
+#pragma unroll
+          for (int hh = 0; hh < 2; ++hh) a[r][hh] = F[((r0 + r) * 2 + hh) * kDxFrag + fidx];
+        }
+#pragma unroll
+      for (int c = 0; c < MT; ++c)
+        if (c < nc) {
+          const u32x4* Fc = F + (2 * RB + (c0 + c) * 2) * kDxFrag + fidx;
+          const u32x4 bh = Fc[0], bl = Fc[kDxFrag];
+#pragma unroll
+          for (int r = 0; r < MT; ++r)
+            if (r < nI) acc[r][c] = mfma3(a[r][0], a[r][1], bh, bl, acc[r][c]);
+        }
+    }
+    float* __restrict__ out = U + pass * m.uplane + (size_t)(16 * r0 + 4 * lk) * ld + 16 * c0 + lrow;
 #pragma unroll
     for (int r = 0; r < MT; ++r)
       if (r < nI) {
@@ -1131,15 +1143,15 @@ __device__ __forceinline__ void vxc_mx_body(const MolDev& m, int item) {
         for (int c = 0; c < MT; ++c)
           if (c < nc) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-              U[(size_t)(16 * (r0 + r) + 4 * lk + i) * ld + 16 * (c0 + c) + lrow] = acc[r][c][i];
+            for (int i = 0; i < 4; ++i) out[(size_t)(16 * r + i) * ld + 16 * c] = acc[r][c][i];
           }
       }
-    return;
   }
-  // U = M + M^T, 64 rows at a time: the strip's 64 columns of M go to LDS transposed
+  if (!diag) return;
+  // M^T, 64 rows at a time: the strip's 64 columns of M go to LDS transposed
   float* T = reinterpret_cast<float*>(&sm.F[0][0]);
   static_assert(sizeof(float) * 64 * PT <= sizeof(sm), "a strip fits the fragment buffers");
+  const int n = 16 * CB;
   for (int s = 0; s < CB; s += 4) {
     __syncthreads();
 #pragma unroll
@@ -1151,19 +1163,12 @@ __device__ __forceinline__ void vxc_mx_body(const MolDev& m, int item) {
             *reinterpret_cast<f32x4*>(T + (16 * (c0 + c - s) + lrow) * PT + 16 * (r0 + r) + 4 * lk) = acc[r][c];
       }
     __syncthreads();
-#pragma unroll
-    for (int r = 0; r < MT; ++r)
-      if (r < nI && r0 + r >= s && r0 + r < s + 4) {
-#pragma unroll
-        for (int c = 0; c < MT; ++c)
-          if (c < nc) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              const int row = 16 * (r0 + r) + 4 * lk + i, col = 16 * (c0 + c) + lrow;
-              U[(size_t)row * ld + col] = acc[r][c][i] + T[(row - 16 * s) * PT + col];
-            }
-          }
-      }
+    float* __restrict__ out = U + m.uplane + (size_t)(16 * s) * ld;
+    const int rows = min(64, n - 16 * s);
+    for (int e = tid; e < rows * (n / 4); e += 256) {
+      const int row = e / (n / 4), col = e % (n / 4) * 4;
+      *reinterpret_cast<f32x4*>(out + (size_t)row * ld + col) = *reinterpret_cast<const f32x4*>(T + row * PT + col);
+    }
   }
 }
 template <int NC, int MT>

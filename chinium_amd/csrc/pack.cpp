@@ -291,7 +291,8 @@ void build_lanes(chx_pack* p) {
 bool stages_ok(const chx_pack* p) { return p->type <= 1 && p->family <= 1; }
 
 void assemble(hipStream_t s, const chx_grid* g, double* V) {
-  launch_assemble<float>(s, g->nbasis, g->d_rowptr.p, g->d_rows.p, g->d_ao_of.p, g->d_U.p, V, g->d_Dres.p, g->d_cpart.p);
+  launch_assemble<float>(s, g->nbasis, g->d_rowptr.p, g->d_rows.p, g->d_ao_of.p, g->d_U.p, V, g->d_Dres.p, g->d_cpart.p,
+                         1, g->u_elems);
 }
 
 // Form 2: the lane's molecules in one launch per stage (the persistent stage

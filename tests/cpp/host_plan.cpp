@@ -138,7 +138,7 @@ void launch_split_d(hipStream_t, int, int, const double*, const int*, const Chun
 void launch_density_mx(hipStream_t, int, int, int, const MolDev& m) { CHECK(at(m.part)); launched(); }
 void launch_make_b_mx(hipStream_t, int, const MolDev& m) { CHECK(at(m.bt)); launched(); }
 void launch_vxc_mx(hipStream_t, int, int, int nitems, const MolDev& m) {
-  for (int k = 0; k < nitems; ++k) CHECK(at(m.cwork + k, sizeof(MxItem)) && at(m.U + m.cwork[k].u));
+  for (int k = 0; k < nitems; ++k) CHECK(at(m.cwork + k, sizeof(MxItem)) && at(m.U + m.cwork[k].u) && at(m.U + m.uplane + m.cwork[k].u));
   launched();
 }
 void launch_reduce_corr(hipStream_t, int, const double*, double* out) { CHECK(at(out)); launched(); }
@@ -149,9 +149,10 @@ void launch_vxc_c64(hipStream_t, int, int nwork, const MxItem*, const double*, c
 int assemble_blocks(int n) { return n; }
 template <class T>
 void launch_assemble(hipStream_t, int n, const int* rowptr, const RowRef* rows, const int*, const T* U, double* V,
-                     const float*, double*, int, size_t) {
+                     const float*, double*, int nmat, size_t sU) {
+  const size_t last = sizeof(T) == 4 ? sU : (nmat - 1) * sU;
   CHECK(at(rowptr, 4 * (n + 1)) && at(V, sizeof(double) * n * n));
-  for (int e = 0; e < rowptr[n]; ++e) CHECK(at(U + rows[e].u, sizeof(T) * rows[e].len));
+  for (int e = 0; e < rowptr[n]; ++e) CHECK(at(U + rows[e].u, sizeof(T) * rows[e].len) && at(U + last + rows[e].u, sizeof(T) * rows[e].len));
   launched();
 }
 template void launch_assemble<float>(hipStream_t, int, const int*, const RowRef*, const int*, const float*, double*,
@@ -251,7 +252,7 @@ void failed_plans() {
     CHECK(chx_grid_set_precision(g, form) == CHX_OK && chx_grid_get_ao(g, 0, 0) == CHX_OK && g->cached);
     CHECK(chx_grid_set_vxc_chunk(g, 4) == CHX_OK);
     CHECK(build(g, xc, D, F) == CHX_OK);
-    const size_t u = g->u_elems, per = form == CHX_PREC_FP64 ? sizeof(double) : sizeof(float);
+    const size_t u = g->u_elems, per = 8;  // (mixed form: two FP32 products)
     // shorter runs: more blocks than there is room for
     fake::budget = fake::used + u * per;
     const unsigned long gen = g->plan_gen;

@@ -120,3 +120,26 @@ def test_no_shell_alive(form, cache):
         assert not g.getEnergyGrad().any()
         assert not any(F.any() for F in g.getFockSkeleton()[0])
         assert not g.getEnergyHess().any()
+
+
+def _constants(nsh, type_=0):
+    """One hydrogen with nsh shells of exponent 0: every s function is 1 everywhere, every Cartesian p shell x, y, z."""
+    mol = ca.Molecule([1], [[0.0, 0.0, 0.0]])
+    for _ in range(nsh):
+        mol.add_shell(0, type_, [0.0], [1.0])
+    return mol
+
+
+@pytest.mark.parametrize("shape", [0, 1])
+def test_products_of_a_run_are_added_in_fp64(shape):
+    """Phi_I^T B_J and B_I^T Phi_J of one run, each a sum of integers below 2^24 and so exact in FP32, add up exactly
+    (in one FP32 accumulator they would pass 2^24 and lose their odd part)."""
+    mol = _constants(200)  # 7 tiles: two groups
+    g = _grid(mol, 0, ca.CHX_PREC_MIXED, run=7)
+    g.setVxcShape(shape)
+    w = g.points()[:, 3]
+    a = np.random.default_rng(8).integers(0, 30000, len(w)) * 2 + 1  # 16 bits: hi + lo holds them
+    assert 7 * 64 * 60000 * 1.05 > 2 ** 24 > 7 * 64 * 30000 * 1.05
+    g.setVrho(2 * a / w)  # the integrand's factor is w v_rho / 2
+    V = g.getFock(1)[0]
+    assert np.array_equal(V, np.full(V.shape, 2.0 * a.sum()))
