@@ -554,16 +554,17 @@ __device__ __forceinline__ void walk_tile_f32(const BasisView& bv, int t, double
 // Density epilogue on one tile at this lane's point, as sums per shell of X Q
 // and X grad Q times R and grad R: with X = Phi D, o[0] = sum_nu X_nu phi_nu and
 // o[1..3] = sum_nu X_nu grad phi_nu; TAU: with X_r = (d_r Phi) D also
-// o[4] = sum_r sum_nu X_r,nu d_r phi_nu, from the same walk over the shells (the
-// walk, not the MFMAs, is most of a GGA density on lists of a few hundred AOs).
+// o[4 + r] = sum_nu X_r,nu d_r phi_nu, from the same walk over the shells (the
+// walk, not the MFMAs, is most of a GGA density on lists of a few hundred AOs). The
+// three directions stay apart: they are added in FP64, where the functional sums tau.
 // X is held in registers (uniform column index: no memory access).
 typedef float f32x32 __attribute__((ext_vector_type(32)));
 constexpr int kXPitch = kBatch + 4;  // of X^T in LDS: 16-byte rows that 16 lanes write without bank conflicts
 template <bool TAU>
 struct DensEpi {
   f32x32 xv[TAU ? 4 : 1];
-  float o[TAU ? 5 : 4] = {};
-  float R, Rx, Ry, Rz, S0, Sx, Sy, Sz, T0, Tx, Ty, Tz;
+  float o[TAU ? 7 : 4] = {};
+  float R, Rx, Ry, Rz, S0, Sx, Sy, Sz, Tx, Ty, Tz, Ux, Uy, Uz;
   // xq: X^T of this tile at this lane's point, xq[col * kXPitch]
   __device__ void load(int d, const float* xq) {
 #pragma unroll
@@ -572,7 +573,7 @@ struct DensEpi {
   __device__ void begin(float a, float ax, float ay, float az) {
     R = a; Rx = ax; Ry = ay; Rz = az;
     S0 = Sx = Sy = Sz = 0.f;
-    if (TAU) T0 = Tx = Ty = Tz = 0.f;
+    if (TAU) Tx = Ty = Tz = Ux = Uy = Uz = 0.f;
   }
   __device__ void comp(int col, float q, float qx, float qy, float qz) {
     const float v = xv[0][col];
@@ -582,10 +583,12 @@ struct DensEpi {
     Sz += v * qz;
     if (TAU) {
       const float vx = xv[TAU ? 1 : 0][col], vy = xv[TAU ? 2 : 0][col], vz = xv[TAU ? 3 : 0][col];
-      T0 += vx * qx + vy * qy + vz * qz;
       Tx += vx * q;
       Ty += vy * q;
       Tz += vz * q;
+      Ux += vx * qx;
+      Uy += vy * qy;
+      Uz += vz * qz;
     }
   }
   __device__ void end() {
@@ -593,7 +596,11 @@ struct DensEpi {
     o[1] += Rx * S0 + R * Sx;
     o[2] += Ry * S0 + R * Sy;
     o[3] += Rz * S0 + R * Sz;
-    if (TAU) o[TAU ? 4 : 0] += R * T0 + Rx * Tx + Ry * Ty + Rz * Tz;
+    if (TAU) {
+      o[TAU ? 4 : 0] += R * Ux + Rx * Tx;
+      o[TAU ? 5 : 0] += R * Uy + Ry * Ty;
+      o[TAU ? 6 : 0] += R * Uz + Rz * Tz;
+    }
   }
 };
 
@@ -788,7 +795,7 @@ struct DensMxMggaSmem {
     u32x4 F[(4 * kDxA + kDxB) * kDxFrag];  // one K step's fragments: A_0..A_3, D
     float X[kGroup * kTile][kXPitch];
   };
-  float red[kGroup][5][kBatch];
+  float red[kGroup][7][kBatch];
   double px[kBatch], py[kBatch], pz[kBatch];
 };
 
@@ -907,15 +914,15 @@ __global__ __launch_bounds__(256, 2) void k_density_mx_mgga(MolDev m) {
   }
   if (wave < nt) walk_tile_f32<true>(bv, j0 + wave, sm.px[lane], sm.py[lane], sm.pz[lane], epi);
 #pragma unroll
-  for (int c = 0; c < 5; ++c) sm.red[wave][c][lane] = epi.o[c];
+  for (int c = 0; c < 7; ++c) sm.red[wave][c][lane] = epi.o[c];
   __syncthreads();
   for (int e = tid; e < 7 * kBatch; e += 256) {
     const int c = e / kBatch, g = e % kBatch;
     double v = 0.0;
-    for (int q = 0; q < nt; ++q) v += c < 5 ? (double)sm.red[q][c][g] : 0.0;
+    for (int q = 0; q < nt; ++q) v += (double)sm.red[q][c][g];
     if (c < 4)
       m.part[(size_t)grp * 4 * kBatch + c * kBatch + g] = v;
-    else  // part_tau: [group][3][64], summed over the directions in the first
+    else  // part_tau: [group][3][64]
       m.part_tau[(size_t)grp * 3 * kBatch + (c - 4) * kBatch + g] = v;
   }
 }

@@ -143,3 +143,15 @@ def test_products_of_a_run_are_added_in_fp64(shape):
     g.setVrho(2 * a / w)  # the integrand's factor is w v_rho / 2
     V = g.getFock(1)[0]
     assert np.array_equal(V, np.full(V.shape, 2.0 * a.sum()))
+
+
+@pytest.mark.parametrize("form", [ca.CHX_PREC_FP64, ca.CHX_PREC_MIXED])
+def test_directions_of_tau_are_added_in_fp64(form):
+    """Of the functions x, y, z each has one constant derivative: tau is half the trace of D, and an entry of 2^26 next to
+    ones of 1 (each exact in FP32) shows a sum over the directions in FP32."""
+    mol = _constants(1, 1)
+    g = _grid(mol, 2, form)
+    a = 65535.0 * 2 ** 10
+    g.getDensity([np.diag([a, 1.0, 1.0])])
+    _, _, tau, w = g.pointDensity()
+    assert np.array_equal(tau[w != 0], np.full((w != 0).sum(), 0.5 * (a + 2.0)))
