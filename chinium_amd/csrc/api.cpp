@@ -184,6 +184,27 @@ int matrices_at_once(size_t per, int nmats) {
 // Stage ids of chx_grid_kernel_times.
 enum { kStPermute = 0, kStDensity = 1, kStFunctional = 2, kStVxc = 3, kStFinalize = 4, kStMakeB = 5, kStCore = 6 };
 
+// FP64 form without AO tables: rho, grad rho and (part_tau not null) tau of a device
+// matrix, D's blocks gathered for a segment of the chunks at a time.
+void density_recomputed(chx_grid* g, const double* dD, double* part, double* part_tau) {
+  hipEvent_t e = nullptr;
+  for (size_t s = 0; s + 1 < g->seg_chunk.size(); ++s) {
+    if (g->seg_chunk[s] == g->seg_chunk[s + 1]) continue;
+    const ChunkDev &c0 = g->chunks[g->seg_chunk[s]], &c1 = g->chunks[g->seg_chunk[s + 1] - 1];
+    const int g0 = g->grp_off[c0.b0], ng = g->grp_off[c1.b0 + c1.nb] - g0;
+    g->mark_begin(kStPermute, &e);
+    launch_gather_d(g->stream, c1.tile0 + c1.ntl - c0.tile0, g->nbasis, dD, g->d_tile_chunk.p, g->d_chunks.p,
+                    g->d_ao_of.p, g->d_Dt.p, nullptr, 0, 1, 0, c0.tile0, c0.doff);
+    g->mark_end(kStPermute, e);
+    g->mark_begin(kStDensity, &e);
+    for (int mode = 0; mode <= (part_tau ? 3 : 0); ++mode)
+      launch_density_f64(g->stream, mode, ng, g->d_grp_batch.p + g0, g->d_grp_tile.p + g0, g->d_grp_ntiles.p + g0,
+                         g->d_b_chunk.p, g->d_chunks.p, g->d_x.p, g->d_y.p, g->d_z.p, g->view(), g->d_Dt.p, c0.doff,
+                         mode ? part_tau + ((size_t)g0 * 3 + mode - 1) * kBatch : part + (size_t)g0 * 4 * kBatch);
+    g->mark_end(kStDensity, e);
+  }
+}
+
 // spin: which of the (up to two) split remainders of D this density's is
 void density_from_device(chx_grid* g, const double* dD, int spin = 0) {
   hipEvent_t e = nullptr;
@@ -214,24 +235,19 @@ void density_from_device(chx_grid* g, const double* dD, int spin = 0) {
     g->have_v = false;
     return;
   }
-  g->mark_begin(kStPermute, &e);
-  ++g->d_gen;
-  gather_d(g, dD, g->d_Dt, g->type >= 2);
-  g->mark_end(kStPermute, e);
-  g->mark_begin(kStDensity, &e);
   if (g->cached) {
+    g->mark_begin(kStPermute, &e);
+    ++g->d_gen;
+    gather_d(g, dD, g->d_Dt, g->type >= 2);
+    g->mark_end(kStPermute, e);
+    g->mark_begin(kStDensity, &e);
     launch_density_c64(g->stream, ng, g->d_grp_batch.p, g->d_grp_tile.p, g->d_grp_ntiles.p, g->d_bt_off.p,
                        g->d_b_chunk.p, g->d_chunks.p, g->d_cache.p, g->d_Dt.p, g->d_asym.p, g->d_gen, g->d_part.p,
                        g->type >= 2 ? g->d_part_tau.p : nullptr);
-  } else {  // AO values recomputed in the kernels
-    launch_density_f64(g->stream, 0, ng, g->d_grp_batch.p, g->d_grp_tile.p, g->d_grp_ntiles.p, g->d_b_chunk.p,
-                         g->d_chunks.p, g->d_x.p, g->d_y.p, g->d_z.p, g->view(), g->d_Dt.p, g->d_part.p);
-    if (g->type >= 2)
-      for (int r = 1; r <= 3; ++r)
-        launch_density_f64(g->stream, r, ng, g->d_grp_batch.p, g->d_grp_tile.p, g->d_grp_ntiles.p, g->d_b_chunk.p,
-                         g->d_chunks.p, g->d_x.p, g->d_y.p, g->d_z.p, g->view(), g->d_Dt.p, g->d_part_tau.p + (size_t)(r - 1) * kBatch);
+    g->mark_end(kStDensity, e);
+  } else {
+    density_recomputed(g, dD, g->d_part.p, g->type >= 2 ? g->d_part_tau.p : nullptr);
   }
-  g->mark_end(kStDensity, e);
   g->have_density = true;
   g->have_eval = false;
   g->have_v = false;
@@ -604,19 +620,18 @@ int chx_grid_get_density_u(chx_grid* g, const double* D, int nmats, int nspin, i
     const size_t rP = Workspace::round(sP), rD = Workspace::round(sD), rI = Workspace::round(nb2);
     const int mb = g->cached ? matrices_at_once(rP + rD + rI, ntot) : 1;
     Workspace ws(g, rI * mb + rP * mb + (mb > 1 ? rD * mb : 0));
-    double *Din = ws.take(rI * mb), *part = ws.take(rP * mb);
-    double* Dt = mb > 1 ? ws.take(rD * mb) : g->d_Dt.alloc_get(std::max<size_t>(1, sD));
+    double *Din = ws.take(rI * mb), *part = ws.take(rP * mb), *Dt = mb > 1 ? ws.take(rD * mb) : g->d_Dt.p;
     for (int m = 0; m < ntot; m += mb) {
       const int k = std::min(mb, ntot - m);
       CHX_HIP(hipMemcpyAsync(Din, D + m * nb2, sizeof(double) * nb2 * k, hipMemcpyHostToDevice, g->stream));
-      launch_gather_d(g->stream, (int)g->tile_chunk.size(), nbasis, Din, g->d_tile_chunk.p, g->d_chunks.p,
-                      g->d_ao_of.p, Dt, nullptr, 0, k, sD);
-      if (g->cached)
+      if (g->cached) {
+        launch_gather_d(g->stream, (int)g->tile_chunk.size(), nbasis, Din, g->d_tile_chunk.p, g->d_chunks.p,
+                        g->d_ao_of.p, Dt, nullptr, 0, k, sD);
         launch_density_c64(g->stream, ng, g->d_grp_batch.p, g->d_grp_tile.p, g->d_grp_ntiles.p, g->d_bt_off.p,
                            g->d_b_chunk.p, g->d_chunks.p, g->d_cache.p, Dt, nullptr, 0, part, nullptr, k, sD, sP);
-      else
-        launch_density_f64(g->stream, 0, ng, g->d_grp_batch.p, g->d_grp_tile.p, g->d_grp_ntiles.p, g->d_b_chunk.p,
-                           g->d_chunks.p, g->d_x.p, g->d_y.p, g->d_z.p, g->view(), Dt, part);
+      } else {
+        density_recomputed(g, Din, part, nullptr);
+      }
       launch_point_rho(g->stream, g->nbatches, g->d_grp_off.p, part, rhou + (size_t)m * 4 * nslots, k, sP);
     }
     CHX_HIP(hipStreamSynchronize(g->stream));

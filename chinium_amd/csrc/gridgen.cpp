@@ -415,8 +415,8 @@ static double shell_reach(int type, int np, const double* e, const double* c, do
 // the list's length in whole tiles, the second term the gather and the scatter
 // in units of one point's contraction. Over (H2O)1 .. (H2O)128, C18 and
 // alkanes, kChunkCost = 256 gives 7 to 23 batches per chunk at 1.2 to 1.7 times
-// the work of single batches' lists.
-static void build_chunks(chx_grid* g, int nwords, const std::vector<unsigned long long>& alive) {
+// the work of single batches' lists. At most `longest` batches make a chunk.
+static void build_chunks(chx_grid* g, int nwords, const std::vector<unsigned long long>& alive, int longest) {
   constexpr double kChunkCost = 256.0;
   const int nb = g->nbatches, nsh = (int)g->sh_type.size();
   std::vector<int> sizes;  // shell sizes present, with the mask of the shells of that size
@@ -446,7 +446,7 @@ static void build_chunks(chx_grid* g, int nwords, const std::vector<unsigned lon
     std::copy_n(&alive[(size_t)b0 * nwords], nwords, cur.begin());
     int b1 = b0 + 1;
     double c = cost(cur.data(), nullptr, 1);
-    while (b1 < nb && b1 - b0 < kChunkMax) {
+    while (b1 < nb && b1 - b0 < longest) {
       const unsigned long long* v = &alive[(size_t)b1 * nwords];
       const double cm = cost(cur.data(), v, b1 - b0 + 1);
       if (cm > c + cost(v, nullptr, 1)) break;
@@ -482,6 +482,25 @@ static void build_chunks(chx_grid* g, int nwords, const std::vector<unsigned lon
   }
   g->chunk_b0.push_back(nb);
   g->tile_seg_off.push_back((int)g->seg.size());
+}
+
+// The form that recomputes AO values: segments of chunks whose blocks of D are gathered
+// together, into at most an eighth of the room (or one chunk's, the matrix at most).
+static void build_segments(chx_grid* g, double room) {
+  const size_t cap = (size_t)(room / 8 / sizeof(double));
+  g->seg_chunk.assign(1, 0);
+  g->seg_elems = 0;
+  size_t cur = 0;
+  for (size_t c = 0; c < g->chunks.size(); ++c) {
+    const size_t n = (size_t)g->chunks[c].ntl * kTile * g->chunks[c].ntl * kTile;
+    if (cur > 0 && cur + n > cap) {
+      g->seg_chunk.push_back((int)c);
+      cur = 0;
+    }
+    cur += n;
+    g->seg_elems = std::max(g->seg_elems, cur);
+  }
+  g->seg_chunk.push_back((int)g->chunks.size());
 }
 
 // Vxc work items: per chunk every block (I, J) of super-tiles of `sup` tiles
@@ -570,16 +589,63 @@ static void build_mwork(chx_grid* g, int sup, int len, std::vector<RowRef>& rows
   }
 }
 
+// u_elems of build_mwork for these groups and runs.
+static size_t run_elems(const chx_grid* g, int sup, int len) {
+  size_t n = 0;
+  for (const ChunkDev& ch : g->chunks) {
+    if (ch.ntl == 0) continue;
+    const int ng = (ch.ntl + sup - 1) / sup;
+    size_t run = 0;
+    for (int I = 0; I < ng; ++I) {
+      const int I0 = ch.ntl * I / ng, I1 = ch.ntl * (I + 1) / ng;
+      run += (size_t)(I1 - I0) * kTile * (ch.ntl - I0) * kTile;
+    }
+    n += run * ((ch.nb + len - 1) / len);
+  }
+  return n;
+}
+
+// Tiles per Vxc group of the cached tables.
+static int group_tiles(const chx_grid* g) {
+  return g->precision == CHX_PREC_MIXED && g->mx_wide ? kMxWideTiles : kMxTiles;
+}
+
+// Run length of the cached tables' Vxc work items: the caller's, or the rule's and not below
+// what the plan found room for.
+static int run_length(const chx_grid* g, int sup) {
+  return g->vxc_chunk > 0 ? g->vxc_chunk : std::max(default_len(g, sup, true), g->min_run);
+}
+
+static double slot_bytes(const chx_grid* g, int nT) {
+  double slots = 0;
+  for (const ChunkDev& ch : g->chunks) slots += (double)ch.nb * ch.ntl;
+  return slots * (g->precision == CHX_PREC_MIXED ? 3.0 * nT * kMxComp * sizeof(unsigned short)
+                                                 : 5.0 * kBatch * kTile * sizeof(double));
+}
+
+// What the tables of the cached forms take (bytes) at a run length. FP64: phi, grad phi
+// and B per slot, the chunks' blocks of D, the runs' blocks of V. Mixed: the split operand
+// cache (nT components in two layouts, 2 bytes an element) and B^T per slot, the core
+// slots' third terms, D's blocks in two terms, either product of the runs.
+static double table_bytes(const chx_grid* g, int nT, const std::vector<char>& core, int len) {
+  const double runs = (double)run_elems(g, group_tiles(g), len);
+  if (g->precision != CHX_PREC_MIXED) return slot_bytes(g, nT) + (g->dt_elems + runs) * sizeof(double);
+  double core_slots = 0;
+  for (size_t b = 0; b < core.size(); ++b) core_slots += core[b] * g->chunks[g->b_chunk[b]].ntl;
+  return slot_bytes(g, nT) + (core_slots * nT * kBatch * kTile + 2.0 * g->dt_elems) * sizeof(unsigned short) +
+         2 * runs * sizeof(float);
+}
+
 // Vxc work items of the cached tables over groups of up to kMxTiles tiles or
 // (mixed form, wide) kMxWideTiles; FP64 form: also every pair of groups for the
 // plain products. Uploads them; the host vectors outlive the copies (synchronises).
 void build_cwork(chx_grid* g) {
   hipStream_t st = g->stream;
   const bool mixed = g->precision == CHX_PREC_MIXED;
-  const int sup = mixed && g->mx_wide ? kMxWideTiles : kMxTiles;
+  const int sup = group_tiles(g);
   std::vector<RowRef> rows;
   std::vector<int> rowptr;
-  build_mwork(g, sup, g->vxc_chunk > 0 ? g->vxc_chunk : default_len(g, sup, true), rows, rowptr);
+  build_mwork(g, sup, run_length(g, sup), rows, rowptr);
   if (mixed) {
     g->d_U64.release();
     g->d_U.alloc(std::max<size_t>(1, 2 * g->u_elems));
@@ -696,7 +762,56 @@ static void make_plan(chx_grid* g) {
       CHX_HIP(hipMemcpyAsync(alive.data(), d_alive.p, sizeof(alive[0]) * alive.size(), hipMemcpyDeviceToHost, st));
     CHX_HIP(hipStreamSynchronize(st));
   }
-  build_chunks(g, nwords, alive);
+  const bool mixed = g->precision == CHX_PREC_MIXED;
+  const int nT = g->type >= 2 ? 4 : 1;
+  if (mixed && g->ntiles > kMxMaxTiles)
+    throw Error(CHX_ERR_UNSUPPORTED, "the mixed-precision form takes at most " + std::to_string(kMxMaxTiles * kTile) +
+                                         " basis functions");
+  if (mixed && g->max_nprim > kSegPrim)
+    throw Error(CHX_ERR_UNSUPPORTED, "the mixed-precision form takes at most " + std::to_string(kSegPrim) +
+                                         " primitives per shell");
+  if (mixed) {  // a previous FP64 plan's tables are not needed any more
+    g->d_cache.release();
+    g->d_bmat.release();
+  }
+  // core batches of the mixed form: any real point within core_radius of a nucleus with Z > 2
+  std::vector<char> core;
+  if (mixed && g->core_radius > 0) {
+    core.assign(nb, 0);
+    const double r2c = g->core_radius * g->core_radius;  // <= 1 bohr: the cells' reach
+    const HeavyCells hc(g->mol);
+    for (int b = 0; b < nb; ++b)
+      for (int q = 0; q < g->batch_n[b] && !core[b]; ++q) {
+        const size_t p = (size_t)b * kBatch + q;
+        core[b] = hc.near(g->hx[p], g->hy[p], g->hz[p], r2c) >= 0;
+      }
+  }
+  // The chunks, and whether their tables have room. D's and V's blocks grow with a list's
+  // square once per chunk and run, the tables only with its length per batch: where the
+  // whole does not fit, runs are made longer (up to the chunk), then chunks (up to
+  // kChunkLong batches, which costs nothing where the lists are alike; where they differ
+  // the chunks stay short and the blocks small).
+  size_t free_b = 0, total_b = 0;
+  CHX_HIP(hipMemGetInfo(&free_b, &total_b));
+  const double room = (mixed ? 0.9 : 0.8) * (double)free_b;
+  g->mx_wide = wide_groups(g);
+  bool fits = false;
+  for (int longest = kChunkMax; !fits; longest *= 2) {
+    build_chunks(g, nwords, alive, longest);
+    g->min_run = 1;
+    fits = table_bytes(g, nT, core, run_length(g, group_tiles(g))) <= room;
+    while (!fits && g->vxc_chunk == 0 && g->min_run < longest) {
+      g->min_run *= 2;
+      fits = table_bytes(g, nT, core, run_length(g, group_tiles(g))) <= room;
+    }
+    if (longest >= kChunkLong || (!mixed && g->cache_mode == 0) || slot_bytes(g, nT) > room) break;
+  }
+  if (mixed && !fits)
+    throw Error(CHX_ERR_DEVICE, "the mixed-precision form needs " +
+                                    std::to_string(table_bytes(g, nT, core, run_length(g, group_tiles(g))) / 1e9) +
+                                    " GB of device memory for its AO cache");
+  g->cached = mixed || g->cache_mode == 1 || (g->cache_mode == -1 && fits);
+  if (!g->cached) build_segments(g, room);
   g->bt_off.assign(nb + 1, 0);
   g->batch_work.assign(nb, 0.0);
   g->slot_batch.clear(); g->slot_tile.clear();
@@ -753,31 +868,6 @@ static void make_plan(chx_grid* g) {
   g->d_chunks.upload(g->chunks, st); g->d_b_chunk.upload(g->b_chunk, st);
   g->d_tile_chunk.upload(g->tile_chunk, st); g->d_ao_of.upload(g->ao_of, st);
   g->d_slot_batch.upload(g->slot_batch, st); g->d_slot_tile.upload(g->slot_tile, st);
-  // The mixed form always runs from the split operand cache (nT components
-  // in two layouts per slot, 2 bytes per element) plus B^T of nT components.
-  const bool mixed = g->precision == CHX_PREC_MIXED;
-  const int nT = g->type >= 2 ? 4 : 1;
-  const double cache_bytes =
-      mixed ? (double)nslot * 3.0 * nT * kMxComp * sizeof(unsigned short)
-            : (double)nslot * (4.0 + 1.0) * kBatch * kTile * sizeof(double);  // phi, grad phi and B
-  if (mixed && g->ntiles > kMxMaxTiles)
-    throw Error(CHX_ERR_UNSUPPORTED, "the mixed-precision form takes at most " + std::to_string(kMxMaxTiles * kTile) +
-                                         " basis functions");
-  if (mixed && g->max_nprim > kSegPrim)
-    throw Error(CHX_ERR_UNSUPPORTED, "the mixed-precision form takes at most " + std::to_string(kSegPrim) +
-                                         " primitives per shell");
-  if (mixed) {  // a previous FP64 plan's tables are not needed any more
-    g->d_cache.release();
-    g->d_bmat.release();
-  }
-  size_t free_b = 0, total_b = 0;
-  CHX_HIP(hipMemGetInfo(&free_b, &total_b));
-  if (mixed && cache_bytes > 0.9 * (double)free_b)
-    throw Error(CHX_ERR_DEVICE, "the mixed-precision form needs " + std::to_string(cache_bytes / 1e9) +
-                                    " GB of device memory for its AO cache");
-  g->cached = mixed || g->cache_mode == 1 || (g->cache_mode == -1 && cache_bytes < 0.8 * (double)free_b);
-  // large bases: Vxc items over groups of up to 5 tiles
-  g->mx_wide = wide_groups(g);
   g->vwork.clear();
   g->mwork.clear();
   if (g->cached) g->d_Mint.release();
@@ -792,23 +882,15 @@ static void make_plan(chx_grid* g) {
       g->bmx_comps = nT;
       g->d_bmx.alloc(std::max<size_t>(1, nslot * (size_t)nT * kMxComp));
       g->d_Dsplit.alloc(std::max<size_t>(1, 2 * g->dt_elems));
-      // core batches: any real point within core_radius of a nucleus with Z > 2
       std::vector<int> core_off(nb, -1), slot_core(std::max<size_t>(1, nslot), -1);
       g->core_grps.clear();
       g->main_grps.clear();
       g->ncore_batches = 0;
       g->core_flops = 0.0;
       int ncore_slots = 0;
-      if (g->core_radius > 0) {
-        const double r2c = g->core_radius * g->core_radius;  // <= 1 bohr: the cells' reach
-        const HeavyCells hc(g->mol);
+      if (!core.empty()) {
         for (int b = 0; b < nb; ++b) {
-          bool core = false;
-          for (int q = 0; q < g->batch_n[b] && !core; ++q) {
-            const size_t p = (size_t)b * kBatch + q;
-            core = hc.near(g->hx[p], g->hy[p], g->hz[p], r2c) >= 0;
-          }
-          if (!core) {
+          if (!core[b]) {
             for (int k = g->grp_off[b]; k < g->grp_off[b + 1]; ++k) g->main_grps.push_back(k);
             continue;
           }
@@ -859,7 +941,7 @@ static void make_plan(chx_grid* g) {
   // per-iteration buffers
   const size_t nslots = (size_t)nb * kBatch;
   if (mixed) g->d_Dt.release();
-  else g->d_Dt.alloc(std::max<size_t>(1, g->dt_elems));
+  else g->d_Dt.alloc(std::max<size_t>(1, g->cached ? g->dt_elems : g->seg_elems));
   g->d_Din.alloc((size_t)g->nbasis * g->nbasis);
   g->d_Vout.alloc((size_t)g->nbasis * g->nbasis);
   g->d_part.alloc(std::max<size_t>(1, g->grp_batch.size() * 4 * kBatch));

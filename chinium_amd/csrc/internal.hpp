@@ -20,6 +20,7 @@ constexpr int kPadAO = 128;    // nbasis is padded to a multiple of this (4 tile
 constexpr int kMxTiles = 4;    // tiles per Vxc group of the cached tables (128 AOs)
 constexpr int kMxWideTiles = 5;  // ... of the mixed form's wide shape (160 AOs)
 constexpr int kChunkMax = 32;  // most consecutive batches that share one AO list
+constexpr int kChunkLong = 512;  // ... where memory is short
 constexpr int kCoef = 5;       // Vxc integrand coefficients per point: a, c_x, c_y, c_z, t
 constexpr double kCoreRadius = 0.3;  // bohr: points this close to a nucleus with Z > 2 are batched apart
 
@@ -121,7 +122,7 @@ struct BasisView {
   const int* sh_atom;       // atom of each shell (XC gradient)
 };
 
-// A chunk: up to kChunkMax consecutive batches (the batch order is spatial) and
+// A chunk: up to kChunkMax (short of memory: kChunkLong) consecutive batches (the batch order is spatial) and
 // the list of the AOs above the screening threshold in any of them, packed in
 // ntl tiles of 32 AOs (tiles tile0 .. tile0 + ntl - 1 of the grid's list). Every
 // batch of the chunk carries all ntl tiles, so slot (batch, tile q) is
@@ -172,14 +173,16 @@ void launch_screen(hipStream_t s, int nbatches, int nshells, int nwords, const d
 // The chunks' dense blocks of D (FP64): block r of the launch gathers the 32
 // rows of tile r from D (reference order, column-major n x n), zero for padding.
 // asym (may be null): *asym = gen when D is not symmetric to within rounding.
+// tile0, d0: first tile, and place in the whole list of blocks of Dt's first element.
 void launch_gather_d(hipStream_t s, int ntiles, int n, const double* D, const int* tile_chunk, const ChunkDev* chunks,
-                     const int* ao_of, double* Dt, int* asym, int gen, int nmat = 1, size_t sO = 0);
+                     const int* ao_of, double* Dt, int* asym, int gen, int nmat = 1, size_t sO = 0, int tile0 = 0,
+                     long d0 = 0);
 void launch_pad_d(hipStream_t s, int n, int npad, const double* D, double* Dpad);
 // mode 0: rho, grad rho / 2 into part ([group][4][64]); mode r = 1..3: the tau
-// partial of direction r (part = component r - 1 of [group][3][64]).
+// partial of direction r (part = component r - 1 of [group][3][64]). d0 as above.
 void launch_density_f64(hipStream_t s, int mode, int ngroups, const int* grp_batch, const int* grp_tile,
                         const int* grp_ntiles, const int* b_chunk, const ChunkDev* chunks, const double* bx,
-                        const double* by, const double* bz, BasisView bv, const double* Dt, double* part);
+                        const double* by, const double* bz, BasisView bv, const double* Dt, long d0, double* part);
 // One molecule of a multi-molecule functional launch: byte offsets of its
 // buffers from the launch's base pointer, its slot count, its first block
 // (entry nmol is a sentinel whose blk0 is the total block count) and its E/N slot.
@@ -478,6 +481,8 @@ struct chx_grid {
   std::vector<int> chunk_b0;           // first batch of each chunk (and the end)
   std::vector<int> b_chunk, tile_chunk, ao_of;
   size_t dt_elems = 0;                 // elements of the chunks' dense blocks of D
+  std::vector<int> seg_chunk;          // AO values recomputed: first chunk of each segment (and the end)
+  size_t seg_elems = 0;                // ... elements of the largest segment's blocks of D
   std::vector<int> bt_off;             // first slot of each batch
   std::vector<int> grp_batch, grp_tile, grp_ntiles, grp_off;  // density work groups
   std::vector<chx::VxcItem> vwork;     // Vxc work items (64-AO super-tiles I <= J), AO values recomputed
@@ -486,6 +491,7 @@ struct chx_grid {
   int cache_mode = -1;               // -1 automatic, 0 never, 1 always
   std::vector<int> slot_batch, slot_tile;
   int vxc_chunk = 0;                 // batches per Vxc work item; 0 = by the item count
+  int min_run = 1;                   // ... and at least this many, where shorter runs' blocks have no room
   int vxc_shape = -1;                // mixed form's Vxc groups: -1 by basis size, 0 up to 4 tiles, 1 up to 5
   int mx_wide = 0;                   // mixed form: Vxc over groups of up to 5 tiles (large bases)
   std::vector<chx::MxItem> mwork;       // Vxc work items of the cached tables

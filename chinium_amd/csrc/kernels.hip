@@ -91,17 +91,17 @@ __global__ __launch_bounds__(256) void k_gather_d(int n, const double* __restric
                                                   const int* __restrict__ tile_chunk,
                                                   const ChunkDev* __restrict__ chunks, const int* __restrict__ ao_of,
                                                   double* __restrict__ Dt, int ntiles, int* __restrict__ asym,
-                                                  int gen, size_t sO) {
+                                                  int gen, size_t sO, int tile0, long d0) {
   D += (size_t)blockIdx.y * n * n;  // the matrix of the launch
   Dt += blockIdx.y * sO;
-  const int t = blockIdx.x;
-  if (t >= ntiles) {  // 1e-13: above the rounding of a product formed in FP64, below what tau shows
-    check_symmetry(t - ntiles, n, D, 1e-13, asym, gen);
+  if ((int)blockIdx.x >= ntiles) {  // 1e-13: above the rounding of a product formed in FP64, below what tau shows
+    check_symmetry(blockIdx.x - ntiles, n, D, 1e-13, asym, gen);
     return;
   }
+  const int t = tile0 + blockIdx.x;
   const ChunkDev c = chunks[tile_chunk[t]];
   const int ld = c.ntl * kTile;
-  double* __restrict__ out = Dt + c.doff + (size_t)(t - c.tile0) * kTile * ld;
+  double* __restrict__ out = Dt + (c.doff - d0) + (size_t)(t - c.tile0) * kTile * ld;
   const int* __restrict__ cols = ao_of + (size_t)c.tile0 * kTile;
   __shared__ int rows[kTile];
   if (threadIdx.x < kTile) rows[threadIdx.x] = ao_of[(size_t)t * kTile + threadIdx.x];
@@ -118,10 +118,10 @@ __global__ __launch_bounds__(256) void k_gather_d(int n, const double* __restric
 }
 
 void launch_gather_d(hipStream_t s, int ntiles, int n, const double* D, const int* tile_chunk, const ChunkDev* chunks,
-                     const int* ao_of, double* Dt, int* asym, int gen, int nmat, size_t sO) {
+                     const int* ao_of, double* Dt, int* asym, int gen, int nmat, size_t sO, int tile0, long d0) {
   if (ntiles == 0) return;
   hipLaunchKernelGGL(k_gather_d, dim3(ntiles + (asym ? symmetry_blocks(n) : 0), nmat), dim3(256), 0, s, n, D,
-                     tile_chunk, chunks, ao_of, Dt, ntiles, asym, gen, sO);
+                     tile_chunk, chunks, ao_of, Dt, ntiles, asym, gen, sO, tile0, d0);
   CHX_HIP(hipGetLastError());
 }
 
@@ -153,7 +153,8 @@ __global__ __launch_bounds__(256) void k_density_f64(const int* __restrict__ grp
                                                      const ChunkDev* __restrict__ chunks,
                                                      const double* __restrict__ bx, const double* __restrict__ by,
                                                      const double* __restrict__ bz, BasisView bv,
-                                                     const double* __restrict__ Dt, double* __restrict__ part) {
+                                                     const double* __restrict__ Dt, long d0,
+                                                     double* __restrict__ part) {
   __shared__ DensSmem sm;
   const int grp = blockIdx.x;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -175,7 +176,7 @@ __global__ __launch_bounds__(256) void k_density_f64(const int* __restrict__ grp
   const int lrow = lane & 15, lk = lane >> 4;
   for (int k = 0; k < ch.ntl; ++k) {
     const int ti = ch.tile0 + k;
-    const double* __restrict__ Drow = Dt + ch.doff + (size_t)k * kTile * ld + col0;
+    const double* __restrict__ Drow = Dt + (ch.doff - d0) + (size_t)k * kTile * ld + col0;
     // zero the Phi tile, then fill the AOs this tile holds
     for (int e = tid; e < kTile * kBatch; e += 256) (&sm.k.A[0][0])[e] = 0.0;
     __syncthreads();
@@ -280,11 +281,11 @@ __global__ __launch_bounds__(256) void k_density_f64(const int* __restrict__ grp
 
 void launch_density_f64(hipStream_t s, int mode, int ngroups, const int* grp_batch, const int* grp_tile,
                         const int* grp_ntiles, const int* b_chunk, const ChunkDev* chunks, const double* bx,
-                        const double* by, const double* bz, BasisView bv, const double* Dt, double* part) {
+                        const double* by, const double* bz, BasisView bv, const double* Dt, long d0, double* part) {
   if (ngroups == 0) return;
 #define CHX_DF64(M)                                                                                       \
   hipLaunchKernelGGL(k_density_f64<M>, dim3(ngroups), dim3(256), 0, s, grp_batch, grp_tile, grp_ntiles, \
-                     b_chunk, chunks, bx, by, bz, bv, Dt, part);
+                     b_chunk, chunks, bx, by, bz, bv, Dt, d0, part);
   switch (mode) {
     case 0: CHX_DF64(0); break;
     case 1: CHX_DF64(1); break;

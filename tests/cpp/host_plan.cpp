@@ -120,8 +120,38 @@ void launch_ao_cache(hipStream_t, int, const int*, const int*, const double*, co
                      double*) { launched(); }
 void launch_ao_cache_mx(hipStream_t, int, const int*, const int*, const double*, const double*, const double*,
                         BasisView, int, int, unsigned short*, const int*, unsigned short*) { launched(); }
-void launch_gather_d(hipStream_t, int, int, const double*, const int*, const ChunkDev*, const int*, double* Dt, int*,
-                     int, int, size_t) { CHECK(at(Dt)); launched(); }
+std::vector<char> gathered;  // chunks whose blocks of D are in place
+size_t density_groups = 0;   // density groups run since it was cleared
+void launch_gather_d(hipStream_t, int ntiles, int, const double*, const int* tile_chunk, const ChunkDev* chunks,
+                     const int*, double* Dt, int*, int, int nmat, size_t sO, int tile0, long d0) {
+  gathered.assign(1 << 16, 0);
+  for (int t = tile0; t < tile0 + ntiles; ++t) {
+    const ChunkDev& c = chunks[tile_chunk[t]];
+    CHECK(c.tile0 >= tile0 && c.tile0 + c.ntl <= tile0 + ntiles);  // whole chunks
+    CHECK(at(Dt + (c.doff - d0)) && at(Dt + (nmat - 1) * sO + (c.doff - d0), 8192 * (size_t)c.ntl * c.ntl));
+    gathered[tile_chunk[t]] = 1;
+  }
+  launched();
+}
+void launch_density_f64(hipStream_t, int mode, int ng, const int* batch, const int* tile, const int*,
+                        const int* b_chunk, const ChunkDev* chunks, const double*, const double*, const double*,
+                        BasisView, const double* Dt, long d0, double* part) {
+  for (int k = 0; k < ng; ++k) {
+    const ChunkDev& c = chunks[b_chunk[batch[k]]];
+    CHECK(gathered[b_chunk[batch[k]]] && tile[k] >= c.tile0 && tile[k] < c.tile0 + c.ntl);
+    CHECK(at(Dt + (c.doff - d0)) && at(Dt + (c.doff - d0), 8192 * (size_t)c.ntl * c.ntl));
+  }
+  CHECK(ng == 0 || at(part, ((size_t)(ng - 1) * (mode ? 3 : 4) + 1) * 512));
+  density_groups += ng;
+  launched();
+}
+void launch_point_rho(hipStream_t, int, const int*, const double* part, double* rhou, int, size_t) {
+  CHECK(at(part) && at(rhou));
+  launched();
+}
+void launch_vxc_f64(hipStream_t, int, int, const VxcItem*, const int*, const double*, const double*, const double*,
+                    const double*, BasisView, double* M, int npad) { CHECK(at(M, 8 * npad * npad)); launched(); }
+void launch_finalize_sym(hipStream_t, int, int, const double*, double* V) { CHECK(at(V)); launched(); }
 void launch_pad_d(hipStream_t, int, int npad, const double*, double* D) {
   CHECK(at(D, sizeof(double) * npad * npad));
   launched();
@@ -287,6 +317,61 @@ void failed_plans() {
   }
 }
 
+// Plans under a byte budget: longer runs, longer chunks, the form without tables and its segments, in
+// this order, and every build within the budget.
+void budgets() {
+  const size_t all = fake::budget;
+  for (int form : {CHX_PREC_FP64, CHX_PREC_MIXED}) {
+    chx_grid* g = grid(4, 160);  // 640 AOs, all alive in most batches
+    chx_xc* xc = functional(1);
+    const int n = g->nbasis;
+    std::vector<double> D((size_t)n * n, 0.1), F((size_t)n * n);
+    CHECK(chx_grid_set_precision(g, form) == CHX_OK && chx_grid_get_ao(g, 0, 0) == CHX_OK && g->cached);
+    size_t slots = 0;
+    for (const chx::ChunkDev& c : g->chunks) slots += (size_t)c.nb * c.ntl;
+    const double table = slots * (form == CHX_PREC_MIXED ? 3.0 * chx::kMxComp * 2 : 5.0 * 2048 * 8);
+    const double blocks = form == CHX_PREC_MIXED ? 4.0 * g->dt_elems + 8.0 * g->u_elems
+                                                 : 8.0 * g->dt_elems + 8.0 * g->u_elems;
+    const size_t u0 = g->u_elems, d0 = g->dt_elems, chunks0 = g->chunks.size();
+    chx_grid_destroy(g);
+    const double share = form == CHX_PREC_MIXED ? 0.9 : 0.8;
+    int longer_runs = 0, longer_chunks = 0, recomputed = 0, refused = 0;
+    for (double f = 1.2; f > 0.02; f *= 0.93) {  // room for the tables and f of their blocks, down to a part of the tables
+      g = grid(4, 160);
+      CHECK(chx_grid_set_precision(g, form) == CHX_OK);
+      const double room = f > 0.1 ? table + f * blocks : table * f / 0.1;
+      fake::budget = fake::used + (size_t)(room / share);
+      const int rc = chx_grid_get_ao(g, 0, 0);
+      if (rc != CHX_OK) {
+        CHECK(form == CHX_PREC_MIXED && room < table + blocks);
+        ++refused;
+      } else {
+        CHECK(g->cached || form == CHX_PREC_FP64);
+        chx::density_groups = 0;
+        CHECK(build(g, xc, D, F) == CHX_OK);
+        if (!g->cached) {
+          CHECK(chx::density_groups == g->grp_batch.size());
+          CHECK(chx_grid_get_density_u(g, D.data(), 1, 1, n) == CHX_OK);
+          CHECK(chx::density_groups == 2 * g->grp_batch.size());
+          ++recomputed;
+        } else if (g->dt_elems < d0) {
+          ++longer_chunks;
+        } else if (g->u_elems < u0) {
+          ++longer_runs;
+        }
+        for (const chx::ChunkDev& c : g->chunks) CHECK(c.nb <= chx::kChunkLong);
+      }
+      fake::budget = all;
+      chx_grid_destroy(g);
+    }
+    std::printf("form %d: %zu chunks; plans with longer runs %d, longer chunks %d, without tables %d, refused %d\n", form,
+                chunks0, longer_runs, longer_chunks, recomputed, refused);
+    CHECK(longer_runs > 0 && longer_chunks > 0);
+    CHECK(form == CHX_PREC_MIXED ? refused > 0 : recomputed > 0);
+    chx_xc_destroy(xc);
+  }
+}
+
 // A shell is in the list of every batch in which one of its components or their derivatives exceeds the
 // threshold: contractions of steep and diffuse primitives of either sign, coarse thresholds, exponents of 0.
 void reaches() {
@@ -349,7 +434,7 @@ void reaches() {
 
 int main(int argc, char** argv) {
   const std::map<std::string, void (*)()> checks = {
-      {"empty_lists", empty_lists}, {"failed_plans", failed_plans}, {"reaches", reaches}};
+      {"empty_lists", empty_lists}, {"failed_plans", failed_plans}, {"budgets", budgets}, {"reaches", reaches}};
   if (argc != 3 || !checks.count(argv[1])) return 2;
   root = argv[2];
   checks.at(argv[1])();
