@@ -349,20 +349,20 @@ class Grid:
         return G.reshape(-1, 3)
 
     def autotune(self, xc, D_ptr, V_ptr, reps=3):
-        """Times each Vxc work-item length, keeps the fastest; returns (chunk, {chunk: ms})."""
+        """Times each Vxc work-item length (0: the default rule's), keeps the fastest; returns (chunk, {chunk: ms})."""
         c = ctypes.c_int()
         ms = (ctypes.c_float * 4)()
         _check(lib().chx_grid_autotune(self.h, xc.h, D_ptr, V_ptr, int(reps), ctypes.byref(c), ms))
-        return c.value, dict(zip((8, 16, 32, 128), list(ms)))
+        return c.value, dict(zip((0, 4, 8, 16), list(ms)))
 
     def autotuneTiles(self, xc, D_ptr, V_ptr, reps=3):
-        """Mixed form: times both Vxc block shapes (0: groups of 4 tiles of 32 AOs, 1: of 5) at
-        each work-item length, keeps the fastest; returns (shape, chunk, {(shape, chunk): ms})."""
+        """Mixed form: times both Vxc block shapes (0: groups of 4 tiles of 32 AOs, 1: of 5) at each
+        work-item length (0: the default rule's), keeps the fastest; returns (shape, chunk, {(shape, chunk): ms})."""
         sh, c = ctypes.c_int(), ctypes.c_int()
         ms = (ctypes.c_float * 8)()
         _check(lib().chx_grid_autotune_tiles(self.h, xc.h, D_ptr, V_ptr, int(reps), ctypes.byref(sh),
                                              ctypes.byref(c), ms))
-        keys = [(a, b) for a in (0, 1) for b in (8, 16, 32, 128)]
+        keys = [(a, b) for a in (0, 1) for b in (0, 4, 8, 16)]
         return sh.value, c.value, dict(zip(keys, list(ms)))
 
     def setVxcChunk(self, chunk):
@@ -709,8 +709,9 @@ class Pack:
         return v.value
 
     def autotune(self, xc, D_ptrs, V_ptrs, reps=3):
-        """Times each Vxc work-item length, keeps the fastest, then picks the lane count;
-        returns (chunk, {chunk: ms})."""
+        """Times the Vxc work-item lengths (8, 16: at most that many batches where the default rule takes more; 32: the
+        rule; 128: whole chunks), keeps the fastest, then picks the block shapes, form and lane count; returns
+        (chunk, {chunk: ms})."""
         c = ctypes.c_int()
         ms = (ctypes.c_float * 4)()
         _check(lib().chx_pack_autotune(self.h, xc.h, self._ptrs(D_ptrs), self._ptrs(V_ptrs), int(reps),

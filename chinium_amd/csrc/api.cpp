@@ -867,7 +867,7 @@ int chx_grid_autotune(chx_grid* g, const chx_xc* xc, const double* D_dev, double
     require(g && xc && D_dev && V_dev && reps > 0, CHX_ERR_ARG, "bad arguments");
     require(g->ao_ready && g->cached, CHX_ERR_STATE, "Grid::getAO (with the AO tables in HBM) must precede tuning");
     require(g->type >= xc->family, CHX_ERR_STATE, "grid type is below the functional family (call setType)");
-    static const int cand[] = {8, 16, 32, 128};
+    static const int cand[] = {0, 4, 8, 16};  // 0: the rule's
     hipEvent_t a, b;
     CHX_HIP(hipEventCreate(&a));
     CHX_HIP(hipEventCreate(&b));
@@ -884,7 +884,13 @@ int chx_grid_autotune(chx_grid* g, const chx_xc* xc, const double* D_dev, double
     int best = -1;
     float best_ms = 0.f;
     for (int k = 0; k < 4; ++k) {
-      set_vxc_chunk(g, cand[k]);
+      try {
+        set_vxc_chunk(g, cand[k]);
+      } catch (const Error&) {  // its blocks do not fit: not a candidate, where the grid kept its plan
+        if (!g->ao_ready) throw;
+        if (ms_out) ms_out[k] = HUGE_VALF;
+        continue;
+      }
       build();  // warm-up
       CHX_HIP(hipEventRecord(a, g->stream));
       for (int r = 0; r < reps; ++r) build();
@@ -902,6 +908,7 @@ int chx_grid_autotune(chx_grid* g, const chx_xc* xc, const double* D_dev, double
     (void)hipEventDestroy(a);
     (void)hipEventDestroy(b);
     g->profile = prof;
+    require(best >= 0, CHX_ERR_DEVICE, "no Vxc work length has room");
     set_vxc_chunk(g, cand[best]);
     if (chunk_out) *chunk_out = cand[best];
   });

@@ -610,11 +610,10 @@ static int group_tiles(const chx_grid* g) {
   return g->precision == CHX_PREC_MIXED && g->mx_wide ? kMxWideTiles : kMxTiles;
 }
 
-// Run length of the cached tables' Vxc work items: the caller's, or the rule's and not below
-// what the plan found room for.
-static int run_length(const chx_grid* g, int sup) {
-  return g->vxc_chunk > 0 ? g->vxc_chunk : std::max(default_len(g, sup, true), g->min_run);
-}
+// Run length of the cached tables' Vxc work items by the rule, not below what the plan found
+// room for; the caller's where it set one.
+int auto_run(const chx_grid* g) { return std::max(default_len(g, group_tiles(g), true), g->min_run); }
+static int run_length(const chx_grid* g) { return g->vxc_chunk > 0 ? g->vxc_chunk : auto_run(g); }
 
 static double slot_bytes(const chx_grid* g, int nT) {
   double slots = 0;
@@ -645,7 +644,7 @@ void build_cwork(chx_grid* g) {
   const int sup = group_tiles(g);
   std::vector<RowRef> rows;
   std::vector<int> rowptr;
-  build_mwork(g, sup, run_length(g, sup), rows, rowptr);
+  build_mwork(g, sup, run_length(g), rows, rowptr);
   if (mixed) {
     g->d_U64.release();
     g->d_U.alloc(std::max<size_t>(1, 2 * g->u_elems));
@@ -799,16 +798,16 @@ static void make_plan(chx_grid* g) {
   for (int longest = kChunkMax; !fits; longest *= 2) {
     build_chunks(g, nwords, alive, longest);
     g->min_run = 1;
-    fits = table_bytes(g, nT, core, run_length(g, group_tiles(g))) <= room;
+    fits = table_bytes(g, nT, core, run_length(g)) <= room;
     while (!fits && g->vxc_chunk == 0 && g->min_run < longest) {
       g->min_run *= 2;
-      fits = table_bytes(g, nT, core, run_length(g, group_tiles(g))) <= room;
+      fits = table_bytes(g, nT, core, run_length(g)) <= room;
     }
     if (longest >= kChunkLong || (!mixed && g->cache_mode == 0) || slot_bytes(g, nT) > room) break;
   }
   if (mixed && !fits)
     throw Error(CHX_ERR_DEVICE, "the mixed-precision form needs " +
-                                    std::to_string(table_bytes(g, nT, core, run_length(g, group_tiles(g))) / 1e9) +
+                                    std::to_string(table_bytes(g, nT, core, run_length(g)) / 1e9) +
                                     " GB of device memory for its AO cache");
   g->cached = mixed || g->cache_mode == 1 || (g->cache_mode == -1 && fits);
   if (!g->cached) build_segments(g, room);

@@ -23,6 +23,7 @@
 #include <array>
 #include <algorithm>
 #include <chrono>
+#include <cmath>
 #include <cstdint>
 #include <cstring>
 #include <string>
@@ -32,6 +33,7 @@
 
 namespace chx {
 void set_vxc_chunk(chx_grid* g, int chunk);
+int auto_run(const chx_grid* g);
 void set_vxc_shape(chx_grid* g, int shape);
 std::string& last_error();
 }
@@ -520,14 +522,23 @@ int chx_pack_autotune(chx_pack* p, const chx_xc* xc, const double* const* D_dev,
                       int* chunk_out, float* ms_out) {
   return pguard([&] {
     prequire(p && xc && D_dev && V_dev && reps > 0, CHX_ERR_ARG, "bad arguments");
+    // 8, 16: at most that many batches where the rule takes more; 32: the rule; 128: whole chunks
     static const int cand[] = {8, 16, 32, 128};
+    auto length = [](const chx_grid* g, int c) { return c < 32 ? std::min(c, auto_run(g)) : c == 32 ? 0 : kMxMaxChunk; };
     hipEvent_t a, b;
     CHX_HIP(hipEventCreate(&a));
     CHX_HIP(hipEventCreate(&b));
     int best = -1;
     float best_ms = 0.f;
     for (int k = 0; k < 4; ++k) {
-      for (chx_grid* g : p->grids) set_vxc_chunk(g, cand[k]);
+      try {
+        for (chx_grid* g : p->grids) set_vxc_chunk(g, length(g, cand[k]));
+      } catch (const Error&) {  // no room for a member's blocks: not a candidate, where it kept its plan
+        for (const chx_grid* g : p->grids)
+          if (!g->ao_ready) throw;
+        if (ms_out) ms_out[k] = HUGE_VALF;
+        continue;
+      }
       build_lanes(p);
       run(p, xc, D_dev, V_dev, nullptr, nullptr);  // capture and warm up
       CHX_HIP(hipEventRecord(a, p->stream));
@@ -543,7 +554,8 @@ int chx_pack_autotune(chx_pack* p, const chx_xc* xc, const double* const* D_dev,
         best_ms = ms;
       }
     }
-    for (chx_grid* g : p->grids) set_vxc_chunk(g, cand[best]);
+    prequire(best >= 0, CHX_ERR_DEVICE, "no Vxc work length has room");
+    for (chx_grid* g : p->grids) set_vxc_chunk(g, length(g, cand[best]));
     // then the Vxc tile shape per molecule, by a basis-size threshold: groups of 5 tiles for
     // npad >= T, of 4 below (T = 0: 5 for all; -1: none)
     static const int thr[] = {-1, 1024, 512, 0};

@@ -217,8 +217,9 @@ int chx_grid_core_flops(const chx_grid* g, double* flops);
 int chx_grid_set_screening(chx_grid* g, double threshold);
 /* Autotuner (no reference counterpart): times `reps` XC builds (D_dev ->
  * V_dev, device pointers, column-major nbasis^2) for each Vxc work-item
- * length (8, 16, 32, 128 batches), keeps the fastest; chunk_out gets it,
- * ms_out[4] the times. Needs the AO tables in HBM (cached or mixed form). */
+ * length (0: the default rule's; 4, 8, 16 batches), keeps the fastest;
+ * chunk_out gets it, ms_out[4] the times (infinite where a length's blocks
+ * do not fit). Needs the AO tables in HBM (cached or mixed form). */
 int chx_grid_autotune(chx_grid* g, const chx_xc* xc, const double* D_dev, double* V_dev, int reps, int* chunk_out,
                       float* ms_out);
 /* Mixed form's Vxc block shape (no reference counterpart): groups of up to 4
@@ -226,8 +227,9 @@ int chx_grid_autotune(chx_grid* g, const chx_xc* xc, const double* D_dev, double
  * from npad 1024 on, else 0. chx_grid_vxc_shape reports the shape in use. */
 int chx_grid_set_vxc_shape(chx_grid* g, int shape);
 /* Vxc work-item length in batches (0: by the number of items, at most 128; an
- * item ends with its chunk of at most 32 batches); the autotuners set it from
- * their timings. */
+ * item ends with its chunk of batches, at most 32 unless memory is short); the
+ * autotuners set it from their timings. A length whose blocks do not fit is
+ * refused and the grid keeps the former one. */
 int chx_grid_set_vxc_chunk(chx_grid* g, int chunk);
 int chx_grid_vxc_shape(const chx_grid* g, int* shape);
 /* chx_grid_autotune over both shapes (mixed form): times the four work
@@ -350,8 +352,10 @@ int chx_pack_xc(chx_pack* p, const chx_xc* xc, const double* const* D_dev, doubl
                 double* N);
 /* 1 (default) replays a captured hipGraph, 0 launches eagerly. */
 int chx_pack_set_graph(chx_pack* p, int enable);
-/* Autotuner: times `reps` builds for each Vxc work-item length (8, 16, 32,
- * 128 batches), keeps the fastest (chunk_out gets it, ms_out[4] the times);
+/* Autotuner: times `reps` builds for each Vxc work-item length (8, 16: at most
+ * that many batches in the molecules where the default rule takes more; 32: the
+ * rule's; 128: whole chunks), keeps the fastest (chunk_out gets it, ms_out[4]
+ * the times, infinite where a length's blocks do not fit);
  * then the Vxc tile shape per molecule (chx_grid_set_vxc_shape) by a
  * basis-size threshold T (groups of 5 tiles for npad >= T: none, 1024, 512,
  * all), keeps the fastest; then the form and lanes (per-molecule kernels or

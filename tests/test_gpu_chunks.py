@@ -155,3 +155,22 @@ def test_directions_of_tau_are_added_in_fp64(form):
     g.getDensity([np.diag([a, 1.0, 1.0])])
     _, _, tau, w = g.pointDensity()
     assert np.array_equal(tau[w != 0], np.full((w != 0).sum(), 0.5 * (a + 2.0)))
+
+
+@pytest.mark.parametrize("form", [ca.CHX_PREC_FP64, ca.CHX_PREC_MIXED])
+def test_autotuner_has_the_default_among_its_lengths(form):
+    """The default rule's run length (1 to 4 batches in FP64 and in small systems) is one of those timed."""
+    from chinium_amd import hip
+    mol, _, D = _system("water sto-3g")
+    xc = ca.ExchangeCorrelation()
+    xc.Read("PBE")
+    g = _grid(mol, 1, form)
+    E, V = ca.xc_build(g, xc, D)
+    n = len(D)
+    dD, dV = hip.DeviceArray(n * n), hip.DeviceArray(n * n)
+    dD.upload(np.asfortranarray(D).ravel(order="F"))
+    chunk, ms = g.autotune(xc, dD.ptr, dV.ptr, reps=1)
+    assert 0 in ms and ms[chunk] == min(ms.values())
+    g.setVxcChunk(0)
+    E0, V0 = ca.xc_build(g, xc, D)
+    assert np.array_equal(V, V0)
