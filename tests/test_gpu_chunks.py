@@ -88,7 +88,7 @@ def test_coarse_threshold_moves_little():
 def test_tau_of_a_nonsymmetric_matrix(name, form):
     """rho and tau are quadratic forms: an antisymmetric part of D adds nothing. A symmetric D takes half of
     tau's products, one with an antisymmetric part all of them; one with rounding-level asymmetry (products
-    like C C^T formed elsewhere) still counts as symmetric. Bounds: the forms' own rounding, 2^-16 of
+    like C C^T formed elsewhere) gives the same by either. Bounds: the forms' own rounding, 2^-16 of
     sum |D| |d phi| |d phi| (mixed), of which tau is about 1/10 at these densities."""
     mol, _, D = _system(name)
     n = len(D)
@@ -174,3 +174,26 @@ def test_autotuner_has_the_default_among_its_lengths(form):
     g.setVxcChunk(0)
     E0, V0 = ca.xc_build(g, xc, D)
     assert np.array_equal(V, V0)
+
+
+@pytest.mark.parametrize("n", [505, 512, 513, 8200])
+def test_assembly_by_basis_size(n):
+    """V's assembly from the runs' blocks: a copy of the sums per wave up to 512 AOs (64 KB of LDS there, and no more
+    than that left over), one for all above, two column ranges from 8193 on; against the form that adds to M. All
+    terms of a density of positive orbitals have one sign: 16 bits per operand give 3 x 2^-17 of V's largest."""
+    print("assembly: %d AOs" % n, flush=True)
+    rng = np.random.default_rng(n)
+    mol = ca.Molecule([1], [[0.0, 0.0, 0.0]])
+    for e in rng.uniform(0.1, 20.0, n):
+        mol.add_shell(0, 0, [e], [(2 * e / np.pi) ** 0.75])
+    C = rng.uniform(0.1, 1.0, (n, 2)) / n
+    D = C @ C.T
+    xc = ca.ExchangeCorrelation()
+    xc.Read("PBE")
+    E0, V0 = ca.xc_build(_grid(mol, 1, ca.CHX_PREC_FP64, 0), xc, D)
+    E, V = ca.xc_build(_grid(mol, 1, ca.CHX_PREC_FP64, 1), xc, D)
+    scale = np.abs(V0).max()
+    assert abs(E - E0) <= 1e-12 * abs(E0) and np.abs(V - V0).max() <= 1e-12 * scale
+    assert np.array_equal(V, V.T)
+    Em, Vm = ca.xc_build(_grid(mol, 1, ca.CHX_PREC_MIXED), xc, D)
+    assert abs(Em - E0) <= 5e-5 * abs(E0) and np.abs(Vm - V0).max() <= 5e-5 * scale

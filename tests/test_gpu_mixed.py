@@ -164,8 +164,8 @@ def test_mixed_meta_grid_after_gga_potentials():
 
 @pytest.mark.parametrize("name", ["h2o16_def2svp_sg2_b3lyp", "c18_def2tzvp_sg3_r2scan"])
 def test_vxc_block_shapes_agree(name):
-    """Both Vxc block shapes of the mixed form (128-AO super-tile pairs; 256-AO groups of each batch
-    chunk's alive-tile union) on bases below the default switch (npad 384 and 640): the same E_xc (the
+    """Both Vxc block shapes of the mixed form (groups of up to 4, or 5, tiles of 32 AOs of each batch
+    chunk's list) on bases below the default switch (npad 384 and 640): the same E_xc (the
     shape only changes Vxc and, through it, E's first-order correction for the split of D,
     sum V . (D - hi - lo), whose size is about 2^-17 |V . D|: the shapes' V differ by their rounding,
     which moves E by far less than 1e-9 Eh), V within the mixed form's rounding of each other and of

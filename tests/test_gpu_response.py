@@ -105,8 +105,8 @@ def test_water_cluster_response():
 
 @pytest.mark.parametrize("nmats", [2, 300])
 def test_perturbations_together_and_alone(nmats):
-    """Several matrices go through one launch (300: more than one set of launches, the last one short): each
-    is what it is by itself, to the bit (the same kernels, sums in a fixed order)."""
+    """Several matrices go through one launch (300: in getFockU more than one set of launches, the last one short):
+    each is what it is by itself, to the bit (the same kernels, sums in a fixed order)."""
     w, mol, D = _h2o()
     rng = np.random.default_rng(12)
     Dxs = []
@@ -115,6 +115,19 @@ def test_perturbations_together_and_alone(nmats):
         Dxs.append(0.1 * (A + A.T))
     grid, xc, Fs = _response(mol, "SG-1", "PBE", D, Dxs, 1)
     for m in sorted({0, 1, nmats // 2, nmats - 2, nmats - 1}):
+        grid.getDensityU([[Dxs[m]]])
+        (F,), = grid.getFockU()
+        assert np.array_equal(F, Fs[m]), m
+
+
+def test_more_perturbations_than_a_launch_takes():
+    """At most 1024 matrices share a launch: 1101 of a small molecule, the last set odd."""
+    mol = ca.Molecule([1, 1], [[0.0, 0.0, 0.0], [0.0, 0.0, 1.4]], "sto-3g")
+    D = wl.density_matrix(mol.overlap(), 1, 2)
+    rng = np.random.default_rng(4)
+    Dxs = [A + A.T for A in rng.standard_normal((1101, 2, 2))]
+    grid, xc, Fs = _response(mol, "SG-1", "PBE", D, Dxs, 1)
+    for m in (0, 1023, 1024, 1100):
         grid.getDensityU([[Dxs[m]]])
         (F,), = grid.getFockU()
         assert np.array_equal(F, Fs[m]), m

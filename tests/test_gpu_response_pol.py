@@ -121,16 +121,16 @@ def test_polarised_response_closed_shell_limit():
 
 
 def test_polarised_perturbations_together_and_alone():
-    """2 x 90 outputs, more than one set of launches: each is what it is by itself, to the bit."""
+    """2 x 150 outputs, more than one set of launches in getFockU: each is what it is by itself, to the bit."""
     Z, xyz, mol, Da, Db = _oh()
     rng = np.random.default_rng(7)
     Xas, Xbs = [], []
-    for _ in range(90):
+    for _ in range(150):
         A, B = rng.standard_normal(Da.shape), rng.standard_normal(Db.shape)
         Xas.append(0.05 * (A + A.T))
         Xbs.append(0.05 * (B + B.T))
     grid, (Fa, Fb) = _gpu_response(mol, "SG-1", "PBE", Da, Db, Xas, Xbs)
-    for m in (0, 44, 89):
+    for m in (0, 44, 89, 149):
         grid.getDensityU([[Xas[m]], [Xbs[m]]])
         (A,), (B,) = grid.getFockU(2)
         assert np.array_equal(A, Fa[m]) and np.array_equal(B, Fb[m]), m

@@ -128,3 +128,36 @@ def test_spin_protocol_errors():
     with pytest.raises(ca.ChxError) as e:  # three spin matrices
         g.getDensity([Da, Db, Da])
     assert e.value.code == -1
+
+
+@pytest.mark.parametrize("n", [4, 24])
+def test_both_spins_together_and_one_after_the_other(n):
+    """FP64, GGA: both spins share their launches while their tables are small (4 waters); the tables of 24 waters are
+    above that line and the spins follow each other. Either way: swapped spins give swapped potentials, equal ones
+    the closed-shell result."""
+    Z, X = wl.water_cluster_angstrom(n, 6.0 if n == 4 else 11.0, 5)
+    mol = ca.Molecule(Z, X * ca.ANGSTROM_TO_BOHR, "def2-svp")
+    Da, Db = _spin_dms(mol, 5 * n, 5 * n - 1, 3)
+    xc, rks = _xc("PBE"), ca.ExchangeCorrelation()
+    rks.Read("PBE")
+    grid = ca.Grid(mol, "SG-2", 1, 0)
+    grid.setAOCache(1)
+    grid.setType(1)
+    grid.getAO(0, 0)
+    grid.profile(True)
+
+    def build(Ds, f):
+        grid.getDensity(Ds)
+        f.Evaluate("ev", grid)
+        return grid.getEnergy(), grid.getFock()
+
+    grid.kernel_times()
+    E, (Va, Vb) = build([Da, Db], xc)
+    assert grid.kernel_times()["density"][1] == (1 if n == 4 else 2)
+    E2, (Vb2, Va2) = build([Db, Da], xc)
+    scale = max(np.abs(Va).max(), np.abs(Vb).max())
+    assert abs(E - E2) <= 1e-12 * abs(E)
+    assert max(np.abs(Va - Va2).max(), np.abs(Vb - Vb2).max()) <= 1e-11 * scale
+    Ec, (Vc,) = build([2 * Da], rks)
+    Ee, Ve = build([Da, Da], xc)
+    assert abs(Ec - Ee) <= 1e-11 * abs(Ec) and max(np.abs(V - Vc).max() for V in Ve) <= 1e-10 * scale
