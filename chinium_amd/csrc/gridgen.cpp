@@ -409,13 +409,18 @@ static double shell_reach(int type, int np, const double* e, const double* c, do
 
 // Cuts the batches into chunks with one AO list each. A batch's own list is
 // short (a few hundred of a large molecule's thousands of AOs), which is what
-// makes the contractions cheap, but a chunk's list is gathered from D and
-// scattered to M once per chunk, so neighbours are merged while the merged
-// list's cost stays below that of the two: cost = n^2 (points + kChunkCost), n
-// the list's length in whole tiles, the second term the gather and the scatter
-// in units of one point's contraction. Over (H2O)1 .. (H2O)128, C18 and
-// alkanes, kChunkCost = 256 gives 7 to 23 batches per chunk at 1.2 to 1.7 times
-// the work of single batches' lists. At most `longest` batches make a chunk.
+// makes the contractions cheap, but a chunk's block of D is gathered once per
+// chunk and its blocks of V are stored and read back once per run, so neighbours
+// are merged while the merged list's cost stays below that of the two: cost =
+// n^2 (points + kChunkCost), n the list's length in whole tiles, the second term
+// those blocks in units of one point's contraction. kChunkCost = 256 gives 7 to
+// 23 batches per chunk at 1.2 to 1.7 times the work of single batches' lists over
+// (H2O)1 .. (H2O)128, C18 and alkanes. Builds in us at 64 / 128 / 256 / 512 /
+// 1024: mixed (H2O)16 730 / 721 / 705 / 726 / 757, (H2O)48 r2SCAN 7940 / 7990 /
+// 8010 / 8410 / 8790, (H2O)128 13650 / 12390 / 11900 / 12300 / 12770, alkane C24
+// 618 / 594 / 582 / 588 / 633; FP64, whose contractions cost more beside the same
+// blocks, (H2O)16 2090 / 2150 / 2220 / 2290 / 2430, C18 8810 / 9390 / 9670 / 9860 /
+// 10010 (one value for both forms is kept here). At most `longest` batches make a chunk.
 static void build_chunks(chx_grid* g, int nwords, const std::vector<unsigned long long>& alive, int longest) {
   constexpr double kChunkCost = 256.0;
   const int nb = g->nbatches, nsh = (int)g->sh_type.size();
@@ -548,7 +553,7 @@ static int default_len(const chx_grid* g, int sup, bool upper) {
   return 1;
 }
 
-// Mixed form: runs of at most len batches of a chunk; per run the groups of its
+// Cached tables: runs of at most len batches of a chunk; per run the groups of its
 // tiles (at most sup, equal to within one) and an item per pair I <= J. U holds
 // per run and group I the row panel of I's rows, columns from I0 to the list's
 // end; rows/rowptr list for every AO its row in every run that holds it, from

@@ -331,8 +331,8 @@ struct MolDev {
   const int* asym;  // == gen: this build's D is not symmetric (meta-GGA)
   int gen, pad2_;
 };
-constexpr int kMxMaxTiles = 512;  // basis size the mixed form takes (npad <= 16384)
-constexpr int kMxMaxChunk = 128;  // batches per Vxc work item in the mixed form
+constexpr int kMxMaxTiles = 512;  // basis size the mixed form takes (npad <= 16384): no kernel's limit, nothing larger was run
+constexpr int kMxMaxChunk = 128;  // longest run a caller may ask for, batches per Vxc work item
 
 // XC nuclear gradient (kernels_grad.hip), FP64 cached form. gpart: kGradCopies
 // partial gradients of 3 natoms.

@@ -93,7 +93,7 @@ void launch_ao_cache(hipStream_t s, int nslots, const int* slot_batch, const int
 // C18 / def2-TZVP / SG-3: 4.6 ms (7.6 in four launches with LDS stages).
 // NM = 2: two matrices (spins, perturbations) against the same phi, which is then
 // read once for both, the epilogue's grad phi too. Radical C7 / UKS, def2-SVP /
-// SG-2: 0.26 ms for both spins, 0.29 in two launches.
+// SG-1: 0.25 ms for both spins, 0.28 in two launches.
 template <bool TAU, int NM>
 __global__ __launch_bounds__(TAU ? 512 : 256, 2) void k_density_c64(
     const int* __restrict__ grp_batch, const int* __restrict__ grp_tile, const int* __restrict__ grp_ntiles,

@@ -33,11 +33,6 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kMxRow = 2 * kTile;             // one AOg row: 32 hi then 32 lo
 constexpr int kMxT = 2 * kTile * kBatch;      // elements per component of AOg, AOt and Bt
-// LDS operand tiles: rows of 4 16-byte chunks (32 bf16), chunk c of row r
-// stored at position c ^ ((r >> 2) & 3). A wave's 16-byte accesses then hit
-// distinct banks both when 16 lanes read one chunk of 16 consecutive rows
-// (MFMA operands) and when they write all 4 chunks of 4 rows (staging).
-__device__ __forceinline__ int swz(int r, int c) { return c ^ ((r >> 2) & 3); }
 
 // float -> bf16, round to nearest even: the hardware conversion
 // (v_cvt_pk_bf16_f32). k_bf16_check compares it with the bit-level rule
@@ -88,8 +83,6 @@ __device__ __forceinline__ f32x4 mfma3(u32x4 ah, u32x4 al, u32x4 bh, u32x4 bl, f
   c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf(ah), as_bf(bl), c, 0, 0, 0);
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf(ah), as_bf(bh), c, 0, 0, 0);
 }
-// value of the pair stored at p (hi) and p + off (lo)
-__device__ __forceinline__ float pair_at(const u16* p, int off) { return bf2f(p[0]) + bf2f(p[off]); }
 
 // ---------------------------------------------------------------------------
 // AO cache in split form: one block per slot. Values are evaluated in FP64,
@@ -259,7 +252,7 @@ __device__ __forceinline__ double block_sum_d(double v) {
 // against 86 shared; (H2O)48 250 us shared against 363 with 4 waves; (H2O)128 700 us
 // against 1430 with 2. With both products of a run, added here in FP64 (def2-SVP /
 // SG-2): (H2O)16 57 us (48 with one FP32 sum), (H2O)48 157 to 201 (157 to 163),
-// (H2O)128 0.79 ms (0.62).
+// (H2O)128 0.78 ms (0.62).
 // The FP64 atomics to HBM that all this replaces, one per element of M and run
 // at about 40 G/s, took most of the Vxc launch. kAsmLds sums per block: larger
 // bases take several column ranges (grid y).
@@ -615,8 +608,9 @@ struct DensEpi {
 // swizzled order from which the MFMA lanes read without bank conflicts.
 // Per step: wait for the step's fragments, read the wave's 12 into registers,
 // barrier, start the DMA of the next step into the same buffer, run the
-// wave's 24 MFMAs while it lands (one 24 KB buffer, so three blocks share a
-// CU and cover each other's barriers). Epilogue: X goes to LDS, wave q loads
+// wave's 24 MFMAs while it lands (one buffer of 24 KB, 28 with the third terms,
+// under X^T's 34: 39.5 KB in all, so four blocks share a CU and cover each
+// other's barriers). Epilogue: X goes to LDS, wave q loads
 // tile q's columns at its lane's point into registers and contracts them with
 // phi / grad phi recomputed in FP32.
 constexpr int kDxFrag = 64;  // u32x4 per fragment
@@ -1046,11 +1040,12 @@ void launch_make_b_mx(hipStream_t s, int ncomp, const MolDev& one) {
 // MT x MT fragments of 16 x 16; MT = 5 is the largest whose two buffers leave
 // room for two blocks per CU).
 // Either product is stored once per run, row-major, the row panel of group I from
-// column I0 on, the second one uplane elements after the first. One accumulator for
-// both and one store, which adds them in FP32, took (H2O)16 / def2-SVP / SG-2 from
-// 190 to 175 us and (H2O)128 from 3.6 to 3.5 ms: their bytes. A second set of
-// accumulators, their FP64 sum stored at the end, is as slow (188 us; with MT = 5 it
-// does not fit the registers).
+// column I0 on, the second one uplane elements after the first; of a block on the
+// diagonal the upper half. (H2O)16 / def2-SVP / SG-2 186 us, (H2O)128 3.55 ms; one
+// accumulator for both and one store, which adds them in FP32, took 175 us and 3.51
+// ms: fewer bytes. A second set of accumulators, their FP64 sum stored at the end, is
+// no faster than two stores (188 us with whole diagonal blocks, 190 so stored; with
+// MT = 5 it does not fit the registers).
 template <int MT>
 struct VxcMxSmem {
   u32x4 F[2][8 * MT * kDxFrag];  // step k in buffer k & 1: row group's fragments, then the column group's
@@ -1148,7 +1143,7 @@ __device__ __forceinline__ void vxc_mx_body(const MolDev& m, int item) {
       if (r < nI) {
 #pragma unroll
         for (int c = 0; c < MT; ++c)
-          if (c < nc) {
+          if (c < nc && (!diag || c0 + c >= r0 + r)) {  // (below the diagonal nothing is read)
 #pragma unroll
             for (int i = 0; i < 4; ++i) out[(size_t)(16 * r + i) * ld + 16 * c] = acc[r][c][i];
           }
@@ -1174,7 +1169,8 @@ __device__ __forceinline__ void vxc_mx_body(const MolDev& m, int item) {
     const int rows = min(64, n - 16 * s);
     for (int e = tid; e < rows * (n / 4); e += 256) {
       const int row = e / (n / 4), col = e % (n / 4) * 4;
-      *reinterpret_cast<f32x4*>(out + (size_t)row * ld + col) = *reinterpret_cast<const f32x4*>(T + row * PT + col);
+      if (col + 3 >= 16 * s + row)
+        *reinterpret_cast<f32x4*>(out + (size_t)row * ld + col) = *reinterpret_cast<const f32x4*>(T + row * PT + col);
     }
   }
 }
