@@ -731,6 +731,18 @@ void set_vxc_shape(chx_grid* g, int shape) {
   else rebuild_runs(g, g->vxc_chunk, shape);
 }
 
+// Bytes of the tables that the grid's former plan holds; with release, they are freed.
+static size_t former_tables(chx_grid* g, bool release) {
+  size_t n = 0;
+  auto add = [&](auto& b) {
+    n += b.n * sizeof(*b.p);
+    if (release) b.release();
+  };
+  add(g->d_cache); add(g->d_bmat); add(g->d_U64); add(g->d_Dt);
+  add(g->d_cmx); add(g->d_bmx); add(g->d_U); add(g->d_Dsplit); add(g->d_cmx3);
+  return n;
+}
+
 // Screening and work plans (Grid::getAO counterpart).
 static void make_plan(chx_grid* g) {
   hipStream_t st = g->stream;
@@ -774,10 +786,6 @@ static void make_plan(chx_grid* g) {
   if (mixed && g->max_nprim > kSegPrim)
     throw Error(CHX_ERR_UNSUPPORTED, "the mixed-precision form takes at most " + std::to_string(kSegPrim) +
                                          " primitives per shell");
-  if (mixed) {  // a previous FP64 plan's tables are not needed any more
-    g->d_cache.release();
-    g->d_bmat.release();
-  }
   // core batches of the mixed form: any real point within core_radius of a nucleus with Z > 2
   std::vector<char> core;
   if (mixed && g->core_radius > 0) {
@@ -797,7 +805,7 @@ static void make_plan(chx_grid* g) {
   // the chunks stay short and the blocks small).
   size_t free_b = 0, total_b = 0;
   CHX_HIP(hipMemGetInfo(&free_b, &total_b));
-  const double room = (mixed ? 0.9 : 0.8) * (double)free_b;
+  const double share = mixed ? 0.9 : 0.8, room = share * (double)(free_b + former_tables(g, false));
   g->mx_wide = wide_groups(g);
   bool fits = false;
   for (int longest = kChunkMax; !fits; longest *= 2) {
@@ -815,6 +823,7 @@ static void make_plan(chx_grid* g) {
                                     std::to_string(table_bytes(g, nT, core, run_length(g)) / 1e9) +
                                     " GB of device memory for its AO cache");
   g->cached = mixed || g->cache_mode == 1 || (g->cache_mode == -1 && fits);
+  if (!g->cached || table_bytes(g, nT, core, run_length(g)) > share * (double)free_b) former_tables(g, true);
   if (!g->cached) build_segments(g, room);
   g->bt_off.assign(nb + 1, 0);
   g->batch_work.assign(nb, 0.0);

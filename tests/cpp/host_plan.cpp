@@ -372,6 +372,34 @@ void budgets() {
   }
 }
 
+// A grid planned again has the room of its former plan: the same tables, also where both would not fit,
+// and the other form's tables in the place of its own.
+void planned_again() {
+  const size_t all = fake::budget;
+  for (int form : {CHX_PREC_FP64, CHX_PREC_MIXED}) {
+    chx_grid* g = grid(2, 160);
+    chx_xc* xc = functional(1);
+    const int n = g->nbasis;
+    std::vector<double> D((size_t)n * n, 0.1), F((size_t)n * n);
+    const size_t before = fake::used;
+    CHECK(chx_grid_set_precision(g, form) == CHX_OK && chx_grid_get_ao(g, 0, 0) == CHX_OK && g->cached);
+    const size_t u = g->u_elems, d = g->dt_elems;
+    fake::budget = before + (fake::used - before) * 3 / 2;
+    for (double thr : {1e-13, 1e-14}) {
+      CHECK(chx_grid_set_screening(g, thr) == CHX_OK && chx_grid_get_ao(g, 0, 0) == CHX_OK && g->cached);
+      CHECK(build(g, xc, D, F) == CHX_OK);
+    }
+    CHECK(g->u_elems == u && g->dt_elems == d && g->min_run == 1);
+    CHECK(chx_grid_set_precision(g, form == CHX_PREC_FP64 ? CHX_PREC_MIXED : CHX_PREC_FP64) == CHX_OK);
+    CHECK(chx_grid_get_ao(g, 0, 0) == CHX_OK && build(g, xc, D, F) == CHX_OK);
+    CHECK(chx_grid_set_precision(g, form) == CHX_OK && chx_grid_get_ao(g, 0, 0) == CHX_OK && g->cached);
+    CHECK(build(g, xc, D, F) == CHX_OK && g->u_elems == u);
+    fake::budget = all;
+    chx_xc_destroy(xc);
+    chx_grid_destroy(g);
+  }
+}
+
 // A shell is in the list of every batch in which one of its components or their derivatives exceeds the
 // threshold: contractions of steep and diffuse primitives of either sign, coarse thresholds, exponents of 0.
 void reaches() {
@@ -434,7 +462,7 @@ void reaches() {
 
 int main(int argc, char** argv) {
   const std::map<std::string, void (*)()> checks = {
-      {"empty_lists", empty_lists}, {"failed_plans", failed_plans}, {"budgets", budgets}, {"reaches", reaches}};
+      {"empty_lists", empty_lists}, {"failed_plans", failed_plans}, {"budgets", budgets}, {"planned_again", planned_again}, {"reaches", reaches}};
   if (argc != 3 || !checks.count(argv[1])) return 2;
   root = argv[2];
   checks.at(argv[1])();

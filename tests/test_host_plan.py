@@ -17,7 +17,7 @@ def host_plan():
     return os.path.join(CPP, "host_plan")
 
 
-@pytest.mark.parametrize("check", ["empty_lists", "failed_plans", "budgets", "reaches"])
+@pytest.mark.parametrize("check", ["empty_lists", "failed_plans", "budgets", "planned_again", "reaches"])
 def test_host_plan(host_plan, check):
     r = subprocess.run([host_plan, check, ca.DATA_ROOT], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout + r.stderr
